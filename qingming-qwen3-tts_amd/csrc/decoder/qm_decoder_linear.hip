@@ -1,5 +1,5 @@
 // qm_decoder_linear.hip — linears of the decoder language models for few token rows (a decode step, a short portion of a
-// prompt) and for the 32-bit mode: weight-streaming dot products; many bf16 rows are handed to the matrix-core kernel.
+// prompt): weight-streaming dot products; many rows are handed to the matrix-core kernels (bf16, and the 32-bit mode's).
 //
 // Bound by HBM: every weight is read once per group of R rows.  A wave owns NR weight rows and streams them 16 bytes a
 // lane, `kDotAhead` pieces of each row requested before the first is used; the input rows live in LDS as T.  Sums are fp32
@@ -52,10 +52,14 @@ static int32_t launch_streaming(const DecLinearParams& prm, hipStream_t stream) 
 }
 
 template <class T>
-static int32_t streaming(const DecLinearParams& prm, hipStream_t stream) {
+static int64_t longest_row_bytes(const DecLinearParams& prm) {
     int k = 0;
     for (int g = 0; g < prm.groups; ++g) k = prm.group[g].k > k ? prm.group[g].k : k;
-    const int64_t row_bytes = static_cast<int64_t>(k) * sizeof(T);
+    return static_cast<int64_t>(k) * sizeof(T);
+}
+template <class T>
+static int32_t streaming(const DecLinearParams& prm, hipStream_t stream) {
+    const int64_t row_bytes = longest_row_bytes<T>(prm);
     if (row_bytes > kDotLds) return QM_ERR_GEOMETRY;
     if (prm.rows > 4 && 8 * row_bytes <= kDotLds) return launch_streaming<T, 8>(prm, stream);
     if (prm.rows > 2 && 4 * row_bytes <= kDotLds) return launch_streaming<T, 4>(prm, stream);
@@ -115,6 +119,17 @@ static int32_t launch_narrow(const DecLinearParams& prm, hipStream_t stream) {
 // Rows from which the matrix cores take over: below, one 64-row tile is mostly empty and the weights' bytes decide.
 constexpr int kDecMatrixRows = 16;
 
+// Whether fp32 rows go to the matrix cores: up to eight rows every weight is streamed once either way, and below about 2^26 products
+// the dot-product kernel's many short chains end first (us, dot products / matrix cores; products in millions: router 32 x 1024 of 1000
+// rows 33: 7.9 / 8.8; 320 x 1024 of 100 rows 33: 7.2 / 8.9; 1024 x 1024 of 64 rows 67: 7.9 / 9.0, of 100 rows 105: 13.4 / 9.2, of 300
+// rows 315: 28.7 / 9.6; 5120 + 2 x 3072 by 1024 of 8 rows 92: 12.3 / 11.5, of 300 rows 3460: 224 / 36).
+static bool split_pays(const DecLinearParams& prm) {
+    if (prm.rows <= 8 || longest_row_bytes<float>(prm) > kDotLds) return false;
+    int64_t products = 0;
+    for (int g = 0; g < prm.groups; ++g) products += static_cast<int64_t>(prm.group[g].n) * prm.group[g].k * (prm.group[g].w_up ? 2 : 1);
+    return products * prm.rows > (int64_t{1} << 26);
+}
+
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream) {
     if (prm.rows < 0 || prm.groups < 1 || prm.groups > kDecGroups) return QM_ERR_ARGUMENT;
     for (int g = 0; g < prm.groups; ++g) {
@@ -123,7 +138,7 @@ int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t 
         if (d.n <= 0 || d.k <= 0 || d.n % (d.w_up ? 128 : 16) || d.k % 128 || d.ldx < d.k || d.ldo < d.n || d.ldx % 8 || d.ldo % 4) return QM_ERR_GEOMETRY;
     }
     if (prm.rows == 0) return QM_OK;
-    if (f32) return streaming<float>(prm, stream);
+    if (f32) return split_pays(prm) ? launch_split_linears(prm, stream) : streaming<float>(prm, stream);
     bool matrix = prm.rows >= kDecMatrixRows;
     if (matrix && prm.groups == 1 && prm.group[0].n <= kNarrowColumns && !prm.group[0].w_up)
         return prm.group[0].n <= 32 ? launch_narrow<2>(prm, stream) : launch_narrow<4>(prm, stream);

@@ -53,6 +53,7 @@ int32_t launch_gated_norm(const GatedNormParams& prm, int rows, int f32, hipStre
 // Many rows of bf16 go to the matrix cores (linears of one launch in one grid, a gate/up pair in its own), few rows and
 // fp32 to the streaming kernel.
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream);
+int32_t launch_split_linears(const DecLinearParams& prm, hipStream_t stream);    // fp32 rows on the matrix cores
 // Rotation and cache write, then the attention.
 int32_t launch_chunk_attention(const ChunkAttentionParams& prm, int f32, hipStream_t stream);
 int32_t launch_chunk_attention_mfma(const ChunkAttentionParams& prm, hipStream_t stream);

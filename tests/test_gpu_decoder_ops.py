@@ -155,6 +155,42 @@ def test_linears(decoder, dev, f32, rows):
     close(get(outs[2]), plain.silu(gate) * (x[2].astype(np.float64) @ up.T), f32, tol32=3e-6, tol16=2e-2)
 
 
+@pytest.mark.parametrize("rows,n,k,pair", [
+    # every tile of the 32-bit mode's matrix-core linears: columns that end inside a tile, reductions of an odd number of steps per share
+    (16, 2128, 2048, False), (9, 3600, 2176, False), (33, 1040, 2048, False), (40, 1040, 1664, False), (129, 6640, 128, False),
+    (300, 6640, 128, False), (10, 1664, 2176, True), (33, 1024, 1152, True), (150, 4096, 128, True), (257, 4096, 128, True)])
+def test_linears_of_many_fp32_rows(decoder, dev, rows, n, k, pair):
+    """Against 64 bits, per output: a sum of k exact products through at most k / 64 + 80 roundings of partial sums that sum |x w| bounds.
+    Columns of x differ by up to 2^40; the last row holds an infinity."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    ldx, ldo = k + 8, n + 12
+    x = torch.randn(rows, ldx, device=dev, generator=gen) * torch.exp2(torch.randint(-20, 21, (ldx,), device=dev, generator=gen).float())
+    w, up = ((torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for _ in range(2))
+    if pair:
+        x /= x.abs().amax(1, keepdim=True)
+    else:
+        x[-1, 3] = float("inf")
+    out = torch.full((rows + 1, ldo), 7.0, device=dev)
+    linear = decoder.DecoderLinear(x=x.data_ptr(), w=w.data_ptr(), w_up=up.data_ptr() if pair else None, out32=None if pair else out.data_ptr(),
+                                   out=out.data_ptr() if pair else None, ldx=ldx, ldo=ldo, n=n, k=k)
+    assert decoder.lib().qm_decoder_linear_rows(C.byref(linear), 1, rows, 1, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert bool((out[rows:] == 7).all()) and bool((out[:, n:] == 7).all())
+    got, wide = out[:rows, :n].double().cpu(), x[:, :k].double().cpu()
+    unit = (k / 64 + 80) * 2.0 ** -24
+    gate, most = wide @ w.double().cpu().T, wide.abs() @ w.double().cpu().abs().T
+    if pair:
+        other, other_most = wide @ up.double().cpu().T, wide.abs() @ up.double().cpu().abs().T
+        want = torch.nn.functional.silu(gate) * other
+        # (silu's slope is at most 1.1; its exponential, reciprocal and product are good to a few units in the last place)
+        bound = unit * (1.1 * most * other.abs() + torch.nn.functional.silu(gate).abs() * other_most) + 8 * 2.0 ** -24 * want.abs() + 1e-12
+    else:
+        assert torch.equal(got[-1].isinf(), w[:, 3].cpu() != 0) and torch.equal(got[-1].sign(), w[:, 3].double().cpu().sign())
+        want, bound, got = gate[:-1], unit * most[:-1], got[:-1]
+    assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() / bound).max())
+
+
 ATTENTION = [
     # heads, kv_heads, dim, vdim, chunk, rot_dims
     (4, 2, 16, 16, 50, 8), (3, 3, 24, 40, 37, 24), (5, 1, 36, 20, 64, 10), (6, 2, 64, 64, 200, 16), (2, 1, 136, 144, 300, 64), (8, 2, 128, 128, 256, 128),
