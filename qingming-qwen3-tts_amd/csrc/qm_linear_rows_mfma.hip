@@ -431,7 +431,11 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
         asm volatile("s_barrier" ::: "memory");                   // everybody's have; and everybody has read this step's stage
         multiply(f1, f0, yes{}, next_at, 1, yes{}, next_at, req, integral_constant<int, 0>{}, integral_constant<int, 0>{});
     }
-    gm_wait_vm<0>();                                              // (the requests past the last step, before the block's LDS goes)
+    // The last step's reads for a step that does not come have to land before their registers, which the compiler takes as
+    // free from here on, hold anything else; and the requests past the last step before the block's LDS goes.
+    arrived(f0, integral_constant<int, 0>{});
+    arrived(f1, integral_constant<int, 0>{});
+    gm_wait_vm<0>();
 
     // ---- epilogue: accumulator register r of a lane is output column 8 (r / 4) + 4 (lane / 32) + r % 4 of the MFMA
     // tile's 32, token row lane % 32 ----
