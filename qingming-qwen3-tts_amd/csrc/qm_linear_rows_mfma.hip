@@ -6,8 +6,9 @@
 // instead of the reference's 32 lane-strided chains: bf16 inputs, fp32 accumulation, the same roundings after the sum,
 // results within the operators' tolerance of the exact-chain kernel (qm_linear_rows.hip), not bit-identical to it.
 //
-// A block of four waves owns a tile of BM token rows x BN output columns: 128 x 128 (waves 2 x 2, each 64 x 64 as 2 x 2
-// MFMA tiles); 64 x 128 for calls whose grid of 128-row tiles would leave CUs empty (waves 4 x 1, each 32 columns x 64
+// A block owns a tile of BM token rows x BN output columns: 128 x 128 (eight waves 2 x 4, each 64 rows x 32 columns, two to a
+// SIMD so that one multiplies while the other waits to issue: three linears of 2048, 2048 and 6144 inputs over 1024 rows 71.3 ->
+// 68.6 us against four waves of 64 x 64; the other tiles gain nothing from it and keep four); 64 x 128 for calls whose grid of 128-row tiles would leave CUs empty (waves 4 x 1, each 32 columns x 64
 // rows); 128 x 192 for a gate/up pair whose 128-column tiles come to between one and two rounds of the CUs and whose
 // 192-column tiles fit in one (1024 tokens x 6144 channels: 256 blocks).  Several linears of one input (q, k, v) share a
 // grid: a column tile's number says which of them it belongs to.  Both operands are K-contiguous rows (x [m][k],
@@ -36,7 +37,6 @@
 
 namespace qm {
 
-constexpr int kGmThreads = 256;
 constexpr int kGmTile = 128;                 // output columns per block (192 for a gate/up pair that it divides), token rows 128 or 64
 constexpr int kGmStep = 64;                  // k per step (32 with the 192-column tile)
 
@@ -87,6 +87,14 @@ struct GmShape {
     static_assert(kStageBytes * kStages <= 160 * 1024 - 1024, "the CU's LDS");
 };
 
+// How the waves share the tile: kAcross of them side by side along the output columns, each with kTn MFMA tiles of columns and
+// kTm of token rows.
+template <int BM, int BN, int WAVES>
+struct GmWaves {
+    static constexpr int kAcross = BM == 128 && (WAVES == 4 || BN == 192) ? 2 : 4;
+    static constexpr int kTn = BN / 32 / kAcross, kTm = BM / 32 / (WAVES / kAcross);
+};
+
 // Where the side operations of a k block stand among its MFMAs.  The MFMAs of a k block run over the wave's tiles (a, b),
 // a the weight tile and b the token tile, b fastest, and for a gate/up pair the gate MFMA before the up MFMA; MFMA number i
 // is followed by slot i.  A matrix-core instruction takes 32 cycles and the wave issues in order, so whatever else the wave
@@ -132,8 +140,8 @@ struct GmSchedule {
     }
 };
 
-template <bool DUAL, int BM, int BN, int KSTEP>
-__global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRowsParams prm) {
+template <bool DUAL, int BM, int BN, int KSTEP, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRowsParams prm) {
     request_arguments(prm);
     extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
     constexpr int kStages = GmShape<DUAL, BM, BN, KSTEP>::kStages;
@@ -143,22 +151,21 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
     constexpr int kWeights = DUAL ? 2 : 1;
     constexpr int kStageBytes = kXBytes + kWeights * kWBytes;
     static_assert(kStageBytes == GmShape<DUAL, BM, BN, KSTEP>::kStageBytes, "");
-    constexpr int kTn = BM == 128 ? BN / 64 : BN / 128;           // MFMA tiles of a wave along the output columns
-    constexpr int kTm = 2;                                        // and along the token rows
+    using Waves = GmWaves<BM, BN, WAVES>;
+    constexpr int kTn = Waves::kTn, kTm = Waves::kTm;
     constexpr int kFragTile = 32 * kRowBytes;                     // LDS bytes from an operand's MFMA tile to its next
     using Schedule = GmSchedule<DUAL, kTn, kTm>;
-    // pieces of 1 KiB (one instruction of a wave) per stage: x, w (, up); dealt to the four waves in turn
+    // pieces of 1 KiB (one instruction of a wave) per stage: x, w (, up); dealt to the waves in turn
     constexpr int kPiecesX = kXBytes / 1024, kPiecesW = kWBytes / 1024;
-    constexpr int kPerWave = (kPiecesX + kWeights * kPiecesW) / 4;
-    static_assert(kPiecesX % 4 == 0 && kPiecesW % 4 == 0, "a wave's piece i is of the same operand in every wave");
-    static_assert(kPerWave * (kStages - 2) <= 63 && kStages >= 2, "the waits count the later stages' pieces");
+    constexpr int kPerWave = (kPiecesX + kWeights * kPiecesW) / WAVES;
+    static_assert(kPiecesX % WAVES == 0 && kPiecesW % WAVES == 0, "a wave's piece i is of the same operand in every wave");
+    static_assert(kStages >= 2, "the waits count the later stages' pieces");
     static_assert(kKb == 4 || kKb == 8, "the step schedule lists the k blocks");
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wave_n = BM == 128 ? (wave & 1) : wave;
-    const int wave_m = BM == 128 ? (wave >> 1) : 0;
+    const int wave_n = wave % Waves::kAcross, wave_m = wave / Waves::kAcross;
     int K = prm.reduction;
     int m0 = static_cast<int>(blockIdx.y) * BM;
     // (several linears of one input in one grid: which of them this block's column tile belongs to)
@@ -200,10 +207,10 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
         matrix_at = static_cast<int64_t>(matrix) * columns * K;
     }
 
-    // ---- this wave's pieces of a stage: instruction q = wave + 4 i covers LDS bytes [1024 q, 1024 q + 1024) of the
+    // ---- this wave's pieces of a stage: instruction q = wave + WAVES i covers LDS bytes [1024 q, 1024 q + 1024) of the
     // stage (x tile, then w, then up); its lane l fills slot l % kSlots of tile row kRowsPerPiece (q within the tile) +
     // l / kSlots with global piece slot ^ slot_key(row).  The tiles are read through buffer descriptors that begin at the
-    // block's first row of each operand: a lane's offset is the same for every piece (4 kRowsPerPiece rows further on,
+    // block's first row of each operand: a lane's offset is the same for every piece (WAVES kRowsPerPiece rows further on,
     // the key of a row is the same), what changes from piece to piece and step to step is a scalar; token rows past the
     // last are out of the descriptor's range and read as zero without touching memory (their results are never stored).
     const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
@@ -217,20 +224,41 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
     const int lane_row = kRowsPerPiece * wave + lane / kSlots;
     const uint32_t lane_off = static_cast<uint32_t>(lane_row) * row_bytes
                             + 16u * static_cast<uint32_t>((lane % kSlots) ^ slot_key<kRowBytes>(lane_row));
-    static_assert((4 * kRowsPerPiece) % (256 / kRowBytes * kSlots) == 0, "a piece further on, a row's key is the same");
+    static_assert((WAVES * kRowsPerPiece) % (256 / kRowBytes * kSlots) == 0, "a piece further on, a row's key is the same");
     // (a block takes piece blockIdx.z of the reduction: all of it unless the launch cut it)
     const int steps = K / KSTEP / prm.reduction_parts;
     const int first_step = static_cast<int>(blockIdx.z) * steps;
     // Piece `i` of this wave's pieces of step `step_`, into stage step_ % kStages.  (Requests past the last step repeat it
     // and land in a stage nobody reads again: the wait before the barrier counts pieces.)
     auto request_piece = [&](int step_, int i) __attribute__((always_inline)) {
-        constexpr int kX = kPiecesX / 4, kW = kPiecesW / 4;
+        constexpr int kX = kPiecesX / WAVES, kW = kPiecesW / WAVES;
         const int j = i < kX ? i : (i < kX + kW ? i - kX : i - kX - kW);
         const uint32_t k_bytes = static_cast<uint32_t>((first_step + min(step_, steps - 1)) * KSTEP * 2);
-        const int scalar = static_cast<int>(k_bytes + static_cast<uint32_t>(4 * kRowsPerPiece * j) * row_bytes);
-        auto* to = (__attribute__((address_space(3))) void*)(gm_smem + (step_ % kStages) * kStageBytes + 1024 * wave + 4096 * i);
+        const int scalar = static_cast<int>(k_bytes + static_cast<uint32_t>(WAVES * kRowsPerPiece * j) * row_bytes);
+        auto* to = (__attribute__((address_space(3))) void*)(gm_smem + (step_ % kStages) * kStageBytes + 1024 * wave + 1024 * WAVES * i);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(i < kX ? x_rsrc : (i < kX + kW ? w_rsrc : u_rsrc), to, 16, static_cast<int>(lane_off),
                                                  scalar, 0, 0);
+    };
+
+    // With two stages a weight line would be asked for one step before its use, less than memory takes: one lane per line of a
+    // later step's weights asks for four bytes of it (into LDS that nobody reads), so that the stage's request finds it in L2.  The
+    // row tiles of a column tile take turns; a lane with nothing to ask for is out of the descriptor's range.  (1024 tokens x 6144
+    // channels of 2048, weights not in any cache: 62 -> 56 us.  With three and four stages it costs more than it brings.)
+    constexpr int kTouchAhead = kStages == 2 ? 4 : 0;
+    constexpr int kTouches = kTouchAhead ? (kWeights * BN + 64 * WAVES - 1) / (64 * WAVES) : 0;     // a wave's requests per step
+    static_assert(kPerWave * (kStages - 2) + kTouches * kTouchAhead <= 63 && (kTouches == 0 || kStages == 2), "the waits count the later stages' pieces");
+    static_assert(kTouches == 0 || kRowBytes == 128, "a row's step is one line");
+    const int sharers = min(static_cast<int>(gridDim.y), 8), turn = static_cast<int>(blockIdx.y) % sharers;
+    auto touch = [&](int step_) __attribute__((always_inline)) {
+#pragma unroll
+        for (int t = 0; t < kTouches; ++t) {
+            const int first = (t * WAVES + wave) * 64, row = first + lane;
+            const bool up = DUAL && first >= BN;
+            const bool wanted = step_ < steps && step_ % sharers == turn && row < kWeights * BN;
+            const uint32_t off = wanted ? static_cast<uint32_t>(up ? row - BN : row) * row_bytes + static_cast<uint32_t>((first_step + step_) * KSTEP * 2) : 0x7ffffff0U;
+            auto* to = (__attribute__((address_space(3))) void*)(gm_smem + kStages * kStageBytes + 256 * wave);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(up ? u_rsrc : w_rsrc, to, 4, static_cast<int>(off), 0, 0, 0);
+        }
     };
 
     f32x16_t acc[kTn][kTm], acc_up[DUAL ? kTn : 1][DUAL ? kTm : 1];
@@ -289,22 +317,27 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
     auto read_all = [&](Frags& f, uint32_t stage_at, int kb) __attribute__((always_inline)) {
         read_nth(f, stage_at, kb, integral_constant<int, 0>{});
         read_nth(f, stage_at, kb, integral_constant<int, 1>{});
-        read_nth(f, stage_at, kb, integral_constant<int, 2>{});
+        if constexpr (Schedule::kReads > 2) read_nth(f, stage_at, kb, integral_constant<int, 2>{});
         if constexpr (Schedule::kReads > 3) read_nth(f, stage_at, kb, integral_constant<int, 3>{});
-        if constexpr (Schedule::kReads > 4) {
-            read_nth(f, stage_at, kb, integral_constant<int, 4>{});
-            read_nth(f, stage_at, kb, integral_constant<int, 5>{});
-        }
-        if constexpr (Schedule::kReads > 6) {
-            read_nth(f, stage_at, kb, integral_constant<int, 6>{});
-            read_nth(f, stage_at, kb, integral_constant<int, 7>{});
-        }
+        if constexpr (Schedule::kReads > 4) read_nth(f, stage_at, kb, integral_constant<int, 4>{});
+        if constexpr (Schedule::kReads > 5) read_nth(f, stage_at, kb, integral_constant<int, 5>{});
+        if constexpr (Schedule::kReads > 6) read_nth(f, stage_at, kb, integral_constant<int, 6>{});
+        if constexpr (Schedule::kReads > 7) read_nth(f, stage_at, kb, integral_constant<int, 7>{});
     };
-    static_assert(Schedule::kReads == 3 || Schedule::kReads == 4 || Schedule::kReads == 6 || Schedule::kReads == 8, "read_all lists them");
+    static_assert(Schedule::kReads >= 2 && Schedule::kReads <= 8, "read_all lists them");
     constexpr int kReads = Schedule::kReads;
     // the fragments of f may be used once at most `later` reads issued after them are outstanding
     auto arrived = [&](Frags& f, auto later) __attribute__((always_inline)) {
-        if constexpr (kTn == 3 && DUAL) {
+        if constexpr (kTm == 1 && kTn == 3 && DUAL) {
+            asm volatile("s_waitcnt lgkmcnt(%7)" : "+v"(f.w[0]), "+v"(f.w[1]), "+v"(f.w[kTn - 1]), "+v"(f.u[0]), "+v"(f.u[1]), "+v"(f.u[kTn - 1]),
+                         "+v"(f.x[0]) : "n"(decltype(later)::value) : "memory");
+        } else if constexpr (kTm == 1 && DUAL) {
+            static_assert(kTm != 1 || !DUAL || kTn == 1 || kTn == 3, "");
+            asm volatile("s_waitcnt lgkmcnt(%3)" : "+v"(f.w[0]), "+v"(f.u[0]), "+v"(f.x[0]) : "n"(decltype(later)::value) : "memory");
+        } else if constexpr (kTm == 1) {
+            static_assert(kTm != 1 || DUAL || kTn == 1, "");
+            asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(f.w[0]), "+v"(f.x[0]) : "n"(decltype(later)::value) : "memory");
+        } else if constexpr (kTn == 3 && DUAL) {
             asm volatile("s_waitcnt lgkmcnt(%8)" : "+v"(f.w[0]), "+v"(f.w[1]), "+v"(f.w[kTn - 1]), "+v"(f.u[0]), "+v"(f.u[1]), "+v"(f.u[kTn - 1]),
                          "+v"(f.x[0]), "+v"(f.x[1]) : "n"(decltype(later)::value) : "memory");
         } else if constexpr (kTn == 2 && DUAL) {
@@ -360,18 +393,15 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
                 slot(integral_constant<int, first + 1>{});
             }
         };
-        unit(integral_constant<int, 0>{}, integral_constant<int, 0>{});
-        unit(integral_constant<int, 0>{}, integral_constant<int, 1>{});
-        if constexpr (kTn >= 2) {
-            unit(integral_constant<int, 1>{}, integral_constant<int, 0>{});
-            unit(integral_constant<int, 1>{}, integral_constant<int, 1>{});
-        }
-        if constexpr (kTn == 3) {
-            unit(integral_constant<int, 2>{}, integral_constant<int, 0>{});
-            unit(integral_constant<int, 2>{}, integral_constant<int, 1>{});
-        }
+        auto across = [&](auto a_) __attribute__((always_inline)) {
+            unit(a_, integral_constant<int, 0>{});
+            if constexpr (kTm == 2) unit(a_, integral_constant<int, 1>{});
+        };
+        across(integral_constant<int, 0>{});
+        if constexpr (kTn >= 2) across(integral_constant<int, 1>{});
+        if constexpr (kTn == 3) across(integral_constant<int, 2>{});
     };
-    static_assert(kTm == 2 && kTn <= 3, "multiply lists the units");
+    static_assert(kTm <= 2 && kTn <= 3, "multiply lists the units");
     using yes = std::true_type;
     using no = std::false_type;
 
@@ -392,7 +422,9 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
     for (int ahead = 0; ahead < kStages - 1; ++ahead)
 #pragma unroll
         for (int i = 0; i < kPerWave; ++i) request_piece(ahead, i);
-    gm_wait_vm<kPerWave * (kStages - 2)>();
+#pragma unroll
+    for (int ahead = 0; ahead < kTouchAhead; ++ahead) touch(kStages - 1 + ahead);
+    gm_wait_vm<kPerWave * (kStages - 2) + kTouches * kTouchAhead>();
     asm volatile("s_barrier" ::: "memory");
     Frags f0, f1;
     read_all(f0, lds_base, 0);
@@ -427,7 +459,8 @@ __global__ __launch_bounds__(kGmThreads) void linear_rows_mfma_kernel(LinearRows
             k_block(integral_constant<int, 6>{});
         }
         arrived(f1, integral_constant<int, 0>{});
-        gm_wait_vm<kPerWave * (kStages - 2)>();                   // this wave's pieces of the next step's stage have landed
+        touch(step + kStages - 1 + kTouchAhead);
+        gm_wait_vm<kPerWave * (kStages - 2) + kTouches>();        // this wave's pieces of the next step's stage have landed
         asm volatile("s_barrier" ::: "memory");                   // everybody's have; and everybody has read this step's stage
         multiply(f1, f0, yes{}, next_at, 1, yes{}, next_at, req, integral_constant<int, 0>{}, integral_constant<int, 0>{});
     }
@@ -544,19 +577,19 @@ __global__ __launch_bounds__(256) void linear_rows_parts_kernel(LinearRowsParams
     *reinterpret_cast<uint2*>(prm.output + static_cast<int64_t>(m) * prm.columns + n) = packed;
 }
 
-template <bool DUAL, int BM, int BN, int KSTEP>
+template <bool DUAL, int BM, int BN, int KSTEP, int WAVES>
 int32_t launch_rows_mfma_as(const LinearRowsParams& prm, hipStream_t stream) {
     using Shape = GmShape<DUAL, BM, BN, KSTEP>;
-    constexpr int smem = Shape::kStages * Shape::kStageBytes;
+    constexpr int smem = Shape::kStages * Shape::kStageBytes + (Shape::kStages == 2 ? 256 * WAVES : 0);
     int column_tiles = prm.columns / BN;
     for (int g = 1; g < prm.groups; ++g) column_tiles += prm.group_columns[g - 1] / BN;
     const dim3 grid(static_cast<unsigned>(column_tiles), static_cast<unsigned>((prm.rows + BM - 1) / BM),
                     static_cast<unsigned>(prm.reduction_parts));
     if (grid.y > 65535u) return QM_ERR_ARGUMENT;
     static std::atomic<bool> lds_raised[kMaxDevices];
-    const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(linear_rows_mfma_kernel<DUAL, BM, BN, KSTEP>), smem, lds_raised);
+    const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(linear_rows_mfma_kernel<DUAL, BM, BN, KSTEP, WAVES>), smem, lds_raised);
     if (rc != QM_OK) return rc;
-    hipLaunchKernelGGL((linear_rows_mfma_kernel<DUAL, BM, BN, KSTEP>), grid, dim3(kGmThreads), smem, stream, prm);
+    hipLaunchKernelGGL((linear_rows_mfma_kernel<DUAL, BM, BN, KSTEP, WAVES>), grid, dim3(64 * WAVES), smem, stream, prm);
     int32_t status = launch_status();
     if (status == QM_OK && prm.reduction_parts > 1) {
         const int64_t quads = static_cast<int64_t>(prm.rows) * (prm.columns / 4);
@@ -593,8 +626,8 @@ int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t str
     if (prm.rows == 0 || prm.columns == 0) return QM_OK;
     if (prm.tile_matrix) {
         if (prm.groups > 1 || prm.reduction_parts != 1 || (prm.tile_rows != 64 && prm.tile_rows != 128) || prm.rows % prm.tile_rows) return QM_ERR_ARGUMENT;
-        if (prm.tile_rows == 64) return dual ? launch_rows_mfma_as<true, 64, 128, 64>(prm, stream) : launch_rows_mfma_as<false, 64, 128, 64>(prm, stream);
-        return dual ? launch_rows_mfma_as<true, 128, 128, 64>(prm, stream) : launch_rows_mfma_as<false, 128, 128, 64>(prm, stream);
+        if (prm.tile_rows == 64) return dual ? launch_rows_mfma_as<true, 64, 128, 64, 4>(prm, stream) : launch_rows_mfma_as<false, 64, 128, 64, 4>(prm, stream);
+        return dual ? launch_rows_mfma_as<true, 128, 128, 64, 4>(prm, stream) : launch_rows_mfma_as<false, 128, 128, 64, 8>(prm, stream);
     }
     // blocks of 64 token rows where blocks of 128 would leave CUs without one (one block per CU either way)
     const int64_t row_tiles = (prm.rows + 127) / 128;
@@ -607,13 +640,13 @@ int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t str
         // of 192 columns, if those fit in one round (1024 tokens x 6144 channels: 384 blocks of 128, 256 of 192)
         const int64_t blocks_192 = static_cast<int64_t>(prm.columns / 192) * row_tiles;
         if (prm.reduction_parts == 1 && prm.columns % 192 == 0 && blocks_128 > 256 && blocks_128 < 512 && blocks_192 <= 256)
-            return launch_rows_mfma_as<true, 128, 192, 64>(prm, stream);
-        return small ? launch_rows_mfma_as<true, 64, 128, 64>(prm, stream) : launch_rows_mfma_as<true, 128, 128, 64>(prm, stream);
+            return launch_rows_mfma_as<true, 128, 192, 64, 4>(prm, stream);
+        return small ? launch_rows_mfma_as<true, 64, 128, 64, 4>(prm, stream) : launch_rows_mfma_as<true, 128, 128, 64, 4>(prm, stream);
     }
     // (64 token rows and a long uncut reduction: steps of 128 k, half as many barriers for the same MFMAs; a short one
     // loses more to the larger first stages than it gains)
-    if (small && prm.reduction_parts == 1 && prm.reduction >= 4096) return launch_rows_mfma_as<false, 64, 128, 128>(prm, stream);
-    return small ? launch_rows_mfma_as<false, 64, 128, 64>(prm, stream) : launch_rows_mfma_as<false, 128, 128, 64>(prm, stream);
+    if (small && prm.reduction_parts == 1 && prm.reduction >= 4096) return launch_rows_mfma_as<false, 64, 128, 128, 4>(prm, stream);
+    return small ? launch_rows_mfma_as<false, 64, 128, 64, 4>(prm, stream) : launch_rows_mfma_as<false, 128, 128, 64, 8>(prm, stream);
 }
 
 }  // namespace qm
