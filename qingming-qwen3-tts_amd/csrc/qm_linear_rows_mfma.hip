@@ -9,7 +9,8 @@
 // A block owns a tile of BM token rows x BN output columns: 128 x 128 (eight waves 2 x 4, each 64 rows x 32 columns, two to a
 // SIMD so that one multiplies while the other waits to issue: three linears of 2048, 2048 and 6144 inputs over 1024 rows 71.3 ->
 // 68.6 us against four waves of 64 x 64; the other tiles gain nothing from it and keep four); 64 x 128 for calls whose grid of 128-row tiles would leave CUs empty (waves 4 x 1, each 32 columns x 64
-// rows); 128 x 192 for a gate/up pair whose 128-column tiles come to between one and two rounds of the CUs and whose
+// rows); 64 x 64 with up to eight stages where most CUs would still be empty and a block's time is its chain of round trips to memory
+// (waves 2 x 2); 128 x 192 for a gate/up pair whose 128-column tiles come to between one and two rounds of the CUs and whose
 // 192-column tiles fit in one (1024 tokens x 6144 channels: 256 blocks).  Several linears of one input (q, k, v) share a
 // grid: a column tile's number says which of them it belongs to.  Both operands are K-contiguous rows (x [m][k],
 // w [n][k]), so one tile layout serves both: KSTEP (64, or 128 for 64-row tiles with a long reduction) k per step, a row
@@ -18,7 +19,7 @@
 // operand and the token rows as B (D = W X^T): a lane then holds, for one token row, runs of four consecutive output
 // columns — 8-byte stores.
 // The tiles go from memory straight into a ring of LDS stages (buffer_load ... lds, no registers, the swizzle chosen by
-// which piece a lane fetches): four stages where they fit in 128 KiB, else three, two for the 192-column tile (64 KiB a
+// which piece a lane fetches): four stages where they fit in 128 KiB (the 64 x 64 tile: eight, or six for a pair), else three, two for the 192-column tile (64 KiB a
 // stage).  A step's one barrier stands between the MFMAs of its last two k blocks, where a wave has read all it needs of
 // the step's stage and waits (vmcnt counts the later stages' pieces still in flight) for its own pieces of the next.
 // Nothing but MFMAs is issued in a bunch: a k block's LDS reads and the requests for the stage just freed stand one or
@@ -33,6 +34,7 @@
 #include "qm_host.h"
 #include "qm_linear_rows_params.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace qm {
@@ -83,7 +85,8 @@ __device__ __forceinline__ uint32_t swiglu_pair(float g0, float g1, float u0, fl
 template <bool DUAL, int BM, int BN, int KSTEP>
 struct GmShape {
     static constexpr int kStageBytes = (BM + (DUAL ? 2 : 1) * BN) * KSTEP * 2;
-    static constexpr int kStages = kStageBytes * 4 <= 128 * 1024 ? 4 : (kStageBytes * 3 <= 144 * 1024 ? 3 : 2);
+    static constexpr int kDeep = 144 * 1024 / kStageBytes < 8 ? 144 * 1024 / kStageBytes : 8;
+    static constexpr int kStages = BN == 64 ? kDeep : kStageBytes * 4 <= 128 * 1024 ? 4 : (kStageBytes * 3 <= 144 * 1024 ? 3 : 2);
     static_assert(kStageBytes * kStages <= 160 * 1024 - 1024, "the CU's LDS");
 };
 
@@ -91,7 +94,7 @@ struct GmShape {
 // kTm of token rows.
 template <int BM, int BN, int WAVES>
 struct GmWaves {
-    static constexpr int kAcross = BM == 128 && (WAVES == 4 || BN == 192) ? 2 : 4;
+    static constexpr int kAcross = BN == 64 || (BM == 128 && (WAVES == 4 || BN == 192)) ? 2 : 4;
     static constexpr int kTn = BN / 32 / kAcross, kTm = BM / 32 / (WAVES / kAcross);
 };
 
@@ -578,7 +581,10 @@ __global__ __launch_bounds__(256) void linear_rows_parts_kernel(LinearRowsParams
 }
 
 template <bool DUAL, int BM, int BN, int KSTEP, int WAVES>
-int32_t launch_rows_mfma_as(const LinearRowsParams& prm, hipStream_t stream) {
+int32_t launch_rows_mfma_as(const LinearRowsParams& given, hipStream_t stream) {
+    LinearRowsParams prm = given;
+    if (BN == 64)                                                 // (given in tiles of 128 columns)
+        for (int& first : prm.group_first_tile) first *= 2;
     using Shape = GmShape<DUAL, BM, BN, KSTEP>;
     constexpr int smem = Shape::kStages * Shape::kStageBytes + (Shape::kStages == 2 ? 256 * WAVES : 0);
     int column_tiles = prm.columns / BN;
@@ -622,6 +628,22 @@ size_t rows_mfma_workspace_bytes(int rows, int columns, int reduction, bool dual
     return static_cast<size_t>(parts) * (dual ? 2 : 1) * rows * columns * sizeof(float);
 }
 
+// The longest chain of 64-k steps that a CU walks if the linears are dealt out in tiles of 64 rows and `bn` columns, a block per CU,
+// long reductions first: the whole work over the CUs, in whole blocks of the shortest reduction.
+static int64_t rows_mfma_chain(const LinearRowsParams& prm, int bn) {
+    const int64_t row_tiles = (prm.rows + 63) / 64;
+    int64_t total = 0, shortest = 0, longest = 0;
+    for (int g = 0; g < prm.groups; ++g) {
+        const int64_t columns = g == 0 ? prm.columns : prm.group_columns[g - 1];
+        const int64_t steps = (g == 0 || !prm.group_reduction[g - 1] ? prm.reduction : prm.group_reduction[g - 1]) / kGmStep;
+        total += columns / bn * row_tiles * steps;
+        shortest = g == 0 || steps < shortest ? steps : shortest;
+        longest = steps > longest ? steps : longest;
+    }
+    const int64_t even = (total + 255) / 256;
+    return std::max(longest, (even + shortest - 1) / shortest * shortest);
+}
+
 int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t stream) {
     if (prm.rows == 0 || prm.columns == 0) return QM_OK;
     if (prm.tile_matrix) {
@@ -635,6 +657,13 @@ int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t str
     for (int g = 1; g < prm.groups; ++g) columns += prm.group_columns[g - 1];
     const int64_t blocks_128 = columns / kGmTile * row_tiles;
     const bool small = blocks_128 < 200;
+    // Measured (us, 64 x 128 / 64 x 64 tiles): 2048 columns of 6144 at 16 / 64 / 300 / 500 rows 24 / 28 / 27 / 28 against 17 / 20 / 20 / 22,
+    // 4096 of 2048 at 128 / 200 / 300 rows 10.9 / 11.1 / 11.4 against 8.7 / 9.5 / 16.2, pairs of 6144 of 2048 at 64 / 128 / 200 rows
+    // 26 / 25 / 25 against 18 / 18 / 30, three linears of 2048, 2048 and 6144 at 200 / 300 / 500 rows 36 / 41 / 44 against 25 / 36 / 52.
+    // Smaller tiles with deeper rings where that shortens the grid's longest chain of steps or leaves it as it is: a step of a 64 x 64
+    // tile takes about 0.7 of a 64 x 128 one's time (seven stages under way instead of three).
+    if (small && prm.reduction_parts == 1 && 7 * rows_mfma_chain(prm, 64) < 10 * rows_mfma_chain(prm, 128))
+        return dual ? launch_rows_mfma_as<true, 64, 64, 64, 4>(prm, stream) : launch_rows_mfma_as<false, 64, 64, 64, 4>(prm, stream);
     if (dual) {
         // a gate/up pair whose grid of 128-column tiles is more than the CUs take at once and less than twice that: tiles
         // of 192 columns, if those fit in one round (1024 tokens x 6144 channels: 384 blocks of 128, 256 of 192)

@@ -244,3 +244,37 @@ def test_qkv_rows_with_an_empty_member(qm, dev, oracle):
         for g, w in zip(got, want):
             assert torch.equal(g, w)
 
+
+
+@pytest.mark.parametrize("rows,cols,red", [
+    # each tile of the matrix-core kernel at a remainder of rows: 64 x 64 (one step, fewer steps than its stages, many), 64 x 128,
+    # 64 x 128 with 128 k a step, 128 x 128 with one and several rounds
+    (17, 128, 128), (65, 256, 256), (190, 2048, 3072), (300, 4096, 256), (129, 16640, 384), (65, 16640, 4096), (1000, 4096, 256), (1030, 8192, 128)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_matrix_core_tiles_against_64_bits(qm, dev, rows, cols, red, pair, rows_kernel):
+    """Every output is the rounding of a sum that is within red * 2^-24 * sum |x w| of the exact one; a pair's roundings of gate, SiLU,
+    up and product follow, half a spacing (2^-9) of the value each, the gate's through a slope of at most 1.1."""
+    import torch
+    if rows_kernel == EXACT:
+        pytest.skip("the exact chain is compared bit for bit above")
+    gen = torch.Generator(device=dev).manual_seed(rows + red)
+    x = torch.randn(rows, red, device=dev, generator=gen).bfloat16()
+    w, up = ((torch.randn(cols, red, device=dev, generator=gen) * red ** -0.5).bfloat16() for _ in range(2))
+    out = torch.full((rows + 1, cols), 7.0, device=dev, dtype=torch.bfloat16)
+    if pair:
+        qm.gate_up_swiglu_rows(x, w, up, out, rows, red, cols)
+    else:
+        qm.linear_rows(x, w, None, None, out, rows, cols, red)
+    torch.cuda.synchronize()
+    assert bool((out[rows:] == 7).all())
+    got, unit, half = out[:rows].double(), red * 2.0 ** -24, 2.0 ** -8
+    s, most = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    want, bound = s, unit * most + half * s.abs()
+    if pair:
+        u, u_most = x.double() @ up.double().t(), x.double().abs() @ up.double().abs().t()
+        act = torch.nn.functional.silu(s)
+        act_bound = 1.1 * bound + half * act.abs()
+        u_bound = unit * u_most + half * u.abs()
+        want = act * u
+        bound = act_bound * u.abs() + u_bound * act.abs() + act_bound * u_bound + half * want.abs()
+    assert bool(((got - want).abs() <= bound + 1e-30).all()), float(((got - want).abs() / (bound + 1e-30)).max())
