@@ -167,13 +167,17 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
     constexpr int kHeld = 4;                   // float4s a thread holds between its two uses of a value
     if (prm.groups == 1 && total % 4 == 0 && prm.ld_o % 4 == 0 && total <= kHeld * 4 * kDecThreads) {
         const int vectors = total >> 2;
-        float4 held[kHeld], g[kHeld];
+        float4 held[kHeld], g[kHeld], weight[kHeld];
         float sq[1] = {0.0f};
 #pragma unroll
         for (int i = 0; i < kHeld; ++i) {
             const int v = tid + i * kDecThreads;
             held[i] = load4_if(v < vectors, o, v);
             g[i] = load4_if(v < vectors, gate, v);
+            weight[i] = prm.weight ? load4_if(v < vectors, prm.weight, v) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+        }
+#pragma unroll
+        for (int i = 0; i < kHeld; ++i) {
             sq[0] = square_sum(held[i], sq[0]);
         }
         block_sums<1>(sq, sh_red);
@@ -182,7 +186,7 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
         for (int i = 0; i < kHeld; ++i) {
             const int v = tid + i * kDecThreads;
             if (v >= vectors) continue;
-            const float4 w = prm.weight ? load4(prm.weight, v) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+            const float4 w = weight[i];
             store4(out, v, held[i].x * inverse * w.x * gate_f32(g[i].x, silu), held[i].y * inverse * w.y * gate_f32(g[i].y, silu),
                    held[i].z * inverse * w.z * gate_f32(g[i].z, silu), held[i].w * inverse * w.w * gate_f32(g[i].w, silu));
         }
@@ -194,29 +198,42 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
         for (int c = tid; c < total; c += kDecThreads)
             out[c] = from_f32<T>(o[c] * inverse * weight_at(c) * gate_f32(gate[c], silu));
     } else {
-        // a wave per slice, a slice of up to 256 values held by its lanes
-        for (int g = wave; g < prm.groups; g += kDecThreads / 64) {
-            float held[4], gates[4], sq = 0.0f;
+        // a wave per slice, a slice of up to 256 values held by its lanes; the values of four slices are asked for at once
+        constexpr int kAtOnce = 4;
+        for (int g0 = wave; g0 < prm.groups; g0 += kAtOnce * (kDecThreads / 64)) {
+            float held[kAtOnce][4], gates[kAtOnce][4], weights[kAtOnce][4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = lane + 64 * i;
-                const bool in = c < prm.size;
-                const int at = g * prm.size + (in ? c : 0);
-                const float value = o[at];
-                gates[i] = gate[at];
-                held[i] = in ? value : 0.0f;
-                sq = fmaf(held[i], held[i], sq);
-            }
-            for (int c = lane + 256; c < prm.size; c += 64) sq = fmaf(o[g * prm.size + c], o[g * prm.size + c], sq);
-            const float inverse = 1.0f / sqrtf(wave_sum(sq) * inv_size + prm.eps);
+            for (int j = 0; j < kAtOnce; ++j) {
+                const int g = min(g0 + j * (kDecThreads / 64), prm.groups - 1);   // (past the last: repeated, not stored)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int c = lane + 64 * i, at = g * prm.size + c;
-                if (c < prm.size) out[at] = from_f32<T>(held[i] * inverse * weight_at(at) * gate_f32(gates[i], silu));
+                for (int i = 0; i < 4; ++i) {
+                    const int c = lane + 64 * i;
+                    const bool in = c < prm.size;
+                    const int at = g * prm.size + (in ? c : 0);
+                    const float value = o[at];
+                    gates[j][i] = gate[at];
+                    weights[j][i] = weight_at(at);
+                    held[j][i] = in ? value : 0.0f;
+                }
             }
-            for (int c = lane + 256; c < prm.size; c += 64) {
-                const int at = g * prm.size + c;
-                out[at] = from_f32<T>(o[at] * inverse * weight_at(at) * gate_f32(gate[at], silu));
+#pragma unroll
+            for (int j = 0; j < kAtOnce; ++j) {
+                const int g = g0 + j * (kDecThreads / 64);
+                if (g >= prm.groups) break;
+                float sq = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sq = fmaf(held[j][i], held[j][i], sq);
+                for (int c = lane + 256; c < prm.size; c += 64) sq = fmaf(o[g * prm.size + c], o[g * prm.size + c], sq);
+                const float inverse = 1.0f / sqrtf(wave_sum(sq) * inv_size + prm.eps);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int c = lane + 64 * i;
+                    if (c < prm.size) out[g * prm.size + c] = from_f32<T>(held[j][i] * inverse * weights[j][i] * gate_f32(gates[j][i], silu));
+                }
+                for (int c = lane + 256; c < prm.size; c += 64) {
+                    const int at = g * prm.size + c;
+                    out[at] = from_f32<T>(o[at] * inverse * weight_at(at) * gate_f32(gate[at], silu));
+                }
             }
         }
     }
@@ -283,12 +300,16 @@ template <class T>
 __device__ __forceinline__ void slice_norm_row(const float* x, const float* weight, int n, int64_t padded, float eps, float* sh_red, T* out) {
     const int tid = threadIdx.x;
     constexpr int kHeld = 4;
-    float held[kHeld], sq[1] = {0.0f};
+    float held[kHeld], weights[kHeld], sq[1] = {0.0f};
 #pragma unroll
     for (int i = 0; i < kHeld; ++i) {
-        const int c = tid + i * kDecThreads;
-        const float value = x[min(c, n - 1)];
-        held[i] = c < n ? value : 0.0f;
+        const int c = min(tid + i * kDecThreads, n - 1);
+        held[i] = x[c];
+        weights[i] = weight[c];
+    }
+#pragma unroll
+    for (int i = 0; i < kHeld; ++i) {
+        held[i] = tid + i * kDecThreads < n ? held[i] : 0.0f;
         sq[0] = fmaf(held[i], held[i], sq[0]);
     }
     for (int c = tid + kHeld * kDecThreads; c < n; c += kDecThreads) sq[0] = fmaf(x[c], x[c], sq[0]);
@@ -297,7 +318,7 @@ __device__ __forceinline__ void slice_norm_row(const float* x, const float* weig
 #pragma unroll
     for (int i = 0; i < kHeld; ++i) {
         const int c = tid + i * kDecThreads;
-        if (c < n) out[c] = from_f32<T>(held[i] * inverse * weight[c]);
+        if (c < n) out[c] = from_f32<T>(held[i] * inverse * weights[i]);
     }
     for (int c = tid + kHeld * kDecThreads; c < n; c += kDecThreads) out[c] = from_f32<T>(x[c] * inverse * weight[c]);
     for (int64_t c = n + tid; c < padded; c += kDecThreads) out[c] = from_f32<T>(0.0f);
