@@ -106,7 +106,13 @@ int32_t launch_layer_out(const LayerOutParams& prm, int f32, hipStream_t stream)
 int32_t launch_argmax(const float* scores, int vocab, int32_t* token, hipStream_t stream);
 // step = the words below: the chosen token is put out and becomes the one to feed, the token that was fed the one before it,
 // and the position moves on by `advance`
-enum StepWord { kStepPosition, kStepBefore, kStepToken, kStepEmitted, kStepChosen, kStepWords };
+enum StepWord { kStepPosition, kStepBefore, kStepToken, kStepEmitted, kStepChosen, kStepTicket, kStepWords };
 int32_t launch_emit(int32_t* step, int32_t* out, int advance, hipStream_t stream);
+// The words from pinned host memory; and `vocab` scores into pinned host memory, each of mail_blocks(vocab) blocks raising its flag
+// (kMailFlagStride words apart) to the ticket behind what it wrote: a host that sees every flag has every score.
+constexpr int kMailBlocks = 16, kMailFlagStride = 16;
+inline int mail_blocks(int vocab) { return vocab < 1024 ? 1 : vocab / 1024 < kMailBlocks ? vocab / 1024 : kMailBlocks; }
+int32_t launch_take_words(const int32_t* host, int32_t* step, hipStream_t stream);
+int32_t launch_mail_scores(const float* scores, int vocab, float* host, uint32_t* flags, const int32_t* ticket, hipStream_t stream);
 
 }  // namespace qm

@@ -133,6 +133,21 @@ __global__ void emit_kernel(int32_t* step, int32_t* out, int advance) {
     step[kStepPosition] += advance;
 }
 
+__global__ void take_words_kernel(const int32_t* host, int32_t* step) {
+    if (threadIdx.x < kStepWords) step[threadIdx.x] = __hip_atomic_load(host + threadIdx.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__global__ __launch_bounds__(kDecThreads) void mail_scores_kernel(const float* scores, int vocab, float* host, uint32_t* flags, const int32_t* ticket) {
+    const uint32_t number = static_cast<uint32_t>(__hip_atomic_load(ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+    const int vectors = vocab >> 2, stride = static_cast<int>(gridDim.x) * kDecThreads;
+    for (int v = static_cast<int>(blockIdx.x) * kDecThreads + threadIdx.x; v < vectors; v += stride)
+        reinterpret_cast<float4*>(host)[v] = reinterpret_cast<const float4*>(scores)[v];
+    if (blockIdx.x == 0 && static_cast<int>(threadIdx.x) < (vocab & 3)) host[4 * vectors + threadIdx.x] = scores[4 * vectors + threadIdx.x];
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) __hip_atomic_store(flags + blockIdx.x * kMailFlagStride, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 static int most_k(const DecLinearParams& prm) {
     int k = 0;
     for (int g = 0; g < prm.groups; ++g) k = prm.group[g].k > k ? prm.group[g].k : k;
@@ -225,6 +240,19 @@ int32_t launch_argmax(const float* scores, int vocab, int32_t* token, hipStream_
     if (!scores || !token) return QM_ERR_NULL;
     if (vocab <= 0) return QM_ERR_ARGUMENT;
     hipLaunchKernelGGL(argmax_kernel, dim3(1), dim3(kArgmaxThreads), 0, stream, scores, vocab, token);
+    return launch_status();
+}
+
+int32_t launch_take_words(const int32_t* host, int32_t* step, hipStream_t stream) {
+    if (!host || !step) return QM_ERR_NULL;
+    hipLaunchKernelGGL(take_words_kernel, dim3(1), dim3(64), 0, stream, host, step);
+    return launch_status();
+}
+
+int32_t launch_mail_scores(const float* scores, int vocab, float* host, uint32_t* flags, const int32_t* ticket, hipStream_t stream) {
+    if (!scores || !host || !flags || !ticket) return QM_ERR_NULL;
+    if (vocab <= 0) return QM_ERR_ARGUMENT;
+    hipLaunchKernelGGL(mail_scores_kernel, dim3(mail_blocks(vocab)), dim3(kDecThreads), 0, stream, scores, vocab, host, flags, ticket);
     return launch_status();
 }
 

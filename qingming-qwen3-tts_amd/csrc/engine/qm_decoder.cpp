@@ -19,6 +19,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -78,6 +79,34 @@ struct DecoderLayer {
     double magnitude = 1.0;
 };
 
+// What a step sends and gets in pinned host memory, so that it is one graph and the host sees the scores as they arrive.  A step
+// has its results before the next one begins, so one mailbox serves every sequence.
+struct Mailbox {
+    char* at = nullptr;
+    uint32_t last = 0;                              // ticket of the last scores asked for
+    Mailbox() = default;
+    Mailbox(const Mailbox&) = delete;
+    Mailbox& operator=(const Mailbox&) = delete;
+    ~Mailbox() {
+        if (at) (void)hipHostFree(at);
+    }
+    void open(int vocab_p) {
+        void* p = nullptr;
+        hip_check(hipHostMalloc(&p, kScores + static_cast<size_t>(vocab_p) * 4, hipHostMallocDefault), "pinned step results");
+        at = static_cast<char*>(p);
+        std::memset(at, 0, kScores);
+    }
+    static constexpr size_t kFlags = 256, kScores = kFlags + qm::kMailBlocks * qm::kMailFlagStride * 4;
+    int32_t* words() const { return reinterpret_cast<int32_t*>(at); }
+    uint32_t* flags() const { return reinterpret_cast<uint32_t*>(at + kFlags); }
+    float* scores() const { return reinterpret_cast<float*>(at + kScores); }
+    bool arrived(int blocks) const {
+        for (int b = 0; b < blocks; ++b)
+            if (__atomic_load_n(flags() + b * qm::kMailFlagStride, __ATOMIC_ACQUIRE) != last) return false;
+        return true;
+    }
+};
+
 struct RunState {                                   // byte offsets inside a sequence's memory
     size_t k = 0, v = 0, decay = 0, delta = 0, latent = 0, key = 0;
 };
@@ -104,10 +133,14 @@ struct qm_decoder {
     qm_engine::DeviceBuffer x[2], h, proj, mlp, attended, gated, y[3], q_rot, raw, ml, acc, scratch, tokens, wanted, head_h, logits, tap, tap_h,
         step_words, q_latent, queries, q_scratch, expanded, expert_logits, expert_scratch;
     std::vector<hipGraphExec_t> graphs;             // one-token step of each sequence
+    std::vector<hipGraphExec_t> mail_graphs;        // the same between the mailbox's words and its scores
+    qm_engine::Mailbox mailbox;
 
     ~qm_decoder() {
-        for (hipGraphExec_t g : graphs)
-            if (g) (void)hipGraphExecDestroy(g);
+        (void)hipDeviceSynchronize();               // (a step returns when its scores are there: its last kernel may not have ended)
+        for (const auto* some : {&graphs, &mail_graphs})
+            for (hipGraphExec_t g : *some)
+                if (g) (void)hipGraphExecDestroy(g);
         if (own_stream && stream) (void)hipStreamDestroy(stream);
     }
 };
@@ -376,6 +409,7 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
         d->before.push_back(-1);
     }
     d->graphs.assign(static_cast<size_t>(sequences), nullptr);
+    d->mail_graphs.assign(static_cast<size_t>(sequences), nullptr);
 
     // activations of a pass
     const size_t rows = static_cast<size_t>(d->max_rows);
@@ -451,6 +485,7 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
     d->head_h = zeros(static_cast<size_t>(kLogitRows) * d->width_p * item);
     d->logits = zeros(static_cast<size_t>(kLogitRows) * d->vocab_p * 4);
     d->step_words = zeros(kStepWords * 4);
+    d->mailbox.open(d->vocab_p);
     hip_check(hipDeviceSynchronize(), "decoder setup");
     return d;
 }
@@ -788,7 +823,28 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
     *stream_out = x;
 }
 
-// Logits of the rows that `places` (host) names, as rows of `out` (host).
+// Row 0 of d.logits into the mailbox; `ticket` names the device word, or the mailbox's own, that holds the ticket.
+void mail_scores(qm_decoder& d, const int32_t* ticket) {
+    op_check(qm::launch_mail_scores(f32_of(d.logits), d.config.vocab, d.mailbox.scores(), d.mailbox.flags(), ticket, d.stream), "scores to the host");
+}
+void next_ticket(qm_decoder& d, int position, int before, int token) {
+    const int32_t words[kStepWords] = {position, before, token, 0, 0, static_cast<int32_t>(++d.mailbox.last)};
+    std::memcpy(d.mailbox.words(), words, sizeof words);
+}
+// The mailbox's scores, once they are there.  Looking at the flags sees them some 10 us before the stream's wait returns; a stream
+// that has longer work ahead is waited for.
+const float* await_scores(qm_decoder& d) {
+    const int blocks = qm::mail_blocks(d.config.vocab);
+    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+    for (int looks = 1; !d.mailbox.arrived(blocks); ++looks) {
+        if (looks % 64 != 0 || std::chrono::steady_clock::now() < until) continue;
+        hip_check(hipStreamSynchronize(d.stream), "step");
+        if (!d.mailbox.arrived(blocks)) throw ApiError(QM_ERR_STATUS, "the step's scores did not arrive");
+    }
+    return d.mailbox.scores();
+}
+
+// Logits of the rows that `places` (host) names, as rows of `out` (host); returns when they are there.
 void run_head(qm_decoder& d, const float* x, const Pending& pending, const int32_t* places, int count, float* out) {
     hipStream_t s = d.stream;
     for (int first = 0; first < count; first += kLogitRows) {
@@ -802,6 +858,12 @@ void run_head(qm_decoder& d, const float* x, const Pending& pending, const int32
         l.group[l.groups++] = linear_of(d.head, d.head_h.raw(), f32_of(d.logits));
         op_check(qm::launch_decoder_linears(l, d.f32, s), "head");
         const size_t vocab_bytes = static_cast<size_t>(d.config.vocab) * 4;
+        if (out && rows == 1) {
+            next_ticket(d, 0, 0, 0);
+            mail_scores(d, d.mailbox.words() + qm::kStepTicket);
+            std::memcpy(out + static_cast<size_t>(first) * d.config.vocab, await_scores(d), vocab_bytes);
+            continue;
+        }
         if (out)
             hip_check(hipMemcpy2DAsync(out + static_cast<size_t>(first) * d.config.vocab, vocab_bytes, d.logits.raw(),
                                        static_cast<size_t>(d.vocab_p) * 4, vocab_bytes, static_cast<size_t>(rows), hipMemcpyDeviceToHost, s),
@@ -916,6 +978,26 @@ void enqueue_one_by_operators(qm_decoder& d, int sequence, int position) {
     op_check(qm::launch_decoder_linears(l, d.f32, d.stream), "head");
 }
 
+// What `enqueue` queues, as a graph.
+template <class F>
+hipGraphExec_t capture(qm_decoder& d, F&& enqueue) {
+    hipGraph_t captured = nullptr;
+    hip_check(hipStreamBeginCapture(d.stream, hipStreamCaptureModeThreadLocal), "step capture");
+    try {
+        enqueue();
+    } catch (...) {
+        (void)hipStreamEndCapture(d.stream, &captured);
+        if (captured) (void)hipGraphDestroy(captured);
+        throw;
+    }
+    hip_check(hipStreamEndCapture(d.stream, &captured), "step capture");
+    hipGraphExec_t graph = nullptr;
+    const hipError_t e = hipGraphInstantiate(&graph, captured, nullptr, nullptr, 0);
+    (void)hipGraphDestroy(captured);
+    hip_check(e, "step graph");
+    return graph;
+}
+
 // One token of the sequence, whose words are in place; logits in row 0 of d.logits.
 void run_one(qm_decoder& d, int sequence) {
     int& length = d.length[static_cast<size_t>(sequence)];
@@ -927,28 +1009,30 @@ void run_one(qm_decoder& d, int sequence) {
         enqueue_one(d, sequence);          // (the first of all sets the kernels' attributes, outside of any capture)
         d.warm = true;
     } else {
-        if (!graph) {
-            hipGraph_t captured = nullptr;
-            hip_check(hipStreamBeginCapture(d.stream, hipStreamCaptureModeThreadLocal), "step capture");
-            try {
-                enqueue_one(d, sequence);
-            } catch (...) {
-                (void)hipStreamEndCapture(d.stream, &captured);
-                if (captured) (void)hipGraphDestroy(captured);
-                throw;
-            }
-            hip_check(hipStreamEndCapture(d.stream, &captured), "step capture");
-            const hipError_t e = hipGraphInstantiate(&graph, captured, nullptr, nullptr, 0);
-            (void)hipGraphDestroy(captured);
-            hip_check(e, "step graph");
-        }
+        if (!graph) graph = capture(d, [&] { enqueue_one(d, sequence); });
         hip_check(hipGraphLaunch(graph, d.stream), "step graph launch");
     }
     ++length;
 }
 
+// A one-token step from the mailbox's words to its scores.
+void run_one_by_mail(qm_decoder& d, int sequence, int before, int token) {
+    int& length = d.length[static_cast<size_t>(sequence)];
+    if (length >= d.capacity) throw ApiError(QM_ERR_SLOT_RANGE, "the sequence exceeds its capacity");
+    hipGraphExec_t& graph = d.mail_graphs[static_cast<size_t>(sequence)];
+    if (!graph)
+        graph = capture(d, [&] {
+            op_check(qm::launch_take_words(d.mailbox.words(), step_words(d), d.stream), "step words");
+            enqueue_one(d, sequence);
+            mail_scores(d, step_words(d) + qm::kStepTicket);
+        });
+    next_ticket(d, length, before, token);
+    hip_check(hipGraphLaunch(graph, d.stream), "step graph launch");
+    ++length;
+}
+
 void put_step_words(qm_decoder& d, int position, int before, int token) {
-    const int32_t words[kStepWords] = {position, before, token, 0, 0};
+    const int32_t words[kStepWords] = {position, before, token, 0, 0, 0};
     hip_check(hipMemcpyAsync(d.step_words.raw(), words, sizeof words, hipMemcpyHostToDevice, d.stream), "step words");
 }
 
@@ -979,6 +1063,14 @@ void step(qm_decoder& d, int sequence, const int32_t* tokens, int count, const i
         d.tap = DeviceBuffer(static_cast<size_t>(d.max_rows) * d.width_p * 4);
         d.tap_h = DeviceBuffer(static_cast<size_t>(d.max_rows) * d.width_p * 4);
     }
+    if (count == 1 && !streams && wanted > 0 && (d.path & 3) == 0 && d.warm) {
+        run_one_by_mail(d, sequence, before, tokens[0]);
+        before = tokens[0];
+        const float* scores = await_scores(d);
+        for (int i = 0; i < wanted; ++i)
+            std::memcpy(logits + static_cast<size_t>(i) * d.config.vocab, scores, static_cast<size_t>(d.config.vocab) * 4);
+        return;
+    }
     if (count == 1 && !streams) {
         put_step_words(d, length, before, tokens[0]);
         run_one(d, sequence);
@@ -989,6 +1081,7 @@ void step(qm_decoder& d, int sequence, const int32_t* tokens, int count, const i
         if (read_back) hip_check(hipStreamSynchronize(d.stream), "step");
         return;
     }
+    bool waited = false;                           // for everything queued so far
     for (int first = 0; first < count; first += d.max_rows) {
         const int rows = std::min(d.max_rows, count - first);
         std::vector<int32_t> places;
@@ -1006,6 +1099,7 @@ void step(qm_decoder& d, int sequence, const int32_t* tokens, int count, const i
         run_layers(d, sequence, rows, length, &x, pending, streams);
         length += rows;
         before = tokens[first + rows - 1];
+        waited = !places.empty();
         if (!places.empty()) {
             std::vector<float> some(places.size() * static_cast<size_t>(d.config.vocab));
             run_head(d, x, pending, places.data(), static_cast<int>(places.size()), some.data());
@@ -1014,7 +1108,7 @@ void step(qm_decoder& d, int sequence, const int32_t* tokens, int count, const i
                             static_cast<size_t>(d.config.vocab) * 4);
         }
     }
-    if (read_back) hip_check(hipStreamSynchronize(d.stream), "step");
+    if (read_back && !waited) hip_check(hipStreamSynchronize(d.stream), "step");
 }
 
 // The prompt, then token by token: the head's scores, the token they give into the step words, the step that reads it.

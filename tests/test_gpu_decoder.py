@@ -144,6 +144,34 @@ def test_wanted_places_in_any_order(decoder, models):
     assert engine.step(engine.open(), m.tokens[:5]).shape == (0, m.cfg["vocab"])
 
 
+@pytest.mark.parametrize("name", ["plain", "mixed"])
+def test_ways_of_stepping_leave_the_same(decoder, models, name):
+    """Steps whose scores come through pinned memory, steps that want none, several copies, queued steps and generation in turn, two
+    sequences of one engine: the scores of every token are those of plain fused launches, bit for bit (77 scores: no multiple of four)."""
+    m = models(name)
+    tokens = m.tokens[:40]
+    plain_engine = decoder.Decoder(m.directory, len(m.tokens), sequences=2)
+    plain_engine.set_path(1)
+    p = plain_engine.open()
+    want = [plain_engine.step(p, tokens[:9], [8])[0]] + [plain_engine.step(p, [t], [0])[0] for t in tokens[9:]]
+    engine = decoder.Decoder(m.directory, len(m.tokens), sequences=2)
+    a, b = engine.open(), engine.open()
+    for s in (a, b):
+        assert np.array_equal(engine.step(s, tokens[:9], [8])[0], want[0])
+    for i, t in enumerate(tokens[9:], 1):
+        for s in (a, b):
+            if (i + s) % 4 == 0:
+                engine.step(s, [t])
+            elif (i + s) % 4 == 1:
+                engine.enqueue(s, [t])
+            else:
+                got = engine.step(s, [t], [0] * (i % 3 + 1))
+                assert got.shape[0] == i % 3 + 1 and all(np.array_equal(row, want[i]) for row in got)
+    made = engine.generate(a, [int(tokens[0])], 5)
+    assert np.array_equal(made, plain_engine.generate(p, [int(tokens[0])], 5))
+    assert np.array_equal(engine.step(a, [1], [0]), plain_engine.step(p, [1], [0]))
+
+
 def greedy(m, prompt, count):
     tokens = list(prompt)
     for _ in range(count):
