@@ -64,6 +64,7 @@ int64_t delta_scratch_floats(int rows, int heads, int dim);
 bool delta_chunks_fit(const DeltaParams& prm);
 int32_t launch_decay_chunks(const DecayAttentionParams& prm, hipStream_t stream);
 int32_t launch_delta_chunks(const DeltaParams& prm, hipStream_t stream);
+int32_t check_general_delta(const DeltaParams& prm);
 int32_t launch_general_delta(const DeltaParams& prm, hipStream_t stream);
 int32_t launch_latent_rows(const LatentRowsParams& prm, int f32, hipStream_t stream);
 // keep: what the step's token leaves in the cache, written by the launch that prepares the queries (NULL: it is there).
@@ -99,8 +100,11 @@ struct LayerOutParams {
     SliceNorm slice;                 // (input 3)
 };
 int32_t launch_layer_in(const LayerInParams& prm, int f32, hipStream_t stream);
-// The attention (rotation and cache write included) beside the decayed linear attention, one token each.
-int32_t launch_mixer_step(const ChunkAttentionParams& attention, const DecayAttentionParams& decay, int f32, hipStream_t stream);
+// The attention (rotation and cache write included) beside the decayed linear attention, and the delta rule, one token each; and
+// beside either one linear whose input is in memory as it is (or none).
+int32_t launch_mixer_step(const ChunkAttentionParams& attention, const DecayAttentionParams& decay, const DecLinearParams& beside, int f32,
+                          hipStream_t stream);
+int32_t launch_delta_step(const DeltaParams& delta, const DecLinearParams& beside, int f32, hipStream_t stream);
 int32_t launch_layer_out(const LayerOutParams& prm, int f32, hipStream_t stream);
 // the id of the highest of `vocab` scores (lowest among equals)
 int32_t launch_argmax(const float* scores, int vocab, int32_t* token, hipStream_t stream);

@@ -69,11 +69,16 @@ static int32_t delta_as(const DeltaParams& prm, hipStream_t stream) {
     return launch_status();
 }
 
-int32_t launch_general_delta(const DeltaParams& prm, hipStream_t stream) {
+int32_t check_general_delta(const DeltaParams& prm) {
     if (!prm.proj || !prm.w2 || !prm.w0 || !prm.a_bias || !prm.state || !prm.out) return QM_ERR_NULL;
     if (prm.rows < 0) return QM_ERR_ARGUMENT;
     if (prm.heads <= 0 || prm.heads > 65535 || prm.dim <= 0 || prm.dim > kDecMaxHead || prm.rank <= 0 || prm.rank > 1024) return QM_ERR_GEOMETRY;
-    if (prm.rows == 0) return QM_OK;
+    return QM_OK;
+}
+
+int32_t launch_general_delta(const DeltaParams& prm, hipStream_t stream) {
+    const int32_t rc = check_general_delta(prm);
+    if (rc != QM_OK || prm.rows == 0) return rc;
     if (prm.scratch && prm.rows >= kChunkedRows && delta_chunks_fit(prm)) return launch_delta_chunks(prm, stream);
     if (prm.dim <= 32) return delta_as<8>(prm, stream);
     if (prm.dim <= 64) return delta_as<16>(prm, stream);

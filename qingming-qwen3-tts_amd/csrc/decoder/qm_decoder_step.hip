@@ -4,6 +4,8 @@
 // its own, while the block's first weights are already on their way.
 //
 // Bound by HBM (each weight is read once) and, for narrow models, by the latency of the launches.
+#include <algorithm>
+
 #include "../qm_host.h"
 #include "qm_decoder_attention.h"
 #include "qm_decoder_dot.h"
@@ -71,9 +73,35 @@ __global__ __launch_bounds__(kDecThreads) void layer_out_kernel(LayerOutParams p
     dot_finish<T, 1, kOutRows>(group, d, piece, xs, 0, 1);
 }
 
+// A tile of a linear whose input is there already.
+template <class T>
+__device__ __forceinline__ void plain_tile(const DecLinearGroup& group, int tile, T* xs) {
+    const DotRows<kOutRows> d = dot_rows<kOutRows>(group, tile);
+    uint4 piece[kDotAhead][kOutRows];
+    dot_request<kOutRows>(d, group.k, piece);
+    constexpr int kVec = 16 / sizeof(T);
+    const T* x = static_cast<const T*>(group.x);
+    for (int c = threadIdx.x * kVec; c < group.k; c += kDecThreads * kVec)
+        *reinterpret_cast<uint4*>(xs + c) = *reinterpret_cast<const uint4*>(x + c);
+    __syncthreads();
+    dot_finish<T, 1, kOutRows>(group, d, piece, xs, 0, 1);
+}
+
+// A mixer is a chain of round trips on few CUs while the layer's down projection waits for nothing but the launch before: its tiles
+// are the blocks behind the mixer's (`beside`), and what follows the mixer has that much less to stream (one token of a parallel layer
+// of width 2048: mixer 9.4 and output linears 12.3 us one after the other).
+template <class T, int RD>
+__global__ __launch_bounds__(kDecThreads) void delta_step_kernel(DeltaParams delta, DecLinearParams beside) {
+    request_arguments(delta, beside);
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    const int slices = (delta.dim + kRecColumns - 1) / kRecColumns, block = static_cast<int>(blockIdx.x);
+    if (block < slices * delta.heads) general_delta_step<RD>(delta, block / slices, block % slices, lds);
+    else plain_tile<T>(beside.group[0], block - slices * delta.heads, reinterpret_cast<T*>(lds));
+}
+
 template <class T, int GQ, int VC>
-__global__ __launch_bounds__(kDecThreads) void mixer_step_kernel(ChunkAttentionParams attention, DecayAttentionParams decay) {
-    request_arguments(attention, decay);
+__global__ __launch_bounds__(kDecThreads) void mixer_step_kernel(ChunkAttentionParams attention, DecayAttentionParams decay, DecLinearParams beside) {
+    request_arguments(attention, decay, beside);
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int attention_blocks = attention.part.splits * attention.kv_heads;
     int block = static_cast<int>(blockIdx.x);
@@ -84,6 +112,10 @@ __global__ __launch_bounds__(kDecThreads) void mixer_step_kernel(ChunkAttentionP
     block -= attention_blocks;
     const int slices = (decay.vdim + kRecColumns - 1) / kRecColumns;
     const int head = block / slices, slice = block % slices;
+    if (head >= decay.heads) {
+        plain_tile<T>(beside.group[0], block - decay.heads * slices, reinterpret_cast<T*>(lds));
+        return;
+    }
     if (decay.dim <= 32) decay_attention_block<8>(decay, head, slice, lds);
     else if (decay.dim <= 64) decay_attention_block<16>(decay, head, slice, lds);
     else if (decay.dim <= 128) decay_attention_block<32>(decay, head, slice, lds);
@@ -209,31 +241,78 @@ int32_t launch_layer_out(const LayerOutParams& prm, int f32, hipStream_t stream)
     return f32 ? layer_out_as<float>(prm, stream) : layer_out_as<uint16_t>(prm, stream);
 }
 
+// The blocks of the linear beside a mixer, and its LDS; negative: an error.
+template <class T>
+static int32_t beside_blocks(const DecLinearParams& beside, size_t mixer_lds, size_t* lds) {
+    *lds = mixer_lds;
+    if (beside.groups == 0) return 0;
+    const DecLinearGroup& d = beside.group[0];
+    if (beside.groups != 1 || beside.rows != 1 || d.w_up) return QM_ERR_ARGUMENT;
+    if (!d.x || !d.w || !d.out32) return QM_ERR_NULL;
+    if (d.n <= 0 || d.n % 128 || d.k <= 0 || d.k % 128 || static_cast<int64_t>(d.k) * sizeof(T) > static_cast<int64_t>(kDotLdsMost)) return QM_ERR_GEOMETRY;
+    *lds = std::max(mixer_lds, d.k * sizeof(T));
+    return dot_tiles_of<kOutRows>(beside);
+}
+
 template <class T, int GQ, int VC>
-static int32_t mixer_step_as(const ChunkAttentionParams& a, const DecayAttentionParams& d, hipStream_t stream) {
+static int32_t mixer_step_as(const ChunkAttentionParams& a, const DecayAttentionParams& d, const DecLinearParams& beside, hipStream_t stream) {
     const int rd = d.dim <= 32 ? 8 : d.dim <= 64 ? 16 : d.dim <= 128 ? 32 : 64;
     const int attention = attention_lds_floats(GQ, a.k_stride, a.v_stride), decay = decay_lds_floats(rd);
-    const int blocks = a.part.splits * a.kv_heads + d.heads * ((d.vdim + kRecColumns - 1) / kRecColumns);
-    hipLaunchKernelGGL((mixer_step_kernel<T, GQ, VC>), dim3(blocks), dim3(kDecThreads), sizeof(float) * (attention > decay ? attention : decay), stream,
-                       a, d);
+    size_t lds = 0;
+    const int more = beside_blocks<T>(beside, sizeof(float) * (attention > decay ? attention : decay), &lds);
+    if (more < 0) return more;
+    static std::atomic<bool> raised[kMaxDevices];
+    const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(mixer_step_kernel<T, GQ, VC>), kDotLdsMost, raised);
+    if (rc != QM_OK) return rc;
+    const int blocks = a.part.splits * a.kv_heads + d.heads * ((d.vdim + kRecColumns - 1) / kRecColumns) + more;
+    hipLaunchKernelGGL((mixer_step_kernel<T, GQ, VC>), dim3(blocks), dim3(kDecThreads), lds, stream, a, d, beside);
     return launch_status();
 }
 template <class T, int GQ>
-static int32_t mixer_step_group(const ChunkAttentionParams& a, const DecayAttentionParams& d, hipStream_t stream) {
-    return a.v_stride <= 128 && a.k_stride <= 128 ? mixer_step_as<T, GQ, 1>(a, d, stream) : mixer_step_as<T, GQ, 2>(a, d, stream);
+static int32_t mixer_step_group(const ChunkAttentionParams& a, const DecayAttentionParams& d, const DecLinearParams& beside, hipStream_t stream) {
+    return a.v_stride <= 128 && a.k_stride <= 128 ? mixer_step_as<T, GQ, 1>(a, d, beside, stream) : mixer_step_as<T, GQ, 2>(a, d, beside, stream);
 }
 template <class T>
-static int32_t mixer_step(const ChunkAttentionParams& a, const DecayAttentionParams& d, hipStream_t stream) {
+static int32_t mixer_step(const ChunkAttentionParams& a, const DecayAttentionParams& d, const DecLinearParams& beside, hipStream_t stream) {
     const int group = a.heads / a.kv_heads;
-    return group == 1 ? mixer_step_group<T, 1>(a, d, stream) : group == 2 ? mixer_step_group<T, 2>(a, d, stream) : mixer_step_group<T, 4>(a, d, stream);
+    return group == 1 ? mixer_step_group<T, 1>(a, d, beside, stream)
+         : group == 2 ? mixer_step_group<T, 2>(a, d, beside, stream) : mixer_step_group<T, 4>(a, d, beside, stream);
 }
 
-int32_t launch_mixer_step(const ChunkAttentionParams& attention, const DecayAttentionParams& decay, int f32, hipStream_t stream) {
+int32_t launch_mixer_step(const ChunkAttentionParams& attention, const DecayAttentionParams& decay, const DecLinearParams& beside, int f32,
+                          hipStream_t stream) {
     int32_t rc = check_attention(attention);
     if (rc == QM_OK) rc = check_decay_attention(decay);
     if (rc != QM_OK) return rc;
     if (attention.rows != 1 || decay.rows != 1) return QM_ERR_ARGUMENT;
-    return f32 ? mixer_step<float>(attention, decay, stream) : mixer_step<uint16_t>(attention, decay, stream);
+    return f32 ? mixer_step<float>(attention, decay, beside, stream) : mixer_step<uint16_t>(attention, decay, beside, stream);
+}
+
+template <class T, int RD>
+static int32_t delta_step_as(const DeltaParams& delta, const DecLinearParams& beside, hipStream_t stream) {
+    size_t lds = 0;
+    const int more = beside_blocks<T>(beside, sizeof(float) * delta_step_lds_floats(RD, delta.rank), &lds);
+    if (more < 0) return more;
+    static std::atomic<bool> raised[kMaxDevices];
+    const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(delta_step_kernel<T, RD>), kDotLdsMost, raised);
+    if (rc != QM_OK) return rc;
+    const int blocks = (delta.dim + kRecColumns - 1) / kRecColumns * delta.heads + more;
+    hipLaunchKernelGGL((delta_step_kernel<T, RD>), dim3(blocks), dim3(kDecThreads), lds, stream, delta, beside);
+    return launch_status();
+}
+template <class T>
+static int32_t delta_step(const DeltaParams& delta, const DecLinearParams& beside, hipStream_t stream) {
+    if (delta.dim <= 32) return delta_step_as<T, 8>(delta, beside, stream);
+    if (delta.dim <= 64) return delta_step_as<T, 16>(delta, beside, stream);
+    if (delta.dim <= 128) return delta_step_as<T, 32>(delta, beside, stream);
+    return delta_step_as<T, 64>(delta, beside, stream);
+}
+
+int32_t launch_delta_step(const DeltaParams& delta, const DecLinearParams& beside, int f32, hipStream_t stream) {
+    const int32_t rc = check_general_delta(delta);
+    if (rc != QM_OK) return rc;
+    if (delta.rows != 1) return QM_ERR_ARGUMENT;
+    return f32 ? delta_step<float>(delta, beside, stream) : delta_step<uint16_t>(delta, beside, stream);
 }
 
 int32_t launch_argmax(const float* scores, int vocab, int32_t* token, hipStream_t stream) {

@@ -899,11 +899,17 @@ void enqueue_one(qm_decoder& d, int sequence) {
         next ^= 1;
         qm::LayerOutParams out = {};
         out.position_dev = step_words(d);
+        out.linears = linears_out(d, w, 1, pending);
+        qm::DecLinearParams beside = {};       // the down projection needs nothing of the mixer
+        if (w.config.ff && !sandwich(w)) {
+            beside.rows = beside.groups = 1;
+            beside.group[0] = out.linears.group[--out.linears.groups];
+        }
         switch (w.config.mixer) {
             case MixerKind::AttentionBesideDecay: {
                 qm_chunk_attention a = attention_of(d, w, d.states[i], sequence, 1, 0);
                 a.position_dev = step_words(d);
-                op_check(qm::launch_mixer_step(a, decay_of(d, w, d.states[i], sequence, 1, 0), d.f32, s), "attention beside decayed attention");
+                op_check(qm::launch_mixer_step(a, decay_of(d, w, d.states[i], sequence, 1, 0), beside, d.f32, s), "attention beside decayed attention");
                 out.part = a.part;
                 out.chunk = a.chunk;
                 out.input[0] = 1;
@@ -911,7 +917,7 @@ void enqueue_one(qm_decoder& d, int sequence) {
                 break;
             }
             case MixerKind::GeneralDelta:
-                op_check(qm::launch_general_delta(delta_of(d, w, d.states[i], sequence, 1), s), "generalized delta rule");
+                op_check(qm::launch_delta_step(delta_of(d, w, d.states[i], sequence, 1), beside, d.f32, s), "generalized delta rule");
                 out.input[0] = 2;
                 break;
             case MixerKind::Retention: {
@@ -936,7 +942,6 @@ void enqueue_one(qm_decoder& d, int sequence) {
                 break;
             }
         }
-        out.linears = linears_out(d, w, 1, pending);
         if (w.config.mixer != MixerKind::LatentAttention) out.gated = gated_of(d, w);
         op_check(qm::launch_layer_out(out, d.f32, s), "output projections");
         if (sandwich(w) && w.config.ff) {
