@@ -23,7 +23,7 @@ namespace qm_engine {
 struct Layer {
     Param input_norm, q_weight, q_bias, k_weight, k_bias, v_weight, v_bias, q_norm, k_norm, o_weight, o_bias, post_norm,
         gate_weight, up_weight, down_weight;
-    DeviceBuffer key_cache, value_cache;
+    uint16_t *key_cache = nullptr, *value_cache = nullptr;      // [kv_heads][max_cache][128] in the engine's `caches`
 };
 
 }  // namespace qm_engine
@@ -38,6 +38,7 @@ struct qm_safefile {
 
 struct qm_talker {
     std::vector<qm_engine::Layer> layers;
+    qm_engine::DeviceBuffer caches;          // every layer's, one behind the other: a request's reset is one fill
     qm_engine::Param final_norm;
     int q_heads = 0, kv_heads = 0, q_dim = 0, kv_dim = 0, intermediate = 0, max_cache = 0, prefill_length = 0;
     hipStream_t stream = nullptr;
@@ -151,9 +152,12 @@ static std::unique_ptr<qm_talker> create_talker(const std::string& model_dir, in
 
     engine->max_cache = max_cache;
     const size_t cache_bytes = static_cast<size_t>(engine->kv_heads) * max_cache * kHeadDim * 2;
+    engine->caches = DeviceBuffer(2 * cache_bytes * engine->layers.size());
+    uint16_t* cache = engine->caches.u16();
     for (Layer& w : engine->layers) {
-        w.key_cache = DeviceBuffer(cache_bytes);
-        w.value_cache = DeviceBuffer(cache_bytes);
+        w.key_cache = cache;
+        w.value_cache = cache + cache_bytes / 2;
+        cache += cache_bytes;
     }
     auto vec = [](int n) { return DeviceBuffer(static_cast<size_t>(n) * 2); };
     engine->hidden_a = vec(kHidden); engine->hidden_b = vec(kHidden);
@@ -180,17 +184,14 @@ static std::unique_ptr<qm_talker> create_talker(const std::string& model_dir, in
 
 static void reset_talker(qm_talker& e, int prefill_length) {
     if (prefill_length < 0 || prefill_length > e.max_cache) throw ApiError(QM_ERR_SLOT_RANGE, "prefill length exceeds the cache");
-    for (Layer& w : e.layers) {
-        hip_check(hipMemsetAsync(w.key_cache.raw(), 0, w.key_cache.bytes(), e.stream), "key cache reset");
-        hip_check(hipMemsetAsync(w.value_cache.raw(), 0, w.value_cache.bytes(), e.stream), "value cache reset");
-    }
+    hip_check(hipMemsetAsync(e.caches.raw(), 0, e.caches.bytes(), e.stream), "cache reset");
     e.prefill_length = prefill_length;
 }
 
 static qm_kv_cache flat_cache_of(const qm_talker& e, const Layer& w) {
     qm_kv_cache cache = {};
-    cache.k_pool = w.key_cache.u16();
-    cache.v_pool = w.value_cache.u16();
+    cache.k_pool = w.key_cache;
+    cache.v_pool = w.value_cache;
     cache.stride_page = 0;
     cache.stride_head = static_cast<int64_t>(e.max_cache) * kHeadDim;
     cache.stride_token = kHeadDim;
@@ -502,8 +503,8 @@ extern "C" int32_t qm_talker_reset(qm_talker* engine, int32_t prefill_length) {
 extern "C" int32_t qm_talker_cache(qm_talker* engine, int32_t layer, uint16_t** key_cache, uint16_t** value_cache) {
     if (!engine || !key_cache || !value_cache) return QM_ERR_NULL;
     if (layer < 0 || layer >= static_cast<int32_t>(engine->layers.size())) return QM_ERR_ARGUMENT;
-    *key_cache = engine->layers[static_cast<size_t>(layer)].key_cache.u16();
-    *value_cache = engine->layers[static_cast<size_t>(layer)].value_cache.u16();
+    *key_cache = engine->layers[static_cast<size_t>(layer)].key_cache;
+    *value_cache = engine->layers[static_cast<size_t>(layer)].value_cache;
     return QM_OK;
 }
 
