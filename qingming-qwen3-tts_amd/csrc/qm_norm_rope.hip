@@ -89,27 +89,51 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(
     out[base + lane + 64] = r.hi;
 }
 
-// The prompt pass's query and key heads in one grid: item = row * (q_heads + kv_heads) + head, the first q_heads of a
-// row its query heads; every head as norm_rope_rows_kernel forms it.
+// The prompt pass's query and key heads in one grid, a block per row, the first q_heads of a row's heads its query heads; every head as
+// norm_rope_rows_kernel forms it.  A wave takes kRopeHeads heads at a time: their values, the row's cosines and sines and the weights
+// are asked for at once (a wave per head was three rounds of waves that each waited for memory: 1000 rows of 24 heads 9.2 -> 7.7 us).
+constexpr int kRopeHeads = 6;
 __global__ __launch_bounds__(256) void qk_norm_rope_rows_kernel(
     const uint16_t* __restrict__ q_in, const uint16_t* __restrict__ k_in, const uint16_t* __restrict__ q_norm_w,
     const uint16_t* __restrict__ k_norm_w, const uint16_t* __restrict__ cos_rows, const uint16_t* __restrict__ sin_rows,
-    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out, int64_t total_heads, int q_heads, int kv_heads, float epsilon) {
-    request_arguments(q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, total_heads, q_heads, kv_heads, epsilon);
-    const int lane = threadIdx.x & 63;
-    const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (item >= total_heads) return;
-    const int per_row = q_heads + kv_heads;
-    const int64_t row = item / per_row;
-    const int head = static_cast<int>(item - row * per_row);
-    const bool is_query = head < q_heads;
-    const uint16_t* in = is_query ? q_in : k_in;
-    uint16_t* out = is_query ? q_out : k_out;
-    const int64_t base = is_query ? (row * q_heads + head) * kDim : (row * kv_heads + (head - q_heads)) * kDim;
-    const HeadPair r = norm_rope_head(in[base + lane], in[base + lane + 64], is_query ? q_norm_w : k_norm_w,
-                                      cos_rows + row * kDim, sin_rows + row * kDim, epsilon, lane);
-    out[base + lane] = r.lo;
-    out[base + lane + 64] = r.hi;
+    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out, int q_heads, int kv_heads, float epsilon) {
+    request_arguments(q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, q_heads, kv_heads, epsilon);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t row = blockIdx.x;
+    const int heads = q_heads + kv_heads;
+    const uint16_t c0 = cos_rows[row * kDim + lane], c1 = cos_rows[row * kDim + lane + 64];
+    const uint16_t s0 = sin_rows[row * kDim + lane], s1 = sin_rows[row * kDim + lane + 64];
+    uint16_t gq[2] = {0, 0}, gk[2] = {0, 0};
+    if (q_norm_w) {
+        gq[0] = q_norm_w[lane];
+        gq[1] = q_norm_w[lane + 64];
+    }
+    if (k_norm_w) {
+        gk[0] = k_norm_w[lane];
+        gk[1] = k_norm_w[lane + 64];
+    }
+    for (int first = wave * kRopeHeads; first < heads; first += 4 * kRopeHeads) {
+        uint16_t x[kRopeHeads][2];
+        auto place = [&](int head) { return head < q_heads ? (row * q_heads + head) * kDim : (row * kv_heads + (head - q_heads)) * kDim; };
+#pragma unroll
+        for (int i = 0; i < kRopeHeads; ++i) {                     // (past the last head: it again, not stored)
+            const int head = min(first + i, heads - 1);
+            const uint16_t* in = (head < q_heads ? q_in : k_in) + place(head);
+            x[i][0] = in[lane];
+            x[i][1] = in[lane + 64];
+        }
+#pragma unroll
+        for (int i = 0; i < kRopeHeads; ++i) {
+            const int head = first + i;
+            if (head >= heads) break;
+            const bool is_query = head < q_heads;
+            const HeadPair r = norm_rope_head_values(x[i][0], x[i][1], (is_query ? q_norm_w : k_norm_w) != nullptr, is_query ? gq[0] : gk[0],
+                                                     is_query ? gq[1] : gk[1], c0, c1, s0, s1, epsilon);
+            uint16_t* out = (is_query ? q_out : k_out) + place(head);
+            out[lane] = r.lo;
+            out[lane + 64] = r.hi;
+        }
+    }
 }
 
 // [rows][kv_heads][128] -> pages; one thread moves 16 bytes of K and 16 bytes of V.
@@ -211,12 +235,9 @@ extern "C" int32_t qm_qk_norm_rope_rows(
     if (!q_in || !k_in || !cos_rows || !sin_rows || !q_out || !k_out) return QM_ERR_NULL;
     if (rows < 0 || q_heads <= 0 || kv_heads <= 0) return QM_ERR_ARGUMENT;
     if (rows == 0) return QM_OK;
-    const int64_t total = static_cast<int64_t>(rows) * (static_cast<int64_t>(q_heads) + kv_heads);
-    const int64_t blocks = (total + 3) / 4;
-    if (blocks > 0x7fffffffLL) return QM_ERR_ARGUMENT;
-    hipLaunchKernelGGL(qm::qk_norm_rope_rows_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
-                       static_cast<hipStream_t>(hip_stream),
-                       q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, total, q_heads, kv_heads, epsilon);
+    if ((static_cast<int64_t>(rows) * (static_cast<int64_t>(q_heads) + kv_heads) + 3) / 4 > 0x7fffffffLL) return QM_ERR_ARGUMENT;
+    hipLaunchKernelGGL(qm::qk_norm_rope_rows_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, static_cast<hipStream_t>(hip_stream),
+                       q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, q_heads, kv_heads, epsilon);
     return qm::launch_status();
 }
 

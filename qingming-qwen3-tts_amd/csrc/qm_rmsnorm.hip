@@ -34,6 +34,29 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_rows_kernel(const uint16
     }
 }
 
+// The same for rows of 256 N columns: a thread's values stay in registers and its weights are asked for with them, so that a row costs
+// one round trip to memory instead of two behind one another (1000 rows of 2048: 7.4 -> 5.2 us; one row 6.5 -> 4.1).
+template <int N>
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_held_rows_kernel(const uint16_t* input, const uint16_t* weight, uint16_t* output,
+                                                                         float epsilon) {
+    request_arguments(input, weight, output, epsilon);
+    __shared__ float sh_waves[8];
+    __shared__ float sh_total;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * (N * kNormThreads) + threadIdx.x;
+    uint16_t x[N], w[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = input[base + i * kNormThreads];
+#pragma unroll
+    for (int i = 0; i < N; ++i) w[i] = weight[threadIdx.x + i * kNormThreads];
+    float sum_squares = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) sum_squares = fmaf(bf2f(x[i]), bf2f(x[i]), sum_squares);
+    const float total = block_sum_256_like_reference(sum_squares, sh_waves, &sh_total);
+    const float inverse_rms = 1.0f / sqrtf(total / static_cast<float>(N * kNormThreads) + epsilon);
+#pragma unroll
+    for (int i = 0; i < N; ++i) output[base + i * kNormThreads] = f2bf(round_bf16(bf2f(x[i]) * inverse_rms) * bf2f(w[i]));
+}
+
 // talker_add_postnorm_fused_kernel (R17:16205-16286): one block.
 __global__ __launch_bounds__(kNormThreads) void add_postnorm_kernel(const uint16_t* hidden, const uint16_t* attention,
                                                                     const uint16_t* norm_weight, uint16_t* residual,
@@ -65,6 +88,16 @@ extern "C" int32_t qm_rmsnorm_rows(const uint16_t* input, const uint16_t* weight
     if (!input || !weight || !output) return QM_ERR_NULL;
     if (rows < 0 || dimension <= 0) return QM_ERR_ARGUMENT;
     if (rows == 0) return QM_OK;
+    const dim3 grid(static_cast<unsigned>(rows)), block(kNormThreads);
+    hipStream_t stream = static_cast<hipStream_t>(hip_stream);
+    if (dimension == 8 * kNormThreads) {
+        hipLaunchKernelGGL(rmsnorm_held_rows_kernel<8>, grid, block, 0, stream, input, weight, output, epsilon);
+        return launch_status();
+    }
+    if (dimension == 4 * kNormThreads) {
+        hipLaunchKernelGGL(rmsnorm_held_rows_kernel<4>, grid, block, 0, stream, input, weight, output, epsilon);
+        return launch_status();
+    }
     hipLaunchKernelGGL(rmsnorm_rows_kernel, dim3(static_cast<unsigned>(rows)), dim3(kNormThreads), 0,
                        static_cast<hipStream_t>(hip_stream), input, weight, output, dimension, epsilon);
     return launch_status();
