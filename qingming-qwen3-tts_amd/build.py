@@ -39,7 +39,7 @@ def build(verbose=True, jobs=4):
 # The decoder language models' library stands alone: its kernels, the kernels it shares with libqm_attn.so (their objects)
 # and its engine, so that a first run of such a model compiles no other model's kernels.
 DECODER_SOURCES = ["decoder/qm_decoder_ops.hip", "decoder/qm_decoder_norm.hip", "decoder/qm_decoder_linear.hip", "decoder/qm_decoder_linear_f32.hip",
-                   "decoder/qm_decoder_attention.hip", "decoder/qm_decoder_attention_mfma.hip",
+                   "decoder/qm_decoder_attention.hip", "decoder/qm_decoder_attention_mfma.hip", "decoder/qm_decoder_attention_f32.hip",
                    "decoder/qm_decoder_recurrent.hip", "decoder/qm_decoder_decay_chunks.hip", "decoder/qm_decoder_delta_chunks.hip",
                    "decoder/qm_decoder_latent.hip", "decoder/qm_decoder_latent_mfma.hip", "decoder/qm_decoder_experts.hip",
                    "decoder/qm_decoder_step.hip"]

@@ -2,8 +2,9 @@
 // floor(. / chunk)), grouped query heads, over a ring cache of keys and values, for gfx950.
 //
 // Chunks count from position 0 of the sequence, so a query needs at most `chunk` keys, all of them in the cache however the
-// prompt was cut.  Two kernels: few rows (decode) deal a chunk's keys to several blocks per key/value head and combine the
-// partial results; many bf16 rows take the matrix-core kernel of qm_decoder_attention_mfma.hip.
+// prompt was cut.  Three kernels: few rows (decode) deal a chunk's keys to several blocks per key/value head and combine the
+// partial results; many bf16 rows take the matrix-core kernel of qm_decoder_attention_mfma.hip, many fp32 rows that of
+// qm_decoder_attention_f32.hip.
 #include "../qm_host.h"
 #include "qm_decoder_attention.h"
 
@@ -133,6 +134,7 @@ int32_t launch_chunk_attention(const ChunkAttentionParams& prm, int f32, hipStre
     if (rc != QM_OK) return rc;
     // (positions that only the device knows belong to one-token steps)
     if (!f32 && prm.rows >= kAttentionMatrixRows && !prm.position_dev && !(prm.options & QM_ATTENTION_ROWS)) return launch_chunk_attention_mfma(prm, stream);
+    if (f32 && attention_f32_pays(prm) && !prm.position_dev && !(prm.options & QM_ATTENTION_ROWS)) return launch_chunk_attention_f32(prm, stream);
     return f32 ? attention_rows<float>(prm, stream) : attention_rows<uint16_t>(prm, stream);
 }
 

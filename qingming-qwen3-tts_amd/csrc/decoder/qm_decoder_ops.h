@@ -57,6 +57,8 @@ int32_t launch_split_linears(const DecLinearParams& prm, hipStream_t stream);   
 // Rotation and cache write, then the attention.
 int32_t launch_chunk_attention(const ChunkAttentionParams& prm, int f32, hipStream_t stream);
 int32_t launch_chunk_attention_mfma(const ChunkAttentionParams& prm, hipStream_t stream);
+bool attention_f32_pays(const ChunkAttentionParams& prm);                         // whether many fp32 rows go to the matrix cores
+int32_t launch_chunk_attention_f32(const ChunkAttentionParams& prm, hipStream_t stream);
 int32_t launch_decay_attention(const DecayAttentionParams& prm, hipStream_t stream);
 // Floats of scratch with which a pass of `rows` tokens is computed in chunks (0: it is not).
 int64_t decay_scratch_floats(int rows, int heads, int dim, int vdim);

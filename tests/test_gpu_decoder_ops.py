@@ -289,6 +289,31 @@ def test_two_attention_kernels_agree(decoder, dev):
     assert np.abs(a - b).max() <= 2e-2 * np.abs(b).max()
 
 
+@pytest.mark.parametrize("shape", [(16, 8, 64, 64, 512, 64), (5, 1, 36, 20, 64, 10), (3, 3, 24, 40, 37, 24), (8, 2, 128, 128, 256, 128), (4, 2, 65, 6, 19, 2)])
+def test_fp32_attention_of_many_rows_against_the_row_kernel(decoder, dev, shape):
+    """Both kernels of fp32 rows stand as close to 64 bits, around the 16 query rows of a block, the 16 keys of a step and
+    the end of a chunk; and a row does not know the values of positions that it does not see, whatever they are."""
+    worst = {False: [], True: []}
+    for rows in (16, 17, 31, 33, 65, 130, 230):
+        case = AttentionCase(shape, rows, seed=rows)
+        want = case.want()
+        for rows_only in (False, True):
+            got = case.run(decoder, dev, True, [rows], rows_only=rows_only)
+            close(got, want, True, tol32=2e-5)
+            worst[rows_only].append(np.sqrt(np.mean((got - want) ** 2)))
+    # (the root mean square over some thousand outputs: 1.5 leaves room for the draw alone)
+    assert np.mean(worst[False]) <= 1.5 * np.mean(worst[True])
+    whole = AttentionCase(shape, 100, seed=3)
+    plain_result = whole.run(decoder, dev, True, [100])
+    for at, what in ((99, np.inf), (50, np.nan), (17, -np.inf), (18, np.inf)):
+        broken = AttentionCase(shape, 100, seed=3)
+        broken.proj[at, broken.v_at:broken.v_at + broken.vdim] = what
+        got = broken.run(decoder, dev, True, [100])
+        sees = np.array([at <= i < at // whole.chunk * whole.chunk + whole.chunk for i in range(100)])
+        assert np.abs(got[~sees] - plain_result[~sees]).max(initial=0.0) <= 4e-6 * np.abs(plain_result).max()
+        assert not np.isfinite(got[at]).all()
+
+
 @pytest.mark.parametrize("chunked", [False, True])
 @pytest.mark.parametrize("heads,dim,vdim", [(3, 16, 24), (2, 20, 36), (1, 48, 16), (4, 64, 128), (2, 132, 200), (1, 256, 256), (2, 7, 9)])
 def test_decay_attention(decoder, dev, chunked, heads, dim, vdim):
