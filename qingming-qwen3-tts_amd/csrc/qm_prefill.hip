@@ -110,7 +110,11 @@ struct PrefillParams {
     int chunk_paged;
 };
 
-constexpr int kChunkRecordFloats = 66 * kPfThreads;   // per thread: 64 of O (unnormalised), the reference maximum, the sum
+// A run's record, value by value of the threads: 16 times four of O (unnormalised), then reference maximum and sum.  (The
+// workspace is aligned for floats.)
+constexpr int kChunkRecordFloats = 66 * kPfThreads;
+typedef float record4_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef float record2_t __attribute__((ext_vector_type(2), aligned(4)));
 
 struct PfStage {
     uint16_t k[kBN * kKS];
@@ -666,14 +670,13 @@ __device__ __forceinline__ void prefill_body(const PrefillParams& prm, const qm_
     if (CHUNK && !PRECISE && to_record) {
         // One run of several: the unnormalised O, the reference maximum and the sum, as register images (thread t of
         // the merge kernel takes what thread t leaves here).
-        float* rec = prm.chunk_records
-                   + ((static_cast<int64_t>(pair) * prm.n_qtiles + qt) * prm.chunk_parts + part) * kChunkRecordFloats + tid;
+        float* rec = prm.chunk_records + ((static_cast<int64_t>(pair) * prm.n_qtiles + qt) * prm.chunk_parts + part) * kChunkRecordFloats;
 #pragma unroll
         for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) rec[(16 * dt + r) * kPfThreads] = o[dt][r];
-        rec[64 * kPfThreads] = m_run;
-        rec[65 * kPfThreads] = l_tot;
+            for (int rq = 0; rq < 4; ++rq)
+                reinterpret_cast<record4_t*>(rec)[(4 * dt + rq) * kPfThreads + tid] = record4_t{o[dt][4 * rq], o[dt][4 * rq + 1], o[dt][4 * rq + 2], o[dt][4 * rq + 3]};
+        reinterpret_cast<record2_t*>(rec + 64 * kPfThreads)[tid] = record2_t{m_run, l_tot};
         return;
     }
 
@@ -745,17 +748,20 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_chunk_kernel(PrefillPar
 }
 
 // Combines the runs of the query tiles that prefill_chunk_kernel split: sum over runs of O * w over sum of l * w,
-// w = exp(maximum of the run - largest maximum), in run order.  grid = pairs * n_qtiles * 8, 256 threads: thread t
+// w = exp(maximum of the run - largest maximum), in run order.  grid = n_qtiles * 8 * pairs, 256 threads: thread t
 // holds what thread t of a run's block held (column = (row % 16, head) of a wave), and a block takes eight of the
-// thread's 64 values, all runs' loads in flight at once.
+// thread's 64 values, all runs' loads in flight at once (MOST: no query tile has more runs).  Pairs are dealt to the dies as by
+// prefill_chunk_kernel: the records are then in the L2 of the die that wrote them.  Bound: the records' bytes and two trips to
+// memory (256 rows at 2048, eight runs, 17 MB: 5.3 -> 4.6 us, of them all 21.0 -> 20.3, against single floats and sixteen
+// runs' loads whatever there are; sixteen slices instead of eight change nothing).
 constexpr int kChunkMaxRuns = 16;
 constexpr int kChunkMergeSlices = 8;
+template <int MOST>
 __global__ __launch_bounds__(kPfThreads) void prefill_chunk_merge_kernel(PrefillParams prm, int round_scores, int gqa_group) {
     request_arguments(prm, round_scores, gqa_group);
-    const int slice = blockIdx.x % kChunkMergeSlices;
-    const int item = blockIdx.x / kChunkMergeSlices;
-    const int pair = item % (prm.batch * prm.kv_heads);
-    const int qt = item / (prm.batch * prm.kv_heads);
+    const int pairs = prm.batch * prm.kv_heads;
+    const int pair = blockIdx.x % pairs, item = blockIdx.x / pairs;
+    const int slice = item % kChunkMergeSlices, qt = item / kChunkMergeSlices;
     const int wave_rows = 32 / gqa_group, block_rows = 4 * wave_rows;
     const int q0 = qt * block_rows;
     const int last_tile = min(q0 + prm.cache_before + block_rows - 1, prm.key_count - 1) / kBN;
@@ -764,41 +770,43 @@ __global__ __launch_bounds__(kPfThreads) void prefill_chunk_merge_kernel(Prefill
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63, col = lane & 31, grp = lane >> 5;
     const float coef = round_scores ? kLog2e : prm.scale * kLog2e;
-    const float* rec = prm.chunk_records + (static_cast<int64_t>(pair) * prm.n_qtiles + qt) * prm.chunk_parts * kChunkRecordFloats + tid;
-    float mv[kChunkMaxRuns], lv[kChunkMaxRuns], ov[kChunkMaxRuns][8];
+    const float* rec = prm.chunk_records + (static_cast<int64_t>(pair) * prm.n_qtiles + qt) * prm.chunk_parts * kChunkRecordFloats;
+    record2_t ml[MOST];
+    constexpr int kQuads = 16 / kChunkMergeSlices;
+    record4_t ov[MOST][kQuads];
 #pragma unroll
-    for (int p = 0; p < kChunkMaxRuns; ++p) {
+    for (int p = 0; p < MOST; ++p) {
         const float* r = rec + static_cast<int64_t>(min(p, runs - 1)) * kChunkRecordFloats;
-        mv[p] = r[64 * kPfThreads];
-        lv[p] = r[65 * kPfThreads];
+        ml[p] = reinterpret_cast<const record2_t*>(r + 64 * kPfThreads)[tid];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) ov[p][i] = r[(8 * slice + i) * kPfThreads];
+        for (int h = 0; h < kQuads; ++h) ov[p][h] = reinterpret_cast<const record4_t*>(r)[(kQuads * slice + h) * kPfThreads + tid];
     }
     float m_all = -INFINITY;
 #pragma unroll
-    for (int p = 0; p < kChunkMaxRuns; ++p) m_all = fmaxf(m_all, mv[p]);
+    for (int p = 0; p < MOST; ++p) m_all = fmaxf(m_all, ml[p][0]);
     const float m_ref = m_all == -INFINITY ? 0.0f : m_all;
-    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    float acc[4 * kQuads] = {};
     float l = 0.0f;
 #pragma unroll
-    for (int p = 0; p < kChunkMaxRuns; ++p) {
-        const float w = p < runs ? fast_exp2((mv[p] - m_ref) * coef) : 0.0f;
-        l = fmaf(lv[p], w, l);
+    for (int p = 0; p < MOST; ++p) {
+        const float w = p < runs ? fast_exp2((ml[p][0] - m_ref) * coef) : 0.0f;
+        l = fmaf(ml[p][1], w, l);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] = fmaf(ov[p][i], w, acc[i]);
+        for (int i = 0; i < 4 * kQuads; ++i) acc[i] = fmaf(ov[p][i / 4][i % 4], w, acc[i]);
     }
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
     const int b = pair / prm.kv_heads, kvh = pair % prm.kv_heads;
     const int row = q0 + wave_rows * wave + col % wave_rows;
     if (row >= prm.seq) return;
     uint16_t* out = prm.out + ((static_cast<int64_t>(b) * prm.seq + row) * (gqa_group * prm.kv_heads) + gqa_group * kvh + col / wave_rows) * kDim;
-    // value 16 dt + 4 rq + j of a thread is dim 32 dt + 8 rq + 4 grp + j: this slice is dt = slice / 2, rq = 2 (slice % 2), + 1
+    // quad 4 dt + rq of a thread is dims 32 dt + 8 rq + 4 grp ..
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kQuads; ++h) {
+        const int quad = kQuads * slice + h;
         uint2 packed;
         packed.x = pack_bf16_pair(acc[4 * h + 0] * inv, acc[4 * h + 1] * inv);
         packed.y = pack_bf16_pair(acc[4 * h + 2] * inv, acc[4 * h + 3] * inv);
-        *reinterpret_cast<uint2*>(out + 32 * (slice >> 1) + 8 * (2 * (slice & 1) + h) + 4 * grp) = packed;
+        *reinterpret_cast<uint2*>(out + 8 * quad + 4 * grp) = packed;
     }
 }
 
@@ -2025,8 +2033,8 @@ static int32_t launch_chunk_kernels(const PrefillParams& prm, const qm_kv_cache&
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(pairs * prm.n_qtiles * prm.chunk_parts)), dim3(kPfThreads), smem, s, prm, cache);
     int32_t rc = launch_status();
     if (rc == QM_OK && prm.chunk_parts > 1) {
-        hipLaunchKernelGGL(prefill_chunk_merge_kernel, dim3(static_cast<unsigned>(pairs * prm.n_qtiles * kChunkMergeSlices)), dim3(kPfThreads), 0, s,
-                           prm, round_scores ? 1 : 0, G);
+        const auto merge = prm.chunk_parts <= 8 ? prefill_chunk_merge_kernel<8> : prefill_chunk_merge_kernel<kChunkMaxRuns>;
+        hipLaunchKernelGGL(merge, dim3(static_cast<unsigned>(pairs * prm.n_qtiles * kChunkMergeSlices)), dim3(kPfThreads), 0, s, prm, round_scores ? 1 : 0, G);
         rc = launch_status();
     }
     return rc;
