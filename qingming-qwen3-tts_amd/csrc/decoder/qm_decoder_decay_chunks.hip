@@ -6,13 +6,26 @@
 // contributions into the state before each chunk (element by element, so the whole state is walked in parallel); every
 // chunk's outputs, all at once.  All products are fp32 on the matrix cores, powers of d have non-negative exponents only.
 // Bound: the bytes of the states between the launches and the fp32 matrix cores, whichever is longer.
+#include <algorithm>
+
 #include "../qm_host.h"
 #include "qm_decoder_mfma32.h"
 
 namespace qm {
 
-constexpr int kDecaySlice = 64;                // value channels staged at once
-constexpr int kDecayVStride = kDecaySlice + 4;
+// Blocks of W waves (4 or 8) take 16 W value channels.
+template <int W>
+struct DecayBlock {
+    static constexpr int kThreads = 64 * W, kSlice = 16 * W, kVStride = kSlice + 4;
+    static constexpr int kRows = kThreads / 16;                    // rows staged at once
+    static constexpr int kPasses = kDecayChunk / kRows;
+};
+constexpr int kDecayPStride = kDecayChunk + 4;
+// More blocks of four waves than CUs share CUs, and every one stages its head's queries and keys and makes their scores anew: then
+// blocks of eight waves, half as many.  Outputs and states (us, four waves / eight): 8 heads of 128 by 256, 777 rows 25.6 / 19.6 and
+// 15.6 / 14.1; 16 heads of 64 by 128, 1024 rows 18.5 / 15.0 and 11.4 / 10.7.  Below, four waves spread over twice the CUs.
+constexpr int kDecayWide = 256;
+constexpr int kScoreTiles = 10;                // 16 x 16 tiles of a chunk's scores on and below the diagonal
 
 // Rotation of every row's q and k in place, k scaled: a block per row, a pair's angle once for all heads.
 __global__ __launch_bounds__(kDecThreads) void decay_rotate_kernel(DecayAttentionParams prm) {
@@ -42,14 +55,15 @@ __global__ __launch_bounds__(kDecThreads) void decay_rotate_kernel(DecayAttentio
 }
 
 // Rows [t0, t0 + 64) of a head's q, k or v columns into LDS, through silu unless they were rotated (zeros past the rows or
-// the head), times factor(j): sixteen threads take 64 columns of a row, four each.  request_rows asks for columns c4 .. c4 + 3
-// of the thread's four rows, put_rows stores them.
-__device__ __forceinline__ void request_rows(const DecayAttentionParams& prm, int t0, int column, int columns, int c, float4 (&x)[4]) {
+// the head), times factor(j): sixteen threads take 64 columns of a row, four each.  request_rows asks for columns c .. c + 3
+// of the thread's rows, put_rows stores them.
+template <int W>
+__device__ __forceinline__ void request_rows(const DecayAttentionParams& prm, int t0, int column, int columns, int c, float4 (&x)[DecayBlock<W>::kPasses]) {
     const int row = threadIdx.x >> 4;
     const bool vectors = ((column | columns | prm.ld_proj) & 3) == 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {              // (rows past the last repeat it, with factor zero: no branch around a load)
-        const float* p = prm.proj + min(t0 + row + 16 * i, prm.rows - 1) * prm.ld_proj + column;
+    for (int i = 0; i < DecayBlock<W>::kPasses; ++i) {             // (rows past the last repeat it, with factor zero: no branch around a load)
+        const float* p = prm.proj + min(t0 + row + DecayBlock<W>::kRows * i, prm.rows - 1) * prm.ld_proj + column;
         if (vectors) {
             x[i] = load4_if(c < columns, p, c >> 2);
         } else {
@@ -63,51 +77,53 @@ __device__ __forceinline__ void request_rows(const DecayAttentionParams& prm, in
         }
     }
 }
-template <class F>
-__device__ __forceinline__ void put_rows(const DecayAttentionParams& prm, float* to, int stride, int t0, int c, float4 (&x)[4], F factor) {
+template <int W, class F>
+__device__ __forceinline__ void put_rows(const DecayAttentionParams& prm, float* to, int stride, int t0, int c, float4 (&x)[DecayBlock<W>::kPasses], F factor) {
     const int row = threadIdx.x >> 4;
     const bool silu = !(prm.options & QM_DECAY_ROTARY);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int j = row + 16 * i;
+    for (int i = 0; i < DecayBlock<W>::kPasses; ++i) {
+        const int j = row + DecayBlock<W>::kRows * i;
         const float f = t0 + j < prm.rows ? factor(j) : 0.0f;
         if (silu) x[i] = make_float4(silu_f32(x[i].x), silu_f32(x[i].y), silu_f32(x[i].z), silu_f32(x[i].w));
         *reinterpret_cast<float4*>(to + j * stride + c) = make_float4(x[i].x * f, x[i].y * f, x[i].z * f, x[i].w * f);
     }
 }
 // `padded`: a multiple of 16
-template <class F>
+template <int W, class F>
 __device__ __forceinline__ void stage_rows(const DecayAttentionParams& prm, float* to, int stride, int t0, int column, int columns, int padded, F factor) {
 #pragma unroll 2
     for (int c = (threadIdx.x & 15) * 4; c < padded; c += 64) {
-        float4 x[4];
-        request_rows(prm, t0, column, columns, c, x);
-        put_rows(prm, to, stride, t0, c, x, factor);
+        float4 x[DecayBlock<W>::kPasses];
+        request_rows<W>(prm, t0, column, columns, c, x);
+        put_rows<W>(prm, to, stride, t0, c, x, factor);
     }
 }
 
-__global__ __launch_bounds__(kDecThreads) void decay_chunk_state_kernel(DecayAttentionParams prm) {
+template <int W>
+__global__ __launch_bounds__(64 * W) void decay_chunk_state_kernel(DecayAttentionParams prm) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, l16 = lane & 15;
-    const int head = static_cast<int>(blockIdx.x), chunk = static_cast<int>(blockIdx.y), e0 = static_cast<int>(blockIdx.z) * kDecaySlice;
+    const int head = static_cast<int>(blockIdx.x), chunk = static_cast<int>(blockIdx.y), e0 = static_cast<int>(blockIdx.z) * DecayBlock<W>::kSlice;
     const int t0 = chunk * kDecayChunk, tokens = min(kDecayChunk, prm.rows - t0);
+    constexpr int kVStride = DecayBlock<W>::kVStride;
     const int dp = mfma32_pad(prm.dim), stride = mfma32_stride(prm.dim);
     const float* powers = prm.powers + head * kDecayPowers;
     float* ks = lds;                           // [64][stride]
-    float* vs = ks + kDecayChunk * stride;     // [64][kDecayVStride]
-    stage_rows(prm, ks, stride, t0, prm.k_column + head * prm.dim, prm.dim, dp, [&](int j) { return powers[tokens - 1 - j]; });
-    stage_rows(prm, vs, kDecayVStride, t0, prm.v_column + head * prm.vdim + e0, prm.vdim - e0, kDecaySlice, [](int) { return 1.0f; });
+    float* vs = ks + kDecayChunk * stride;     // [64][kVStride]
+    stage_rows<W>(prm, ks, stride, t0, prm.k_column + head * prm.dim, prm.dim, dp, [&](int j) { return powers[tokens - 1 - j]; });
+    stage_rows<W>(prm, vs, kVStride, t0, prm.v_column + head * prm.vdim + e0, prm.vdim - e0, DecayBlock<W>::kSlice, [](int) { return 1.0f; });
     __syncthreads();
     float* out = prm.scratch + (static_cast<int64_t>(chunk) * prm.heads + head) * prm.dim * prm.vdim;
-    for (int d0 = 16 * wave; d0 < dp; d0 += 64) {
-        f32x4_t acc[4] = {};
+    for (int d0 = 16 * wave; d0 < dp; d0 += 16 * W) {
+        f32x4_t acc[W] = {};
         for (int j0 = 0; j0 < kDecayChunk; j0 += 4) {
             const float a = ks[(j0 + g) * stride + d0 + l16];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) acc[e] = mfma32(a, vs[(j0 + g) * kDecayVStride + 16 * e + l16], acc[e]);
+            for (int e = 0; e < W; ++e) acc[e] = mfma32(a, vs[(j0 + g) * kVStride + 16 * e + l16], acc[e]);
         }
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < W; ++e) {
             const int column = e0 + 16 * e + l16;
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -142,21 +158,24 @@ __global__ __launch_bounds__(kDecThreads) void decay_chunk_walk_kernel(DecayAtte
     prm.state[at] = s;
 }
 
-__global__ __launch_bounds__(kDecThreads) void decay_chunk_output_kernel(DecayAttentionParams prm) {
+template <int W>
+__global__ __launch_bounds__(64 * W) void decay_chunk_output_kernel(DecayAttentionParams prm) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, l16 = lane & 15;
     const int head = static_cast<int>(blockIdx.x), chunk = static_cast<int>(blockIdx.y);
-    const int t0 = chunk * kDecayChunk, e0 = static_cast<int>(blockIdx.z) * kDecaySlice;
+    const int t0 = chunk * kDecayChunk, e0 = static_cast<int>(blockIdx.z) * DecayBlock<W>::kSlice;
+    constexpr int kVStride = DecayBlock<W>::kVStride;
     const int dp = mfma32_pad(prm.dim), stride = mfma32_stride(prm.dim);
     const float* powers = prm.powers + head * kDecayPowers;
     float* qs = lds;                           // [64][stride]
-    float* ks = qs + kDecayChunk * stride;     // [64][stride], then the weights and the values, [64][kDecayVStride] each
+    float* ks = qs + kDecayChunk * stride;     // [64][stride], then the weights, [64][kDecayPStride], and the values, [64][kVStride]
     float* ps = ks;
-    float* vs = ks + kDecayChunk * kDecayVStride;
+    float* vs = ks + kDecayChunk * kDecayPStride;
     auto one = [](int) { return 1.0f; };
     const int c4 = (threadIdx.x & 15) * 4;
-    float4 value[4];
-    request_rows(prm, t0, prm.v_column + head * prm.vdim + e0, prm.vdim - e0, c4, value);
+    float4 value[W / 4][DecayBlock<W>::kPasses];
+#pragma unroll
+    for (int x = 0; x < W / 4; ++x) request_rows<W>(prm, t0, prm.v_column + head * prm.vdim + e0, prm.vdim - e0, c4 + 64 * x, value[x]);
     const float* before = prm.scratch + (static_cast<int64_t>(chunk) * prm.heads + head) * prm.dim * prm.vdim;
     const int column = e0 + 16 * wave + l16;
     auto request_state = [&](int d0, float (&s)[4]) __attribute__((always_inline)) {          // (q is zero past the head)
@@ -167,25 +186,37 @@ __global__ __launch_bounds__(kDecThreads) void decay_chunk_output_kernel(DecayAt
     float state[kAhead][4];
 #pragma unroll
     for (int u = 0; u < kAhead; ++u) request_state(16 * u, state[u]);
-    stage_rows(prm, qs, stride, t0, prm.q_column + head * prm.dim, prm.dim, dp, one);
-    stage_rows(prm, ks, stride, t0, prm.k_column + head * prm.dim, prm.dim, dp, one);
+    stage_rows<W>(prm, qs, stride, t0, prm.q_column + head * prm.dim, prm.dim, dp, one);
+    stage_rows<W>(prm, ks, stride, t0, prm.k_column + head * prm.dim, prm.dim, dp, one);
     __syncthreads();
-    f32x4_t score[4] = {};                     // rows of tile `wave`, column tiles 0 .. wave
-    for (int d0 = 0; d0 < dp; d0 += 16) {
-        const float4 a = *reinterpret_cast<const float4*>(qs + (16 * wave + l16) * stride + d0 + 4 * g);
+    // The score tiles go round the waves: whole rows of tiles each would leave the last wave with four of the ten.
+    constexpr int kEach = (kScoreTiles + W - 1) / W;
+    f32x4_t score[kEach] = {};
+    int tile_row[kEach], tile_column[kEach];
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            if (j <= wave) score[j] = mfma32_block(a, *reinterpret_cast<const float4*>(ks + (16 * j + l16) * stride + d0 + 4 * g), score[j]);
+    for (int n = 0; n < kEach; ++n) {
+        const int t = wave + W * n;
+        tile_row[n] = (t >= 1) + (t >= 3) + (t >= 6);
+        tile_column[n] = t - tile_row[n] * (tile_row[n] + 1) / 2;
+    }
+    for (int d0 = 0; d0 < dp; d0 += 16) {
+#pragma unroll
+        for (int n = 0; n < kEach; ++n) {
+            if (wave + W * n >= kScoreTiles) continue;
+            score[n] = mfma32_block(*reinterpret_cast<const float4*>(qs + (16 * tile_row[n] + l16) * stride + d0 + 4 * g),
+                                    *reinterpret_cast<const float4*>(ks + (16 * tile_column[n] + l16) * stride + d0 + 4 * g), score[n]);
+        }
     }
     __syncthreads();
-    put_rows(prm, vs, kDecayVStride, t0, c4, value, one);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        if (j > wave) continue;
+    for (int x = 0; x < W / 4; ++x) put_rows<W>(prm, vs, kVStride, t0, c4 + 64 * x, value[x], one);
+#pragma unroll
+    for (int n = 0; n < kEach; ++n) {
+        if (wave + W * n >= kScoreTiles) continue;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const int row = 16 * wave + 4 * g + r, column = 16 * j + l16;
-            ps[row * kDecayVStride + column] = column <= row ? score[j][r] * powers[row - column] : 0.0f;
+            const int row = 16 * tile_row[n] + 4 * g + r, column = 16 * tile_column[n] + l16;
+            ps[row * kDecayPStride + column] = column <= row ? score[n][r] * powers[row - column] : 0.0f;
         }
     }
     float decayed[4];                          // d^(i+1) of the lane's row of each tile
@@ -210,11 +241,11 @@ __global__ __launch_bounds__(kDecThreads) void decay_chunk_output_kernel(DecayAt
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const float* v = vs + (16 * j + 4 * g) * kDecayVStride + 16 * wave + l16;
-        const float4 b = make_float4(v[0], v[kDecayVStride], v[2 * kDecayVStride], v[3 * kDecayVStride]);
+        const float* v = vs + (16 * j + 4 * g) * kVStride + 16 * wave + l16;
+        const float4 b = make_float4(v[0], v[kVStride], v[2 * kVStride], v[3 * kVStride]);
 #pragma unroll
         for (int i = j; i < 4; ++i)
-            acc[i] = mfma32_block(*reinterpret_cast<const float4*>(ps + (16 * i + l16) * kDecayVStride + 16 * j + 4 * g), b, acc[i]);
+            acc[i] = mfma32_block(*reinterpret_cast<const float4*>(ps + (16 * i + l16) * kDecayPStride + 16 * j + 4 * g), b, acc[i]);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i)
@@ -230,24 +261,32 @@ int64_t decay_scratch_floats(int rows, int heads, int dim, int vdim) {
     return static_cast<int64_t>((rows + kDecayChunk - 1) / kDecayChunk) * heads * dim * vdim;
 }
 
-int32_t launch_decay_chunks(const DecayAttentionParams& prm, hipStream_t stream) {
-    const int chunks = (prm.rows + kDecayChunk - 1) / kDecayChunk;
-    const int stride = mfma32_stride(prm.dim), slices = (prm.vdim + kDecaySlice - 1) / kDecaySlice;
-    const int state_lds = static_cast<int>(sizeof(float)) * kDecayChunk * (stride + kDecayVStride);
-    const int output_lds = static_cast<int>(sizeof(float)) * kDecayChunk * (stride + (stride > 2 * kDecayVStride ? stride : 2 * kDecayVStride));
+template <int W>
+static int32_t decay_chunks_as(const DecayAttentionParams& prm, int chunks, hipStream_t stream) {
+    using Block = DecayBlock<W>;
+    const int stride = mfma32_stride(prm.dim), slices = (prm.vdim + Block::kSlice - 1) / Block::kSlice;
+    const int state_lds = static_cast<int>(sizeof(float)) * kDecayChunk * (stride + Block::kVStride);
+    const int output_lds = static_cast<int>(sizeof(float)) * kDecayChunk * (stride + std::max(stride, kDecayPStride + Block::kVStride));
     static std::atomic<bool> raised[2][kMaxDevices];
-    int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decay_chunk_state_kernel), kDotLdsMost, raised[0]);
-    if (rc == QM_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decay_chunk_output_kernel), kDotLdsMost, raised[1]);
+    int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decay_chunk_state_kernel<W>), kDotLdsMost, raised[0]);
+    if (rc == QM_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decay_chunk_output_kernel<W>), kDotLdsMost, raised[1]);
     if (rc != QM_OK) return rc;
-    if (output_lds > kDotLdsMost || chunks > 65535 || prm.scratch_floats < decay_scratch_floats(prm.rows, prm.heads, prm.dim, prm.vdim)) return QM_ERR_WORKSPACE;
+    if (output_lds > kDotLdsMost) return QM_ERR_WORKSPACE;
     if (prm.options & QM_DECAY_ROTARY)
         hipLaunchKernelGGL(decay_rotate_kernel, dim3(prm.rows), dim3(kDecThreads), sizeof(float) * (prm.rot_dims + 1), stream, prm);
-    hipLaunchKernelGGL(decay_chunk_state_kernel, dim3(prm.heads, chunks, slices), dim3(kDecThreads), state_lds, stream, prm);
+    hipLaunchKernelGGL(decay_chunk_state_kernel<W>, dim3(prm.heads, chunks, slices), dim3(Block::kThreads), state_lds, stream, prm);
     const int64_t plane = static_cast<int64_t>(prm.heads) * prm.dim * prm.vdim;
     hipLaunchKernelGGL(decay_chunk_walk_kernel, dim3(static_cast<unsigned>((plane + kDecThreads - 1) / kDecThreads)), dim3(kDecThreads), 0, stream, prm,
                        chunks);
-    hipLaunchKernelGGL(decay_chunk_output_kernel, dim3(prm.heads, chunks, slices), dim3(kDecThreads), output_lds, stream, prm);
+    hipLaunchKernelGGL(decay_chunk_output_kernel<W>, dim3(prm.heads, chunks, slices), dim3(Block::kThreads), output_lds, stream, prm);
     return launch_status();
+}
+
+int32_t launch_decay_chunks(const DecayAttentionParams& prm, hipStream_t stream) {
+    const int chunks = (prm.rows + kDecayChunk - 1) / kDecayChunk;
+    if (chunks > 65535 || prm.scratch_floats < decay_scratch_floats(prm.rows, prm.heads, prm.dim, prm.vdim)) return QM_ERR_WORKSPACE;
+    const int64_t blocks = static_cast<int64_t>(prm.heads) * chunks * ((prm.vdim + DecayBlock<4>::kSlice - 1) / DecayBlock<4>::kSlice);
+    return prm.vdim > DecayBlock<4>::kSlice && blocks > kDecayWide ? decay_chunks_as<8>(prm, chunks, stream) : decay_chunks_as<4>(prm, chunks, stream);
 }
 
 }  // namespace qm

@@ -346,6 +346,27 @@ def test_decay_attention(decoder, dev, chunked, heads, dim, vdim):
         close(get(s), state, True, tol32=5e-6)
 
 
+@pytest.mark.parametrize("heads,dim,vdim,rows", [(8, 20, 200, 573), (6, 64, 129, 961), (16, 132, 72, 530), (8, 128, 256, 512), (8, 128, 256, 513)])
+def test_decay_attention_in_wide_blocks(decoder, dev, heads, dim, vdim, rows):
+    """Passes of around and of more than 256 blocks of 64 value channels, which blocks of 128 take over."""
+    import torch
+    rng = np.random.default_rng(rows)
+    decay = np.array([0.999, 1.0, 0.3, 0.0, 0.9, 0.99, 0.5, 0.75] * 2)[:heads]
+    proj = rng.standard_normal((rows, heads * (2 * dim + vdim))).astype(np.float32)
+    part = lambda at, count, size: plain.silu(proj[:, at:at + count * size].astype(np.float64)).reshape(rows, count, size)
+    want, state = plain.decayed_linear_attention(part(0, heads, dim), part(heads * dim, heads, dim), part(2 * heads * dim, heads, vdim), decay)
+    powers = put(np.power(decay[:, None], np.arange(decoder.DECAY_POWERS)[None]).astype(np.float32), dev)
+    pd, s, out = put(proj, dev), torch.zeros((heads, dim, vdim), device=dev), torch.full((rows, heads * vdim), 7.0, device=dev)
+    floats = decoder.lib().qm_decay_attention_scratch_floats(rows, heads, dim, vdim)
+    scratch = torch.full((floats,), float("nan"), device=dev)
+    op = decoder.DecayAttention(proj=pd.data_ptr(), powers=powers.data_ptr(), state=s.data_ptr(), out=out.data_ptr(), scratch=scratch.data_ptr(),
+                                ld_proj=proj.shape[1], scratch_floats=floats, rows=rows, heads=heads, dim=dim, vdim=vdim, q_column=0,
+                                k_column=heads * dim, v_column=2 * heads * dim)
+    assert decoder.lib().qm_decay_attention_rows(C.byref(op), torch.cuda.current_stream().cuda_stream) == 0
+    close(get(out), want.reshape(rows, -1), True, tol32=5e-6)          # (as in the smaller passes: the sums are the same)
+    close(get(s), state, True, tol32=5e-6)
+
+
 @pytest.mark.parametrize("chunked", [False, True])
 @pytest.mark.parametrize("heads,dim,rank", [(3, 16, 5), (2, 20, 16), (1, 48, 64), (4, 64, 8), (2, 100, 33), (2, 128, 64), (1, 160, 300), (1, 256, 24)])
 def test_general_delta(decoder, dev, chunked, heads, dim, rank):
