@@ -1,7 +1,8 @@
 // qm_decoder_step.hip — one token through a layer run in three launches, for gfx950: everything that reads the layer's
-// norm, the mixer, everything that leaves the layer.  The small vector work between two linears (residual sum, norms, the
-// attention's merge, gates) is repeated by every block that needs its result rather than handed over through a launch of
-// its own, while the block's first weights are already on their way.
+// norm, the mixer (and beside it the down projection, which does not wait for it), everything that leaves the mixer.  The
+// small vector work between two linears (residual sum, norms, the attention's merge, gates) is repeated by every block that
+// needs its result rather than handed over through a launch of its own, while the block's first weights are already on
+// their way.
 //
 // Bound by HBM (each weight is read once) and, for narrow models, by the latency of the launches.
 #include <algorithm>

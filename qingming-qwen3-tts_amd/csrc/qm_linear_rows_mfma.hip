@@ -7,20 +7,20 @@
 // results within the operators' tolerance of the exact-chain kernel (qm_linear_rows.hip), not bit-identical to it.
 //
 // A block owns a tile of BM token rows x BN output columns: 128 x 128 (eight waves 2 x 4, each 64 rows x 32 columns, two to a
-// SIMD so that one multiplies while the other waits to issue: three linears of 2048, 2048 and 6144 inputs over 1024 rows 71.3 ->
-// 68.6 us against four waves of 64 x 64; the other tiles gain nothing from it and keep four); 64 x 128 for calls whose grid of 128-row tiles would leave CUs empty (waves 4 x 1, each 32 columns x 64
-// rows); 64 x 64 with up to eight stages where most CUs would still be empty and a block's time is its chain of round trips to memory
-// (waves 2 x 2); 128 x 192 for a gate/up pair whose 128-column tiles come to between one and two rounds of the CUs and whose
-// 192-column tiles fit in one (1024 tokens x 6144 channels: 256 blocks).  Several linears of one input (q, k, v) share a
-// grid: a column tile's number says which of them it belongs to.  Both operands are K-contiguous rows (x [m][k],
+// SIMD so that one multiplies while the other waits to issue: three linears of 2048, 2048 and 6144 inputs over 1024 rows
+// 71.3 -> 68.6 us against four waves of 64 x 64; the other tiles gain nothing from it and keep four); 64 x 128 for calls whose
+// grid of 128-row tiles would leave CUs without a block; 64 x 64 with up to eight stages where most CUs would still be empty
+// and a block's time is its chain of round trips to memory (waves 2 x 2); 128 x 192 for a gate/up pair whose 128-column tiles
+// come to between one and two rounds of the CUs and whose 192-column tiles fit in one (1024 tokens x 6144 channels: 256
+// blocks).  Several linears of one input (q, k, v) share a grid: a column tile's number says which of them it belongs to.  Both operands are K-contiguous rows (x [m][k],
 // w [n][k]), so one tile layout serves both: KSTEP (64, or 128 for 64-row tiles with a long reduction) k per step, a row
 // of a tile is KSTEP / 8 16-byte pieces in LDS, piece q of row r stored in slot q ^ key(r), the key chosen so that the
 // sixteen rows a fragment read touches in a cycle spread over all 64 banks.  An MFMA takes the weight rows as its A
 // operand and the token rows as B (D = W X^T): a lane then holds, for one token row, runs of four consecutive output
 // columns — 8-byte stores.
 // The tiles go from memory straight into a ring of LDS stages (buffer_load ... lds, no registers, the swizzle chosen by
-// which piece a lane fetches): four stages where they fit in 128 KiB (the 64 x 64 tile: eight, or six for a pair), else three, two for the 192-column tile (64 KiB a
-// stage).  A step's one barrier stands between the MFMAs of its last two k blocks, where a wave has read all it needs of
+// which piece a lane fetches): four stages where they fit in 128 KiB (the 64 x 64 tile: eight, or six for a pair), else three,
+// two for the 192-column tile (64 KiB a stage).  A step's one barrier stands between the MFMAs of its last two k blocks, where a wave has read all it needs of
 // the step's stage and waits (vmcnt counts the later stages' pieces still in flight) for its own pieces of the next.
 // Nothing but MFMAs is issued in a bunch: a k block's LDS reads and the requests for the stage just freed stand one or
 // two to a slot between its MFMAs (GmSchedule), because the wave issues in order and an MFMA hides 32 cycles of other

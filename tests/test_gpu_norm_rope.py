@@ -161,6 +161,27 @@ def test_query_and_key_rows_in_one_launch_are_the_two_calls(oracle, qm, dev, row
     assert f(*a, 0, q_heads, kv_heads, 1e-6, None) == 0
 
 
+@pytest.mark.parametrize("q_heads,kv_heads", [(5, 1), (6, 1), (16, 8), (24, 1), (32, 8), (48, 1)])
+def test_query_and_key_heads_around_a_block_s_share(oracle, qm, dev, q_heads, kv_heads):
+    """A wave takes six heads of a row and a block 24 at a time: fewer, as many and more, also in place, bit for bit."""
+    import torch
+    rows = 3
+    q, k = (oracle.normal_bf16((rows, heads, 128), 700 + heads) for heads in (q_heads, kv_heads))
+    gq, gk = (oracle.normal_bf16((128,), seed, 1.0, 0.1) for seed in (702, 703))
+    cos, sin = oracle.rope_table(rows, 9)
+    want_q, want_k = np.zeros_like(q), np.zeros_like(k)
+    assert oracle.norm_rope_rows(q, gq, cos, sin, want_q, rows, q_heads) == 0
+    assert oracle.norm_rope_rows(k, gk, cos, sin, want_k, rows, kv_heads) == 0
+    qd, kd = to_dev(q, dev), to_dev(k, dev)
+    rest = [to_dev(a, dev) for a in (gq, gk, cos, sin)]
+    got_q, got_k = (torch.full(t.shape, 0x7fc0, dtype=torch.int16, device=dev) for t in (qd, kd))
+    qm.qk_norm_rope_rows(qd, kd, *rest, got_q, got_k, rows, q_heads, kv_heads)
+    qm.qk_norm_rope_rows(qd, kd, *rest, qd, kd, rows, q_heads, kv_heads)
+    torch.cuda.synchronize()
+    assert np.array_equal(to_u16(got_q), want_q) and np.array_equal(to_u16(got_k), want_k)
+    assert torch.equal(qd, got_q) and torch.equal(kd, got_k)
+
+
 def test_scatter_kv_paged_and_flat(oracle, qm, dev):
     import torch
     rows, first = 75, 9
