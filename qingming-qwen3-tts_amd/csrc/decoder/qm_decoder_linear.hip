@@ -73,7 +73,6 @@ static int32_t streaming(const DecLinearParams& prm, hipStream_t stream) {
 // L2), and the four sums meet in LDS.  Bound by the latency of a wave's loads.
 constexpr int kNarrowRows = 16;                        // token rows of a block
 constexpr int kNarrowColumns = 64;                     // most columns
-constexpr int kDecNarrowRows = 16;                     // fewest token rows: the dot products end first below
 template <int TILES>
 __global__ __launch_bounds__(kDecThreads) void narrow_linear_kernel(DecLinearGroup group, int rows) {
     __shared__ float sums[4][TILES * 16 * (kNarrowRows + 1)];
@@ -117,13 +116,11 @@ static int32_t launch_narrow(const DecLinearParams& prm, hipStream_t stream) {
     return launch_status();
 }
 
-// Whether bf16 rows go to the matrix cores: beyond eight rows the dot products stream every weight twice, and from five rows on the
-// rows' own LDS reads slow a long reduction (us, dot products / matrix cores: inputs 10240 + 2 x 6144 by 2048 of 4 / 5 / 9 / 15 rows
-// 23 / 29 / 43 / 44 against 28 to 29; outputs of 2048, 2048 and 6144 inputs 15 / 23 / 31 / 39 against 17 to 20; 5120 + 2 x 3072 by 1024
-// of 5 / 8 / 9 rows 11 / 12 / 16 against 13 to 14).
-static bool matrix_pays(const DecLinearParams& prm) {
-    return prm.rows > 8 || (prm.rows > 4 && longest_row_bytes<uint16_t>(prm) >= 8192);
-}
+// Rows from which bf16 goes to the matrix cores.  Below, one tile is mostly empty, and a pair's gate and up would be rounded to bf16
+// before their product, where the dot products keep them in fp32 and round once: up to 15 rows the results are the dot products',
+// whatever rows go together.  (The matrix cores would end earlier from nine rows on, and from five where a reduction is long: us, dot
+// products / matrix cores, inputs 10240 + 2 x 6144 by 2048 of 9 / 15 rows 43 / 44 against 28 to 29.)
+constexpr int kDecMatrixRows = 16;
 
 // Whether fp32 rows go to the matrix cores: up to eight rows every weight is streamed once either way, and below about 2^26 products
 // the dot-product kernel's many short chains end first (us, dot products / matrix cores; products in millions: router 32 x 1024 of 1000
@@ -145,8 +142,8 @@ int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t 
     }
     if (prm.rows == 0) return QM_OK;
     if (f32) return split_pays(prm) ? launch_split_linears(prm, stream) : streaming<float>(prm, stream);
-    bool matrix = matrix_pays(prm);
-    if (prm.rows >= kDecNarrowRows && prm.groups == 1 && prm.group[0].n <= kNarrowColumns && !prm.group[0].w_up)
+    bool matrix = prm.rows >= kDecMatrixRows;
+    if (matrix && prm.groups == 1 && prm.group[0].n <= kNarrowColumns && !prm.group[0].w_up)
         return prm.group[0].n <= 32 ? launch_narrow<2>(prm, stream) : launch_narrow<4>(prm, stream);
     for (int g = 0; g < prm.groups; ++g) matrix = matrix && prm.group[g].n % 128 == 0 && prm.group[g].ldx == prm.group[g].k && prm.group[g].ldo == prm.group[g].n;
     if (!matrix) return streaming<uint16_t>(prm, stream);

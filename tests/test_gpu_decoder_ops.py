@@ -155,6 +155,39 @@ def test_linears(decoder, dev, f32, rows):
     close(get(outs[2]), plain.silu(gate) * (x[2].astype(np.float64) @ up.T), f32, tol32=3e-6, tol16=2e-2)
 
 
+@pytest.mark.parametrize("rows,k", [(5, 4096), (8, 6144), (9, 256), (12, 2048), (15, 640)])
+@pytest.mark.parametrize("pair", [False, True])
+def test_few_bf16_rows_give_the_same_bits_together_and_alone(decoder, dev, rows, k, pair):
+    """Up to 15 rows a row is the dot products': fp32 sums in one order, a pair rounded once behind its product."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    n = 256
+    x = torch.randn(rows, k, device=dev, generator=gen).bfloat16()
+    w, up = ((torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for _ in range(2))
+    dtype = torch.bfloat16 if pair else torch.float32
+
+    def run(first, count):
+        out = torch.full((count, n), 7.0, device=dev, dtype=dtype)
+        linear = decoder.DecoderLinear(x=x.data_ptr() + 2 * k * first, w=w.data_ptr(), w_up=up.data_ptr() if pair else None, out32=None if pair else out.data_ptr(),
+                                       out=out.data_ptr() if pair else None, ldx=k, ldo=n, n=n, k=k)
+        assert decoder.lib().qm_decoder_linear_rows(C.byref(linear), 1, count, 0, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return out
+
+    assert torch.equal(run(0, rows), torch.cat([run(i, 1) for i in range(rows)]))
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 15])
+def test_a_reduction_too_long_for_the_dot_products_is_refused(decoder, dev, rows):
+    import torch
+    n, k = 128, 65536 + 128
+    x, w = torch.zeros(rows, k, device=dev, dtype=torch.bfloat16), torch.zeros(n, k, device=dev, dtype=torch.bfloat16)
+    out = torch.full((rows, n), 7.0, device=dev)
+    linear = decoder.DecoderLinear(x=x.data_ptr(), w=w.data_ptr(), out32=out.data_ptr(), ldx=k, ldo=n, n=n, k=k)
+    assert decoder.lib().qm_decoder_linear_rows(C.byref(linear), 1, rows, 0, torch.cuda.current_stream().cuda_stream) == -2
+    assert bool((out == 7).all())
+
+
 @pytest.mark.parametrize("rows,n,k,pair", [
     # every tile of the 32-bit mode's matrix-core linears: columns that end inside a tile, reductions of an odd number of steps per share
     (16, 2128, 2048, False), (9, 3600, 2176, False), (33, 1040, 2048, False), (40, 1040, 1664, False), (129, 6640, 128, False),
