@@ -11,8 +11,8 @@
 // LDS stages (a row's 16-byte pieces swizzled over the banks).  Bound: three times the bf16 matrix-core flops of the shape.
 #include <algorithm>
 
-#include "qm_decoder_device.h"
 #include "../qm_host.h"
+#include "qm_decoder_dot.h"
 
 namespace qm {
 
@@ -34,6 +34,13 @@ __device__ __forceinline__ uint32_t take_upper(float& x) {
     const uint32_t upper = (bits | nan) & 0xffff0000U;
     x = finite ? x - __uint_as_float(upper) : 0.0f;
     return upper;
+}
+
+// x . w in one chain.
+__device__ __forceinline__ float plain_dot(const float* x, const uint16_t* w, int k) {
+    float sum = 0.0f;
+    for (int c = 0; c < k; c += 8) sum = dot8(*reinterpret_cast<const uint4*>(w + c), x + c, sum);
+    return sum;
 }
 
 template <int BT, int TN, int KS>
@@ -179,6 +186,7 @@ __global__ __launch_bounds__(kDecThreads * KS, KS > 2 ? KS : 2) void split_linea
                 for (int b = 0; b < BT; ++b) sum[a][b] += others[((other * TN + a) * BT + b) * kDecThreads + tid];
     }
     // a lane holds columns 4 g .. 4 g + 3 of a tile's sixteen for token row l16
+    bool finite = true;
 #pragma unroll
     for (int b = 0; b < BT; ++b) {
         const int row = row0 + 16 * b + l16;
@@ -192,6 +200,7 @@ __global__ __launch_bounds__(kDecThreads * KS, KS > 2 ? KS : 2) void split_linea
                 v.z = silu_f32(sum[0][b][2]) * sum[1][b][2];
                 v.w = silu_f32(sum[0][b][3]) * sum[1][b][3];
                 *reinterpret_cast<float4*>(to) = v;
+                finite = finite && v.x == v.x && v.y == v.y && v.z == v.z && v.w == v.w;
             }
         } else {
 #pragma unroll
@@ -200,8 +209,26 @@ __global__ __launch_bounds__(kDecThreads * KS, KS > 2 ? KS : 2) void split_linea
                 if (channel >= group.n) continue;
                 *reinterpret_cast<float4*>(group.out32 + static_cast<int64_t>(row) * group.ldo + channel + 4 * g) =
                     make_float4(sum[a][b][0], sum[a][b][1], sum[a][b][2], sum[a][b][3]);
+#pragma unroll
+                for (int r = 0; r < 4; ++r) finite = finite && sum[a][b][r] == sum[a][b][r];
             }
         }
+    }
+    // The zeros among an input's lower parts make a NaN of an infinite weight, where the input itself makes an infinity of it.  Outputs
+    // that are no number are therefore formed again from the inputs as they are.
+    if (finite) return;
+    const float* const inputs = static_cast<const float*>(group.x);
+    float* const outputs = pair ? static_cast<float*>(group.out) : group.out32;
+#pragma unroll 1
+    for (int i = 0; i < 4 * BT * (pair ? 1 : TN); ++i) {
+        const int row = row0 + 16 * (i / 4 % BT) + l16, channel = channel0 + 16 * (i / (4 * BT)) + 4 * g + i % 4;
+        if (row >= rows || channel >= group.n) continue;
+        float* const at = outputs + static_cast<int64_t>(row) * group.ldo + channel;
+        if (*at == *at) continue;
+        const float* const x_row = inputs + static_cast<int64_t>(row) * group.ldx;
+        const int64_t w_row = static_cast<int64_t>(channel) * k;
+        const float first = plain_dot(x_row, group.w + w_row, k);
+        *at = pair ? silu_f32(first) * plain_dot(x_row, group.w_up + w_row, k) : first;
     }
 }
 

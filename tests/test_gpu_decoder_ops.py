@@ -188,10 +188,13 @@ def test_a_reduction_too_long_for_the_dot_products_is_refused(decoder, dev, rows
     assert bool((out == 7).all())
 
 
-@pytest.mark.parametrize("rows,n,k,pair", [
+SPLIT_LINEARS = [
     # every tile of the 32-bit mode's matrix-core linears: columns that end inside a tile, reductions of an odd number of steps per share
     (16, 2128, 2048, False), (9, 3600, 2176, False), (33, 1040, 2048, False), (40, 1040, 1664, False), (129, 6640, 128, False),
-    (300, 6640, 128, False), (10, 1664, 2176, True), (33, 1024, 1152, True), (150, 4096, 128, True), (257, 4096, 128, True)])
+    (300, 6640, 128, False), (10, 1664, 2176, True), (33, 1024, 1152, True), (150, 4096, 128, True), (257, 4096, 128, True)]
+
+
+@pytest.mark.parametrize("rows,n,k,pair", SPLIT_LINEARS)
 def test_linears_of_many_fp32_rows(decoder, dev, rows, n, k, pair):
     """Against 64 bits, per output: a sum of k exact products through at most k / 64 + 80 roundings of partial sums that sum |x w| bounds.
     Columns of x differ by up to 2^40; the last row holds an infinity."""
@@ -222,6 +225,34 @@ def test_linears_of_many_fp32_rows(decoder, dev, rows, n, k, pair):
         assert torch.equal(got[-1].isinf(), w[:, 3].cpu() != 0) and torch.equal(got[-1].sign(), w[:, 3].double().cpu().sign())
         want, bound, got = gate[:-1], unit * most[:-1], got[:-1]
     assert bool(((got - want).abs() <= bound).all()), float(((got - want).abs() / bound).max())
+
+
+@pytest.mark.parametrize("rows,n,k,pair", SPLIT_LINEARS)
+def test_many_fp32_rows_meet_infinite_weights(decoder, dev, rows, n, k, pair):
+    """Infinities and NaNs stand where the dot products of few rows have them: infinite weights against inputs with nothing behind their
+    upper bits, zeros, subnormals and infinities."""
+    import torch
+    inf = float("inf")
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    x = torch.randn(rows, k, device=dev, generator=gen)
+    x[0], x[1], x[2, 3], x[3, :64], x[-2] = 1.0, 0.5, 0.0, 1e-41, x[-2].bfloat16().float()
+    x[-1, 3] = inf
+    w, up = ((torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for _ in range(2))
+    w[5, 3], w[7, 2], w[9, 4], w[11, 0], w[11, 1], w[n - 1, k - 1], w[n // 2, 100] = inf, -inf, float("nan"), inf, -inf, -inf, inf
+    up[5, 9], up[6, 3], up[n // 2 + 1, 5] = -inf, inf, inf
+
+    def run(first, count):
+        out = torch.full((count, n), 7.0, device=dev)
+        linear = decoder.DecoderLinear(x=x.data_ptr() + 4 * k * first, w=w.data_ptr(), w_up=up.data_ptr() if pair else None, out32=None if pair else out.data_ptr(),
+                                       out=out.data_ptr() if pair else None, ldx=k, ldo=n, n=n, k=k)
+        assert decoder.lib().qm_decoder_linear_rows(C.byref(linear), 1, count, 1, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return out
+
+    got, want = run(0, rows), torch.cat([run(i, min(8, rows - i)) for i in range(0, rows, 8)])
+    assert bool(want.isinf().any()) and bool(want.isnan().any())
+    for same in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(same(got), same(want))
 
 
 ATTENTION = [
