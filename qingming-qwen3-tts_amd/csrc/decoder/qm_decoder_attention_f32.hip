@@ -39,7 +39,7 @@ __global__ __launch_bounds__(WAVES * 64) void chunk_attention_f32_kernel(ChunkAt
     const int query_row = min(row0 + l16, total - 1);
     const int position = position_at(query_row), lo = chunk_start(position);
 
-    float4 q[C / 16];                          // (channels past the head: zeros, against whatever the clamped loads bring)
+    float4 q[C / 16];                          // (channels past the head: zeros here and in the keys, whose clamped loads repeat the last four)
     const float* q_row = static_cast<const float*>(prm.q_rot) +
                          (static_cast<int64_t>(query_row / group) * prm.heads + kv_head * group + query_row % group) * prm.k_stride;
 #pragma unroll
@@ -82,6 +82,11 @@ __global__ __launch_bounds__(WAVES * 64) void chunk_attention_f32_kernel(ChunkAt
         f32x4_t s[kF32AttentionSums];
 #pragma unroll
         for (int i = 0; i < kF32AttentionSums; ++i) s[i] = none;
+        if (prm.k_stride < C) {
+#pragma unroll
+            for (int kb = 0; kb < C / 16; ++kb)
+                if (16 * kb + 4 * g >= prm.k_stride) k[kb] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
 #pragma unroll
         for (int kb = 0; kb < C / 16; ++kb) {
             f32x4_t* sums = s + 4 * (kb & 3);

@@ -378,6 +378,21 @@ def test_fp32_attention_of_many_rows_against_the_row_kernel(decoder, dev, shape)
         assert not np.isfinite(got[at]).all()
 
 
+@pytest.mark.parametrize("shape", [(4, 2, 40, 40, 50, 8), (3, 3, 24, 40, 37, 8), (2, 1, 72, 16, 60, 8), (4, 2, 64, 64, 50, 8)])
+def test_fp32_attention_of_many_rows_meets_infinite_keys(decoder, dev, shape):
+    """An infinity in a key's last channel decides by the query's sign: a score of -inf is a weight of zero, one of +inf leaves no number."""
+    case = AttentionCase(shape, 100, seed=11)
+    for at, head in ((3, 0), (61, shape[1] - 1)):
+        case.proj[at, case.k_at + head * case.dim + case.dim - 1] = np.inf
+    with np.errstate(invalid="ignore"):
+        want = case.want()
+    got = case.run(decoder, dev, True, [100])
+    finite = np.isfinite(want)
+    assert not finite.all() and finite[61:case.chunk * 2].any()
+    assert np.array_equal(np.isfinite(got), finite)
+    close(got[finite], want[finite], True, tol32=2e-5)
+
+
 @pytest.mark.parametrize("chunked", [False, True])
 @pytest.mark.parametrize("heads,dim,vdim", [(3, 16, 24), (2, 20, 36), (1, 48, 16), (4, 64, 128), (2, 132, 200), (1, 256, 256), (2, 7, 9)])
 def test_decay_attention(decoder, dev, chunked, heads, dim, vdim):
