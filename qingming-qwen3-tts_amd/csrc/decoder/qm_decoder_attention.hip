@@ -3,7 +3,7 @@
 //
 // Chunks count from position 0 of the sequence, so a query needs at most `chunk` keys, all of them in the cache however the
 // prompt was cut.  Three kernels: few rows (decode) deal a chunk's keys to several blocks per key/value head and combine the
-// partial results; many bf16 rows take the matrix-core kernel of qm_decoder_attention_mfma.hip, many fp32 rows that of
+// partial results; many bf16 rows take the matrix-core kernel of qm_decoder_attention_mfma.hip, many fp32 rows, where it ends first, that of
 // qm_decoder_attention_f32.hip.
 #include "../qm_host.h"
 #include "qm_decoder_attention.h"

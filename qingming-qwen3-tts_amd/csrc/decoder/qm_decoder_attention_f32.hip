@@ -9,6 +9,8 @@
 // No sum has longer chains than in the kernel of few rows: scores are kept in sixteen sums, and a step's share of the values
 // is summed apart, in two, before it joins the rest.  Root mean square error against 64 bits, 16 query heads over 8 key/value
 // heads of 64 channels, chunks of 512: 1.04e-7 at 16 rows, 1.18e-7 at 300 (the kernel of few rows: 1.07e-7, 1.21e-7).
+#include <algorithm>
+
 #include "../qm_host.h"
 #include "qm_decoder_mfma32.h"
 
@@ -232,14 +234,34 @@ static int32_t attention_f32_as(const ChunkAttentionParams& prm, hipStream_t str
     return launch_status();
 }
 
-// Measured with the rotation's launch, 16 query heads over 8 key/value heads, chunks of 512, here and by the kernel of few rows
-// (us): heads of 64 channels 9.2 and 15.5 at 16 rows, 10.5 and 23.0 at 100, 15.8 and 54.4 at 300, 43.5 and 172 at 1024; of 128
-// channels 11.6 and 16.8 at 16 rows, 68.5 and 180 at 1024.  The bf16 rows' line is also the one behind which the caller provides
-// no splits of the keys.  Heads past 128 channels stay with the kernel of few rows: the registers of 256 spill (4 query heads over
-// one of 256 channels, 300 rows: 54 and 51).
+// Whether the rows take this kernel: its time against that of the kernel of few rows, which deals a row's keys to several blocks if
+// the caller cut them.  Both are a start and a block's chain, in tenths of a microsecond as measured, times the rounds of blocks: here
+// a step of 64 keys 14 (heads of more than 64 channels: 21) and a block per CU; there a pass of 128 keys 30 for up to two query heads
+// of a key/value head, 39 for every four, two blocks per CU, and 0.07 for every block launched beyond that.
+// Measured with the rotation's launch (us, here / kernel of few rows).  16 query heads over 8 of 64 channels, chunks of 512: 9.2 / 15.5
+// at 16 rows, 10.5 / 23.0 at 100, 15.8 / 54.4 at 300, 43.5 / 172 at 1024; of 128 channels 11.6 / 16.8 at 16 rows, 68.5 / 180 at 1024.
+// The last 16 rows of 1016, two heads over one of 128 channels: 41 / 31.  16 rows at position 8000 in a chunk of 8192, 16 heads over 8
+// of 64 channels: 175 / 177 uncut and 65 in four pieces, of 128 channels 263 / 187 and 68; 4 heads over one of 64: 174 / 247 and 29 in
+// sixteen; 150 rows 180 / 255 and 115.
+// Heads past 128 channels stay with the kernel of few rows: the registers of 256 spill (4 query heads over one of 256 channels, 300
+// rows: 54 / 51).
 bool attention_f32_pays(const ChunkAttentionParams& prm) {
-    const int64_t blocks = (static_cast<int64_t>(prm.rows) * (prm.heads / prm.kv_heads) + kF32AttentionRows - 1) / kF32AttentionRows;
-    return prm.rows >= kAttentionMatrixRows && prm.dim <= 128 && prm.vdim <= 128 && blocks <= 65535 && (reinterpret_cast<uintptr_t>(prm.out) & 15) == 0;
+    const int64_t group = prm.heads / prm.kv_heads, chunk = prm.chunk;
+    auto pieces = [](int64_t n, int64_t of) { return (n + of - 1) / of; };
+    if (prm.rows < kAttentionMatrixRows || prm.dim > 128 || prm.vdim > 128 || pieces(prm.rows * group, kF32AttentionRows) > 65535 ||
+        (reinterpret_cast<uintptr_t>(prm.out) & 15) != 0)
+        return false;
+    const int64_t before = prm.position % chunk;
+    const int64_t keys = std::min(before + prm.rows, chunk);       // the most that a row sees
+    const int64_t first = std::min<int64_t>(prm.rows, chunk - before), more = prm.rows - first, last = more % chunk;
+    const int64_t all_keys = first * before + first * (first + 1) / 2 + more / chunk * (chunk * (chunk + 1) / 2) + last * (last + 1) / 2;
+    const int64_t rows = pieces(all_keys, keys);                   // as many as see that many for the same work
+    const int64_t here = 75 + pieces(keys, 64) * (std::max(prm.dim, prm.vdim) <= 64 ? 14 : 21) *
+                                  pieces(pieces(rows * group, kF32AttentionRows) * prm.kv_heads, 256);
+    const int64_t piece = std::min<int64_t>(keys, prm.part.keys_per_split);
+    const int64_t there = 120 + pieces(piece, 128) * (group <= 2 ? 30 : 39 * pieces(group, 4)) * pieces(pieces(keys, piece) * prm.kv_heads * rows, 512) +
+                          std::max<int64_t>(static_cast<int64_t>(prm.part.splits) * prm.kv_heads * prm.rows - 512, 0) * 7 / 100;
+    return here <= there;
 }
 
 int32_t launch_chunk_attention_f32(const ChunkAttentionParams& prm, hipStream_t stream) {

@@ -393,6 +393,17 @@ def test_fp32_attention_of_many_rows_meets_infinite_keys(decoder, dev, shape):
     close(got[finite], want[finite], True, tol32=2e-5)
 
 
+@pytest.mark.parametrize("shape,before,splits,here", [
+    ((2, 1, 128, 128, 1024, 64), 1000, 1, False), ((4, 1, 64, 64, 2048, 64), 2000, 16, False), ((4, 1, 64, 64, 2048, 64), 2000, 1, True),
+    ((16, 8, 64, 64, 512, 64), 200, 1, True), ((16, 8, 64, 64, 512, 64), 200, 4, True)])
+def test_long_chunks_of_few_fp32_rows_take_the_row_kernel(decoder, dev, shape, before, splits, here):
+    """Where few blocks would walk a long chunk that the caller cut, or one of wide heads, the row kernel ends first and is taken."""
+    case = AttentionCase(shape, before + 16, seed=4)
+    got, rows_kernel = (case.run(decoder, dev, True, [before, 16], splits=splits, rows_only=only)[before:] for only in (False, True))
+    close(got, rows_kernel, True, tol32=2e-5)
+    assert np.array_equal(got, rows_kernel) != here
+
+
 @pytest.mark.parametrize("chunked", [False, True])
 @pytest.mark.parametrize("heads,dim,vdim", [(3, 16, 24), (2, 20, 36), (1, 48, 16), (4, 64, 128), (2, 132, 200), (1, 256, 256), (2, 7, 9)])
 def test_decay_attention(decoder, dev, chunked, heads, dim, vdim):
