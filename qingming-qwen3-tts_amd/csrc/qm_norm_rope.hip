@@ -89,52 +89,59 @@ __global__ __launch_bounds__(256) void norm_rope_rows_kernel(
     out[base + lane + 64] = r.hi;
 }
 
-// The prompt pass's query and key heads in one grid, a block per row, the first q_heads of a row's heads its query heads; every head as
-// norm_rope_rows_kernel forms it.  A wave takes kRopeHeads heads at a time: their values, the row's cosines and sines and the weights
-// are asked for at once (a wave per head was three rounds of waves that each waited for memory: 1000 rows of 24 heads 9.2 -> 7.7 us).
-constexpr int kRopeHeads = 6;
+// The prompt pass's query and key heads in one grid, the first q_heads of a row's heads its query heads; every head as
+// norm_rope_rows_kernel forms it.  A wave takes H heads of a row: their values, the row's cosines and sines and the weights are asked
+// for at once.
+template <int H>
 __global__ __launch_bounds__(256) void qk_norm_rope_rows_kernel(
     const uint16_t* __restrict__ q_in, const uint16_t* __restrict__ k_in, const uint16_t* __restrict__ q_norm_w,
     const uint16_t* __restrict__ k_norm_w, const uint16_t* __restrict__ cos_rows, const uint16_t* __restrict__ sin_rows,
-    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out, int q_heads, int kv_heads, float epsilon) {
-    request_arguments(q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, q_heads, kv_heads, epsilon);
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t row = blockIdx.x;
-    const int heads = q_heads + kv_heads;
+    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_out, int64_t waves, int q_heads, int kv_heads, float epsilon) {
+    request_arguments(q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, waves, q_heads, kv_heads, epsilon);
+    const int lane = threadIdx.x & 63;
+    const int64_t item = static_cast<int64_t>(blockIdx.x) * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (item >= waves) return;
+    const int heads = q_heads + kv_heads, per_row = (heads + H - 1) / H;
+    const int64_t row = item / per_row;
+    const int first = static_cast<int>(item - row * per_row) * H;
     const uint16_t c0 = cos_rows[row * kDim + lane], c1 = cos_rows[row * kDim + lane + 64];
     const uint16_t s0 = sin_rows[row * kDim + lane], s1 = sin_rows[row * kDim + lane + 64];
     uint16_t gq[2] = {0, 0}, gk[2] = {0, 0};
-    if (q_norm_w) {
+    if (q_norm_w && first < q_heads) {
         gq[0] = q_norm_w[lane];
         gq[1] = q_norm_w[lane + 64];
     }
-    if (k_norm_w) {
+    if (k_norm_w && first + H > q_heads) {
         gk[0] = k_norm_w[lane];
         gk[1] = k_norm_w[lane + 64];
     }
-    for (int first = wave * kRopeHeads; first < heads; first += 4 * kRopeHeads) {
-        uint16_t x[kRopeHeads][2];
-        auto place = [&](int head) { return head < q_heads ? (row * q_heads + head) * kDim : (row * kv_heads + (head - q_heads)) * kDim; };
+    uint16_t x[H][2];
+    auto place = [&](int head) { return head < q_heads ? (row * q_heads + head) * kDim : (row * kv_heads + (head - q_heads)) * kDim; };
 #pragma unroll
-        for (int i = 0; i < kRopeHeads; ++i) {                     // (past the last head: it again, not stored)
-            const int head = min(first + i, heads - 1);
-            const uint16_t* in = (head < q_heads ? q_in : k_in) + place(head);
-            x[i][0] = in[lane];
-            x[i][1] = in[lane + 64];
-        }
+    for (int i = 0; i < H; ++i) {              // (past the last head: it again, not stored)
+        const int head = min(first + i, heads - 1);
+        const uint16_t* in = (head < q_heads ? q_in : k_in) + place(head);
+        x[i][0] = in[lane];
+        x[i][1] = in[lane + 64];
+    }
 #pragma unroll
-        for (int i = 0; i < kRopeHeads; ++i) {
-            const int head = first + i;
-            if (head >= heads) break;
-            const bool is_query = head < q_heads;
-            const HeadPair r = norm_rope_head_values(x[i][0], x[i][1], (is_query ? q_norm_w : k_norm_w) != nullptr, is_query ? gq[0] : gk[0],
-                                                     is_query ? gq[1] : gk[1], c0, c1, s0, s1, epsilon);
-            uint16_t* out = (is_query ? q_out : k_out) + place(head);
-            out[lane] = r.lo;
-            out[lane + 64] = r.hi;
-        }
+    for (int i = 0; i < H; ++i) {
+        const int head = first + i;
+        if (head >= heads) break;
+        const bool is_query = head < q_heads;
+        const HeadPair r = norm_rope_head_values(x[i][0], x[i][1], (is_query ? q_norm_w : k_norm_w) != nullptr, is_query ? gq[0] : gk[0],
+                                                 is_query ? gq[1] : gk[1], c0, c1, s0, s1, epsilon);
+        uint16_t* out = (is_query ? q_out : k_out) + place(head);
+        out[lane] = r.lo;
+        out[lane + 64] = r.hi;
     }
 }
+
+// Some 8000 waves are resident at once.  While a wave per head about fills them, its one round trip is the whole time; with more heads
+// each wave asks for four at once instead of waiting in its turn.  (us, one / four heads a wave: 24 heads of 16 rows 2.1 / 3.1, of 300
+// 3.6 / 3.7, of 400 4.0 / 4.3, of 500 4.5 / 4.4, of 1000 7.6 / 6.9, of 4000 21.9 / 17.4; 72 heads of 16 rows 2.2 / 3.1, of 150 4.5 / 4.4;
+// five heads of 1500 rows 3.5 / 4.0, of 4000 6.7 / 6.4.)
+constexpr int64_t kRopeManyHeads = 10240;
 
 // [rows][kv_heads][128] -> pages; one thread moves 16 bytes of K and 16 bytes of V.
 __global__ __launch_bounds__(256) void scatter_kv_kernel(
@@ -235,9 +242,13 @@ extern "C" int32_t qm_qk_norm_rope_rows(
     if (!q_in || !k_in || !cos_rows || !sin_rows || !q_out || !k_out) return QM_ERR_NULL;
     if (rows < 0 || q_heads <= 0 || kv_heads <= 0) return QM_ERR_ARGUMENT;
     if (rows == 0) return QM_OK;
-    if ((static_cast<int64_t>(rows) * (static_cast<int64_t>(q_heads) + kv_heads) + 3) / 4 > 0x7fffffffLL) return QM_ERR_ARGUMENT;
-    hipLaunchKernelGGL(qm::qk_norm_rope_rows_kernel, dim3(static_cast<unsigned>(rows)), dim3(256), 0, static_cast<hipStream_t>(hip_stream),
-                       q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, q_heads, kv_heads, epsilon);
+    const int64_t heads = static_cast<int64_t>(q_heads) + kv_heads;
+    if ((rows * heads + 3) / 4 > 0x7fffffffLL) return QM_ERR_ARGUMENT;
+    const bool many = rows * heads > qm::kRopeManyHeads;
+    const int64_t waves = many ? rows * ((heads + 3) / 4) : rows * heads;
+    const auto kernel = many ? qm::qk_norm_rope_rows_kernel<4> : qm::qk_norm_rope_rows_kernel<1>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, static_cast<hipStream_t>(hip_stream),
+                       q_in, k_in, q_norm_w, k_norm_w, cos_rows, sin_rows, q_out, k_out, waves, q_heads, kv_heads, epsilon);
     return qm::launch_status();
 }
 

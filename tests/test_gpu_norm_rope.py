@@ -163,7 +163,7 @@ def test_query_and_key_rows_in_one_launch_are_the_two_calls(oracle, qm, dev, row
 
 @pytest.mark.parametrize("q_heads,kv_heads", [(5, 1), (6, 1), (16, 8), (24, 1), (32, 8), (48, 1)])
 def test_query_and_key_heads_around_a_block_s_share(oracle, qm, dev, q_heads, kv_heads):
-    """A wave takes six heads of a row and a block 24 at a time: fewer, as many and more, also in place, bit for bit."""
+    """A wave takes a head, a block four: rows of six to 49 heads, also in place, bit for bit."""
     import torch
     rows = 3
     q, k = (oracle.normal_bf16((rows, heads, 128), 700 + heads) for heads in (q_heads, kv_heads))
@@ -180,6 +180,23 @@ def test_query_and_key_heads_around_a_block_s_share(oracle, qm, dev, q_heads, kv
     torch.cuda.synchronize()
     assert np.array_equal(to_u16(got_q), want_q) and np.array_equal(to_u16(got_k), want_k)
     assert torch.equal(qd, got_q) and torch.equal(kd, got_k)
+
+
+@pytest.mark.parametrize("rows,q_heads,kv_heads", [(5200, 1, 1), (3501, 2, 1), (2100, 4, 1), (700, 16, 8), (301, 33, 2)])
+def test_many_query_and_key_heads(oracle, qm, dev, rows, q_heads, kv_heads):
+    """Past 10240 heads a wave takes four of a row, the last of a row fewer: bit for bit as one by one, also in place."""
+    import torch
+    q, k = (to_dev(oracle.normal_bf16((rows, heads, 128), 710 + heads), dev) for heads in (q_heads, kv_heads))
+    gq, gk = (to_dev(oracle.normal_bf16((128,), seed, 1.0, 0.1), dev) for seed in (712, 713))
+    cos, sin = (to_dev(a, dev) for a in oracle.rope_table(rows, 3))
+    want_q, want_k, got_q, got_k = (torch.full(t.shape, 0x7fc0, dtype=torch.int16, device=dev) for t in (q, k, q, k))
+    qm.norm_rope_rows(q, gq, cos, sin, want_q, rows, q_heads)
+    qm.norm_rope_rows(k, gk, cos, sin, want_k, rows, kv_heads)
+    qm.qk_norm_rope_rows(q, k, gq, gk, cos, sin, got_q, got_k, rows, q_heads, kv_heads)
+    qm.qk_norm_rope_rows(q, k, gq, gk, cos, sin, q, k, rows, q_heads, kv_heads)
+    torch.cuda.synchronize()
+    assert torch.equal(got_q, want_q) and torch.equal(got_k, want_k)
+    assert torch.equal(q, want_q) and torch.equal(k, want_k)
 
 
 def test_scatter_kv_paged_and_flat(oracle, qm, dev):
