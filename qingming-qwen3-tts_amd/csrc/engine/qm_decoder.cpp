@@ -24,6 +24,7 @@
 #include <cstring>
 #include <memory>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "../decoder/qm_decoder_ops.h"
@@ -831,13 +832,18 @@ void next_ticket(qm_decoder& d, int position, int before, int token) {
     const int32_t words[kStepWords] = {position, before, token, 0, 0, static_cast<int32_t>(++d.mailbox.last)};
     std::memcpy(d.mailbox.words(), words, sizeof words);
 }
-// The mailbox's scores, once they are there.  Looking at the flags sees them some 10 us before the stream's wait returns; a stream
-// that has longer work ahead is waited for.
+// The mailbox's scores, once they are there.  Looking at the flags sees them some 10 us before the stream's wait returns (which spends
+// the core as well, all the time: 71 of 71 ms of a wait measured); past the time of a short step the core is left to others that want
+// it, and a stream that has longer work ahead is waited for.
 const float* await_scores(qm_decoder& d) {
     const int blocks = qm::mail_blocks(d.config.vocab);
-    const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
+    const auto begin = std::chrono::steady_clock::now();
     for (int looks = 1; !d.mailbox.arrived(blocks); ++looks) {
-        if (looks % 64 != 0 || std::chrono::steady_clock::now() < until) continue;
+        __builtin_ia32_pause();
+        if (looks % 16 != 0) continue;
+        const auto waited = std::chrono::steady_clock::now() - begin;
+        if (waited > std::chrono::milliseconds(1)) std::this_thread::yield();
+        if (waited < std::chrono::milliseconds(20)) continue;
         hip_check(hipStreamSynchronize(d.stream), "step");
         if (!d.mailbox.arrived(blocks)) throw ApiError(QM_ERR_STATUS, "the step's scores did not arrive");
     }

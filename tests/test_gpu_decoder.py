@@ -172,6 +172,34 @@ def test_ways_of_stepping_leave_the_same(decoder, models, name):
     assert np.array_equal(engine.step(a, [1], [0]), plain_engine.step(p, [1], [0]))
 
 
+def test_steps_behind_long_work(decoder, models, dev):
+    """Scores that tens of milliseconds of other work on the stream are ahead of: waited for, and the step's own."""
+    import torch
+    m = models("plain")
+    stream = torch.cuda.Stream()
+    engine = decoder.Decoder(m.directory, len(m.tokens), stream=stream.cuda_stream)
+
+    def run(before):
+        s = engine.open()
+        got = []
+        for tokens in (m.tokens[:9], m.tokens[9:10], m.tokens[10:11]):
+            before()
+            got.append(engine.step(s, tokens, [len(tokens) - 1])[0])
+        engine.close(s)
+        return got
+
+    a = torch.ones(4096, 4096, device=dev)
+    torch.cuda.synchronize()
+
+    def work():
+        with torch.cuda.stream(stream):
+            for _ in range(80):
+                a @ a
+
+    for got, want in zip(run(work), run(lambda: None)):
+        assert np.array_equal(got, want)
+
+
 def greedy(m, prompt, count):
     tokens = list(prompt)
     for _ in range(count):
