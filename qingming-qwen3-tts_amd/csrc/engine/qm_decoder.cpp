@@ -80,8 +80,9 @@ struct DecoderLayer {
     double magnitude = 1.0;
 };
 
-// What a step sends and gets in pinned host memory, so that it is one graph and the host sees the scores as they arrive.  A step
-// has its results before the next one begins, so one mailbox serves every sequence.
+// What a step sends and gets in pinned host memory, so that it is one graph and the host sees the scores as they arrive: while the
+// graph's last kernel runs, so the memory has to be coherent whatever the runtime takes for its default.  A step has its results before
+// the next one begins, so one mailbox serves every sequence.
 struct Mailbox {
     char* at = nullptr;
     uint32_t last = 0;                              // ticket of the last scores asked for
@@ -93,7 +94,7 @@ struct Mailbox {
     }
     void open(int vocab_p) {
         void* p = nullptr;
-        hip_check(hipHostMalloc(&p, kScores + static_cast<size_t>(vocab_p) * 4, hipHostMallocDefault), "pinned step results");
+        hip_check(hipHostMalloc(&p, kScores + static_cast<size_t>(vocab_p) * 4, hipHostMallocCoherent), "pinned step results");
         at = static_cast<char*>(p);
         std::memset(at, 0, kScores);
     }

@@ -172,6 +172,24 @@ def test_ways_of_stepping_leave_the_same(decoder, models, name):
     assert np.array_equal(engine.step(a, [1], [0]), plain_engine.step(p, [1], [0]))
 
 
+@pytest.mark.parametrize("vocab", [2047, 2049, 5122, 16384 + 3])
+def test_scores_of_large_vocabularies_through_pinned_memory(decoder, tmp_path, vocab):
+    """One block, two, five and sixteen write a step's scores, each raising a flag of its own, the last vocabulary's remainder by the first:
+    every score is the plain launches', bit for bit, and none the step before's."""
+    cfg = cases.config(vocab, 64, [cases.general_delta(2, 16, 32)])
+    cases.write_model(str(tmp_path), cfg, cases.weights(cfg))
+    tokens = cases.tokens_of(cfg, 40)
+    rows = []
+    for path in (1, 0):
+        engine = decoder.Decoder(str(tmp_path), 64)
+        engine.set_path(path)
+        s = engine.open()
+        rows.append([engine.step(s, tokens[:7], [6])[0]] + [engine.step(s, [t], [0])[0] for t in tokens[7:]])
+    for i, (want, got) in enumerate(zip(*rows)):
+        assert np.array_equal(got, want), i
+        assert i == 0 or (got != rows[1][i - 1]).mean() > 0.9
+
+
 def test_steps_behind_long_work(decoder, models, dev):
     """Scores that tens of milliseconds of other work on the stream are ahead of: waited for, and the step's own."""
     import torch
