@@ -139,7 +139,6 @@ struct qm_decoder {
     qm_engine::Mailbox mailbox;
 
     ~qm_decoder() {
-        (void)hipDeviceSynchronize();               // (a step returns when its scores are there: its last kernel may not have ended)
         for (const auto* some : {&graphs, &mail_graphs})
             for (hipGraphExec_t g : *some)
                 if (g) (void)hipGraphExecDestroy(g);
@@ -1190,7 +1189,7 @@ extern "C" int32_t qm_decoder_create(const char* model_dir, int32_t f32, int32_t
 }
 
 extern "C" void qm_decoder_destroy(qm_decoder* decoder) {
-    if (decoder) (void)hipStreamSynchronize(decoder->stream);
+    if (decoder) (void)hipStreamSynchronize(decoder->stream);      // (a step returns when its scores are there: its last kernel may not have ended)
     delete decoder;
 }
 
