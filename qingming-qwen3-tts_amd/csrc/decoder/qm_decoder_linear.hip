@@ -128,6 +128,8 @@ constexpr int kDecMatrixRows = 16;
 // rows 315: 28.7 / 9.6; 5120 + 2 x 3072 by 1024 of 8 rows 92: 12.3 / 11.5, of 300 rows 3460: 224 / 36).
 static bool split_pays(const DecLinearParams& prm) {
     if (prm.rows <= 8 || longest_row_bytes<float>(prm) > kDotLds) return false;
+    for (int g = 0; g < prm.groups; ++g)       // (four columns a store there, single ones here)
+        if (reinterpret_cast<uintptr_t>(prm.group[g].w_up ? prm.group[g].out : prm.group[g].out32) & 15) return false;
     int64_t products = 0;
     for (int g = 0; g < prm.groups; ++g) products += static_cast<int64_t>(prm.group[g].n) * prm.group[g].k * (prm.group[g].w_up ? 2 : 1);
     return products * prm.rows > (int64_t{1} << 26);

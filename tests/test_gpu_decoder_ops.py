@@ -255,6 +255,32 @@ def test_many_fp32_rows_meet_infinite_weights(decoder, dev, rows, n, k, pair):
         assert torch.equal(same(got), same(want))
 
 
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("shift", [0, 1, 2, 3])
+def test_many_fp32_rows_into_any_float_address(decoder, dev, pair, shift):
+    """Outputs that are no multiple of 16 bytes are the dot products', which store single floats."""
+    import torch
+    rows, n, k, ldo = 40, 1024, 2048, 1028
+    gen = torch.Generator(device=dev).manual_seed(3)
+    x = torch.randn(rows, k, device=dev, generator=gen)
+    w, up = ((torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for _ in range(2))
+
+    def run(first, count, shift):
+        out = torch.full((count * ldo + 8,), 7.0, device=dev)
+        at = out.data_ptr() + 4 * shift
+        linear = decoder.DecoderLinear(x=x.data_ptr() + 4 * k * first, w=w.data_ptr(), w_up=up.data_ptr() if pair else None, out32=None if pair else at,
+                                       out=at if pair else None, ldx=k, ldo=ldo, n=n, k=k)
+        assert decoder.lib().qm_decoder_linear_rows(C.byref(linear), 1, count, 1, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        assert bool((out[:shift] == 7).all()) and bool((out[shift + count * ldo:] == 7).all())
+        return out[shift:shift + count * ldo].reshape(count, ldo)
+
+    got, want = run(0, rows, shift), torch.cat([run(i, 8, 0) for i in range(0, rows, 8)])
+    assert bool((got[:, n:] == 7).all())
+    assert torch.equal(got, want) == (shift != 0)
+    assert float((got - want).abs().max()) <= 4e-6 * float(want[:, :n].abs().max())
+
+
 ATTENTION = [
     # heads, kv_heads, dim, vdim, chunk, rot_dims
     (4, 2, 16, 16, 50, 8), (3, 3, 24, 40, 37, 24), (5, 1, 36, 20, 64, 10), (6, 2, 64, 64, 200, 16), (2, 1, 136, 144, 300, 64), (8, 2, 128, 128, 256, 128),
