@@ -1,9 +1,11 @@
 // qm_decoder_linear_f32.hip — linears of the 32-bit mode over several token rows on the bf16 matrix cores (gfx950).
 //
-// An fp32 input is the exact sum of three bf16 numbers (its upper eight significant bits, the next eight, the last eight) and
-// the weights are bf16 as they are, so three bf16 products with fp32 accumulation form what fp32 products form: every product
-// is exact.  The sums are taken in two levels — 64 terms, the smallest parts first, then those sums one after the other — which
-// keeps the chains of roundings as short as a wave's lanes keep them in the dot-product kernel.
+// An fp32 input of at least 2^-110 is the exact sum of three bf16 numbers (its upper eight significant bits, the next eight, the
+// last eight: splitting a number over several narrow products is the common way to a wide product on narrow matrix cores) and the
+// weights are bf16 as they are, so three bf16 products with fp32 accumulation form what fp32 products form: every product is exact.
+// Of a smaller input what lies under 2^-133 is lost, so outputs so small that it could tell are formed again in fp32.  The sums are
+// taken in two levels — 64 terms, the smallest parts first, then those sums one after the other — which keeps the chains of
+// roundings as short as a wave's lanes keep them in the dot-product kernel.
 //
 // A block of four waves takes 16 BT token rows and 64 TN weight rows (a gate/up pair: 32 TN channels, gate and up rows in the
 // same lanes), 64 k a step.  Weights are a wave's own and go straight to its registers, requested two steps ahead, a row's
@@ -17,6 +19,7 @@
 namespace qm {
 
 constexpr int kF32Step = 64;                   // k per step
+constexpr float kF32Small = 0x1p-80f;          // what inputs lose under 2^-133 is no 2^-24th of this for weights that sum to 2^29
 
 typedef uint32_t split_u32x4_t __attribute__((ext_vector_type(4)));
 
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(kDecThreads * KS, KS > 2 ? KS : 2) void split_linea
                 for (int b = 0; b < BT; ++b) sum[a][b] += others[((other * TN + a) * BT + b) * kDecThreads + tid];
     }
     // a lane holds columns 4 g .. 4 g + 3 of a tile's sixteen for token row l16
-    bool finite = true;
+    bool good = true;
 #pragma unroll
     for (int b = 0; b < BT; ++b) {
         const int row = row0 + 16 * b + l16;
@@ -200,7 +203,7 @@ __global__ __launch_bounds__(kDecThreads * KS, KS > 2 ? KS : 2) void split_linea
                 v.z = silu_f32(sum[0][b][2]) * sum[1][b][2];
                 v.w = silu_f32(sum[0][b][3]) * sum[1][b][3];
                 *reinterpret_cast<float4*>(to) = v;
-                finite = finite && v.x == v.x && v.y == v.y && v.z == v.z && v.w == v.w;
+                good = good && v.x == v.x && v.y == v.y && v.z == v.z && v.w == v.w;
             }
         } else {
 #pragma unroll
@@ -210,13 +213,13 @@ __global__ __launch_bounds__(kDecThreads * KS, KS > 2 ? KS : 2) void split_linea
                 *reinterpret_cast<float4*>(group.out32 + static_cast<int64_t>(row) * group.ldo + channel + 4 * g) =
                     make_float4(sum[a][b][0], sum[a][b][1], sum[a][b][2], sum[a][b][3]);
 #pragma unroll
-                for (int r = 0; r < 4; ++r) finite = finite && sum[a][b][r] == sum[a][b][r];
+                for (int r = 0; r < 4; ++r) good = good && (fabsf(sum[a][b][r]) >= kF32Small || sum[a][b][r] == 0.0f);
             }
         }
     }
     // The zeros among an input's lower parts make a NaN of an infinite weight, where the input itself makes an infinity of it.  Outputs
-    // that are no number are therefore formed again from the inputs as they are.
-    if (finite) return;
+    // that are no number, or small (a pair's product of such would be zero), are therefore formed again from the inputs as they are.
+    if (good) return;
     const float* const inputs = static_cast<const float*>(group.x);
     float* const outputs = pair ? static_cast<float*>(group.out) : group.out32;
 #pragma unroll 1
@@ -224,7 +227,7 @@ __global__ __launch_bounds__(kDecThreads * KS, KS > 2 ? KS : 2) void split_linea
         const int row = row0 + 16 * (i / 4 % BT) + l16, channel = channel0 + 16 * (i / (4 * BT)) + 4 * g + i % 4;
         if (row >= rows || channel >= group.n) continue;
         float* const at = outputs + static_cast<int64_t>(row) * group.ldo + channel;
-        if (*at == *at) continue;
+        if (pair ? *at == *at : fabsf(*at) >= kF32Small) continue;
         const float* const x_row = inputs + static_cast<int64_t>(row) * group.ldx;
         const int64_t w_row = static_cast<int64_t>(channel) * k;
         const float first = plain_dot(x_row, group.w + w_row, k);

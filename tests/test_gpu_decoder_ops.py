@@ -255,6 +255,24 @@ def test_many_fp32_rows_meet_infinite_weights(decoder, dev, rows, n, k, pair):
         assert torch.equal(same(got), same(want))
 
 
+@pytest.mark.parametrize("exponent", [-122, -112, -108, -60])
+@pytest.mark.parametrize("rows,n,k", [shape[:3] for shape in SPLIT_LINEARS if not shape[3]])
+def test_many_fp32_rows_of_small_inputs(decoder, dev, rows, n, k, exponent):
+    """Rows of normal numbers down to the smallest keep all their bits: one small input among others does as well."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    x = (torch.rand(rows, k, device=dev, generator=gen) + 1) * torch.randint(0, 2, (rows, k), device=dev, generator=gen).mul(2).sub(1).float() * 2.0 ** exponent
+    x[rows // 2, k // 2] = 1.0
+    w = (torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16()
+    out = torch.full((rows, n), 7.0, device=dev)
+    linear = decoder.DecoderLinear(x=x.data_ptr(), w=w.data_ptr(), out32=out.data_ptr(), ldx=k, ldo=n, n=n, k=k)
+    assert decoder.lib().qm_decoder_linear_rows(C.byref(linear), 1, rows, 1, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    want = x.double() @ w.double().T
+    # (2-norms: the errors of a chain of k roundings scatter like the root of k: 2^-24 sqrt(2176) = 2.8e-6 at most; twice that)
+    assert bool(((out.double() - want).norm(dim=1) <= 6e-6 * want.norm(dim=1)).all())
+
+
 @pytest.mark.parametrize("pair", [False, True])
 @pytest.mark.parametrize("shift", [0, 1, 2, 3])
 def test_many_fp32_rows_into_any_float_address(decoder, dev, pair, shift):
