@@ -57,14 +57,22 @@ static int64_t longest_row_bytes(const DecLinearParams& prm) {
     for (int g = 0; g < prm.groups; ++g) k = prm.group[g].k > k ? prm.group[g].k : k;
     return static_cast<int64_t>(k) * sizeof(T);
 }
+// Token rows that a block of the dot products takes (0: a row does not fit its LDS).
+static int streaming_rows(int rows, int64_t row_bytes) {
+    if (row_bytes > kDotLds) return 0;
+    if (rows > 4 && 8 * row_bytes <= kDotLds) return 8;
+    if (rows > 2 && 4 * row_bytes <= kDotLds) return 4;
+    return rows > 1 && 2 * row_bytes <= kDotLds ? 2 : 1;
+}
 template <class T>
 static int32_t streaming(const DecLinearParams& prm, hipStream_t stream) {
-    const int64_t row_bytes = longest_row_bytes<T>(prm);
-    if (row_bytes > kDotLds) return QM_ERR_GEOMETRY;
-    if (prm.rows > 4 && 8 * row_bytes <= kDotLds) return launch_streaming<T, 8>(prm, stream);
-    if (prm.rows > 2 && 4 * row_bytes <= kDotLds) return launch_streaming<T, 4>(prm, stream);
-    if (prm.rows > 1 && 2 * row_bytes <= kDotLds) return launch_streaming<T, 2>(prm, stream);
-    return launch_streaming<T, 1>(prm, stream);
+    switch (streaming_rows(prm.rows, longest_row_bytes<T>(prm))) {
+        case 8: return launch_streaming<T, 8>(prm, stream);
+        case 4: return launch_streaming<T, 4>(prm, stream);
+        case 2: return launch_streaming<T, 2>(prm, stream);
+        case 1: return launch_streaming<T, 1>(prm, stream);
+        default: return QM_ERR_GEOMETRY;
+    }
 }
 
 // A linear of few columns (a router) over many bf16 rows: the large tiles of the matrix-core kernel would leave most CUs
@@ -125,14 +133,28 @@ constexpr int kDecMatrixRows = 16;
 // Whether fp32 rows go to the matrix cores: up to eight rows every weight is streamed once either way, and below about 2^26 products
 // the dot-product kernel's many short chains end first (us, dot products / matrix cores; products in millions: router 32 x 1024 of 1000
 // rows 33: 7.9 / 8.8; 320 x 1024 of 100 rows 33: 7.2 / 8.9; 1024 x 1024 of 64 rows 67: 7.9 / 9.0, of 100 rows 105: 13.4 / 9.2, of 300
-// rows 315: 28.7 / 9.6; 5120 + 2 x 3072 by 1024 of 8 rows 92: 12.3 / 11.5, of 300 rows 3460: 224 / 36).
+// rows 315: 28.7 / 9.6; 5120 + 2 x 3072 by 1024 of 8 rows 92: 12.3 / 11.5, of 300 rows 3460: 224 / 36).  Beyond, the matrix cores' time
+// is one block's chain while the dot products' grows with their rounds of blocks, so that long reductions to few columns stay with
+// those as long as they fit a round or two (1024 x 3072 of 32 / 33 rows 15.1 / 20.7 and 23.5 / 20.8; 2048 x 6144 of 16 / 17 rows 31.6 /
+// 33.4 and 42.3 / 36.3; 2048 x 2048 of 32 / 33 rows 13.2 / 14.4 and 18.5 / 14.3).  Both in tenths of a microsecond, as measured.
 static bool split_pays(const DecLinearParams& prm) {
-    if (prm.rows <= 8 || longest_row_bytes<float>(prm) > kDotLds) return false;
-    for (int g = 0; g < prm.groups; ++g)       // (four columns a store there, single ones here)
-        if (reinterpret_cast<uintptr_t>(prm.group[g].w_up ? prm.group[g].out : prm.group[g].out32) & 15) return false;
+    const int64_t row_bytes = longest_row_bytes<float>(prm), k = row_bytes / 4;
+    const int64_t together = streaming_rows(prm.rows, row_bytes);
+    if (prm.rows <= 8 || together == 0) return false;
     int64_t products = 0;
-    for (int g = 0; g < prm.groups; ++g) products += static_cast<int64_t>(prm.group[g].n) * prm.group[g].k * (prm.group[g].w_up ? 2 : 1);
-    return products * prm.rows > (int64_t{1} << 26);
+    bool pair = false;
+    for (int g = 0; g < prm.groups; ++g) {     // (four columns a store there, single ones here)
+        const DecLinearGroup& d = prm.group[g];
+        if (reinterpret_cast<uintptr_t>(d.w_up ? d.out : d.out32) & 15) return false;
+        products += static_cast<int64_t>(d.n) * d.k * (d.w_up ? 2 : 1);
+        pair = pair || d.w_up;
+    }
+    if (products * prm.rows <= (int64_t{1} << 26)) return false;
+    const int64_t blocks = dot_tiles_of<kLinearRows>(prm) * ((prm.rows + together - 1) / together), pass = k * together / 8;
+    // (two blocks of the dot products to a CU, where a CU that ends early takes the next; or one)
+    const int64_t dots = 2 * together * row_bytes <= 160 * 1024 ? std::max<int64_t>(blocks, 512) * (20 + pass * 53 / 1024) / 512
+                                                                 : (blocks + 255) / 256 * (20 + pass * 42 / 1024);
+    return dots > 33 + k * (pair ? 85 : prm.rows <= 16 ? 46 : 56) / 1024;
 }
 
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream) {

@@ -191,7 +191,9 @@ def test_a_reduction_too_long_for_the_dot_products_is_refused(decoder, dev, rows
 SPLIT_LINEARS = [
     # every tile of the 32-bit mode's matrix-core linears: columns that end inside a tile, reductions of an odd number of steps per share
     (16, 2128, 2048, False), (9, 3600, 2176, False), (33, 1040, 2048, False), (40, 1040, 1664, False), (129, 6640, 128, False),
-    (300, 6640, 128, False), (10, 1664, 2176, True), (33, 1024, 1152, True), (150, 4096, 128, True), (257, 4096, 128, True)]
+    (300, 6640, 128, False), (10, 1664, 2176, True), (33, 1024, 1152, True), (150, 4096, 128, True), (257, 4096, 128, True),
+    # (and those of the above that a single round of the dot products' blocks covers, with more rows or columns)
+    (81, 1040, 2048, False), (81, 1040, 1664, False), (81, 1024, 1152, True), (10, 4096, 2176, True)]
 
 
 @pytest.mark.parametrize("rows,n,k,pair", SPLIT_LINEARS)
@@ -273,12 +275,35 @@ def test_many_fp32_rows_of_small_inputs(decoder, dev, rows, n, k, exponent):
     assert bool(((out.double() - want).norm(dim=1) <= 6e-6 * want.norm(dim=1)).all())
 
 
+@pytest.mark.parametrize("rows,n,k,pair,dots", [
+    (32, 1024, 3072, False, True), (33, 1024, 3072, False, False), (16, 2048, 6144, False, True), (17, 2048, 6144, False, False),
+    (32, 2048, 2048, False, True), (33, 2048, 2048, False, False), (33, 1024, 2048, True, True), (57, 1024, 2048, True, False), (16, 4096, 2048, False, False), (10, 1664, 2176, True, True), (9, 6144, 2048, True, False)])
+def test_fp32_rows_that_the_dot_products_end_first(decoder, dev, rows, n, k, pair, dots):
+    """Long reductions to few columns stay with the dot products while their blocks fit a round: the bits of eight rows at a time."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(5)
+    x = torch.randn(rows, k, device=dev, generator=gen)
+    w, up = ((torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for _ in range(2))
+
+    def run(first, count):
+        out = torch.full((count, n), 7.0, device=dev)
+        linear = decoder.DecoderLinear(x=x.data_ptr() + 4 * k * first, w=w.data_ptr(), w_up=up.data_ptr() if pair else None, out32=None if pair else out.data_ptr(),
+                                       out=out.data_ptr() if pair else None, ldx=k, ldo=n, n=n, k=k)
+        assert decoder.lib().qm_decoder_linear_rows(C.byref(linear), 1, count, 1, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return out
+
+    got, want = run(0, rows), torch.cat([run(i, min(8, rows - i)) for i in range(0, rows, 8)])
+    assert torch.equal(got, want) == dots
+    assert float((got - want).abs().max()) <= 4e-6 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("pair", [False, True])
 @pytest.mark.parametrize("shift", [0, 1, 2, 3])
 def test_many_fp32_rows_into_any_float_address(decoder, dev, pair, shift):
     """Outputs that are no multiple of 16 bytes are the dot products', which store single floats."""
     import torch
-    rows, n, k, ldo = 40, 1024, 2048, 1028
+    rows, n, k, ldo = 104, 1024, 2048, 1028
     gen = torch.Generator(device=dev).manual_seed(3)
     x = torch.randn(rows, k, device=dev, generator=gen)
     w, up = ((torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for _ in range(2))
