@@ -748,20 +748,21 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_chunk_kernel(PrefillPar
 }
 
 // Combines the runs of the query tiles that prefill_chunk_kernel split: sum over runs of O * w over sum of l * w,
-// w = exp(maximum of the run - largest maximum), in run order.  grid = n_qtiles * 8 * pairs, 256 threads: thread t
-// holds what thread t of a run's block held (column = (row % 16, head) of a wave), and a block takes eight of the
-// thread's 64 values, all runs' loads in flight at once (MOST: no query tile has more runs).  Pairs are dealt to the dies as by
-// prefill_chunk_kernel: the records are then in the L2 of the die that wrote them.  Bound: the records' bytes and two trips to
-// memory (256 rows at 2048, eight runs, 17 MB: 5.3 -> 4.6 us, of them all 21.0 -> 20.3, against single floats and sixteen
-// runs' loads whatever there are; sixteen slices instead of eight change nothing).
+// w = exp(maximum of the run - largest maximum), in run order.  grid = n_qtiles * SLICES * pairs, 256 threads: thread t
+// holds what thread t of a run's block held (column = (row % 16, head) of a wave), and a block takes 64 / SLICES of the
+// thread's 64 values, all runs' loads in flight at once (MOST: no query tile has more runs; left to itself the compiler asks
+// for a few runs at a time, in fewer registers).  Pairs are dealt to the dies as by prefill_chunk_kernel: the records are then
+// in the L2 of the die that wrote them.  Bound: the records' bytes and two trips to memory (a whole call, against single
+// floats and sixteen runs' loads whatever there are: 256 rows at 2048, eight runs, 17 MB, 21.0 -> 20.0 us; sixteen runs in
+// slices of four values: 100 rows at 8000 32.3 -> 31.7, 16 at 8000 22.4 -> 22.1, 40 at 4000 17.1 -> 16.3; in slices of eight 22.7
+// and 16.9 for the last two, and up to 25.3 for the 23.2 of 300 at 4096 with a few runs' loads at a time).
 constexpr int kChunkMaxRuns = 16;
-constexpr int kChunkMergeSlices = 8;
-template <int MOST>
+template <int MOST, int SLICES>
 __global__ __launch_bounds__(kPfThreads) void prefill_chunk_merge_kernel(PrefillParams prm, int round_scores, int gqa_group) {
     request_arguments(prm, round_scores, gqa_group);
     const int pairs = prm.batch * prm.kv_heads;
     const int pair = blockIdx.x % pairs, item = blockIdx.x / pairs;
-    const int slice = item % kChunkMergeSlices, qt = item / kChunkMergeSlices;
+    const int slice = item % SLICES, qt = item / SLICES;
     const int wave_rows = 32 / gqa_group, block_rows = 4 * wave_rows;
     const int q0 = qt * block_rows;
     const int last_tile = min(q0 + prm.cache_before + block_rows - 1, prm.key_count - 1) / kBN;
@@ -772,7 +773,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_chunk_merge_kernel(Prefill
     const float coef = round_scores ? kLog2e : prm.scale * kLog2e;
     const float* rec = prm.chunk_records + (static_cast<int64_t>(pair) * prm.n_qtiles + qt) * prm.chunk_parts * kChunkRecordFloats;
     record2_t ml[MOST];
-    constexpr int kQuads = 16 / kChunkMergeSlices;
+    constexpr int kQuads = 16 / SLICES;
     record4_t ov[MOST][kQuads];
 #pragma unroll
     for (int p = 0; p < MOST; ++p) {
@@ -781,6 +782,7 @@ __global__ __launch_bounds__(kPfThreads) void prefill_chunk_merge_kernel(Prefill
 #pragma unroll
         for (int h = 0; h < kQuads; ++h) ov[p][h] = reinterpret_cast<const record4_t*>(r)[(kQuads * slice + h) * kPfThreads + tid];
     }
+    __builtin_amdgcn_sched_barrier(0);
     float m_all = -INFINITY;
 #pragma unroll
     for (int p = 0; p < MOST; ++p) m_all = fmaxf(m_all, ml[p][0]);
@@ -2033,8 +2035,8 @@ static int32_t launch_chunk_kernels(const PrefillParams& prm, const qm_kv_cache&
     hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(pairs * prm.n_qtiles * prm.chunk_parts)), dim3(kPfThreads), smem, s, prm, cache);
     int32_t rc = launch_status();
     if (rc == QM_OK && prm.chunk_parts > 1) {
-        const auto merge = prm.chunk_parts <= 8 ? prefill_chunk_merge_kernel<8> : prefill_chunk_merge_kernel<kChunkMaxRuns>;
-        hipLaunchKernelGGL(merge, dim3(static_cast<unsigned>(pairs * prm.n_qtiles * kChunkMergeSlices)), dim3(kPfThreads), 0, s, prm, round_scores ? 1 : 0, G);
+        const auto merge = prm.chunk_parts <= 8 ? prefill_chunk_merge_kernel<8, 8> : prefill_chunk_merge_kernel<kChunkMaxRuns, 16>;
+        hipLaunchKernelGGL(merge, dim3(static_cast<unsigned>(pairs * prm.n_qtiles * (prm.chunk_parts <= 8 ? 8 : 16))), dim3(kPfThreads), 0, s, prm, round_scores ? 1 : 0, G);
         rc = launch_status();
     }
     return rc;
