@@ -154,10 +154,69 @@ __device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int
 // The factor that a gate's projection g becomes.
 __device__ __forceinline__ float gate_f32(float g, bool silu) { return silu ? silu_f32(g) : sigmoid_f32(g); }
 
-// One row of the gated norm by a block of 256 threads; sh_red: 4 floats of LDS.
-template <class T>
+// One row of the gated norm's slices, a wave per slice, a slice of up to 256 values held by its lanes.  The values of AT_ONCE slices are
+// asked for at once, and with more than one their weights.
+template <class T, int AT_ONCE>
+__device__ __forceinline__ void gated_norm_slices(const GatedNormParams& prm, const float* o, const float* gate, T* out) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool silu = prm.silu != 0;
+    const float inv_size = 1.0f / static_cast<float>(prm.size);
+    auto weight_at = [&](int at) { return prm.weight ? prm.weight[at] : 1.0f; };
+    for (int g0 = wave; g0 < prm.groups; g0 += AT_ONCE * (kDecThreads / 64)) {
+        float held[AT_ONCE][4], gates[AT_ONCE][4], weights[AT_ONCE][4];
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; ++j) {
+            const int g = min(g0 + j * (kDecThreads / 64), prm.groups - 1);   // (past the last: repeated, not stored)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int c = lane + 64 * i;
+                const bool in = c < prm.size;
+                const int at = g * prm.size + (in ? c : 0);
+                const float value = o[at];
+                gates[j][i] = gate[at];
+                if (AT_ONCE > 1) weights[j][i] = weight_at(at);
+                held[j][i] = in ? value : 0.0f;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < AT_ONCE; ++j) {
+            const int g = g0 + j * (kDecThreads / 64);
+            if (g >= prm.groups) break;
+            float sq = 0.0f;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sq = fmaf(held[j][i], held[j][i], sq);
+            for (int c = lane + 256; c < prm.size; c += 64) sq = fmaf(o[g * prm.size + c], o[g * prm.size + c], sq);
+            const float inverse = 1.0f / sqrtf(wave_sum(sq) * inv_size + prm.eps);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int c = lane + 64 * i, at = g * prm.size + c;
+                if (c < prm.size) out[at] = from_f32<T>(held[j][i] * inverse * (AT_ONCE > 1 ? weights[j][i] : weight_at(at)) * gate_f32(gates[j][i], silu));
+            }
+            for (int c = lane + 256; c < prm.size; c += 64) {
+                const int at = g * prm.size + c;
+                out[at] = from_f32<T>(o[at] * inverse * weight_at(at) * gate_f32(gate[at], silu));
+            }
+        }
+    }
+}
+
+// Whether a wave asks for up to four of its slices at once: where more than four values a lane come of it, and for few rows, each a
+// chain of round trips, from three slices on.  One by one a kernel has registers for more waves, which hides as much where rows are
+// many; slices past 256 values are read twice then, from caches that fewer waves spare.  (us, one by one / four: 16 x 128 of 1 row
+// 4.1 / 3.4, of 1024 7.9 / 6.5; 8 x 256 of 12 rows 3.7 / 3.0, of 4000 16.4 / 14.3; 16 x 64 of 12 rows 3.8 / 3.5, of 1024 5.1 / 5.2; 8 x
+// 128 of 12 rows 3.0 / 2.9, of 1024 4.0 / 4.5; 8 x 64 of 1024 3.5 / 4.2; 8 x 512 of 1024 rows 13.3 / 11.2, of 2048 17.5 / 19.8.)
+inline bool gated_norm_many(const GatedNormParams& prm, int rows) {
+    const int slices = (prm.groups + 3) / 4;
+    const bool wide = (slices < 4 ? slices : 4) * (prm.size < 256 ? prm.size : 256) > 256;
+    return (wide && (prm.size <= 256 || rows <= 1024)) || (slices >= 3 && rows <= 512);
+}
+
+// One row of the gated norm by a block of 256 threads; sh_red: 4 floats of LDS.  AT_ONCE: how slices are taken; 0: in a
+// one-token step, where they go by four and a single slice's weights are asked for with its values as well (the block has few waves
+// beside it whatever its registers: 48 tokens of the second design 7990 us, 8160 by the rule for rows).
+template <class T, int AT_ONCE = 0>
 __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64_t row, float* sh_red, T* out) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x;
     const float* o = prm.o + row * prm.ld_o;
     const float* gate = prm.gate + row * prm.ld_gate;
     const bool silu = prm.silu != 0;
@@ -165,8 +224,9 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
     const float inv_size = 1.0f / static_cast<float>(prm.size);
     auto weight_at = [&](int at) { return prm.weight ? prm.weight[at] : 1.0f; };
     constexpr int kHeld = 4;                   // float4s a thread holds between its two uses of a value
-    if (prm.groups == 1 && total % 4 == 0 && prm.ld_o % 4 == 0 && total <= kHeld * 4 * kDecThreads) {
+    if (AT_ONCE <= 1 && prm.groups == 1 && total % 4 == 0 && prm.ld_o % 4 == 0 && total <= kHeld * 4 * kDecThreads) {
         const int vectors = total >> 2;
+        auto weight4 = [&](int v) { return prm.weight ? load4_if(v < vectors, prm.weight, v) : make_float4(1.0f, 1.0f, 1.0f, 1.0f); };
         float4 held[kHeld], g[kHeld], weight[kHeld];
         float sq[1] = {0.0f};
 #pragma unroll
@@ -174,23 +234,21 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
             const int v = tid + i * kDecThreads;
             held[i] = load4_if(v < vectors, o, v);
             g[i] = load4_if(v < vectors, gate, v);
-            weight[i] = prm.weight ? load4_if(v < vectors, prm.weight, v) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+            if (AT_ONCE == 0) weight[i] = weight4(v);
         }
 #pragma unroll
-        for (int i = 0; i < kHeld; ++i) {
-            sq[0] = square_sum(held[i], sq[0]);
-        }
+        for (int i = 0; i < kHeld; ++i) sq[0] = square_sum(held[i], sq[0]);
         block_sums<1>(sq, sh_red);
         const float inverse = 1.0f / sqrtf(sq[0] * inv_size + prm.eps);
 #pragma unroll
         for (int i = 0; i < kHeld; ++i) {
             const int v = tid + i * kDecThreads;
             if (v >= vectors) continue;
-            const float4 w = weight[i];
+            const float4 w = AT_ONCE == 0 ? weight[i] : weight4(v);
             store4(out, v, held[i].x * inverse * w.x * gate_f32(g[i].x, silu), held[i].y * inverse * w.y * gate_f32(g[i].y, silu),
                    held[i].z * inverse * w.z * gate_f32(g[i].z, silu), held[i].w * inverse * w.w * gate_f32(g[i].w, silu));
         }
-    } else if (prm.groups == 1) {
+    } else if (AT_ONCE <= 1 && prm.groups == 1) {
         float sq[1] = {0.0f};
         for (int c = tid; c < total; c += kDecThreads) sq[0] = fmaf(o[c], o[c], sq[0]);
         block_sums<1>(sq, sh_red);
@@ -198,44 +256,7 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
         for (int c = tid; c < total; c += kDecThreads)
             out[c] = from_f32<T>(o[c] * inverse * weight_at(c) * gate_f32(gate[c], silu));
     } else {
-        // a wave per slice, a slice of up to 256 values held by its lanes; the values of four slices are asked for at once
-        constexpr int kAtOnce = 4;
-        for (int g0 = wave; g0 < prm.groups; g0 += kAtOnce * (kDecThreads / 64)) {
-            float held[kAtOnce][4], gates[kAtOnce][4], weights[kAtOnce][4];
-#pragma unroll
-            for (int j = 0; j < kAtOnce; ++j) {
-                const int g = min(g0 + j * (kDecThreads / 64), prm.groups - 1);   // (past the last: repeated, not stored)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int c = lane + 64 * i;
-                    const bool in = c < prm.size;
-                    const int at = g * prm.size + (in ? c : 0);
-                    const float value = o[at];
-                    gates[j][i] = gate[at];
-                    weights[j][i] = weight_at(at);
-                    held[j][i] = in ? value : 0.0f;
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < kAtOnce; ++j) {
-                const int g = g0 + j * (kDecThreads / 64);
-                if (g >= prm.groups) break;
-                float sq = 0.0f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) sq = fmaf(held[j][i], held[j][i], sq);
-                for (int c = lane + 256; c < prm.size; c += 64) sq = fmaf(o[g * prm.size + c], o[g * prm.size + c], sq);
-                const float inverse = 1.0f / sqrtf(wave_sum(sq) * inv_size + prm.eps);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int c = lane + 64 * i;
-                    if (c < prm.size) out[g * prm.size + c] = from_f32<T>(held[j][i] * inverse * weights[j][i] * gate_f32(gates[j][i], silu));
-                }
-                for (int c = lane + 256; c < prm.size; c += 64) {
-                    const int at = g * prm.size + c;
-                    out[at] = from_f32<T>(o[at] * inverse * weight_at(at) * gate_f32(gate[at], silu));
-                }
-            }
-        }
+        gated_norm_slices<T, AT_ONCE == 1 ? 1 : 4>(prm, o, gate, out);
     }
     for (int c = total + tid; c < prm.ld_out; c += kDecThreads) out[c] = from_f32<T>(0.0f);
 }

@@ -13,11 +13,11 @@ __global__ __launch_bounds__(kDecThreads) void residual_norm_kernel(ResidualPara
     residual_norm_row<T, NV>(prm, row, sh_red, static_cast<T*>(prm.h) + row * prm.ld_h, true);
 }
 
-template <class T>
+template <class T, int AT_ONCE>
 __global__ __launch_bounds__(kDecThreads) void gated_norm_kernel(GatedNormParams prm) {
     __shared__ float sh_red[4];
     const int64_t row = blockIdx.x;
-    gated_norm_row<T>(prm, row, sh_red, static_cast<T*>(prm.out) + row * prm.ld_out);
+    gated_norm_row<T, AT_ONCE>(prm, row, sh_red, static_cast<T*>(prm.out) + row * prm.ld_out);
 }
 
 int32_t check_residual(const ResidualParams& prm) {
@@ -57,8 +57,10 @@ int32_t launch_gated_norm(const GatedNormParams& prm, int rows, int f32, hipStre
     if (rows < 0 || prm.groups <= 0 || prm.size <= 0 || prm.ld_out < static_cast<int64_t>(prm.groups) * prm.size) return QM_ERR_ARGUMENT;
     if (!prm.o || !prm.gate || !prm.out) return QM_ERR_NULL;
     if (rows == 0) return QM_OK;
-    if (f32) hipLaunchKernelGGL(gated_norm_kernel<float>, dim3(rows), dim3(kDecThreads), 0, stream, prm);
-    else hipLaunchKernelGGL(gated_norm_kernel<uint16_t>, dim3(rows), dim3(kDecThreads), 0, stream, prm);
+    const bool many = prm.groups > 1 && gated_norm_many(prm, rows);
+    const auto kernel = f32 ? (many ? gated_norm_kernel<float, 4> : gated_norm_kernel<float, 1>)
+                            : (many ? gated_norm_kernel<uint16_t, 4> : gated_norm_kernel<uint16_t, 1>);
+    hipLaunchKernelGGL(kernel, dim3(rows), dim3(kDecThreads), 0, stream, prm);
     return launch_status();
 }
 

@@ -116,6 +116,27 @@ def test_gated_norm(decoder, dev, f32, groups, size, ld, silu):
 
 
 @pytest.mark.parametrize("f32", [True, False])
+@pytest.mark.parametrize("groups,size", [(4, 65), (5, 128), (5, 129), (8, 128), (8, 129), (9, 3), (9, 64), (9, 86), (16, 64), (17, 256), (8, 300)])
+@pytest.mark.parametrize("rows", [1, 512, 513, 1025])
+def test_gated_norm_in_slices_at_once(decoder, dev, f32, groups, size, rows):
+    """Slices one by one and four at a time, around the lines between them in rows, slices and sizes."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(groups * size)
+    n = groups * size
+    ld = (n + 127) // 128 * 128
+    o, gate, weight = torch.randn(rows, n, device=dev, generator=gen), torch.randn(rows, n, device=dev, generator=gen), torch.randn(n, device=dev, generator=gen)
+    out = torch.full((rows + 1, ld), 7.0, device=dev, dtype=activation(f32))
+    op = decoder.GatedNorm(o=o.data_ptr(), weight=weight.data_ptr(), gate=gate.data_ptr(), out=out.data_ptr(), ld_o=n, ld_gate=n, ld_out=ld, groups=groups,
+                           size=size, eps=0.02)
+    assert decoder.lib().qm_gated_norm_rows(C.byref(op), rows, int(f32), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    wide = o.double().reshape(rows, groups, size)
+    want = (wide / (wide.square().mean(2, keepdim=True) + 0.02).sqrt()).reshape(rows, n) * weight.double() * torch.sigmoid(gate.double())
+    close(out[:rows, :n].float().cpu().numpy(), want.cpu().numpy(), f32)
+    assert bool((out[:rows, n:] == 0).all()) and bool((out[rows:] == 7).all())
+
+
+@pytest.mark.parametrize("f32", [True, False])
 @pytest.mark.parametrize("n", [16, 48, 64, 80])
 @pytest.mark.parametrize("rows,k,ldx,ldo", [(1, 128, 128, 128), (7, 256, 264, 132), (16, 128, 128, 128), (33, 384, 392, 140), (200, 2048, 2048, 128)])
 def test_linear_of_few_columns(decoder, dev, f32, rows, k, ldx, ldo, n):
