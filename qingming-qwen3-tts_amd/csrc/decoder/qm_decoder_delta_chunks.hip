@@ -44,6 +44,9 @@ inline int delta_prepare_lds(int dim) {
     return kDeltaChunk + half + (half > squares ? half : squares);
 }
 
+// AHEAD: a block asks for its keys, queries and rates before it forms the decays, and holds them meanwhile.  Without, they are asked for
+// as they are used, in registers for twice as many blocks of a CU (170 and 108).
+template <bool AHEAD>
 __global__ __launch_bounds__(kDecThreads) void delta_chunk_prepare_kernel(DeltaParams prm) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, l16 = lane & 15;
@@ -69,11 +72,13 @@ __global__ __launch_bounds__(kDecThreads) void delta_chunk_prepare_kernel(DeltaP
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int i = i0 + e * kDecThreads, t = i / z_stride, r = i - t * z_stride;
+            if (i - tid >= kDeltaChunk * z_stride) break;          // (for all threads at once)
             z[e] = prm.proj[(t0 + min(t, tokens - 1)) * prm.ld_proj + prm.z_column + min(r, prm.rank - 1)];
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int i = i0 + e * kDecThreads, t = i / z_stride, r = i - t * z_stride;
+            if (i - tid >= kDeltaChunk * z_stride) break;
             if (i < kDeltaChunk * z_stride) zs[i] = t < tokens && r < prm.rank ? tanhf(z[e]) : 0.0f;
         }
     }
@@ -91,19 +96,26 @@ __global__ __launch_bounds__(kDecThreads) void delta_chunk_prepare_kernel(DeltaP
         sq[e] = wave_sum(sq[e]);
         if (lane == 0 && t < tokens) inverse[t] = 1.0f / sqrtf(sq[e] + prm.unit_eps);
     }
-    // k, r and a of the thread's channel and sixteen tokens (of the first 128 channels: further ones when their turn comes)
-    float k_of[16], r_of[16], a_of[16];
-    auto request_tokens = [&](int i) __attribute__((always_inline)) {
-        const int c = i % dp, first = i / dp * 16;
+    // k, r and a of the thread's channel and four tokens, of its sixteen (ahead: those of the first 128 channels; further ones when their
+    // turn comes)
+    float k_of[AHEAD ? 4 : 1][4], r_of[AHEAD ? 4 : 1][4], a_of[AHEAD ? 4 : 1][4];
+    auto request_tokens = [&](int i, int quad, int to) __attribute__((always_inline)) {
+        const int c = i % dp, first = i / dp * 16 + 4 * quad;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
+        for (int e = 0; e < 4; ++e) {
             const float* p = prm.proj + min(t0 + first + e, prm.rows - 1) * prm.ld_proj + head * dim + min(c, dim - 1);
-            k_of[e] = p[prm.k_column];
-            r_of[e] = p[prm.r_column];
-            a_of[e] = p[prm.a_column];
+            k_of[to][e] = p[prm.k_column];
+            r_of[to][e] = p[prm.r_column];
+            a_of[to][e] = p[prm.a_column];
         }
     };
-    request_tokens(min(tid, 2 * dp - 1));
+    auto request_all = [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int quad = 0; quad < 4; ++quad) request_tokens(i, quad, quad);
+    };
+    if constexpr (AHEAD) {
+        if (64 * wave < 2 * dp) request_all(min(tid, 2 * dp - 1));
+    }
     __syncthreads();
     const int all = prm.heads * dim;
     for (int i = tid; i < 2 * dp; i += kDecThreads) {              // decays: a thread takes a channel of sixteen tokens
@@ -114,7 +126,7 @@ __global__ __launch_bounds__(kDecThreads) void delta_chunk_prepare_kernel(DeltaP
         for (int t = 0; t < 16; ++t) z[t] = bias;
         if (c < dim) {
             const float* w2 = prm.w2 + head * dim + c;
-#pragma unroll 8
+#pragma unroll(AHEAD ? 8 : 4)
             for (int r = 0; r < prm.rank; r += 4) {
                 float w[4];
 #pragma unroll
@@ -157,17 +169,20 @@ __global__ __launch_bounds__(kDecThreads) void delta_chunk_prepare_kernel(DeltaP
         const int i = tid + n * kDecThreads, c = i % dp, first = i / dp * 16;
         if (i >= 2 * dp) break;
         const float bias = c < dim ? prm.a_bias[head * dim + c] : 0.0f;
-        if (n > 0) request_tokens(i);
-#pragma unroll
+        if constexpr (AHEAD) {
+            if (n > 0) request_all(i);
+        }
+#pragma unroll(AHEAD ? 4 : 1)
         for (int quad = 3; quad >= 0; --quad) {
-            const int t1 = first + 4 * quad;
+            const int t1 = first + 4 * quad, from = AHEAD ? quad : 0;
+            if constexpr (!AHEAD) request_tokens(i, quad, 0);
             float k[4], r[4], a[4], at_[4], kt_[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const bool in = t1 + e < tokens && c < dim;
-                k[e] = in ? k_of[4 * quad + e] : 0.0f;
-                r[e] = in ? r_of[4 * quad + e] : 0.0f;
-                a[e] = a_of[4 * quad + e];
+                k[e] = in ? k_of[from][e] : 0.0f;
+                r[e] = in ? r_of[from][e] : 0.0f;
+                a[e] = a_of[from][e];
             }
 #pragma unroll
             for (int e = 3; e >= 0; --e) {
@@ -428,14 +443,21 @@ int64_t delta_scratch_floats(int rows, int heads, int dim) {
 // (the rank-sized projection's tanh shares the LDS of three matrices)
 bool delta_chunks_fit(const DeltaParams& prm) { return delta_z_stride(prm.rank) <= 3 * mfma32_stride(prm.dim); }
 
+// Ahead while no CU has more than two blocks, or LDS for no more.  (us, the whole rule, as used / ahead: 32 heads of 64 over 300 rows, 320
+// blocks, 45.9 / 44.9, over 1024 86.8 / 98.2; 64 heads of 32 over 512 rows 57.0 / 66; 16 heads of 128, two blocks' LDS, over 1024 115.4 /
+// 110.7, over 2048 221 / 213.)
+static bool delta_ahead(int64_t blocks, int lds) { return blocks <= 512 || 3 * lds > 160 * 1024; }
+
 int32_t launch_delta_chunks(const DeltaParams& prm, hipStream_t stream) {
     const int chunks = (prm.rows + kDeltaChunk - 1) / kDeltaChunk;
     const int lds = static_cast<int>(sizeof(float)) * delta_prepare_lds(prm.dim);
-    static std::atomic<bool> raised[kMaxDevices];
-    const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(delta_chunk_prepare_kernel), kDotLdsMost, raised);
+    static std::atomic<bool> raised[2][kMaxDevices];
+    int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(delta_chunk_prepare_kernel<false>), kDotLdsMost, raised[0]);
+    if (rc == QM_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(delta_chunk_prepare_kernel<true>), kDotLdsMost, raised[1]);
     if (rc != QM_OK) return rc;
     if (lds > kDotLdsMost || prm.scratch_floats < delta_scratch_floats(prm.rows, prm.heads, prm.dim)) return QM_ERR_WORKSPACE;
-    hipLaunchKernelGGL(delta_chunk_prepare_kernel, dim3(chunks, prm.heads), dim3(kDecThreads), lds, stream, prm);
+    const auto prepare = delta_ahead(static_cast<int64_t>(chunks) * prm.heads, lds) ? delta_chunk_prepare_kernel<true> : delta_chunk_prepare_kernel<false>;
+    hipLaunchKernelGGL(prepare, dim3(chunks, prm.heads), dim3(kDecThreads), lds, stream, prm);
     const dim3 grid(prm.heads, (prm.dim + 15) / 16);
     if (prm.dim <= 64) hipLaunchKernelGGL(delta_chunk_walk_kernel<1>, grid, dim3(kDecThreads), 0, stream, prm, chunks);
     else if (prm.dim <= 128) hipLaunchKernelGGL(delta_chunk_walk_kernel<2>, grid, dim3(kDecThreads), 0, stream, prm, chunks);

@@ -582,6 +582,33 @@ def test_general_delta(decoder, dev, chunked, heads, dim, rank):
         close(get(s), state, True, tol32=2e-5)
 
 
+@pytest.mark.parametrize("heads,dim,rank,rows", [(33, 20, 7, 530), (35, 64, 36, 513), (32, 16, 4, 512), (32, 16, 3, 545)])
+def test_general_delta_in_many_blocks(decoder, dev, heads, dim, rank, rows):
+    """Passes around 512 blocks and more of small heads, which ask for a chunk's rows as they use them."""
+    import torch
+    rng = np.random.default_rng(rows)
+    every = heads * dim
+    proj = rng.standard_normal((rows, 4 * every + rank)).astype(np.float32)
+    columns = dict(r_column=0, k_column=every, v_column=2 * every, a_column=3 * every, z_column=4 * every)
+    w2 = (rng.standard_normal((rank, every)) * 2 * rank ** -0.5).astype(np.float32)
+    w0, bias = (rng.standard_normal(every) * 3 - 2).astype(np.float32), rng.standard_normal(every).astype(np.float32)
+    p = proj.astype(np.float64)
+    part = lambda name: p[:, columns[name]:columns[name] + every].reshape(rows, heads, dim)
+    w = np.exp(-np.exp(-0.5) * plain.sigmoid(np.tanh(p[:, 4 * every:]) @ w2 + w0)).reshape(rows, heads, dim)
+    a = plain.sigmoid(part("a_column") + bias.reshape(heads, dim))
+    want, state = plain.generalized_delta(part("r_column"), w, part("k_column"), part("v_column"), a)
+    d = [put(v, dev) for v in (proj, w2, w0, bias)]
+    s, out = torch.zeros((heads, dim, dim), device=dev), torch.full((rows, every), 7.0, device=dev)
+    floats = decoder.lib().qm_general_delta_scratch_floats(rows, heads, dim)
+    scratch = torch.full((floats,), float("nan"), device=dev)
+    op = decoder.GeneralDelta(proj=d[0].data_ptr(), w2=d[1].data_ptr(), w0=d[2].data_ptr(), a_bias=d[3].data_ptr(), state=s.data_ptr(), out=out.data_ptr(),
+                              scratch=scratch.data_ptr(), ld_proj=proj.shape[1], scratch_floats=floats, rows=rows, heads=heads, dim=dim, rank=rank,
+                              unit_eps=1e-6, **columns)
+    assert decoder.lib().qm_general_delta_rows(C.byref(op), torch.cuda.current_stream().cuda_stream) == 0
+    close(get(out), want.reshape(rows, -1), True, tol32=2e-5)          # (as in the smaller passes)
+    close(get(s), state, True, tol32=2e-5)
+
+
 @pytest.mark.parametrize("chunked", [False, True])
 @pytest.mark.parametrize("heads,dim,vdim,rot_dims", [(3, 16, 24, 16), (2, 20, 36, 6), (1, 48, 16, 0), (4, 64, 128, 64), (2, 132, 200, 130), (2, 256, 64, 256)])
 def test_retention(decoder, dev, chunked, heads, dim, vdim, rot_dims):
