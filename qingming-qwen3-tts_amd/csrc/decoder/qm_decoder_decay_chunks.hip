@@ -21,10 +21,7 @@ struct DecayBlock {
     static constexpr int kPasses = kDecayChunk / kRows;
 };
 constexpr int kDecayPStride = kDecayChunk + 4;
-// More blocks of four waves than CUs share CUs, and every one stages its head's queries and keys and makes their scores anew: then
-// blocks of eight waves, half as many.  Outputs and states (us, four waves / eight): 8 heads of 128 by 256, 777 rows 25.6 / 19.6 and
-// 15.6 / 14.1; 16 heads of 64 by 128, 1024 rows 18.5 / 15.0 and 11.4 / 10.7.  Below, four waves spread over twice the CUs.
-constexpr int kDecayWide = 256;
+constexpr int kDecayCus = 256;
 constexpr int kScoreTiles = 10;                // 16 x 16 tiles of a chunk's scores on and below the diagonal
 
 // Rotation of every row's q and k in place, k scaled: a block per row, a pair's angle once for all heads.
@@ -262,11 +259,33 @@ int64_t decay_scratch_floats(int rows, int heads, int dim, int vdim) {
 }
 
 template <int W>
+static int decay_output_lds(int dim) {
+    const int stride = mfma32_stride(dim);
+    return static_cast<int>(sizeof(float)) * kDecayChunk * (stride + std::max(stride, kDecayPStride + DecayBlock<W>::kVStride));
+}
+
+// More blocks of four waves than CUs share CUs, and every one stages its head's queries and keys and makes their scores anew: then
+// blocks of eight waves, half as many.  Outputs and states (us, four waves / eight): 8 heads of 128 by 256, 777 rows 25.6 / 19.6 and
+// 15.6 / 14.1; 16 heads of 64 by 128, 1024 rows 18.5 / 15.0 and 11.4 / 10.7.  Below, four waves spread over twice the CUs.
+// Beyond one round of the wide blocks, heads of up to some 64 channels, of which a CU takes three narrow blocks, go back to those where the
+// wide ones' last round or last slice would be mostly empty (a whole pass, four waves / eight: 16 heads of 64 by 128, 1300 rows 39.3 / 41.7,
+// 1800 52.5 / 45.5; 12 of 64 by 192, 850 rows 34.1 / 40.2; 32 of 32 by 96, 700 rows 30.9 / 32.7, 850 40.3 / 35.3; 16 heads of 128 by 128,
+// 1300 rows 70.4 / 69.1).
+static bool decay_wide(const DecayAttentionParams& prm, int chunks) {
+    if (prm.vdim <= DecayBlock<4>::kSlice) return false;
+    const int64_t pairs = static_cast<int64_t>(prm.heads) * chunks;
+    const int64_t narrow = pairs * ((prm.vdim + DecayBlock<4>::kSlice - 1) / DecayBlock<4>::kSlice);
+    const int64_t wide = pairs * ((prm.vdim + DecayBlock<8>::kSlice - 1) / DecayBlock<8>::kSlice), rounds = (wide + kDecayCus - 1) / kDecayCus;
+    if (narrow <= kDecayCus) return false;
+    return rounds == 1 || 3 * decay_output_lds<4>(prm.dim) > 160 * 1024 || 20 * narrow >= 17 * 2 * kDecayCus * rounds;
+}
+
+template <int W>
 static int32_t decay_chunks_as(const DecayAttentionParams& prm, int chunks, hipStream_t stream) {
     using Block = DecayBlock<W>;
     const int stride = mfma32_stride(prm.dim), slices = (prm.vdim + Block::kSlice - 1) / Block::kSlice;
     const int state_lds = static_cast<int>(sizeof(float)) * kDecayChunk * (stride + Block::kVStride);
-    const int output_lds = static_cast<int>(sizeof(float)) * kDecayChunk * (stride + std::max(stride, kDecayPStride + Block::kVStride));
+    const int output_lds = decay_output_lds<W>(prm.dim);
     static std::atomic<bool> raised[2][kMaxDevices];
     int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decay_chunk_state_kernel<W>), kDotLdsMost, raised[0]);
     if (rc == QM_OK) rc = ensure_dynamic_lds(reinterpret_cast<const void*>(decay_chunk_output_kernel<W>), kDotLdsMost, raised[1]);
@@ -285,8 +304,7 @@ static int32_t decay_chunks_as(const DecayAttentionParams& prm, int chunks, hipS
 int32_t launch_decay_chunks(const DecayAttentionParams& prm, hipStream_t stream) {
     const int chunks = (prm.rows + kDecayChunk - 1) / kDecayChunk;
     if (chunks > 65535 || prm.scratch_floats < decay_scratch_floats(prm.rows, prm.heads, prm.dim, prm.vdim)) return QM_ERR_WORKSPACE;
-    const int64_t blocks = static_cast<int64_t>(prm.heads) * chunks * ((prm.vdim + DecayBlock<4>::kSlice - 1) / DecayBlock<4>::kSlice);
-    return prm.vdim > DecayBlock<4>::kSlice && blocks > kDecayWide ? decay_chunks_as<8>(prm, chunks, stream) : decay_chunks_as<4>(prm, chunks, stream);
+    return decay_wide(prm, chunks) ? decay_chunks_as<8>(prm, chunks, stream) : decay_chunks_as<4>(prm, chunks, stream);
 }
 
 }  // namespace qm

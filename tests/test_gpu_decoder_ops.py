@@ -526,9 +526,10 @@ def test_decay_attention(decoder, dev, chunked, heads, dim, vdim):
         close(get(s), state, True, tol32=5e-6)
 
 
-@pytest.mark.parametrize("heads,dim,vdim,rows", [(8, 20, 200, 573), (6, 64, 129, 961), (16, 132, 72, 530), (8, 128, 256, 512), (8, 128, 256, 513)])
+@pytest.mark.parametrize("heads,dim,vdim,rows", [(8, 20, 200, 573), (6, 64, 129, 961), (16, 132, 72, 530), (8, 128, 256, 512), (8, 128, 256, 513),
+                                                   (12, 64, 192, 700), (16, 20, 66, 1800)])
 def test_decay_attention_in_wide_blocks(decoder, dev, heads, dim, vdim, rows):
-    """Passes of around and of more than 256 blocks of 64 value channels, which blocks of 128 take over."""
+    """Passes of around and of more than 256 blocks of 64 value channels, which blocks of 128 take over, and past one round of those."""
     import torch
     rng = np.random.default_rng(rows)
     decay = np.array([0.999, 1.0, 0.3, 0.0, 0.9, 0.99, 0.5, 0.75] * 2)[:heads]
