@@ -455,8 +455,8 @@ def test_fp32_attention_of_many_rows_against_the_row_kernel(decoder, dev, shape)
             got = case.run(decoder, dev, True, [rows], rows_only=rows_only)
             close(got, want, True, tol32=2e-5)
             worst[rows_only].append(np.sqrt(np.mean((got - want) ** 2)))
-    # (the root mean square over some thousand outputs: 1.5 leaves room for the draw alone)
-    assert np.mean(worst[False]) <= 1.5 * np.mean(worst[True])
+    # (over 24 draws of five shapes the ratio was 0.98 to 1.02, and one draw's scatters by 0.07: seven draws' mean by 0.03; five times that)
+    assert np.mean(worst[False]) <= 1.15 * np.mean(worst[True])
     whole = AttentionCase(shape, 100, seed=3)
     plain_result = whole.run(decoder, dev, True, [100])
     for at, what in ((99, np.inf), (50, np.nan), (17, -np.inf), (18, np.inf)):
