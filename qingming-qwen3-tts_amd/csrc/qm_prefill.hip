@@ -110,11 +110,11 @@ struct PrefillParams {
     int chunk_paged;
 };
 
-// A run's record, value by value of the threads: 16 times four of O (unnormalised), then reference maximum and sum.  (The
-// workspace is aligned for floats.)
+// A run's record, value by value of the threads: 16 times four of O (unnormalised), then reference maximum and sum.  (Both entries
+// refuse a workspace that is not aligned to 256 bytes, and a record is a multiple of that.)
 constexpr int kChunkRecordFloats = 66 * kPfThreads;
-typedef float record4_t __attribute__((ext_vector_type(4), aligned(4)));
-typedef float record2_t __attribute__((ext_vector_type(2), aligned(4)));
+typedef float record4_t __attribute__((ext_vector_type(4)));
+typedef float record2_t __attribute__((ext_vector_type(2)));
 
 struct PfStage {
     uint16_t k[kBN * kKS];
