@@ -45,6 +45,7 @@
 #include "qm_host.h"
 #include "qm_norm_rope_head.h"
 #include "qm_predictor_chain.h"
+#include "qm_resident.h"
 #include "qm_sampler_block.h"
 
 namespace qm {
@@ -152,19 +153,11 @@ struct FrParams {
 };
 
 struct FrShared {
-    float waves[8];
-    float total;
+    __attribute__((aligned(16))) float waves[8];    // the eight 32-lane sums of a norm
     int abort;
     int code;
     float residual[8];              // [row of the pass][the block's four down_proj rows]
 };
-
-__device__ __forceinline__ uint32_t agent_load(const uint32_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void agent_store(uint32_t* p, uint32_t v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // This thread's words tid, tid + 256, ... of a tagged vector, all requested at once, again and again until
 // every one carries `tag`.  False when the wait gave up (or another block did).
@@ -201,15 +194,36 @@ __device__ __forceinline__ void request_rows(const uint16_t* src, int rows, unsi
     }
 }
 
-// One M = 1 linear operator, this block's R outputs (channels if DUAL).  The weights are in LDS already (requested
-// long before); the input vector arrives as tagged words (or plain bf16 for the step's first operator) and
-// becomes fp32 in LDS, through the fused prologue if there is one:
+// A row segment's weights of one lane as fp32, from what lds_read_* brought.
+template <bool PAIRS, int STEPS>
+__device__ __forceinline__ void widen_weights(uint32_t (&raw)[STEPS], float (&w)[PAIRS ? 2 * STEPS : STEPS]) {
+#pragma unroll
+    for (int j = 0; j < STEPS; ++j) {
+        if constexpr (PAIRS) {
+            w[2 * j] = lo_bf16(raw[j]);
+            w[2 * j + 1] = hi_bf16(raw[j]);
+        } else {
+            w[j] = bf2f(static_cast<uint16_t>(raw[j]));
+        }
+    }
+}
+
+// One M = 1 linear operator, this block's R outputs (channels if DUAL).  The weights are in LDS already: they were requested a layer
+// ago, and every operator since has seen all of its wave's requests land before its barrier.  So a thread takes its weights into
+// registers, widened, BEFORE it waits for the input: behind the arrival of the input lie only the norm, its exchange and the sums.
+// (Cycles from the input vector to the outputs, weights read and widened then / before: Q/K/V 1700 / 850, o_proj 1600 / 750,
+// gate/up 2880 / 1570, down_proj 2320 / 1000; three frames with four talker layers 4.83 -> 4.43 ms.)  The reads are written out (qm_resident.h): the compiler would have each of its own wait for the
+// requests just made for the next layer.
+// The input vector arrives as tagged words (or plain bf16 for the step's first operator) and becomes fp32 in LDS, through the fused
+// prologue if there is one:
 //   PRE 1: RMSNorm(input) * norm_w (rmsnorm_kernel, R17:8276-8338);
 //   PRE 2: residual = bf16(input + addend), then RMSNorm(residual) * norm_w (R17:16205-16286), the block keeping
 //          the residual of its own down_proj rows.
 // Then 32 threads per output walk the reference's 32 chains (PAIRS: lane l takes the pairs k = 2l, 2l + 1, then
 // + 64, ... as the predictor's kernels do, R17:12110-12120; else k = l, l + 32, ... as the talker's), the
 // reference's shuffle tree adds them and lane 0 rounds, adds what the operator adds and stores the tagged word.
+// The input lies in LDS so that a lane reads four values of its chain with one instruction: element j of lane l's chain in
+// 16-byte piece 32 (j / 4) + l.
 template <bool DUAL, int PRE, bool PAIRS, int K, int R>
 __device__ __forceinline__ bool linear_phase(FrShared& sh, unsigned char* smem, int lds_weights,
                                              const uint32_t* x_words, uint32_t x_tag, const uint16_t* x_plain,
@@ -219,8 +233,15 @@ __device__ __forceinline__ bool linear_phase(FrShared& sh, unsigned char* smem, 
                                              const uint32_t* abort_word, unsigned spin_limit, int row = 0) {
     constexpr int N = K / kFrThreads;                   // input columns per thread: tid, tid + 256, ...
     constexpr int kStride = fr_row_stride(K);
+    constexpr int kPasses = (R + 7) / 8;                // eight outputs (channels) at a time
+    constexpr int kSteps = PAIRS ? K / 64 : K / 32;     // LDS reads of a lane per weight row
+    constexpr int kChain = K / 32;                      // products of a lane per output
+    static_assert(R % 2 == 0 && kChain % 4 == 0, "a wave's two outputs both exist or neither does");
     float* lin_x = reinterpret_cast<float*>(smem + kFrLdsScratch);
     const int tid = threadIdx.x;
+    const int l = tid & 31;             // reference lane
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool works = 2 * wave < R;    // (R = 4: two waves have no output)
 
     uint32_t norm_raw[N];
     if (PRE != 0) {
@@ -228,7 +249,40 @@ __device__ __forceinline__ bool linear_phase(FrShared& sh, unsigned char* smem, 
         for (int u = 0; u < N; ++u) norm_raw[u] = norm_w[tid + kFrThreads * u];
     }
     uint32_t bias_raw = 0;
-    if (bias && (tid & 31) == 0 && (tid >> 5) < R) bias_raw = bias[first_out + (tid >> 5)];
+    if (bias && l == 0 && (tid >> 5) < R) bias_raw = bias[first_out + (tid >> 5)];
+
+    float w[kPasses][kChain], wu[DUAL ? kPasses : 1][DUAL ? kChain : 1];
+    if (works) {
+        uint32_t raw[kPasses][kSteps], raw_up[DUAL ? kPasses : 1][DUAL ? kSteps : 1];
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+            const int c = 8 * p + (tid >> 5);           // (an output that does not exist takes the first one's weights)
+            const uint32_t at = lds_at(smem + lds_weights) + static_cast<uint32_t>((c < R ? (DUAL ? 2 * c : c) : 0) * kStride);
+            if constexpr (PAIRS) {
+                lds_read_b32<0, kSteps, 128>(at + 4u * l, raw[p]);
+                if constexpr (DUAL) lds_read_b32<0, kSteps, 128>(at + kStride + 4u * l, raw_up[p]);
+            } else {
+                lds_read_u16<0, kSteps, 64>(at + 2u * l, raw[p]);
+                if constexpr (DUAL) lds_read_u16<0, kSteps, 64>(at + kStride + 2u * l, raw_up[p]);
+            }
+        }
+        lds_wait();
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+            pin<0, kSteps>(raw[p]);
+            if constexpr (DUAL) pin<0, kSteps>(raw_up[p]);
+        }
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+            widen_weights<PAIRS, kSteps>(raw[p], w[p]);
+            pin<0, kChain>(w[p]);
+            if constexpr (DUAL) {
+                widen_weights<PAIRS, kSteps>(raw_up[p], wu[p]);
+                pin<0, kChain>(wu[p]);
+            }
+        }
+    }
 
     uint32_t x_raw[N], add_raw[N];
     bool ok = true;
@@ -241,10 +295,14 @@ __device__ __forceinline__ bool linear_phase(FrShared& sh, unsigned char* smem, 
     if (PRE == 2) ok = poll_words<N>(add_words, add_tag, abort_word, spin_limit, add_raw) && ok;
     if (!ok) sh.abort = 1;
 
+    // where this thread's columns tid, tid + 256, ... lie: 256 words apart in either order
+    const int place = PAIRS ? (tid >> 7) * 128 + ((tid >> 1) & 31) * 4 + ((tid >> 6) & 1) * 2 + (tid & 1)
+                            : (tid >> 7) * 128 + (tid & 31) * 4 + ((tid >> 5) & 3);
     if (PRE == 0) {
 #pragma unroll
-        for (int u = 0; u < N; ++u) lin_x[tid + kFrThreads * u] = bf2f(static_cast<uint16_t>(x_raw[u]));
+        for (int u = 0; u < N; ++u) lin_x[place + kFrThreads * u] = bf2f(static_cast<uint16_t>(x_raw[u]));
     } else {
+        float value[N];
         float local_sum = 0.0f;
 #pragma unroll
         for (int u = 0; u < N; ++u) {
@@ -254,96 +312,68 @@ __device__ __forceinline__ bool linear_phase(FrShared& sh, unsigned char* smem, 
                 v = bf2f(f2bf(v + bf2f(static_cast<uint16_t>(add_raw[u]))));
                 if (k >= keep_residual_first && k < keep_residual_first + 4) sh.residual[4 * row + k - keep_residual_first] = v;
             }
-            lin_x[k] = v;
+            value[u] = v;
             local_sum = fmaf(v, v, local_sum);
         }
-        const float total = block_sum_256_like_reference(local_sum, sh.waves, &sh.total);
+        // block_sum_256_like_reference with one barrier: every thread adds the eight groups' sums in the second tree's order
+        // (its leaves past the eighth are +0, and a sum of squares is not -0)
+        const float tree = half_wave_tree_sum(local_sum);
+        if (l == 0) sh.waves[tid >> 5] = tree;
+        __syncthreads();
+        const float4 even = *reinterpret_cast<const float4*>(sh.waves), odd = *reinterpret_cast<const float4*>(sh.waves + 4);
+        const float total = ((even.x + odd.x) + (even.z + odd.z)) + ((even.y + odd.y) + (even.w + odd.w));
         const float inverse_rms = 1.0f / sqrtf(total / static_cast<float>(K) + epsilon);
 #pragma unroll
-        for (int u = 0; u < N; ++u) {
-            const int k = tid + kFrThreads * u;
-            lin_x[k] = round_bf16(round_bf16(lin_x[k] * inverse_rms) * bf2f(static_cast<uint16_t>(norm_raw[u])));
-        }
+        for (int u = 0; u < N; ++u)
+            lin_x[place + kFrThreads * u] = round_bf16(round_bf16(value[u] * inverse_rms) * bf2f(static_cast<uint16_t>(norm_raw[u])));
     }
-    __builtin_amdgcn_s_waitcnt(0);      // this wave's weight pieces have landed
+    __builtin_amdgcn_s_waitcnt(0);      // everything this wave has requested so far has landed: the operators behind this one read it
     __syncthreads();
-    if (sh.abort) return false;
-
-    const int l = tid & 31;             // reference lane
-    // This lane's share of the input vector, read once for all passes; then per output all of its weights are
-    // requested from LDS before the chain starts, so that the chain waits for additions, not for reads.
-    constexpr int kSteps = PAIRS ? K / 64 : K / 32;
-    float2 x_pair[PAIRS ? kSteps : 1];
-    float x_one[PAIRS ? 1 : kSteps];
-    if (PAIRS) {
-        const float2* xp = reinterpret_cast<const float2*>(lin_x) + l;
+    const int aborted = sh.abort;       // (looked at before anything leaves)
+    if (works) {
+        float acc[kPasses], up[kPasses];
 #pragma unroll
-        for (int j = 0; j < kSteps; ++j) x_pair[j] = xp[32 * j];
-    } else {
-        const float* xs = lin_x + l;
+        for (int p = 0; p < kPasses; ++p) acc[p] = up[p] = 0.0f;
+        const float4* xp = reinterpret_cast<const float4*>(lin_x) + l;
+        float4 x[kChain / 4];
 #pragma unroll
-        for (int j = 0; j < kSteps; ++j) x_one[j] = xs[32 * j];
-    }
-#pragma unroll 1
-    for (int c0 = 0; c0 < R; c0 += 8) {
-        const int c = c0 + (tid >> 5);
-        const bool live = c < R;
-        const unsigned char* row0 = smem + lds_weights + (live ? (DUAL ? 2 * c : c) : 0) * kStride;
-        const unsigned char* row1 = row0 + kStride;                 // DUAL only: the up row
-        float acc = 0.0f, up = 0.0f;
-        if (PAIRS) {
-            const uint32_t* p0 = reinterpret_cast<const uint32_t*>(row0) + l;
-            const uint32_t* p1 = reinterpret_cast<const uint32_t*>(row1) + l;
-            uint32_t a[kSteps], b[DUAL ? kSteps : 1];
+        for (int j = 0; j < kChain / 4; ++j) x[j] = xp[32 * j];
 #pragma unroll
-            for (int j = 0; j < kSteps; ++j) {
-                a[j] = p0[32 * j];
-                if (DUAL) b[j] = p1[32 * j];
-            }
+        for (int j = 0; j < kChain / 4; ++j) {
+            const float v[4] = {x[j].x, x[j].y, x[j].z, x[j].w};
 #pragma unroll
-            for (int j = 0; j < kSteps; ++j) {
-                acc = fmaf(x_pair[j].x, lo_bf16(a[j]), acc);
-                acc = fmaf(x_pair[j].y, hi_bf16(a[j]), acc);
-                if (DUAL) {
-                    up = fmaf(x_pair[j].x, lo_bf16(b[j]), up);
-                    up = fmaf(x_pair[j].y, hi_bf16(b[j]), up);
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int p = 0; p < kPasses; ++p) {
+                    acc[p] = fmaf(v[e], w[p][4 * j + e], acc[p]);
+                    if constexpr (DUAL) up[p] = fmaf(v[e], wu[p][4 * j + e], up[p]);
                 }
             }
-        } else {
-            const uint16_t* w0 = reinterpret_cast<const uint16_t*>(row0) + l;
-            const uint16_t* w1 = reinterpret_cast<const uint16_t*>(row1) + l;
-            uint32_t a[kSteps], b[DUAL ? kSteps : 1];
-#pragma unroll
-            for (int j = 0; j < kSteps; ++j) {
-                a[j] = w0[32 * j];
-                if (DUAL) b[j] = w1[32 * j];
-            }
-#pragma unroll
-            for (int j = 0; j < kSteps; ++j) {
-                acc = fmaf(x_one[j], bf2f(static_cast<uint16_t>(a[j])), acc);
-                if (DUAL) up = fmaf(x_one[j], bf2f(static_cast<uint16_t>(b[j])), up);
-            }
         }
-        // the reference's shuffle tree over its 32 lanes; lane 0 holds the sum
-        acc = half_wave_tree_sum(acc);
-        if (DUAL) up = half_wave_tree_sum(up);
-        if (l == 0 && live) {
-            uint16_t bits;
-            if (DUAL) {
-                const float gv = bf2f(f2bf(acc));
-                const uint16_t act = f2bf(gv / (1.0f + expf(-gv)));
-                bits = f2bf(bf2f(act) * bf2f(f2bf(up)));
-            } else {
-                float r = acc;
-                if (bias) r += bf2f(static_cast<uint16_t>(bias_raw));
-                bits = f2bf(r);
-                if (add_residual) bits = f2bf(sh.residual[4 * row + c] + bf2f(bits));
+#pragma unroll
+        for (int p = 0; p < kPasses; ++p) {
+            const int c = 8 * p + (tid >> 5);
+            // the reference's shuffle tree over its 32 lanes; lane 0 holds the sum
+            acc[p] = half_wave_tree_sum(acc[p]);
+            if (DUAL) up[p] = half_wave_tree_sum(up[p]);
+            if (l == 0 && c < R && !aborted) {
+                uint16_t bits;
+                if (DUAL) {
+                    const float gv = bf2f(f2bf(acc[p]));
+                    const uint16_t act = f2bf(gv / (1.0f + expf(-gv)));
+                    bits = f2bf(bf2f(act) * bf2f(f2bf(up[p])));
+                } else {
+                    float r = acc[p];
+                    if (bias) r += bf2f(static_cast<uint16_t>(bias_raw));
+                    bits = f2bf(r);
+                    if (add_residual) bits = f2bf(sh.residual[4 * row + c] + bf2f(bits));
+                }
+                agent_store(out_words + first_out + c, (out_tag << 16) | bits);
             }
-            agent_store(out_words + first_out + c, (out_tag << 16) | bits);
         }
     }
-    __syncthreads();                    // every read of the weights and of the input vector is done
-    return true;
+    __syncthreads();                    // every read of the input vector is done
+    return !aborted;
 }
 
 // QK-norm + RoPE + cache append + attention of one kv head for one step (R17:12133-12290, 12314-12575): the head's
@@ -523,6 +553,7 @@ __global__ __launch_bounds__(kFrThreads, 1) void predictor_frame_kernel(FrParams
     const bool samples = b == kFrBlocks - 1;
     unsigned long long rng = 0;
     if (tid == 0) rng = *prm.rng_state;        // every block keeps the generator's state: all draw, the last one stores it
+    __builtin_amdgcn_s_waitcnt(0);             // (the first operator reads its weights before it waits for anything else)
     __syncthreads();
 
     uint32_t* const hidden = ws + kFrWsHidden;
@@ -665,6 +696,7 @@ __global__ __launch_bounds__(kFrThreads, 1) void predictor_frame_kernel(FrParams
             float score[kSmpPerThread];
 #pragma unroll
             for (int j = 0; j < kSmpPerThread; ++j) score[j] = j < kFrVocab / kFrThreads ? bf2f(static_cast<uint16_t>(raw[j])) : 0.0f;
+            __builtin_amdgcn_s_waitcnt(0);     // (the projection's weights, which the next pass may read first thing)
             __syncthreads();
             if (sh.abort) break;
             SamplerParams sp = {};

@@ -52,6 +52,13 @@ __device__ __forceinline__ void pin(uint32_t (&v)[N]) {
         pin<J + 1, N>(v);
     }
 }
+template <int J, int N>
+__device__ __forceinline__ void pin(float (&v)[N]) {
+    if constexpr (J < N) {
+        asm volatile("" : "+v"(v[J]));
+        pin<J + 1, N>(v);
+    }
+}
 __device__ __forceinline__ uint32_t lds_word(const void* p) {
     uint32_t v;
     asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(v) : "v"(lds_at(p)) : "memory");
