@@ -378,108 +378,112 @@ __device__ __forceinline__ bool linear_phase(FrShared& sh, unsigned char* smem, 
 
 // QK-norm + RoPE + cache append + attention of one kv head for one step (R17:12133-12290, 12314-12575): the head's
 // K/V rows of this frame live in LDS for the whole launch (and are written to the caller's caches as they come).
+// Everybody else waits for the eight blocks that run this, so it is two barriers long: a wave takes its own head's words (no
+// exchange before the norm), a wave's keys are scored side by side, every wave forms its head's softmax for itself (4 400 -> 3 500
+// cycles from the projections' arrival to the context; three frames 4.43 -> 4.35 ms).
 __device__ __forceinline__ bool attention_phase(FrShared& sh, unsigned char* smem, const FrParams& prm, const FrLayer& w, int kvh,
                                                 int position, const uint32_t* qkv_words, uint32_t in_tag, uint32_t* ctx_words,
                                                 uint32_t out_tag, const uint32_t* abort_word, unsigned spin_limit) {
-    uint16_t* xq = reinterpret_cast<uint16_t*>(smem + kFrLdsScratch);   // [2][128] the two heads' projections, then rotated
-    uint16_t* xk = xq + 2 * kDim;                                       // [128]
-    uint16_t* xv = xk + kDim;                                           // [128]
-    float* probs = reinterpret_cast<float*>(xv + kDim);                 // [2][16] scores, then probabilities
+    uint16_t* xq = reinterpret_cast<uint16_t*>(smem + kFrLdsScratch);   // [2][128] the two rotated query heads
+    float* scores = reinterpret_cast<float*>(xq + 2 * kDim);            // [2][16]
     uint16_t* kc = reinterpret_cast<uint16_t*>(smem + kFrLdsCache);     // [16][128]
     uint16_t* vc = kc + kFrCache * kDim;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
-    // what the norm needs besides the projections, requested before the wait
+    // waves 0, 1: the two query heads; wave 2: the key; wave 3 moves the value row
     uint16_t g0 = 0, g1 = 0, c0 = 0, c1 = 0, s0 = 0, s1 = 0;
-    if (wave < 3) {
+    if (wave < 3) {                                                     // (requested before the wait)
         const uint16_t* gamma = wave < 2 ? w.q_norm : w.k_norm;
         g0 = gamma[lane]; g1 = gamma[lane + 64];
         c0 = prm.cosine[position * kDim + lane]; c1 = prm.cosine[position * kDim + lane + 64];
         s0 = prm.sine[position * kDim + lane]; s1 = prm.sine[position * kDim + lane + 64];
     }
-    // this thread's two words: one of the head pair's 256 query values, one of the 128 + 128 key / value values
-    const uint32_t* first = qkv_words + 2 * kDim * kvh + tid;
-    const uint32_t* second = qkv_words + (tid < kDim ? kFrQDim + kDim * kvh + tid : kFrQDim + kFrKvDim + kDim * kvh + (tid - kDim));
+    const uint32_t* words = qkv_words + lane
+        + (wave < 2 ? kDim * (2 * kvh + wave) : kFrQDim + (wave == 2 ? 0 : kFrKvDim) + kDim * kvh);
     uint32_t a = 0, b = 0;
     bool ok = false;
     for (unsigned spins = 0;; ++spins) {
-        a = agent_load(first);
-        b = agent_load(second);
+        a = agent_load(words);
+        b = agent_load(words + 64);
         if ((a >> 16) == in_tag && (b >> 16) == in_tag) { ok = true; break; }
         if (spins >= spin_limit) break;
         if ((spins & 255u) == 255u && agent_load(abort_word) != 0u) break;
         __builtin_amdgcn_s_sleep(1);
     }
     if (!ok) sh.abort = 1;
-    xq[tid] = static_cast<uint16_t>(a);
-    if (tid < kDim) xk[tid] = static_cast<uint16_t>(b); else xv[tid - kDim] = static_cast<uint16_t>(b);
-    __syncthreads();
-    if (sh.abort) return false;
-
-    // waves 0, 1: the two query heads; wave 2: the key; wave 3 moves the value row
+    const bool arrived = __builtin_amdgcn_ballot_w64(!ok) == 0;          // this wave's head is whole
     const int64_t cache_at = (static_cast<int64_t>(kvh) * kFrCache + position) * kDim;
     if (wave < 3) {
-        uint16_t* x = wave < 2 ? xq + kDim * wave : xk;
-        const HeadPair r = norm_rope_head_values(x[lane], x[lane + 64], true, g0, g1, c0, c1, s0, s1, prm.epsilon);
+        const HeadPair r = norm_rope_head_values(static_cast<uint16_t>(a), static_cast<uint16_t>(b), true, g0, g1, c0, c1, s0, s1, prm.epsilon);
         if (wave < 2) {
-            x[lane] = r.lo; x[lane + 64] = r.hi;
+            xq[kDim * wave + lane] = r.lo; xq[kDim * wave + lane + 64] = r.hi;
         } else {
             kc[position * kDim + lane] = r.lo; kc[position * kDim + lane + 64] = r.hi;
-            w.key_cache[cache_at + lane] = r.lo; w.key_cache[cache_at + lane + 64] = r.hi;
+            if (arrived) { w.key_cache[cache_at + lane] = r.lo; w.key_cache[cache_at + lane + 64] = r.hi; }
         }
     } else {
         // V is appended as it is (R17:12279-12288)
-        const uint16_t v0 = xv[lane], v1 = xv[lane + 64];
+        const uint16_t v0 = static_cast<uint16_t>(a), v1 = static_cast<uint16_t>(b);
         vc[position * kDim + lane] = v0; vc[position * kDim + lane + 64] = v1;
-        w.value_cache[cache_at + lane] = v0; w.value_cache[cache_at + lane + 64] = v1;
+        if (arrived) { w.value_cache[cache_at + lane] = v0; w.value_cache[cache_at + lane + 64] = v1; }
     }
     __syncthreads();
+    if (sh.abort) return false;
 
-    // scores: a 32-lane half wave per (head, key); reference lane l accumulates dims l, l + 32, l + 64, l + 96, then the
-    // shuffle tree; bf16(sum), bf16(that * scale) (R17:12386-12418)
+    // scores: a 32-lane half wave per (head, key), a wave the keys wave, wave + 4, ... side by side; reference lane l accumulates
+    // dims l, l + 32, l + 64, l + 96, then the shuffle tree; bf16(sum), bf16(that * scale) (R17:12386-12418)
     {
-        const int half = tid >> 5, l = tid & 31, g = half & 1;
+        const int g = (tid >> 5) & 1, l = tid & 31;
         const float scale = __uint_as_float(0x3db504f3U);   // kAttentionScaleBits, R17:9354-9356
         float q4[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) q4[c] = bf2f(xq[kDim * g + l + 32 * c]);
-        for (int j = half >> 1; j <= position; j += 4) {
-            float acc = 0.0f;
+#pragma unroll 1
+        for (int j = wave; j <= position; j += 8) {         // (rows past the position hold zeros or an older frame's keys: not stored)
+            float acc[2] = {0.0f, 0.0f};
+            uint16_t k4[2][4];
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc = fmaf(q4[c], bf2f(kc[j * kDim + l + 32 * c]), acc);
-            acc = half_wave_tree_sum(acc);
-            if (l == 0) probs[16 * g + j] = rbf(rbf(acc) * scale);
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) k4[u][c] = kc[min(j + 4 * u, kFrCache - 1) * kDim + l + 32 * c];
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) acc[u] = fmaf(q4[c], bf2f(k4[u][c]), acc[u]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u) acc[u] = half_wave_tree_sum(acc[u]);
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (l == 0 && j + 4 * u <= position) scores[16 * g + j + 4 * u] = rbf(rbf(acc[u]) * scale);
         }
     }
-    __syncthreads();
-    // softmax: 16 lanes per head; the sum in the shuffle tree's order (R17:12449-12509)
-    if (tid < 32) {
-        const int t = tid & 15;
-        const bool inside = t <= position;
-        const float score = inside ? probs[tid] : -INFINITY;
-        float maximum = score;
+    // P.V: thread (head, d) (R17:12515-12574); its column of V is on its way while the scores are exchanged
+    const int g = wave >> 1, d = tid & 127;
+    float vcol[kFrCache];
 #pragma unroll
-        for (int offset = 8; offset > 0; offset >>= 1) maximum = fmaxf(maximum, __shfl_xor(maximum, offset, 16));
-        const float e = inside ? expf(score - maximum) : 0.0f;
-        float total = e;
-#pragma unroll
-        for (int offset = 8; offset > 0; offset >>= 1) total += __shfl_xor(total, offset, 16);
-        probs[tid] = inside ? rbf(e / total) : 0.0f;
-    }
+    for (int j = 0; j < kFrCache; ++j) vcol[j] = bf2f(vc[j * kDim + d]);
     __syncthreads();
-    // P.V: thread (head, d) (R17:12515-12574)
-    {
-        const int g = tid >> 7, d = tid & 127;
-        float vcol[kFrCache];
+    // softmax of the wave's head in each of its 16-lane rows; the sum in the shuffle tree's order (R17:12449-12509): a rotation by 8,
+    // 4, 2, 1 inside the row brings a lane the value its xor partner holds
+    const bool inside = (lane & 15) <= position;
+    const float score = inside ? scores[16 * g + (lane & 15)] : -INFINITY;
+    float maximum = score;
+    maximum = fmaxf(maximum, row_ror<8>(maximum));
+    maximum = fmaxf(maximum, row_ror<4>(maximum));
+    maximum = fmaxf(maximum, row_ror<2>(maximum));
+    maximum = fmaxf(maximum, row_ror<1>(maximum));
+    const float e = inside ? expf(score - maximum) : 0.0f;
+    const float total = row16_allreduce_sum(e);
+    const float weight = inside ? rbf(e / total) : 0.0f;
+    float probs[kFrCache];
 #pragma unroll
-        for (int j = 0; j < kFrCache; ++j) vcol[j] = bf2f(vc[j * kDim + d]);
-        const float o = pv_limited(probs + 16 * g, vcol, position + 1);
-        const uint16_t bits = __builtin_bit_cast(uint16_t, static_cast<__bf16>(o));
-        agent_store(ctx_words + kDim * (2 * kvh + g) + d, (out_tag << 16) | bits);
-    }
-    __syncthreads();
+    for (int j = 0; j < kFrCache; ++j) probs[j] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(weight), j));
+    const float o = pv_limited(probs, vcol, position + 1);
+    const uint16_t bits = __builtin_bit_cast(uint16_t, static_cast<__bf16>(o));
+    agent_store(ctx_words + kDim * (2 * kvh + g) + d, (out_tag << 16) | bits);
+    __syncthreads();                    // every read of the scores is done
     return true;
 }
 
