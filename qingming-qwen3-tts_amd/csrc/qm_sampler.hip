@@ -12,20 +12,16 @@
 // so the first `keep` entries of the sorted sequence are a property of the scores, not of the
 // sorting algorithm.  Thread 0 then sums exp(score / T - maximum) over them in double, in that
 // order, draws one SplitMix64 number and walks the running sum.  Here the first `keep` entries
-// are found without sorting the rest: every score becomes a 64-bit key (order-preserving image
-// of the float above, inverted id below), the keep-th largest key is found by a radix select
-// over the key's 44 significant bits (histogram passes of 8 bits, one bin per thread, ended as
-// soon as the bin of the keep-th key is wanted whole: two passes for typical scores), the
-// `keep` keys at or above it are gathered and ranked by counting.  The exponentials are computed
-// by `keep` threads at once; the sums stay one thread's, in the reference's order: the running
-// sum of the second loop repeats the partial sums of the first, so one pass gives both.
+// are found without sorting the rest (qm_sampler_block.h): a radix select, a gather of the few keys from its
+// bin on up, ranks by counting.  The exponentials are computed by `keep` threads at once; the sums stay one thread's, in
+// the reference's order: the running sum of the second loop repeats the partial sums of the first, so one pass gives both.
 // One block of 256 threads; vocab <= 4096 (the reference's sort size), top_k <= 256.
 //
 // The kernel is a chain of short dependent steps, so what costs is latency.  Measured with cycle
 // stamps, 2048 bf16 scores, top 50 (21 us at first, 7.5 us now, of which about 5 are the launch):
 // a load per element inside the arithmetic waits for each in turn (16 x 1 100 cycles; now all
-// requested at once: 1 900); LDS additions to one address take turns (a pass 2 400 cycles;
-// with eight counters per bin, prefix sums by DPP instead of shuffles and three barriers: 1 000);
+// requested at once: 1 900); LDS additions to one address take turns (a pass of 8-bit digits 2 400
+// cycles; of 12-bit digits, prefix sums by DPP instead of shuffles and three barriers: about 1 000);
 // a counter handed round for the gather (3 000; now a prefix sum over per-thread counts); the
 // unrolled pass loop made the compiler compute all passes' digits ahead and spill (40 000).
 //
@@ -38,6 +34,8 @@
 
 namespace qm {
 
+// NARROW: the scores are bf16 and are taken as they are.
+template <bool NARROW>
 __global__ __launch_bounds__(kSmpThreads) void sampler_kernel(SamplerParams prm) {
     request_arguments(prm);
     __shared__ SamplerScratch scratch;
@@ -62,7 +60,7 @@ __global__ __launch_bounds__(kSmpThreads) void sampler_kernel(SamplerParams prm)
     unsigned long long rng = 0;
     if (tid == 0 && prm.top_k > 0 && !prm.process_only) rng = *prm.rng_state;
     const unsigned long long before = rng;
-    const int32_t chosen = sampler_block(prm, scratch, score, rng);
+    const int32_t chosen = sampler_block<NARROW>(prm, scratch, score, rng);
     if (tid != 0 || chosen == -2) return;
     if (rng != before) *prm.rng_state = rng;
     prm.output_id[0] = chosen;
@@ -120,7 +118,8 @@ inline int32_t launch_sampler(const SamplerParams& prm, void* hip_stream) {
     if (prm.vocab <= 0 || prm.offset < 0) return QM_ERR_ARGUMENT;
     if (prm.vocab > kSmpMaxVocab || prm.top_k > kSmpMaxKeep) return QM_ERR_GEOMETRY;
     if (prm.top_k > 0 && !(prm.temperature > 0.0f)) return QM_ERR_ARGUMENT;
-    hipLaunchKernelGGL(sampler_kernel, dim3(1), dim3(kSmpThreads), 0, static_cast<hipStream_t>(hip_stream), prm);
+    if (prm.is_bf16 && !prm.process) hipLaunchKernelGGL(sampler_kernel<true>, dim3(1), dim3(kSmpThreads), 0, static_cast<hipStream_t>(hip_stream), prm);
+    else hipLaunchKernelGGL(sampler_kernel<false>, dim3(1), dim3(kSmpThreads), 0, static_cast<hipStream_t>(hip_stream), prm);
     return launch_status();
 }
 

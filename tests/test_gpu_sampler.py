@@ -155,3 +155,22 @@ def test_sampler_argument_errors(qm, dev):
                                   None, None) == -1
     assert L.qm_final_head_sample(x.data_ptr(), o.data_ptr(), -1, 3072, 2150, 1024, 1.05, 50, 0.9, st.data_ptr(),
                                   o.data_ptr(), None, None) == -5
+
+
+@pytest.mark.parametrize("top_k", [1, 49, 50, 64, 65, 128, 200, 256])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_selection_where_the_bound_lets_many_keys_through(oracle, qm, dev, top_k, bf16):
+    """The select looks at each thread's largest score first (ids t, t + 256, ... are thread t's) and ranks what reaches the bound:
+    equal scores, one thread with all of the largest, vocabularies around top_k, 64, 128 and 256 candidates."""
+    rng = np.random.default_rng(top_k + (1000 if bf16 else 0))
+    draws = rng.standard_normal(4096).astype(np.float32)
+    crowded = np.where(np.arange(4096) % 256 == 77, draws + 40.0, draws)
+    cases = [(draws, 4096), (crowded, 4096), (np.full(4096, -0.75), 4096), (np.round(draws), 2048), (np.where(draws > 1.5, 3.0, draws), 3000),
+             (np.where(draws > 0, 0.0, -0.0), 700), (-np.abs(draws) - 1000.0, 2048)]
+    cases += [(draws, max(1, top_k + d)) for d in (-1, 0, 1)] + [(np.round(draws), n) for n in (63, 64, 65, 127, 129, 255, 256, 257)]
+    for i, (scores, vocab) in enumerate(cases):
+        scores = np.ascontiguousarray(scores[:vocab], dtype=np.float32)
+        if bf16:
+            scores = oracle.f32_to_bf16(scores)
+        want = _cpu_sample(oracle, scores, bf16, 0, vocab, top_k, 0.9, 31 + i, draws=12)
+        assert _gpu_sample(qm, dev, scores, bf16, 0, vocab, top_k, 0.9, 31 + i, draws=12) == want, (i, vocab)
