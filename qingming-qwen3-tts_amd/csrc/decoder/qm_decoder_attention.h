@@ -218,8 +218,8 @@ __device__ __forceinline__ void chunk_attention_block(const ChunkAttentionParams
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
                     float v = acc[g][x][e];
-                    v += __shfl_xor(v, 16, 64);
-                    v += __shfl_xor(v, 32, 64);
+                    v = xor16_sum(v);
+                    v = xor32_sum(v);
                     const int c = x * 128 + l16 * 8 + e;
                     if (sub == 0 && c < prm.v_stride) combine[(wave * GQ + g) * prm.v_stride + c] = v;
                 }

@@ -110,8 +110,8 @@ __global__ __launch_bounds__(WAVES * 64) void chunk_attention_f32_kernel(ChunkAt
             p[r] = whole || (key >= lo && key <= position) ? score : -INFINITY;
             largest = fmaxf(largest, p[r]);
         }
-        largest = fmaxf(largest, __shfl_xor(largest, 16, 64));
-        largest = fmaxf(largest, __shfl_xor(largest, 32, 64));
+        largest = xor16_max(largest);
+        largest = xor32_max(largest);
         const float before = m;
         m = fmaxf(m, largest);
         const float reference = m == -INFINITY ? 0.0f : m;                 // (a row that has seen no key yet: all its weights are zero)
@@ -172,8 +172,8 @@ __global__ __launch_bounds__(WAVES * 64) void chunk_attention_f32_kernel(ChunkAt
     }
 
     // the waves' shares of the keys, combined by all threads
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = xor16_sum(l);
+    l = xor32_sum(l);
     float* sh_ml = sh_sums + WAVES * kF32AttentionRows * kStride;
     float* own = sh_sums + (wave * kF32AttentionRows + l16) * kStride + 16 * g;
 #pragma unroll

@@ -159,7 +159,7 @@ __global__ __launch_bounds__(kFlashThreads) void chunk_attention_mfma_kernel(Chu
         float largest = p[0];
 #pragma unroll
         for (int r = 1; r < 16; ++r) largest = fmaxf(largest, p[r]);
-        largest = fmaxf(largest, __shfl_xor(largest, 32, 64));
+        largest = xor32_max(largest);
         const float before = m;
         m = fmaxf(m, largest);
         const float reference = m == -INFINITY ? 0.0f : m;         // (a row that has seen no key yet: all its weights are zero)
@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kFlashThreads) void chunk_attention_mfma_kernel(Chu
     }
 
     // the four parts of the keys, combined by the first
-    l += __shfl_xor(l, 32, 64);
+    l = xor32_sum(l);
     constexpr int kAtOnce = Shape::kCombineTiles;
     float* shared = reinterpret_cast<float*>(smem);
     float* sh_ml = shared + 2 * (kFlashParts - 1) * kAtOnce * 16 * 64;         // [2 pairs][parts - 1][2][32]

@@ -26,14 +26,16 @@ __device__ __forceinline__ float silu_f32(float z) { return z * sigmoid_f32(z); 
 // Sum / maximum over the 64 lanes of a wave, in every lane.
 __device__ __forceinline__ float wave_sum(float v) {
     v = row16_allreduce_sum(v);
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
+    v = xor16_sum(v);
+    v = xor32_sum(v);
     return v;
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int m = 1; m < 64; m *= 2) v = fmaxf(v, __shfl_xor(v, m, 64));
-    return v;
+    v = fmaxf(v, row_ror<8>(v));
+    v = fmaxf(v, row_ror<4>(v));
+    v = fmaxf(v, row_ror<2>(v));
+    v = fmaxf(v, row_ror<1>(v));
+    return xor32_max(xor16_max(v));
 }
 
 // N sums over the 256 threads of a block at once, in every thread.  sh: 4 * N floats of LDS, free again for the next call

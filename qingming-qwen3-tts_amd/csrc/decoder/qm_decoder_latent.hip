@@ -81,9 +81,9 @@ __global__ __launch_bounds__(kDecThreads) void latent_query_kernel(LatentAttenti
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             float v = acc[r][e];
-            v += __shfl_xor(v, 8, 64);
-            v += __shfl_xor(v, 16, 64);
-            v += __shfl_xor(v, 32, 64);
+            v += row_ror<8>(v);
+            v = xor16_sum(v);
+            v = xor32_sum(v);
             if (lane < 8) sh_sum[(wave * R + r) * 64 + lane * 8 + e] = v;
         }
     __syncthreads();

@@ -135,8 +135,8 @@ __global__ __launch_bounds__(kDecThreads) void latent_partials_mfma_kernel(Laten
             p[i] = 16 * (i >> 2) + (i & 3) <= last ? s[i >> 2][i & 3] * to_log2 : -INFINITY;
             largest = fmaxf(largest, p[i]);
         }
-        largest = fmaxf(largest, __shfl_xor(largest, 16, 64));
-        largest = fmaxf(largest, __shfl_xor(largest, 32, 64));
+        largest = xor16_max(largest);
+        largest = xor32_max(largest);
         const float before = m;
         m = fmaxf(m, largest);
         const float reference = m == -INFINITY ? 0.0f : m;         // (a query that has seen no key yet: all its weights are zero)
@@ -172,8 +172,8 @@ __global__ __launch_bounds__(kDecThreads) void latent_partials_mfma_kernel(Laten
         }
     }
     // the two parts of the keys, combined by the first
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    l = xor16_sum(l);
+    l = xor32_sum(l);
     float* shared = reinterpret_cast<float*>(smem) + half * (kTiles * 4 * 64 + 128);
     __syncthreads();
     if (part == 1) {

@@ -33,8 +33,8 @@ __device__ __forceinline__ void store_state(const float (&s)[RD], float* state, 
     }
 }
 __device__ __forceinline__ float quarter_sum(float v) {
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
+    v = xor16_sum(v);
+    v = xor32_sum(v);
     return v;
 }
 

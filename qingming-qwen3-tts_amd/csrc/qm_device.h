@@ -109,6 +109,25 @@ __device__ __forceinline__ float row16_allreduce_sum(float v) {
     return v;
 }
 
+// v + the value of lane ^ 16 (^ 32) of the wave, and the larger of the two, in every lane.  v_permlane16_swap (v_permlane32_swap) of a
+// register with itself leaves both values in every lane, in one order or the other; a shuffle goes through LDS, some 130 cycles more.
+__device__ __forceinline__ float xor16_sum(float v) {
+    const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+}
+__device__ __forceinline__ float xor32_sum(float v) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(both[0]) + __uint_as_float(both[1]);
+}
+__device__ __forceinline__ float xor16_max(float v) {
+    const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+}
+__device__ __forceinline__ float xor32_max(float v) {
+    const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(both[0]), __uint_as_float(both[1]));
+}
+
 // Logical-token -> page mapping precomputed on the host (a shift when page_size is a power
 // of two, page 0 when the sequence has a single page).
 struct PageMap {
