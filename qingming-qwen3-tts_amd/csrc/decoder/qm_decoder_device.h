@@ -82,8 +82,13 @@ __device__ __forceinline__ float4 weighted(float4 acc, float f, float4 y, float4
     return make_float4(fmaf(f * y.x, w.x, acc.x), fmaf(f * y.y, w.y, acc.y), fmaf(f * y.z, w.z, acc.z), fmaf(f * y.w, w.w, acc.w));
 }
 
-template <class T, int NV>
-__device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int row, float* sh_red, T* h, bool write_x) {
+// `behind` is called when the row's loads have been asked for: a wave's loads come back in the order they were made, and what it asks for
+// (weights, by the megabyte) the sums do not wait for.  EARLY: the norms' weights are among the first loads too (registers).
+struct NothingBehind {
+    __device__ __forceinline__ void operator()() const {}
+};
+template <class T, int NV, bool EARLY = false, class Behind = NothingBehind>
+__device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int row, float* sh_red, T* h, bool write_x, Behind&& behind = Behind()) {
     const int tid = threadIdx.x;
     const int64_t src = prm.row_map ? prm.row_map[row] : row;
     const int vectors = static_cast<int>(prm.ld_h >> 2);
@@ -114,6 +119,20 @@ __device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int
 #pragma unroll
         for (int t = 0; t < 3; ++t) y[t][i] = y_row[t] ? load4_if(in, y_row[t], v) : zero;
     }
+    float4 y_weight[3][EARLY ? NV : 1], step_vec[EARLY ? NV : 1], weight[EARLY ? NV : 1];
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            const int v = tid + i * kDecThreads, from = v < vectors ? v : 0;
+#pragma unroll
+            for (int t = 0; t < 3; ++t) y_weight[t][i] = normed[t] ? load4(prm.term[t].norm_w, from) : one;
+            step_vec[i] = prm.step_vec ? load4(prm.step_vec, from) : zero;
+            weight[i] = load4(prm.norm_w, from);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    behind();
+    __builtin_amdgcn_sched_barrier(0);
     const float inv_width = 1.0f / static_cast<float>(prm.width);
     float factor[3] = {0.0f, 0.0f, 0.0f};
     if (normed[0] || normed[1] || normed[2]) {
@@ -136,9 +155,9 @@ __device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int
         float4 add = zero;
 #pragma unroll
         for (int t = 0; t < 3; ++t)
-            if (y_row[t]) add = weighted(add, factor[t], y[t][i], normed[t] ? load4(prm.term[t].norm_w, v) : one);
+            if (y_row[t]) add = weighted(add, factor[t], y[t][i], EARLY ? y_weight[t][EARLY ? i : 0] : normed[t] ? load4(prm.term[t].norm_w, v) : one);
         x[i] = weighted(x[i], 1.0f, add, one);
-        if (prm.step_vec) x[i] = weighted(x[i], 1.0f, load4(prm.step_vec, v), one);
+        if (prm.step_vec) x[i] = weighted(x[i], 1.0f, EARLY ? step_vec[EARLY ? i : 0] : load4(prm.step_vec, v), one);
         if (write_x && prm.x_out) reinterpret_cast<float4*>(prm.x_out + static_cast<int64_t>(row) * prm.ld_h)[v] = x[i];
         total[0] = square_sum(x[i], total[0]);
     }
@@ -148,7 +167,7 @@ __device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int
     for (int i = 0; i < NV; ++i) {
         const int v = tid + i * kDecThreads;
         if (v >= vectors) continue;
-        const float4 w = load4(prm.norm_w, v);
+        const float4 w = EARLY ? weight[EARLY ? i : 0] : load4(prm.norm_w, v);
         store4(h, v, x[i].x * inverse * w.x, x[i].y * inverse * w.y, x[i].z * inverse * w.z, x[i].w * inverse * w.w);
     }
 }
@@ -158,8 +177,8 @@ __device__ __forceinline__ float gate_f32(float g, bool silu) { return silu ? si
 
 // One row of the gated norm's slices, a wave per slice, a slice of up to 256 values held by its lanes.  The values of AT_ONCE slices are
 // asked for at once, and with more than one their weights.
-template <class T, int AT_ONCE>
-__device__ __forceinline__ void gated_norm_slices(const GatedNormParams& prm, const float* o, const float* gate, T* out) {
+template <class T, int AT_ONCE, class Behind>
+__device__ __forceinline__ void gated_norm_slices(const GatedNormParams& prm, const float* o, const float* gate, T* out, Behind&& behind) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const bool silu = prm.silu != 0;
     const float inv_size = 1.0f / static_cast<float>(prm.size);
@@ -180,6 +199,7 @@ __device__ __forceinline__ void gated_norm_slices(const GatedNormParams& prm, co
                 held[j][i] = in ? value : 0.0f;
             }
         }
+        if (g0 == wave) behind();
 #pragma unroll
         for (int j = 0; j < AT_ONCE; ++j) {
             const int g = g0 + j * (kDecThreads / 64);
@@ -215,9 +235,10 @@ inline bool gated_norm_many(const GatedNormParams& prm, int rows) {
 
 // One row of the gated norm by a block of 256 threads; sh_red: 4 floats of LDS.  AT_ONCE: how slices are taken; 0: in a
 // one-token step, where they go by four and a single slice's weights are asked for with its values as well (the block has few waves
-// beside it whatever its registers: 48 tokens of the second design 7990 us, 8160 by the rule for rows).
-template <class T, int AT_ONCE = 0>
-__device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64_t row, float* sh_red, T* out) {
+// beside it whatever its registers: 48 tokens of the second design 7990 us, 8160 by the rule for rows).  `behind` is called by every wave once,
+// where that can be when its first loads have been asked for.
+template <class T, int AT_ONCE = 0, class Behind = NothingBehind>
+__device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64_t row, float* sh_red, T* out, Behind&& behind = Behind()) {
     const int tid = threadIdx.x;
     const float* o = prm.o + row * prm.ld_o;
     const float* gate = prm.gate + row * prm.ld_gate;
@@ -238,6 +259,7 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
             g[i] = load4_if(v < vectors, gate, v);
             if (AT_ONCE == 0) weight[i] = weight4(v);
         }
+        behind();
 #pragma unroll
         for (int i = 0; i < kHeld; ++i) sq[0] = square_sum(held[i], sq[0]);
         block_sums<1>(sq, sh_red);
@@ -251,6 +273,7 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
                    held[i].z * inverse * w.z * gate_f32(g[i].z, silu), held[i].w * inverse * w.w * gate_f32(g[i].w, silu));
         }
     } else if (AT_ONCE <= 1 && prm.groups == 1) {
+        behind();
         float sq[1] = {0.0f};
         for (int c = tid; c < total; c += kDecThreads) sq[0] = fmaf(o[c], o[c], sq[0]);
         block_sums<1>(sq, sh_red);
@@ -258,44 +281,81 @@ __device__ __forceinline__ void gated_norm_row(const GatedNormParams& prm, int64
         for (int c = tid; c < total; c += kDecThreads)
             out[c] = from_f32<T>(o[c] * inverse * weight_at(c) * gate_f32(gate[c], silu));
     } else {
-        gated_norm_slices<T, AT_ONCE == 1 ? 1 : 4>(prm, o, gate, out);
+        if (static_cast<int>(threadIdx.x >> 6) >= prm.groups) behind();        // (a wave without a slice)
+        gated_norm_slices<T, AT_ONCE == 1 ? 1 : 4>(prm, o, gate, out, behind);
     }
     for (int c = total + tid; c < prm.ld_out; c += kDecThreads) out[c] = from_f32<T>(0.0f);
 }
 
-// One row's heads, combined, by a block of 256 threads; `active` splits hold keys.  sh_w: heads * active floats of LDS.
-template <class T>
-__device__ __forceinline__ void merge_attention_row(const AttentionPartials& p, int64_t row, int active, float* sh_w, T* out, int64_t ld_out) {
+// One row's heads, combined, by a block of 256 threads; `active` splits hold keys.  sh_w: heads * active floats of LDS.  The statistics of four
+// heads a wave and the values of eight splits for two vectors a thread are asked for first, `behind` is called then.
+template <class T, class Behind = NothingBehind>
+__device__ __forceinline__ void merge_attention_row(const AttentionPartials& p, int64_t row, int active, float* sh_w, T* out, int64_t ld_out,
+                                                    Behind&& behind = Behind()) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    for (int h = wave; h < p.heads; h += kDecThreads / 64) {      // each split's factor: a wave per head, a lane per split
-        const int64_t at = ((row * p.heads + h) * p.splits + min(lane, active - 1)) * 2;
-        const float m_read = p.ml[at], l_read = p.ml[at + 1];
-        const float m = lane < active ? m_read : -INFINITY, l = lane < active ? l_read : 0.0f;
-        const float w = fast_exp2((m - wave_max(m)) * kLog2e);
-        const float total = wave_sum(w * l);
-        if (lane < active) sh_w[h * active + lane] = w / total;
-    }
-    __syncthreads();
     const int n = p.heads * p.vdim;
     const float* acc = p.acc + row * p.heads * p.splits * p.vdim;
-    if (p.vdim % 4 == 0) {
-        const int per_head = p.vdim >> 2;
-        for (int i = threadIdx.x; i < n >> 2; i += kDecThreads) {
-            const int h = i / per_head, e = i - h * per_head;
-            const float4* from = reinterpret_cast<const float4*>(acc + static_cast<int64_t>(h) * p.splits * p.vdim) + e;
-            float4 sum = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-            for (int s0 = 0; s0 < active; s0 += 8) {               // (splits past the last: the last one, with factor zero)
-                float4 v[8];
+    const bool vectors = p.vdim % 4 == 0;
+    const int per_head = p.vdim >> 2, all = n >> 2;
+    constexpr int kHeads = 4, kVectors = 2, kSplits = 8;
+    float m_read[kHeads], l_read[kHeads];
+    auto read_heads = [&](int h0) __attribute__((always_inline)) {
 #pragma unroll
-                for (int s = 0; s < 8; ++s) v[s] = from[min(s0 + s, active - 1) * per_head];
+        for (int j = 0; j < kHeads; ++j) {                         // (past the last: repeated, not stored)
+            const int h = min(h0 + j * (kDecThreads / 64), p.heads - 1);
+            const int64_t at = ((row * p.heads + h) * p.splits + min(lane, active - 1)) * 2;
+            m_read[j] = p.ml[at];
+            l_read[j] = p.ml[at + 1];
+        }
+    };
+    float4 v[kVectors][kSplits];
+    auto read_vectors = [&](int i0, int s0) __attribute__((always_inline)) {
 #pragma unroll
-                for (int s = 0; s < 8; ++s) {
-                    const float w = s0 + s < active ? sh_w[h * active + min(s0 + s, active - 1)] : 0.0f;
-                    sum.x = fmaf(w, v[s].x, sum.x); sum.y = fmaf(w, v[s].y, sum.y);
-                    sum.z = fmaf(w, v[s].z, sum.z); sum.w = fmaf(w, v[s].w, sum.w);
+        for (int j = 0; j < kVectors; ++j) {                       // (splits past the last: the last one, with factor zero)
+            const int i = min(i0 + j * kDecThreads, all - 1), h = i / per_head;
+            const float4* from = reinterpret_cast<const float4*>(acc + static_cast<int64_t>(h) * p.splits * p.vdim) + (i - h * per_head);
+#pragma unroll
+            for (int s = 0; s < kSplits; ++s) v[j][s] = from[min(s0 + s, active - 1) * per_head];
+        }
+    };
+    read_heads(wave);
+    if (vectors) read_vectors(static_cast<int>(threadIdx.x), 0);
+    __builtin_amdgcn_sched_barrier(0);
+    behind();
+    __builtin_amdgcn_sched_barrier(0);
+    for (int h0 = wave; h0 < p.heads; h0 += kHeads * (kDecThreads / 64)) {     // each split's factor: a wave per head, a lane per split
+        if (h0 != wave) read_heads(h0);
+#pragma unroll
+        for (int j = 0; j < kHeads; ++j) {
+            const int h = h0 + j * (kDecThreads / 64);
+            const float m = lane < active ? m_read[j] : -INFINITY, l = lane < active ? l_read[j] : 0.0f;
+            const float w = fast_exp2((m - wave_max(m)) * kLog2e);
+            const float total = wave_sum(w * l);
+            if (lane < active && h < p.heads) sh_w[h * active + lane] = w / total;
+        }
+    }
+    __syncthreads();
+    if (vectors) {
+        for (int i0 = threadIdx.x; i0 < all; i0 += kVectors * kDecThreads) {
+            float4 sum[kVectors];
+#pragma unroll
+            for (int j = 0; j < kVectors; ++j) sum[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            for (int s0 = 0; s0 < active; s0 += kSplits) {
+                if (i0 != static_cast<int>(threadIdx.x) || s0 != 0) read_vectors(i0, s0);
+#pragma unroll
+                for (int j = 0; j < kVectors; ++j) {
+                    const int h = min(i0 + j * kDecThreads, all - 1) / per_head;
+#pragma unroll
+                    for (int s = 0; s < kSplits; ++s) {
+                        const float w = s0 + s < active ? sh_w[h * active + min(s0 + s, active - 1)] : 0.0f;
+                        sum[j].x = fmaf(w, v[j][s].x, sum[j].x); sum[j].y = fmaf(w, v[j][s].y, sum[j].y);
+                        sum[j].z = fmaf(w, v[j][s].z, sum[j].z); sum[j].w = fmaf(w, v[j][s].w, sum[j].w);
+                    }
                 }
             }
-            store4(out, i, sum.x, sum.y, sum.z, sum.w);
+#pragma unroll
+            for (int j = 0; j < kVectors; ++j)
+                if (i0 + j * kDecThreads < all) store4(out, i0 + j * kDecThreads, sum[j].x, sum[j].y, sum[j].z, sum[j].w);
         }
     } else {
         for (int i = threadIdx.x; i < n; i += kDecThreads) {
@@ -319,8 +379,9 @@ __device__ __forceinline__ void rotary(int position, double frequency, float& co
 
 // n values divided by their root mean square and weighted, by a block of 256 threads, zeros behind them up to `padded`;
 // sh_red: 4 floats of LDS.
-template <class T>
-__device__ __forceinline__ void slice_norm_row(const float* x, const float* weight, int n, int64_t padded, float eps, float* sh_red, T* out) {
+template <class T, class Behind = NothingBehind>
+__device__ __forceinline__ void slice_norm_row(const float* x, const float* weight, int n, int64_t padded, float eps, float* sh_red, T* out,
+                                               Behind&& behind = Behind()) {
     const int tid = threadIdx.x;
     constexpr int kHeld = 4;
     float held[kHeld], weights[kHeld], sq[1] = {0.0f};
@@ -330,6 +391,7 @@ __device__ __forceinline__ void slice_norm_row(const float* x, const float* weig
         held[i] = x[c];
         weights[i] = weight[c];
     }
+    behind();
 #pragma unroll
     for (int i = 0; i < kHeld; ++i) {
         held[i] = tid + i * kDecThreads < n ? held[i] : 0.0f;

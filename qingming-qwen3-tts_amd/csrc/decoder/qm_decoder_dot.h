@@ -67,13 +67,18 @@ template <int NR>
 __device__ __forceinline__ void dot_request(const DotRows<NR>& d, int k, uint4 (&piece)[kDotAhead][NR]) {
     const int lane = threadIdx.x & 63;
 #pragma unroll
-    for (int u = 0; u < kDotAhead; ++u) dot_request_one<NR>(d, k, u * 512 + lane * 8, piece[u]);
+    for (int u = 0; u < kDotAhead; ++u)
+        if (u * 512 < k) dot_request_one<NR>(d, k, u * 512 + lane * 8, piece[u]);
 }
+struct NoRefill {
+    __device__ __forceinline__ void operator()(int) const {}
+};
 
-// One tile: xs holds R input rows [R][k] in LDS, `piece` the first pieces.
-template <class T, int R, int NR>
+// One tile: xs holds R input rows [R][k] in LDS, `piece` the first pieces.  `refill` is called with a piece's number when the tile has no
+// more use for it.
+template <class T, int R, int NR, class Refill = NoRefill>
 __device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRows<NR>& d, uint4 (&piece)[kDotAhead][NR], const T* xs, int row0,
-                                           int rows) {
+                                           int rows, Refill&& refill = Refill()) {
     const int lane = threadIdx.x & 63;
     const int k = g.k;
     float acc[NR][R];
@@ -92,6 +97,7 @@ __device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRow
                     for (int i = 0; i < NR; ++i) acc[i][r] = dot8(piece[u][i], xs + r * k + at, acc[i][r]);
             }
             if (k0 + kDotAhead * 512 < k) dot_request_one<NR>(d, k, at + kDotAhead * 512, piece[u]);
+            else refill(u);
         }
     }
 #pragma unroll

@@ -28,20 +28,30 @@ __global__ __launch_bounds__(kDecThreads) void layer_in_kernel(LayerInParams prm
     int g = dot_group<kInRows>(prm.linears, tile);
     DotRows<kInRows> d = dot_rows<kInRows>(prm.linears.group[g], tile);
     uint4 piece[kDotAhead][kInRows];
-    dot_request<kInRows>(d, prm.linears.group[g].k, piece);
-    residual_norm_row<T, NV>(prm.residual, 0, sh_red, hs, blockIdx.x == 0);
+    // Rows of up to 1024 columns: the norm's inputs are asked for before the weights and do not come back behind them (48 tokens of the second
+    // design at that width 7920 -> 7820 us).  Longer rows want the weights under way at once (of the first design at 2048: 7210, 7340 the other way).
+    const int k = prm.residual.ld_h;                                           // (every linear's)
+    const auto weights = [&] { dot_request<kInRows>(d, k, piece); };
+    if constexpr (NV > 1) weights();
+    if constexpr (NV > 1) residual_norm_row<T, NV>(prm.residual, 0, sh_red, hs, blockIdx.x == 0);
+    else residual_norm_row<T, NV, true>(prm.residual, 0, sh_red, hs, blockIdx.x == 0, weights);
     __syncthreads();
     if (prm.residual.h && blockIdx.x == 0) {
         T* out = static_cast<T*>(prm.residual.h);
         for (int c = threadIdx.x; c < prm.residual.ld_h; c += kDecThreads) out[c] = hs[c];
     }
     for (int next = static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x);; next += static_cast<int>(gridDim.x)) {
-        dot_finish<T, 1, kInRows>(prm.linears.group[g], d, piece, hs, 0, 1);
-        if (next >= tiles) break;
+        if (next >= tiles) {
+            dot_finish<T, 1, kInRows>(prm.linears.group[g], d, piece, hs, 0, 1);
+            break;
+        }
         tile = next;
-        g = dot_group<kInRows>(prm.linears, tile);
-        d = dot_rows<kInRows>(prm.linears.group[g], tile);
-        dot_request<kInRows>(d, prm.linears.group[g].k, piece);
+        const int then = dot_group<kInRows>(prm.linears, tile);
+        const DotRows<kInRows> rows = dot_rows<kInRows>(prm.linears.group[then], tile);
+        const int lane = threadIdx.x & 63;
+        dot_finish<T, 1, kInRows>(prm.linears.group[g], d, piece, hs, 0, 1, [&](int u) { dot_request_one<kInRows>(rows, k, u * 512 + lane * 8, piece[u]); });
+        g = then;
+        d = rows;
     }
 }
 
@@ -56,15 +66,16 @@ __global__ __launch_bounds__(kDecThreads) void layer_out_kernel(LayerOutParams p
     const DecLinearGroup& group = prm.linears.group[g];
     const DotRows<kOutRows> d = dot_rows<kOutRows>(group, tile);
     uint4 piece[kDotAhead][kOutRows];
-    dot_request<kOutRows>(d, group.k, piece);
+    const auto weights = [&] { dot_request<kOutRows>(d, group.k, piece); };    // (behind what makes the input)
     if (prm.input[g] == 1) {
         merge_attention_row<T>(prm.part, 0, attention_active_splits(*prm.position_dev, prm.chunk, prm.part.keys_per_split),
-                               reinterpret_cast<float*>(xs + most_k), xs, group.k);
+                               reinterpret_cast<float*>(xs + most_k), xs, group.k, weights);
     } else if (prm.input[g] == 2) {
-        gated_norm_row<T>(prm.gated, 0, sh_red, xs);
+        gated_norm_row<T>(prm.gated, 0, sh_red, xs, weights);
     } else if (prm.input[g] == 3) {
-        slice_norm_row<T>(prm.slice.x, prm.slice.weight, prm.slice.n, group.k, prm.slice.eps, sh_red, xs);
+        slice_norm_row<T>(prm.slice.x, prm.slice.weight, prm.slice.n, group.k, prm.slice.eps, sh_red, xs, weights);
     } else {
+        weights();
         constexpr int kVec = 16 / sizeof(T);
         const T* x = static_cast<const T*>(group.x);
         for (int c = threadIdx.x * kVec; c < group.k; c += kDecThreads * kVec)
