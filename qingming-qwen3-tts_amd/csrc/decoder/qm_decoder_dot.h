@@ -31,16 +31,16 @@ __device__ __forceinline__ float dot8(uint4 w, const float* x, float acc) {
     return acc;
 }
 
-// The weight rows of a wave in tile `tile` of the linear.
-template <int NR>
+// The weight rows of a wave in tile `tile` of the linear.  STREAM: read with the non-temporal hint.
+template <int NR, bool STREAM>
 struct DotRows {
     const uint16_t* row[NR];
     int channel;                               // first output of the wave
 };
-template <int NR>
-__device__ __forceinline__ DotRows<NR> dot_rows(const DecLinearGroup& g, int tile) {
+template <int NR, bool STREAM = false>
+__device__ __forceinline__ DotRows<NR, STREAM> dot_rows(const DecLinearGroup& g, int tile) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    DotRows<NR> d;
+    DotRows<NR, STREAM> d;
     if (g.w_up) {
         d.channel = tile * dot_tile_outputs<NR>(g) + wave * (NR / 2);
 #pragma unroll
@@ -56,19 +56,32 @@ __device__ __forceinline__ DotRows<NR> dot_rows(const DecLinearGroup& g, int til
     return d;
 }
 
-template <int NR>
-__device__ __forceinline__ void dot_request_one(const DotRows<NR>& d, int k, int at, uint4 (&piece)[NR]) {
+template <int NR, bool STREAM>
+__device__ __forceinline__ void dot_request_one(const DotRows<NR, STREAM>& d, int k, int at, uint4 (&piece)[NR]) {
     const int from = at < k ? at : 0;          // (past the end: not used; a load under a condition would stand behind a branch)
 #pragma unroll
-    for (int i = 0; i < NR; ++i) piece[i] = *reinterpret_cast<const uint4*>(d.row[i] + from);
+    for (int i = 0; i < NR; ++i) {
+        if constexpr (STREAM) {
+            typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+            const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(d.row[i] + from));
+            piece[i] = make_uint4(v.x, v.y, v.z, v.w);
+        } else {
+            piece[i] = *reinterpret_cast<const uint4*>(d.row[i] + from);
+        }
+    }
 }
 // Requests the first pieces of a wave's weight rows; they may be asked for before the input rows are known.
-template <int NR>
-__device__ __forceinline__ void dot_request(const DotRows<NR>& d, int k, uint4 (&piece)[kDotAhead][NR]) {
+template <int NR, bool STREAM>
+__device__ __forceinline__ void dot_request(const DotRows<NR, STREAM>& d, int k, uint4 (&piece)[kDotAhead][NR]) {
     const int lane = threadIdx.x & 63;
+    if (k >= kDotAhead * 512) {
+#pragma unroll
+        for (int u = 0; u < kDotAhead; ++u) dot_request_one(d, k, u * 512 + lane * 8, piece[u]);
+        return;
+    }
 #pragma unroll
     for (int u = 0; u < kDotAhead; ++u)
-        if (u * 512 < k) dot_request_one<NR>(d, k, u * 512 + lane * 8, piece[u]);
+        if (u * 512 < k) dot_request_one(d, k, u * 512 + lane * 8, piece[u]);
 }
 struct NoRefill {
     __device__ __forceinline__ void operator()(int) const {}
@@ -76,8 +89,8 @@ struct NoRefill {
 
 // One tile: xs holds R input rows [R][k] in LDS, `piece` the first pieces.  `refill` is called with a piece's number when the tile has no
 // more use for it.
-template <class T, int R, int NR, class Refill = NoRefill>
-__device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRows<NR>& d, uint4 (&piece)[kDotAhead][NR], const T* xs, int row0,
+template <class T, int R, int NR, bool STREAM, class Refill = NoRefill>
+__device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRows<NR, STREAM>& d, uint4 (&piece)[kDotAhead][NR], const T* xs, int row0,
                                            int rows, Refill&& refill = Refill()) {
     const int lane = threadIdx.x & 63;
     const int k = g.k;
@@ -96,7 +109,7 @@ __device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRow
 #pragma unroll
                     for (int i = 0; i < NR; ++i) acc[i][r] = dot8(piece[u][i], xs + r * k + at, acc[i][r]);
             }
-            if (k0 + kDotAhead * 512 < k) dot_request_one<NR>(d, k, at + kDotAhead * 512, piece[u]);
+            if (k0 + kDotAhead * 512 < k) dot_request_one(d, k, at + kDotAhead * 512, piece[u]);
             else refill(u);
         }
     }

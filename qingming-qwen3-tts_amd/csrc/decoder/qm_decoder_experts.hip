@@ -90,10 +90,10 @@ __global__ __launch_bounds__(kDecThreads) void expert_in_kernel(ExpertParams prm
     g.out = static_cast<T*>(s.act) + static_cast<int64_t>(at) * prm.ff_p;
     g.ldo = g.n = prm.ff_p;
     g.k = prm.width_p;
-    const DotRows<kExpertInRows> d = dot_rows<kExpertInRows>(g, tile);
+    const auto d = dot_rows<kExpertInRows>(g, tile);
     uint4 piece[kDotAhead][kExpertInRows];
-    dot_request<kExpertInRows>(d, g.k, piece);
-    dot_finish<T, 1, kExpertInRows>(g, d, piece, xs, 0, 1);
+    dot_request(d, g.k, piece);
+    dot_finish<T, 1>(g, d, piece, xs, 0, 1);
 }
 
 // Down of row blockIdx.y: the chosen experts' reductions one behind the other, each weighted.

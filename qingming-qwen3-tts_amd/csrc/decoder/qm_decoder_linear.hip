@@ -25,9 +25,9 @@ __global__ __launch_bounds__(kDecThreads) void decoder_linear_kernel(DecLinearPa
     const int row0 = static_cast<int>(blockIdx.y) * R;
     const int rows = min(R, prm.rows - row0);
     const int k = group.k;
-    const DotRows<kLinearRows> d = dot_rows<kLinearRows>(group, tile);
+    const auto d = dot_rows<kLinearRows>(group, tile);
     uint4 piece[kDotAhead][kLinearRows];
-    dot_request<kLinearRows>(d, k, piece);
+    dot_request(d, k, piece);
     constexpr int kVec = 16 / sizeof(T);
     for (int r = 0; r < R; ++r) {
         const int src = row0 + min(r, rows - 1);               // (a row past the end repeats the last one, never stored)
@@ -36,7 +36,7 @@ __global__ __launch_bounds__(kDecThreads) void decoder_linear_kernel(DecLinearPa
             *reinterpret_cast<uint4*>(xs + r * k + c) = *reinterpret_cast<const uint4*>(x + c);
     }
     __syncthreads();
-    dot_finish<T, R, kLinearRows>(group, d, piece, xs, row0, rows);
+    dot_finish<T, R>(group, d, piece, xs, row0, rows);
 }
 
 template <class T, int R>

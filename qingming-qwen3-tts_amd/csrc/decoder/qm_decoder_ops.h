@@ -23,6 +23,7 @@ constexpr int kDotLdsMost = 159 * 1024;   // dynamic LDS of one block
 struct DecLinearParams {
     qm_decoder_linear group[kDecGroups];
     int groups, rows;
+    int streaming;                   // a one-token step's weights with the non-temporal hint (qm_decoder_dot.h)
 };
 using ResidualParams = qm_residual_norm;
 using GatedNormParams = qm_gated_norm;

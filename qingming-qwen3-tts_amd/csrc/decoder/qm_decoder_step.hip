@@ -18,23 +18,25 @@ constexpr int kInRows = 4;                     // weight rows per wave: input li
 constexpr int kOutRows = 2;                    // output linears (few, long rows)
 constexpr int kInBlocks = 1024;                // most blocks of the input launch: each repeats the norm
 
-template <class T, int NV>
-__global__ __launch_bounds__(kDecThreads) void layer_in_kernel(LayerInParams prm, int tiles) {
-    request_arguments(prm);
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    __shared__ float sh_red[16];
-    T* hs = reinterpret_cast<T*>(smem);                                        // [ld_h]
+// STREAM: the weights with the non-temporal hint, for a model whose weights the last-level cache does not keep from token to token (24 tokens
+// behind 12 of the first design at width 2048, by MiB of weights a token: 400, 3975 -> 3620 us; 272, 2700 -> 2600; 256, 2480 both ways; 144 and
+// less the same or up to 3 % slower).
+template <class T, int NV, bool STREAM>
+__device__ __forceinline__ void layer_in_block(const LayerInParams& prm, int tiles, T* hs, float* sh_red) {
     int tile = static_cast<int>(blockIdx.x);
     int g = dot_group<kInRows>(prm.linears, tile);
-    DotRows<kInRows> d = dot_rows<kInRows>(prm.linears.group[g], tile);
+    auto d = dot_rows<kInRows, STREAM>(prm.linears.group[g], tile);
     uint4 piece[kDotAhead][kInRows];
     // Rows of up to 1024 columns: the norm's inputs are asked for before the weights and do not come back behind them (48 tokens of the second
     // design at that width 7920 -> 7820 us).  Longer rows want the weights under way at once (of the first design at 2048: 7210, 7340 the other way).
     const int k = prm.residual.ld_h;                                           // (every linear's)
-    const auto weights = [&] { dot_request<kInRows>(d, k, piece); };
-    if constexpr (NV > 1) weights();
-    if constexpr (NV > 1) residual_norm_row<T, NV>(prm.residual, 0, sh_red, hs, blockIdx.x == 0);
-    else residual_norm_row<T, NV, true>(prm.residual, 0, sh_red, hs, blockIdx.x == 0, weights);
+    const auto weights = [&] { dot_request(d, k, piece); };
+    if constexpr (NV > 1) {
+        weights();
+        residual_norm_row<T, NV>(prm.residual, 0, sh_red, hs, blockIdx.x == 0);
+    } else {
+        residual_norm_row<T, NV, true>(prm.residual, 0, sh_red, hs, blockIdx.x == 0, weights);
+    }
     __syncthreads();
     if (prm.residual.h && blockIdx.x == 0) {
         T* out = static_cast<T*>(prm.residual.h);
@@ -42,31 +44,37 @@ __global__ __launch_bounds__(kDecThreads) void layer_in_kernel(LayerInParams prm
     }
     for (int next = static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x);; next += static_cast<int>(gridDim.x)) {
         if (next >= tiles) {
-            dot_finish<T, 1, kInRows>(prm.linears.group[g], d, piece, hs, 0, 1);
+            dot_finish<T, 1>(prm.linears.group[g], d, piece, hs, 0, 1);
             break;
         }
         tile = next;
         const int then = dot_group<kInRows>(prm.linears, tile);
-        const DotRows<kInRows> rows = dot_rows<kInRows>(prm.linears.group[then], tile);
+        const auto rows = dot_rows<kInRows, STREAM>(prm.linears.group[then], tile);
         const int lane = threadIdx.x & 63;
-        dot_finish<T, 1, kInRows>(prm.linears.group[g], d, piece, hs, 0, 1, [&](int u) { dot_request_one<kInRows>(rows, k, u * 512 + lane * 8, piece[u]); });
+        dot_finish<T, 1>(prm.linears.group[g], d, piece, hs, 0, 1, [&](int u) { dot_request_one(rows, k, u * 512 + lane * 8, piece[u]); });
         g = then;
         d = rows;
     }
 }
 
-template <class T>
-__global__ __launch_bounds__(kDecThreads) void layer_out_kernel(LayerOutParams prm, int most_k) {
+template <class T, int NV>
+__global__ __launch_bounds__(kDecThreads) void layer_in_kernel(LayerInParams prm, int tiles) {
     request_arguments(prm);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    __shared__ float sh_red[4];
-    T* xs = reinterpret_cast<T*>(smem);
+    __shared__ float sh_red[16];
+    T* hs = reinterpret_cast<T*>(smem);                                        // [ld_h]
+    if (prm.linears.streaming) layer_in_block<T, NV, true>(prm, tiles, hs, sh_red);
+    else layer_in_block<T, NV, false>(prm, tiles, hs, sh_red);
+}
+
+template <class T, bool STREAM>
+__device__ __forceinline__ void layer_out_block(const LayerOutParams& prm, int most_k, T* xs, float* sh_red) {
     int tile = static_cast<int>(blockIdx.x);
     const int g = dot_group<kOutRows>(prm.linears, tile);
     const DecLinearGroup& group = prm.linears.group[g];
-    const DotRows<kOutRows> d = dot_rows<kOutRows>(group, tile);
+    const auto d = dot_rows<kOutRows, STREAM>(group, tile);
     uint4 piece[kDotAhead][kOutRows];
-    const auto weights = [&] { dot_request<kOutRows>(d, group.k, piece); };    // (behind what makes the input)
+    const auto weights = [&] { dot_request(d, group.k, piece); };              // (behind what makes the input)
     if (prm.input[g] == 1) {
         merge_attention_row<T>(prm.part, 0, attention_active_splits(*prm.position_dev, prm.chunk, prm.part.keys_per_split),
                                reinterpret_cast<float*>(xs + most_k), xs, group.k, weights);
@@ -82,21 +90,36 @@ __global__ __launch_bounds__(kDecThreads) void layer_out_kernel(LayerOutParams p
             *reinterpret_cast<uint4*>(xs + c) = *reinterpret_cast<const uint4*>(x + c);
     }
     __syncthreads();
-    dot_finish<T, 1, kOutRows>(group, d, piece, xs, 0, 1);
+    dot_finish<T, 1>(group, d, piece, xs, 0, 1);
+}
+
+template <class T>
+__global__ __launch_bounds__(kDecThreads) void layer_out_kernel(LayerOutParams prm, int most_k) {
+    request_arguments(prm);
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    __shared__ float sh_red[4];
+    T* xs = reinterpret_cast<T*>(smem);
+    if (prm.linears.streaming) layer_out_block<T, true>(prm, most_k, xs, sh_red);
+    else layer_out_block<T, false>(prm, most_k, xs, sh_red);
 }
 
 // A tile of a linear whose input is there already.
-template <class T>
-__device__ __forceinline__ void plain_tile(const DecLinearGroup& group, int tile, T* xs) {
-    const DotRows<kOutRows> d = dot_rows<kOutRows>(group, tile);
+template <class T, bool STREAM>
+__device__ __forceinline__ void plain_tile_as(const DecLinearGroup& group, int tile, T* xs) {
+    const auto d = dot_rows<kOutRows, STREAM>(group, tile);
     uint4 piece[kDotAhead][kOutRows];
-    dot_request<kOutRows>(d, group.k, piece);
+    dot_request(d, group.k, piece);
     constexpr int kVec = 16 / sizeof(T);
     const T* x = static_cast<const T*>(group.x);
     for (int c = threadIdx.x * kVec; c < group.k; c += kDecThreads * kVec)
         *reinterpret_cast<uint4*>(xs + c) = *reinterpret_cast<const uint4*>(x + c);
     __syncthreads();
-    dot_finish<T, 1, kOutRows>(group, d, piece, xs, 0, 1);
+    dot_finish<T, 1>(group, d, piece, xs, 0, 1);
+}
+template <class T>
+__device__ __forceinline__ void plain_tile(const DecLinearParams& linears, int tile, T* xs) {
+    if (linears.streaming) plain_tile_as<T, true>(linears.group[0], tile, xs);
+    else plain_tile_as<T, false>(linears.group[0], tile, xs);
 }
 
 // A mixer is a chain of round trips on few CUs while the layer's down projection waits for nothing but the launch before: its tiles
@@ -108,7 +131,7 @@ __global__ __launch_bounds__(kDecThreads) void delta_step_kernel(DeltaParams del
     extern __shared__ __attribute__((aligned(16))) float lds[];
     const int slices = (delta.dim + kRecColumns - 1) / kRecColumns, block = static_cast<int>(blockIdx.x);
     if (block < slices * delta.heads) general_delta_step<RD>(delta, block / slices, block % slices, lds);
-    else plain_tile<T>(beside.group[0], block - slices * delta.heads, reinterpret_cast<T*>(lds));
+    else plain_tile<T>(beside, block - slices * delta.heads, reinterpret_cast<T*>(lds));
 }
 
 template <class T, int GQ, int VC>
@@ -125,7 +148,7 @@ __global__ __launch_bounds__(kDecThreads) void mixer_step_kernel(ChunkAttentionP
     const int slices = (decay.vdim + kRecColumns - 1) / kRecColumns;
     const int head = block / slices, slice = block % slices;
     if (head >= decay.heads) {
-        plain_tile<T>(beside.group[0], block - decay.heads * slices, reinterpret_cast<T*>(lds));
+        plain_tile<T>(beside, block - decay.heads * slices, reinterpret_cast<T*>(lds));
         return;
     }
     if (decay.dim <= 32) decay_attention_block<8>(decay, head, slice, lds);

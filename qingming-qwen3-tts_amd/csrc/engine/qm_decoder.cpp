@@ -129,6 +129,7 @@ struct qm_decoder {
     qm_engine::Matrix embed, bigram, head;
     int capacity = 0, max_rows = 0, f32 = 0, path = 0;
     bool warm = false;
+    bool streaming = false;                         // a token's weights with the non-temporal hint
     int width_p = 0, vocab_p = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
@@ -346,6 +347,18 @@ int latent_splits(int capacity) { return std::clamp((capacity + qm::kLatentKeys 
 int keys_per_split(int chunk) { return padded(std::max(128, (chunk + 15) / 16), 128); }
 int key_splits(int chunk) { return (chunk + keys_per_split(chunk) - 1) / keys_per_split(chunk); }
 
+// Bytes of weights that one token reads.  Where they are more than the last-level cache (256 MiB) keeps from token to token, the step's
+// linears read them with the non-temporal hint: what is read once and gone displaces nothing, and streams faster.
+int64_t token_bytes(const qm_decoder& d) {
+    auto bytes = [](const Matrix& m) { return static_cast<int64_t>(m.n) * m.k * 2; };
+    int64_t all = bytes(d.head);
+    for (const DecoderLayer& w : d.layers)
+        all += bytes(w.in) + bytes(w.o_left) + bytes(w.o_right) + bytes(w.q_up) + bytes(w.up_latent) + bytes(w.router)
+             + (w.config.experts ? w.config.top : 1) * (2 * bytes(w.gate) + bytes(w.down));
+    return all;
+}
+constexpr int64_t kStreamingTokenBytes = 256ll << 20;
+
 std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int capacity, int sequences, int max_rows, hipStream_t stream) {
     if (capacity <= 0 || sequences <= 0 || max_rows < 0 || (f32 != 0 && f32 != 1))
         throw ApiError(QM_ERR_ARGUMENT, "capacity and sequences must be positive");
@@ -487,6 +500,7 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
     d->logits = zeros(static_cast<size_t>(kLogitRows) * d->vocab_p * 4);
     d->step_words = zeros(kStepWords * 4);
     d->mailbox.open(d->vocab_p);
+    d->streaming = token_bytes(*d) > kStreamingTokenBytes;
     hip_check(hipDeviceSynchronize(), "decoder setup");
     return d;
 }
@@ -880,6 +894,11 @@ void run_head(qm_decoder& d, const float* x, const Pending& pending, const int32
 
 // ---- one token -----------------------------------------------------------------------------------------------------------
 
+qm::DecLinearParams streamed(const qm_decoder& d, qm::DecLinearParams linears) {
+    linears.streaming = d.streaming;
+    return linears;
+}
+
 int32_t* step_words(const qm_decoder& d) { return static_cast<int32_t*>(d.step_words.raw()); }
 
 // The token and position that the step words name, through every layer run and the head: logits in row 0 of d.logits.
@@ -899,14 +918,14 @@ void enqueue_one(qm_decoder& d, int sequence) {
         float* x_new = f32_of(d.x[next]);
         qm::LayerInParams in = {};
         in.residual = residual(x_new, step_vec_of(d, run), f32_of(w.norm1));
-        in.linears = linears_in(d, w, 1);
+        in.linears = streamed(d, linears_in(d, w, 1));
         op_check(qm::launch_layer_in(in, d.f32, s), "residual + norm + input projections");
         x = x_new;
         next ^= 1;
         qm::LayerOutParams out = {};
         out.position_dev = step_words(d);
-        out.linears = linears_out(d, w, 1, pending);
-        qm::DecLinearParams beside = {};       // the down projection needs nothing of the mixer
+        out.linears = streamed(d, linears_out(d, w, 1, pending));
+        qm::DecLinearParams beside = streamed(d, {});       // the down projection needs nothing of the mixer
         if (w.config.ff && !sandwich(w)) {
             beside.rows = beside.groups = 1;
             beside.group[0] = out.linears.group[--out.linears.groups];
@@ -940,6 +959,7 @@ void enqueue_one(qm_decoder& d, int sequence) {
                 qm::LayerOutParams up = {};
                 up.linears.rows = 1;
                 up.linears.group[up.linears.groups++] = linear_of(w.q_up, nullptr, f32_of(d.queries));
+                up.linears = streamed(d, up.linears);
                 up.input[0] = 3;
                 up.slice = {rows.proj + rows.q_column, rows.q_norm, rows.q_rank, rows.eps};
                 op_check(qm::launch_layer_out(up, d.f32, s), "queries");
@@ -955,7 +975,7 @@ void enqueue_one(qm_decoder& d, int sequence) {
             qm::LayerInParams feed = {};
             feed.residual = residual(x_new, nullptr, f32_of(w.norm2));
             if (w.config.experts) feed.residual.h = d.h.raw();
-            feed.linears = feed_in(d, w, 1);
+            feed.linears = streamed(d, feed_in(d, w, 1));
             op_check(qm::launch_layer_in(feed, d.f32, s), "residual + norm + feed-forward");
             x = x_new;
             next ^= 1;
@@ -963,7 +983,7 @@ void enqueue_one(qm_decoder& d, int sequence) {
                 op_check(qm::launch_experts(experts_of(d, w, 1, f32_of(d.y[0])), d.f32, s), "experts");
             } else {
                 qm::LayerOutParams down = {};
-                down.linears = feed_out(d, w, 1);
+                down.linears = streamed(d, feed_out(d, w, 1));
                 op_check(qm::launch_layer_out(down, d.f32, s), "feed-forward");
             }
             pending = feed_term(d, w);
@@ -973,6 +993,7 @@ void enqueue_one(qm_decoder& d, int sequence) {
     head.residual = residual(nullptr, nullptr, f32_of(d.final_norm));
     head.linears.rows = 1;
     head.linears.group[head.linears.groups++] = linear_of(d.head, nullptr, f32_of(d.logits));
+    head.linears = streamed(d, head.linears);
     op_check(qm::launch_layer_in(head, d.f32, s), "final norm + head");
 }
 

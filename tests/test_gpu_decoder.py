@@ -381,3 +381,30 @@ def test_generate_program(decoder, models):
                        input="\n".join(map(json.dumps, prompts)) + "\n", capture_output=True, text=True, timeout=100)
     assert p.returncode == 0, p.stderr
     assert [json.loads(line) for line in p.stdout.splitlines()] == [greedy(m, prompt, 6) for prompt in prompts]
+
+
+@pytest.mark.parametrize("design", ["parallel", "sandwich"])
+def test_weights_beyond_the_cache_give_the_same_bits(decoder, tmp_path, design):
+    """A model whose head alone is more than the last-level cache keeps reads a step's weights with the non-temporal hint: the small model's scores, bit for
+    bit (the large vocabulary's rows repeat the small one's)."""
+    small, times = 1000, 1100                                  # 1 100 000 x 128 values of two bytes: 268 MiB
+    if design == "parallel":
+        layers = [cases.parallel(cases.left(4, 2, 32, 48, 40, 16), cases.right(2, 32, 64, [0.9, 0.99]), 300), cases.general_delta(2, 32, 200)]
+        make = lambda vocab: cases.config(vocab, 128, layers)
+    else:
+        layers = [cases.latent(4, 16, 8, 24, 48, 40, cases.moe(6, 2, 48)), cases.retention(2, 16, 24, [0.9, 0.99], cases.dense(300))]
+        make = lambda vocab: cases.sandwich(vocab, 128, layers, (11, 6, 7))
+    weights = cases.weights(make(small))
+    tokens = cases.tokens_of(make(small), 30)
+    rows = []
+    for count in (1, times):
+        where = tmp_path / str(count)
+        where.mkdir()
+        cases.write_model(str(where), make(small * count), {name: np.tile(w, (count, 1)) if name in ("embed", "head") else w for name, w in weights.items()})
+        engine = decoder.Decoder(str(where), 32)
+        s = engine.open()
+        rows.append([engine.step(s, tokens[:5], [4])[0]] + [engine.step(s, [t], [0])[0] for t in tokens[5:]])
+        engine.close(s)
+        del engine
+    for want, got in zip(*rows):
+        assert np.array_equal(got, np.tile(want, times))
