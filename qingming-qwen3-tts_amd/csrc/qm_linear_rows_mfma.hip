@@ -173,6 +173,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
     int m0 = static_cast<int>(blockIdx.y) * BM;
     // (several linears of one input in one grid: which of them this block's column tile belongs to)
     int tile = static_cast<int>(blockIdx.x);
+    if (tile >= prm.column_tiles) return;                         // (the grid's width is rounded up)
     if (!DUAL && prm.linear_by_linear) {
         int at = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x), first = 0, next = prm.group_first_tile[0];
         for (int g = 1; g < prm.groups && at >= static_cast<int>(gridDim.y) * (next - first); ++g) {
@@ -589,6 +590,11 @@ int32_t launch_rows_mfma_as(const LinearRowsParams& given, hipStream_t stream) {
     constexpr int smem = Shape::kStages * Shape::kStageBytes + (Shape::kStages == 2 ? 256 * WAVES : 0);
     int column_tiles = prm.columns / BN;
     for (int g = 1; g < prm.groups; ++g) column_tiles += prm.group_columns[g - 1] / BN;
+    prm.column_tiles = column_tiles;
+    // Blocks go to the eight dies in turn: where 8 divides the column tiles, the row tiles of one read its weights on one die.  Many column tiles are
+    // rounded up to that, the blocks beyond end at once (1024 tokens, 81 column tiles of 2048: 64.8 -> 56.1 us, 80: 54.2); of few the dies' shares would
+    // be too uneven.
+    if (column_tiles > 40 && prm.rows > BM && !prm.linear_by_linear) column_tiles = (column_tiles + 7) / 8 * 8;
     const dim3 grid(static_cast<unsigned>(column_tiles), static_cast<unsigned>((prm.rows + BM - 1) / BM),
                     static_cast<unsigned>(prm.reduction_parts));
     if (grid.y > 65535u) return QM_ERR_ARGUMENT;

@@ -42,6 +42,8 @@ struct LinearRowsParams {
     // tile_rows rows (64 or 128) takes matrix tile_matrix[t], or is left out where that is negative
     const int32_t* tile_matrix;
     int tile_rows;
+    // (matrix cores) column tiles of the launch, which sets it: the grid may be wider
+    int column_tiles;
 };
 
 // The row linears on the matrix cores (qm_linear_rows_mfma.hip).  `dual`: weight[0] / weight[1] are the gate and up

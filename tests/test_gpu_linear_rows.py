@@ -279,3 +279,20 @@ def test_matrix_core_tiles_against_64_bits(qm, dev, rows, cols, red, pair, rows_
         want = act * u
         bound = act_bound * u.abs() + u_bound * act.abs() + act_bound * u_bound + half * want.abs()
     assert bool(((got - want).abs() <= bound + 1e-30).all()), float(((got - want).abs() / (bound + 1e-30)).max())
+
+
+@pytest.mark.parametrize("rows,cols,red", [(129, 5248, 128), (65, 5376, 256), (300, 5248, 128), (1024, 5888, 128)])
+@pytest.mark.parametrize("rows_kernel", [MATRIX], indirect=True)
+def test_more_than_forty_column_tiles_that_eight_does_not_divide(qm, dev, rows, cols, red, rows_kernel):
+    """The grid's width is rounded up and the blocks beyond the last tile end: every output is written, and nothing behind them."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows + cols)
+    x = torch.randn(rows, red, device=dev, generator=gen).bfloat16()
+    w = torch.randn(cols, red, device=dev, generator=gen).bfloat16()
+    out = torch.full((rows + 1, cols), float("nan"), dtype=torch.bfloat16, device=dev)
+    qm.linear_rows(x, w, None, None, out, rows, cols, red)
+    want = x.double() @ w.double().t()
+    # half a bf16 spacing of the sum, and the fp32 sum's own error: red * 2^-24 of the sum of magnitudes
+    bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * red * 2.0 ** -24
+    assert bool(((out[:rows].double() - want).abs() <= bound).all())
+    assert bool(out[rows].isnan().all())
