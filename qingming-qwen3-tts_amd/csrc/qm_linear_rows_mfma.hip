@@ -72,12 +72,23 @@ __device__ __forceinline__ uint32_t finish_pair(float s0, float s1, bool has_bia
     return v;
 }
 
+// g / (1 + exp(-g)) of a bf16 value, good for its rounding to bf16: the bits that expf and the correctly rounded division give, for every one of
+// the 65 536 (compared exhaustively on the device), in ten instructions where those take some forty.  The denominator is kept down by 2^32, so that its
+// reciprocal does not go below the normal numbers where exp(-g) is near the largest; one Newton step makes the reciprocal good to the last bit.
+// (The pair's epilogue is as long as five of its steps: 1000 tokens x 6144 channels of 2048 54.6 -> 52.1 us, 777 x 3072 of 1024 22.1 -> 20.9.)
+__device__ __forceinline__ float silu_of_bf16(float g) {
+    const float s = fmaf(__builtin_amdgcn_exp2f(g * -kLog2e), 0x1p-32f, 0x1p-32f);
+    const float r = __builtin_amdgcn_rcpf(s);
+    const float refined = fmaf(fmaf(-s, r, 1.0f), r, r);
+    return g * ((s == INFINITY ? 0.0f : refined) * 0x1p-32f);
+}
+
 // Gate/up: swiglu_kernel (R17:8746-8770) on the rounded gate and up values.
 __device__ __forceinline__ uint32_t swiglu_pair(float g0, float g1, float u0, float u1) {
     float gv0, gv1, uv0, uv1, a0, a1;
     round_bf16_pair(g0, g1, gv0, gv1);
     round_bf16_pair(u0, u1, uv0, uv1);
-    round_bf16_pair(gv0 / (1.0f + expf(-gv0)), gv1 / (1.0f + expf(-gv1)), a0, a1);
+    round_bf16_pair(silu_of_bf16(gv0), silu_of_bf16(gv1), a0, a1);
     return pack_bf16_pair(a0 * uv0, a1 * uv1);
 }
 

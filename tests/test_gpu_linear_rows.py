@@ -296,3 +296,23 @@ def test_more_than_forty_column_tiles_that_eight_does_not_divide(qm, dev, rows, 
     bound = want.abs() * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * red * 2.0 ** -24
     assert bool(((out[:rows].double() - want).abs() <= bound).all())
     assert bool(out[rows].isnan().all())
+
+
+@pytest.mark.parametrize("rows_kernel", [MATRIX], indirect=True)
+def test_swiglu_of_every_bf16_gate(qm, dev, rows_kernel):
+    """Each gate value once, through an identity on the matrix cores: the bits of the exact chain's expf and division (a NaN is a NaN)."""
+    import torch
+    x = torch.eye(128, device=dev).bfloat16()
+    up = torch.ones(128, 128, device=dev).bfloat16()
+    for part in range(4):
+        bits = (torch.arange(16384, dtype=torch.int32, device=dev) + 16384 * part).to(torch.int16).view(128, 128)
+        gate = bits.view(torch.bfloat16)
+        gate = torch.where(gate.float().isfinite(), gate, torch.zeros_like(gate)).contiguous()    # (0 times infinity is no gate)
+        got = []
+        for kernel in (MATRIX, EXACT):
+            qm.set_option(qm.OPT_LINEAR_ROWS_KERNEL, kernel)
+            out = torch.zeros(128, 128, dtype=torch.int16, device=dev)
+            qm.gate_up_swiglu_rows(x, gate, up, out, 128, 128, 128)
+            got.append(out)
+        torch.cuda.synchronize()
+        assert bool((got[0] == got[1]).all()), part
