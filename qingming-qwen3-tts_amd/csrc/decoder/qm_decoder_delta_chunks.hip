@@ -12,6 +12,8 @@
 // never below exp(-e^(-1/2)) = 0.545, so 1 / W stays under 3e8 and everything fits fp32; A and K enter the state already
 // multiplied by W.  All products are fp32 on the matrix cores.
 // Bound: the walk, a chain of rows / 32 dependent steps.
+#include <utility>
+
 #include "../qm_host.h"
 #include "qm_decoder_mfma32.h"
 #include "qm_decoder_recurrent.h"
@@ -310,6 +312,16 @@ struct DeltaStep {
     float v[2][4], own[2];
 };
 
+// f(0), f(1), ... f(N - 1), the number known to the compiler.
+template <int N, class F, int... I>
+__device__ __forceinline__ void unrolled_as(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void unrolled(F&& f) {
+    unrolled_as<N>(f, std::make_integer_sequence<int, N>{});
+}
+
 // A barrier for what went into LDS: unlike __syncthreads it leaves the loads under way (the next chunk's) in flight.
 __device__ __forceinline__ void block_exchange() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
@@ -337,65 +349,84 @@ __global__ __launch_bounds__(kDecThreads) void delta_chunk_walk_kernel(DeltaPara
     // (a token past the last meets zeros, a column past the head is not stored: both repeat the last, no branch around a load)
     const float* values = prm.proj + prm.v_column + head * dim + min(column, dim - 1);
     auto value_at = [&](int token) { return values[min(token, prm.rows - 1) * prm.ld_proj]; };
-    auto request = [&](int chunk, DeltaStep<TW>& f) __attribute__((always_inline)) {
-        const float* from = prm.scratch + (static_cast<int64_t>(chunk) * prm.heads + head) * at.floats;
-#pragma unroll
-        for (int i = 0; i < TW; ++i) {
-            const int tile = wave + 4 * i;
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const int operand = ((2 * tile + b) * 64 + lane) * 4;
-                f.m[b][i] = *reinterpret_cast<const float4*>(from + at.m + operand);
-                f.x[b][i] = *reinterpret_cast<const float4*>(from + at.x + operand);
-                f.at[i][b] = *reinterpret_cast<const float4*>(from + at.at + operand);
-                f.kt[i][b] = *reinterpret_cast<const float4*>(from + at.kt + operand);
-            }
-            f.w[i] = *reinterpret_cast<const float4*>(from + at.w + 16 * tile + 4 * g);
-        }
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
+    // The loads of a step, by number: for each of the wave's tiles its shares of the four matrices and the decays, then per half of the chunk the
+    // terms of N and Y and the values.
+    constexpr int kTileLoads = 9, kHalfLoads = 7, kLoads = TW * kTileLoads + 2 * kHalfLoads;
+    const int64_t chunk_floats = static_cast<int64_t>(prm.heads) * at.floats;
+    const float* const matrices = prm.scratch + static_cast<int64_t>(head) * at.floats;
+    auto request = [&](int chunk, DeltaStep<TW>& f, auto number) __attribute__((always_inline)) {
+        constexpr int N = decltype(number)::value;
+        const float* from = matrices + chunk * chunk_floats;
+        if constexpr (N < TW * kTileLoads) {
+            constexpr int i = N / kTileLoads, b = N % kTileLoads & 1, which = N % kTileLoads / 2;
+            const int tile = wave + 4 * i, operand = ((2 * tile + b) * 64 + lane) * 4;
+            if constexpr (which == 0) f.m[b][i] = *reinterpret_cast<const float4*>(from + at.m + operand);
+            else if constexpr (which == 1) f.x[b][i] = *reinterpret_cast<const float4*>(from + at.x + operand);
+            else if constexpr (which == 2) f.kt[i][b] = *reinterpret_cast<const float4*>(from + at.kt + operand);
+            else if constexpr (which == 3) f.at[i][b] = *reinterpret_cast<const float4*>(from + at.at + operand);
+            else f.w[i] = *reinterpret_cast<const float4*>(from + at.w + 16 * tile + 4 * g);
+        } else if constexpr (N < kLoads) {
+            constexpr int b = (N - TW * kTileLoads) / kHalfLoads, which = (N - TW * kTileLoads) % kHalfLoads;
             const int row = (16 * b + l16) * kDeltaChunk + 16 * part + 4 * g + pair;
-            f.n[b] = *reinterpret_cast<const float2*>(from + at.n + row);
-            f.y[b] = *reinterpret_cast<const float2*>(from + at.y + row);
-#pragma unroll
-            for (int t = 0; t < 4; ++t) f.v[b][t] = value_at(chunk * kDeltaChunk + 16 * b + 4 * g + t);
-            f.own[b] = value_at(chunk * kDeltaChunk + 16 * part + 4 * g + pair + b);
+            if constexpr (which == 0) f.n[b] = *reinterpret_cast<const float2*>(from + at.n + row);
+            else if constexpr (which == 1) f.y[b] = *reinterpret_cast<const float2*>(from + at.y + row);
+            else if constexpr (which == 2) f.own[b] = value_at(chunk * kDeltaChunk + 16 * part + 4 * g + pair + b);
+            else f.v[b][which - 3] = value_at(chunk * kDeltaChunk + 16 * b + 4 * g + which - 3);
         }
     };
+    // They stand one or two to a slot between the products of a step: the wave issues in order, a matrix instruction hides 32 cycles of other issue, and
+    // asked for in a bunch they took 1 830 cycles of a step's 6 050 (16 heads of 128, 1024 rows: 81 -> 65.5 us; of 64, 300 rows: 19.5 -> 17.2).
+    constexpr int kSlots = 8 * TW + 4 + 8 * TW, kPerSlot = (kLoads + kSlots - 1) / kSlots;
     auto walk = [&](int chunk, DeltaStep<TW>& f, DeltaStep<TW>& next) __attribute__((always_inline)) {
-        // this chunk's loads, a whole step under way, have to be there; then the next one's go out
+        // this chunk's loads, most of a step under way, have to be there
         __builtin_amdgcn_s_waitcnt((7 << 4) | (15 << 8));          // vmcnt(0), nothing else
-        __builtin_amdgcn_sched_barrier(0);
-        request(min(chunk + 1, chunks - 1), next);
-        __builtin_amdgcn_sched_barrier(0);
+        const int then = min(chunk + 1, chunks - 1);
+        auto slot = [&](auto number) __attribute__((always_inline)) {
+            constexpr int first = decltype(number)::value * kPerSlot;
+            __builtin_amdgcn_sched_barrier(0);
+            request(then, next, std::integral_constant<int, first>{});
+            if constexpr (kPerSlot > 1) request(then, next, std::integral_constant<int, first + 1>{});
+            static_assert(kPerSlot <= 2, "");
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto element = [](const float4& v, auto e) __attribute__((always_inline)) {
+            constexpr int E = decltype(e)::value;
+            if constexpr (E == 0) return v.x;
+            else if constexpr (E == 1) return v.y;
+            else if constexpr (E == 2) return v.z;
+            else return v.w;
+        };
         f32x4_t p[2] = {}, o[2] = {};
-#pragma unroll
-        for (int i = 0; i < TW; ++i) {
-            const float4 b = make_float4(s[i][0], s[i][1], s[i][2], s[i][3]);
-#pragma unroll
-            for (int half = 0; half < 2; ++half) {
-                p[half] = mfma32_block(f.m[half][i], b, p[half]);
-                o[half] = mfma32_block(f.x[half][i], b, o[half]);
-            }
-        }
+        unrolled<8 * TW>([&](auto number) __attribute__((always_inline)) {
+            constexpr int n = decltype(number)::value, i = n / 8, half = n / 4 % 2, e = n % 4;
+            p[half] = mfma32(element(f.m[half][i], std::integral_constant<int, e>{}), s[i][e], p[half]);
+            o[half] = mfma32(element(f.x[half][i], std::integral_constant<int, e>{}), s[i][e], o[half]);
+            slot(number);
+        });
+        unrolled<4>([&](auto number) __attribute__((always_inline)) {
+            constexpr int half = decltype(number)::value / 2, e = decltype(number)::value % 2;
+            p[half] = mfma32(e == 0 ? f.n[half].x : f.n[half].y, f.own[e], p[half]);
+            o[half] = mfma32(e == 0 ? f.y[half].x : f.y[half].y, f.own[e], o[half]);
+            slot(std::integral_constant<int, 8 * TW + decltype(number)::value>{});
+        });
         float (*mine)[kDeltaChunk * kStride] = sh[chunk & 1][wave];
 #pragma unroll
-        for (int half = 0; half < 2; ++half) {
-            p[half] = mfma32(f.n[half].y, f.own[1], mfma32(f.n[half].x, f.own[0], p[half]));
-            o[half] = mfma32(f.y[half].y, f.own[1], mfma32(f.y[half].x, f.own[0], o[half]));
+        for (int half = 0; half < 2; ++half)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 mine[0][(16 * half + 4 * g + r) * kStride + l16] = p[half][r];
                 mine[1][(16 * half + 4 * g + r) * kStride + l16] = o[half][r];
             }
-        }
         // (what does not need P, while the others arrive)
 #pragma unroll
         for (int i = 0; i < TW; ++i) {
             s[i][0] *= f.w[i].x; s[i][1] *= f.w[i].y; s[i][2] *= f.w[i].z; s[i][3] *= f.w[i].w;
-#pragma unroll
-            for (int b = 0; b < 2; ++b) s[i] = mfma32_block(f.kt[i][b], make_float4(f.v[b][0], f.v[b][1], f.v[b][2], f.v[b][3]), s[i]);
         }
+        unrolled<8 * TW>([&](auto number) __attribute__((always_inline)) {
+            constexpr int n = decltype(number)::value, b = n / (4 * TW), e = n / TW % 4, i = n % TW;
+            s[i] = mfma32(element(f.kt[i][b], std::integral_constant<int, e>{}), f.v[b][e], s[i]);
+            slot(std::integral_constant<int, 8 * TW + 4 + n>{});
+        });
         block_exchange();
         float share[4][2][4], read[2][4];
 #pragma unroll
@@ -421,7 +452,7 @@ __global__ __launch_bounds__(kDecThreads) void delta_chunk_walk_kernel(DeltaPara
         }
     };
     DeltaStep<TW> even, odd;
-    request(0, even);
+    unrolled<kLoads>([&](auto number) __attribute__((always_inline)) { request(0, even, number); });
     for (int chunk = 0; chunk < chunks; chunk += 2) {
         walk(chunk, even, odd);
         if (chunk + 1 < chunks) walk(chunk + 1, odd, even);
