@@ -87,8 +87,10 @@ __device__ __forceinline__ float4 weighted(float4 acc, float f, float4 y, float4
 struct NothingBehind {
     __device__ __forceinline__ void operator()() const {}
 };
-template <class T, int NV, bool EARLY = false, class Behind = NothingBehind>
-__device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int row, float* sh_red, T* h, bool write_x, Behind&& behind = Behind()) {
+// MORE: the last term's further pieces are added to it.
+template <class T, int NV, bool EARLY = false, bool MORE = false, class Behind = NothingBehind>
+__device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int row, float* sh_red, T* h, bool write_x, Behind&& behind = Behind(),
+                                                  const MoreOfTerm& more = MoreOfTerm()) {
     const int tid = threadIdx.x;
     const int64_t src = prm.row_map ? prm.row_map[row] : row;
     const int vectors = static_cast<int>(prm.ld_h >> 2);
@@ -109,7 +111,7 @@ __device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int
         }
     }
     const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f), one = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
-    float4 x[NV], y[3][NV];
+    float4 x[NV], y[3][NV], pieces[MORE ? kMorePlanes : 1][MORE ? NV : 1];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
         const int v = tid + i * kDecThreads;
@@ -118,6 +120,11 @@ __device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int
         if (bigram) x[i] = weighted(x[i], 1.0f, load4_if(in, bigram, v), one);
 #pragma unroll
         for (int t = 0; t < 3; ++t) y[t][i] = y_row[t] ? load4_if(in, y_row[t], v) : zero;
+        if constexpr (MORE) {
+            const float* piece = more.sums + src * prm.term[prm.terms - 1].ld;
+#pragma unroll
+            for (int p = 0; p < kMorePlanes; ++p) pieces[p][i] = p < more.planes ? load4_if(in, piece + p * more.plane, v) : zero;
+        }
     }
     float4 y_weight[3][EARLY ? NV : 1], step_vec[EARLY ? NV : 1], weight[EARLY ? NV : 1];
     if constexpr (EARLY) {
@@ -133,6 +140,16 @@ __device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int
     __builtin_amdgcn_sched_barrier(0);
     behind();
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (MORE) {
+#pragma unroll
+        for (int t = 0; t < 3; ++t)
+            if (t == prm.terms - 1) {
+#pragma unroll
+                for (int i = 0; i < NV; ++i)
+#pragma unroll
+                    for (int p = 0; p < kMorePlanes; ++p) y[t][i] = weighted(y[t][i], 1.0f, pieces[p][i], one);
+            }
+    }
     const float inv_width = 1.0f / static_cast<float>(prm.width);
     float factor[3] = {0.0f, 0.0f, 0.0f};
     if (normed[0] || normed[1] || normed[2]) {

@@ -5,6 +5,8 @@
 // lane, `kDotAhead` pieces of each row requested before the first is used; the input rows live in LDS as T.  Sums are fp32
 // (packed bf16 dot products, or fmaf in the 32-bit mode), combined over the wave's lanes at the end.
 #include <algorithm>
+#include <map>
+#include <numeric>
 
 #include "qm_decoder_device.h"
 #include "../qm_host.h"
@@ -157,7 +159,53 @@ static bool split_pays(const DecLinearParams& prm) {
     return dots > 33 + k * (pair ? 85 : prm.rows <= 16 ? 46 : 56) / 1024;
 }
 
-int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream) {
+// Steps of 64 k that the busiest CU walks when blocks of 128 x 128 outputs are dealt out long reductions first, the last one in `parts` pieces; a
+// block's first stages and its outputs are about three steps more.
+static int64_t steps_of_busiest(const DecLinearParams& prm, int parts) {
+    int64_t count[kDecGroups], steps[kDecGroups];
+    int order[kDecGroups] = {0, 1, 2};
+    for (int g = 0; g < prm.groups; ++g) {
+        const int pieces = g == prm.groups - 1 ? parts : 1;
+        count[g] = static_cast<int64_t>(prm.group[g].n / 128) * ((prm.rows + 127) / 128) * pieces;
+        steps[g] = prm.group[g].k / 64 / pieces + 3;
+    }
+    std::stable_sort(order, order + prm.groups, [&](int a, int b) { return steps[a] > steps[b]; });
+    std::map<int64_t, int64_t> cus = {{0, 256}};                               // steps dealt so far -> how many CUs have as many
+    for (int i = 0; i < prm.groups; ++i)
+        for (int64_t left = count[order[i]]; left > 0;) {
+            const auto [at, many] = *cus.begin();
+            const int64_t taken = std::min(left, many);
+            cus.erase(cus.begin());
+            if (many > taken) cus[at] = many - taken;
+            cus[at + steps[order[i]]] += taken;
+            left -= taken;
+        }
+    return cus.rbegin()->first;
+}
+// Into how many pieces the last linear's reduction is cut: where the linears' blocks leave CUs idle behind the longest reduction, its pieces
+// fill them.  (us, 1024 rows, 2048 outputs of 6144: beside 2048 of 2048, three pieces, 66 -> 55; beside twice that, two pieces, 70 -> 65; the norm
+// behind, which adds the pieces, 11.5 -> 14.)  A piece more is a plane of sums written and read, rows x outputs x 8 bytes: a step's time (0.73 us)
+// for each 3 MB.
+static int reduction_pieces(const DecLinearParams& prm) {
+    const DecLinearGroup& last = prm.group[prm.groups - 1];
+    int64_t blocks = 0;
+    for (int g = 0; g < prm.groups; ++g) blocks += static_cast<int64_t>(prm.group[g].n / 128) * ((prm.rows + 127) / 128);
+    if (prm.groups < 2 || blocks < 200) return 1;                              // (fewer take smaller tiles)
+    int best = 1;
+    int64_t least = steps_of_busiest(prm, 1);
+    for (int parts = 2; parts <= 1 + kMorePlanes; ++parts) {
+        if (last.k % (128 * parts)) continue;
+        const int64_t steps = steps_of_busiest(prm, parts) + (parts - 1) * (static_cast<int64_t>(prm.rows) * last.n * 8 / 3000000 + 1);
+        if (steps < least) {
+            least = steps;
+            best = parts;
+        }
+    }
+    return best;
+}
+
+int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut) {
+    if (cut) cut->planes = 0;
     if (prm.rows < 0 || prm.groups < 1 || prm.groups > kDecGroups) return QM_ERR_ARGUMENT;
     for (int g = 0; g < prm.groups; ++g) {
         const DecLinearGroup& d = prm.group[g];
@@ -172,10 +220,31 @@ int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t 
     for (int g = 0; g < prm.groups; ++g) matrix = matrix && prm.group[g].n % 128 == 0 && prm.group[g].ldx == prm.group[g].k && prm.group[g].ldo == prm.group[g].n;
     if (!matrix) return streaming<uint16_t>(prm, stream);
     LinearRowsParams plain = {};
-    int order[kDecGroups] = {0, 1, 2};         // long reductions first
-    std::stable_sort(order, order + prm.groups, [&](int a, int b) { return prm.group[a].k > prm.group[b].k; });
-    for (int i = 0; i < prm.groups; ++i) {
-        const DecLinearGroup& d = prm.group[order[i]];
+    static_assert(kDecGroups + kMorePlanes <= kRowsGroups, "the pieces of a reduction are linears of their own");
+    DecLinearGroup all[kDecGroups + kMorePlanes];
+    int pitch[kDecGroups + kMorePlanes], order[kDecGroups + kMorePlanes], count = prm.groups;
+    for (int g = 0; g < count; ++g) {
+        all[g] = prm.group[g];
+        pitch[g] = prm.group[g].k;
+        if (prm.group[g].w_up) cut = nullptr;
+    }
+    if (cut) {
+        const int pieces = reduction_pieces(prm);
+        DecLinearGroup& last = all[count - 1];
+        last.k /= pieces;
+        cut->plane = static_cast<int64_t>(prm.rows) * last.n;
+        for (; cut->planes < pieces - 1; ++cut->planes, ++count) {
+            all[count] = last;
+            all[count].x = static_cast<const uint16_t*>(last.x) + (cut->planes + 1) * last.k;
+            all[count].w += (cut->planes + 1) * last.k;
+            all[count].out32 = cut->sums + cut->planes * cut->plane;
+            pitch[count] = pitch[prm.groups - 1];
+        }
+    }
+    std::iota(order, order + count, 0);        // long reductions first
+    std::stable_sort(order, order + count, [&](int a, int b) { return all[a].k > all[b].k; });
+    for (int i = 0; i < count; ++i) {
+        const DecLinearGroup& d = all[order[i]];
         if (d.w_up) {
             LinearRowsParams pair = {};
             pair.input = static_cast<const uint16_t*>(d.x);
@@ -192,6 +261,7 @@ int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t 
             plain.weight[0] = plain.weight[1] = d.w;
             plain.sums = d.out32;
             plain.rows = prm.rows; plain.columns = d.n; plain.reduction = d.k;
+            plain.pitch = pitch[order[i]];
             plain.reduction_parts = 1;
         } else {
             const int at = plain.groups - 1;
@@ -202,6 +272,7 @@ int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t 
             plain.group_sums[at] = d.out32;
             plain.group_columns[at] = d.n;
             plain.group_reduction[at] = d.k;
+            plain.group_pitch[at] = pitch[order[i]];
         }
         ++plain.groups;
     }

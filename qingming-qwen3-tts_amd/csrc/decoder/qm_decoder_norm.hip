@@ -6,11 +6,11 @@
 
 namespace qm {
 
-template <class T, int NV>
-__global__ __launch_bounds__(kDecThreads) void residual_norm_kernel(ResidualParams prm) {
+template <class T, int NV, bool MORE>
+__global__ __launch_bounds__(kDecThreads) void residual_norm_kernel(ResidualParams prm, MoreOfTerm more) {
     __shared__ float sh_red[16];
     const int row = static_cast<int>(blockIdx.x);
-    residual_norm_row<T, NV>(prm, row, sh_red, static_cast<T*>(prm.h) + row * prm.ld_h, true);
+    residual_norm_row<T, NV, false, MORE>(prm, row, sh_red, static_cast<T*>(prm.h) + row * prm.ld_h, true, NothingBehind(), more);
 }
 
 template <class T, int AT_ONCE>
@@ -33,24 +33,29 @@ int32_t check_residual(const ResidualParams& prm) {
     return QM_OK;
 }
 
-template <class T>
-static int32_t residual_as(const ResidualParams& prm, int rows, hipStream_t stream) {
+template <class T, bool MORE>
+static int32_t residual_as(const ResidualParams& prm, int rows, const MoreOfTerm& more, hipStream_t stream) {
     switch (row_vectors(prm.ld_h)) {
-        case 1: hipLaunchKernelGGL((residual_norm_kernel<T, 1>), dim3(rows), dim3(kDecThreads), 0, stream, prm); break;
-        case 2: hipLaunchKernelGGL((residual_norm_kernel<T, 2>), dim3(rows), dim3(kDecThreads), 0, stream, prm); break;
-        case 4: hipLaunchKernelGGL((residual_norm_kernel<T, 4>), dim3(rows), dim3(kDecThreads), 0, stream, prm); break;
-        default: hipLaunchKernelGGL((residual_norm_kernel<T, 12>), dim3(rows), dim3(kDecThreads), 0, stream, prm); break;
+        case 1: hipLaunchKernelGGL((residual_norm_kernel<T, 1, MORE>), dim3(rows), dim3(kDecThreads), 0, stream, prm, more); break;
+        case 2: hipLaunchKernelGGL((residual_norm_kernel<T, 2, MORE>), dim3(rows), dim3(kDecThreads), 0, stream, prm, more); break;
+        case 4: hipLaunchKernelGGL((residual_norm_kernel<T, 4, MORE>), dim3(rows), dim3(kDecThreads), 0, stream, prm, more); break;
+        default: hipLaunchKernelGGL((residual_norm_kernel<T, 12, MORE>), dim3(rows), dim3(kDecThreads), 0, stream, prm, more); break;
     }
     return launch_status();
 }
 
-int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipStream_t stream) {
+int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipStream_t stream, const MoreOfTerm& more) {
     const int32_t rc = check_residual(prm);
     if (rc != QM_OK) return rc;
     if (rows < 0) return QM_ERR_ARGUMENT;
     if (!prm.h) return QM_ERR_NULL;
     if (rows == 0) return QM_OK;
-    return f32 ? residual_as<float>(prm, rows, stream) : residual_as<uint16_t>(prm, rows, stream);
+    if (more.planes > 0) {                     // (only the matrix cores' bf16 rows leave a term in pieces)
+        if (!more.sums) return QM_ERR_NULL;
+        if (more.planes > kMorePlanes || prm.terms == 0 || f32) return QM_ERR_ARGUMENT;
+        return residual_as<uint16_t, true>(prm, rows, more, stream);
+    }
+    return f32 ? residual_as<float, false>(prm, rows, more, stream) : residual_as<uint16_t, false>(prm, rows, more, stream);
 }
 
 int32_t launch_gated_norm(const GatedNormParams& prm, int rows, int f32, hipStream_t stream) {

@@ -49,11 +49,25 @@ inline int row_vectors(int64_t ld) { return ld <= 1024 ? 1 : ld <= 2048 ? 2 : ld
 int32_t check_residual(const ResidualParams& prm);
 int32_t check_attention(const ChunkAttentionParams& prm);
 int32_t check_decay_attention(const DecayAttentionParams& prm);
-int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipStream_t stream);
+// The last term in pieces: `planes` more of them, `plane` floats apart, laid out as the term's own and added to it in order.
+constexpr int kMorePlanes = 2;
+struct MoreOfTerm {
+    const float* sums = nullptr;
+    int64_t plane = 0;
+    int planes = 0;
+};
+int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipStream_t stream, const MoreOfTerm& more = MoreOfTerm());
 int32_t launch_gated_norm(const GatedNormParams& prm, int rows, int f32, hipStream_t stream);
 // Many rows of bf16 go to the matrix cores (linears of one launch in one grid, a gate/up pair in its own), few rows and
 // fp32 to the streaming kernel.
-int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream);
+// cut: the last linear's reduction may be taken in pieces, whose sums behind the first's go to cut->sums (room for kMorePlanes planes of
+// [rows][n]); how many do is left in cut->planes.
+struct ReductionCut {
+    float* sums;
+    int64_t plane;
+    int planes;
+};
+int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut = nullptr);
 int32_t launch_split_linears(const DecLinearParams& prm, hipStream_t stream);    // fp32 rows on the matrix cores
 // Rotation and cache write, then the attention.
 int32_t launch_chunk_attention(const ChunkAttentionParams& prm, int f32, hipStream_t stream);

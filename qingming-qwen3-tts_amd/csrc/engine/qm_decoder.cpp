@@ -133,7 +133,7 @@ struct qm_decoder {
     int width_p = 0, vocab_p = 0;
     hipStream_t stream = nullptr;
     bool own_stream = false;
-    qm_engine::DeviceBuffer x[2], h, proj, mlp, attended, gated, y[3], q_rot, raw, ml, acc, scratch, tokens, wanted, head_h, logits, tap, tap_h,
+    qm_engine::DeviceBuffer x[2], h, proj, mlp, attended, gated, y[3], y_more, q_rot, raw, ml, acc, scratch, tokens, wanted, head_h, logits, tap, tap_h,
         step_words, q_latent, queries, q_scratch, expanded, expert_logits, expert_scratch;
     std::vector<hipGraphExec_t> graphs;             // one-token step of each sequence
     std::vector<hipGraphExec_t> mail_graphs;        // the same between the mailbox's words and its scores
@@ -483,6 +483,9 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
     d->attended = zeros(rows * attended * item);
     d->gated = zeros(rows * gated * item);
     for (DeviceBuffer& y : d->y) y = zeros(rows * d->width_p * 4);
+    if (!f32)
+        for (const DecoderLayer& w : d->layers)
+            if (w.config.ff && w.config.form != LayerForm::Sandwich && !d->y_more.raw()) d->y_more = zeros(qm::kMorePlanes * rows * d->width_p * 4);
     d->q_rot = zeros(rows * q_rot * item);
     d->raw = zeros(rows * raw * 4);
     d->ml = zeros(ml * 4);
@@ -511,6 +514,7 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
 struct Pending {
     qm_residual_term term[3] = {};
     int count = 0;
+    qm::MoreOfTerm more;                            // of the last term
 };
 
 qm_residual_norm residual_of(const qm_decoder& d, const Pending& pending, const float* x_in, float* x_out, const float* step_vec, const float* norm,
@@ -792,7 +796,7 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
         const LayerRun& run = d.runs[i];
         const DecoderLayer& w = d.layers[static_cast<size_t>(run.layer)];
         float* x_new = f32_of(d.x[next]);
-        op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, step_vec_of(d, run), f32_of(w.norm1), d.h.raw()), rows, d.f32, s),
+        op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, step_vec_of(d, run), f32_of(w.norm1), d.h.raw()), rows, d.f32, s, pending.more),
                  "residual + norm");
         x = x_new;
         next ^= 1;
@@ -814,10 +818,13 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
             op_check(qm::launch_general_delta(delta_of(d, w, d.states[i], sequence, rows), s), "generalized delta rule");
         }
         if (w.config.mixer != MixerKind::LatentAttention) op_check(qm::launch_gated_norm(gated_of(d, w), rows, d.f32, s), "gated norm");
-        op_check(qm::launch_decoder_linears(linears_out(d, w, rows, pending), d.f32, s), "output projections");
+        const qm::DecLinearParams outputs = linears_out(d, w, rows, pending);
+        qm::ReductionCut cut = {f32_of(d.y_more), 0, 0};
+        op_check(qm::launch_decoder_linears(outputs, d.f32, s, cut.sums ? &cut : nullptr), "output projections");
+        pending.more = {cut.sums, cut.plane, cut.planes};
         if (sandwich(w) && w.config.ff) {
             x_new = f32_of(d.x[next]);
-            op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, nullptr, f32_of(w.norm2), d.h.raw()), rows, d.f32, s), "residual + norm");
+            op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, nullptr, f32_of(w.norm2), d.h.raw()), rows, d.f32, s, pending.more), "residual + norm");
             x = x_new;
             next ^= 1;
             op_check(qm::launch_decoder_linears(feed_in(d, w, rows), d.f32, s), "feed-forward");
@@ -827,7 +834,7 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
         }
         if (taps) {
             // the stream behind this run, before anything is added ahead of the next one
-            op_check(qm::launch_residual_norm(residual_of(d, pending, x, f32_of(d.tap), nullptr, f32_of(d.final_norm), d.tap_h.raw()), rows, d.f32, s),
+            op_check(qm::launch_residual_norm(residual_of(d, pending, x, f32_of(d.tap), nullptr, f32_of(d.final_norm), d.tap_h.raw()), rows, d.f32, s, pending.more),
                      "stream");
             const size_t row_bytes = static_cast<size_t>(d.config.width) * 4;
             hip_check(hipMemcpy2DAsync(taps + i * rows * d.config.width, row_bytes, d.tap.raw(), static_cast<size_t>(d.width_p) * 4, row_bytes,
@@ -872,7 +879,7 @@ void run_head(qm_decoder& d, const float* x, const Pending& pending, const int32
         hip_check(hipMemcpyAsync(d.wanted.raw(), places + first, static_cast<size_t>(rows) * 4, hipMemcpyHostToDevice, s), "wanted rows");
         qm_residual_norm p = residual_of(d, pending, x, nullptr, nullptr, f32_of(d.final_norm), d.head_h.raw());
         p.row_map = static_cast<const int32_t*>(d.wanted.raw());
-        op_check(qm::launch_residual_norm(p, rows, d.f32, s), "final norm");
+        op_check(qm::launch_residual_norm(p, rows, d.f32, s, pending.more), "final norm");
         qm::DecLinearParams l = {};
         l.rows = rows;
         l.group[l.groups++] = linear_of(d.head, d.head_h.raw(), f32_of(d.logits));

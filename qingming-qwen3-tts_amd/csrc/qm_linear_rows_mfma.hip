@@ -180,7 +180,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wave_n = wave % Waves::kAcross, wave_m = wave / Waves::kAcross;
-    int K = prm.reduction;
+    int K = prm.reduction, pitch = prm.pitch;
     int m0 = static_cast<int>(blockIdx.y) * BM;
     // (several linears of one input in one grid: which of them this block's column tile belongs to)
     int tile = static_cast<int>(blockIdx.x);
@@ -202,7 +202,9 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
     float* sums = prm.sums;
     int columns = prm.columns;
     if (!DUAL && prm.groups > 1) {
-        const int g = (tile >= prm.group_first_tile[0]) + (prm.groups > 2 && tile >= prm.group_first_tile[1]);
+        int g = 0;
+#pragma unroll
+        for (int i = 0; i + 1 < kRowsGroups; ++i) g += i + 1 < prm.groups && tile >= prm.group_first_tile[i];
         if (g > 0) {
             tile -= prm.group_first_tile[g - 1];
             weight0 = prm.group_weight[g - 1];
@@ -212,9 +214,11 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
             columns = prm.group_columns[g - 1];
             if (prm.group_input[g - 1]) input = prm.group_input[g - 1];
             if (prm.group_reduction[g - 1]) K = prm.group_reduction[g - 1];
+            pitch = prm.group_pitch[g - 1];
         }
     }
     const int n0 = tile * BN;
+    if (pitch == 0) pitch = K;
     int64_t matrix_at = 0;
     if (prm.tile_matrix) {
         const int matrix = prm.tile_matrix[blockIdx.y];
@@ -228,14 +232,14 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
     // block's first row of each operand: a lane's offset is the same for every piece (WAVES kRowsPerPiece rows further on,
     // the key of a row is the same), what changes from piece to piece and step to step is a scalar; token rows past the
     // last are out of the descriptor's range and read as zero without touching memory (their results are never stored).
-    const uint32_t row_bytes = static_cast<uint32_t>(K) * 2u;
+    const uint32_t row_bytes = static_cast<uint32_t>(pitch) * 2u;
     const int x_rows = min(prm.rows - m0, BM);
     const __amdgpu_buffer_rsrc_t x_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(input + static_cast<int64_t>(m0) * K), 0, static_cast<int>(x_rows * row_bytes), 0x00020000);
+        const_cast<uint16_t*>(input + static_cast<int64_t>(m0) * pitch), 0, static_cast<int>(x_rows * row_bytes), 0x00020000);
     const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>(weight0 + matrix_at + static_cast<int64_t>(n0) * K), 0, static_cast<int>(BN * row_bytes), 0x00020000);
+        const_cast<uint16_t*>(weight0 + matrix_at + static_cast<int64_t>(n0) * pitch), 0, static_cast<int>(BN * row_bytes), 0x00020000);
     const __amdgpu_buffer_rsrc_t u_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint16_t*>((DUAL ? prm.weight[1] : weight0) + matrix_at + static_cast<int64_t>(n0) * K), 0, static_cast<int>(BN * row_bytes), 0x00020000);
+        const_cast<uint16_t*>((DUAL ? prm.weight[1] : weight0) + matrix_at + static_cast<int64_t>(n0) * pitch), 0, static_cast<int>(BN * row_bytes), 0x00020000);
     const int lane_row = kRowsPerPiece * wave + lane / kSlots;
     const uint32_t lane_off = static_cast<uint32_t>(lane_row) * row_bytes
                             + 16u * static_cast<uint32_t>((lane % kSlots) ^ slot_key<kRowBytes>(lane_row));

@@ -6,6 +6,8 @@
 
 namespace qm {
 
+constexpr int kRowsGroups = 5;
+
 struct LinearRowsParams {
     const uint16_t* input;        // [rows][reduction]
     const uint16_t* weight[2];    // [columns][reduction]; [1] = the up matrix (DUAL)
@@ -19,22 +21,24 @@ struct LinearRowsParams {
     // pieces in order and rounds.  1: every block takes the whole reduction and rounds its sums itself.
     int reduction_parts;
     float* partials;
-    // (matrix cores, no gate/up pair) up to three linears of the same input in one grid: the column tiles of linear g
+    // (matrix cores, no gate/up pair) up to kRowsGroups linears of the same input in one grid: the column tiles of linear g
     // start at tile group_first_tile[g] (group 0 at 0), and a block of group g > 0 takes weight / bias / output / columns
     // from group_*[g - 1] instead of the fields above.  groups = 1: one linear.
     int groups;
-    int group_first_tile[2];
-    const uint16_t* group_weight[2];
-    const uint16_t* group_bias[2];
-    uint16_t* group_output[2];
-    int group_columns[2];
+    int group_first_tile[kRowsGroups - 1];
+    const uint16_t* group_weight[kRowsGroups - 1];
+    const uint16_t* group_bias[kRowsGroups - 1];
+    uint16_t* group_output[kRowsGroups - 1];
+    int group_columns[kRowsGroups - 1];
     // (matrix cores, no gate/up pair, reduction uncut) sums != NULL: the fp32 sums as they are go to sums /
     // group_sums[g - 1] ([rows][columns] floats) and nothing to the outputs; bias and residual are not read.
     float* sums;
-    float* group_sums[2];
+    float* group_sums[kRowsGroups - 1];
     // a linear of its own input and reduction (a multiple of 128 as well): NULL / 0 = the first one's
-    const uint16_t* group_input[2];
-    int group_reduction[2];
+    const uint16_t* group_input[kRowsGroups - 1];
+    int group_reduction[kRowsGroups - 1];
+    // elements from a row of input and weights to the next, where a linear takes a piece of longer rows; 0: its reduction
+    int pitch, group_pitch[kRowsGroups - 1];
     // blocks in the order linear by linear (all row tiles of the first, then of the next) instead of row tile by row
     // tile: the linears with the long reductions first, so that none of them starts late
     int linear_by_linear;

@@ -408,3 +408,30 @@ def test_weights_beyond_the_cache_give_the_same_bits(decoder, tmp_path, design):
         del engine
     for want, got in zip(*rows):
         assert np.array_equal(got, np.tile(want, times))
+
+
+@pytest.mark.parametrize("layer,width,rows", [
+    (cases.general_delta(32, 64, 6144), 2048, 1000),                                                             # in three pieces
+    (cases.parallel(cases.left(16, 4, 128, 128, 512, 64), cases.right(16, 64, 128, [0.95] * 16), 6144), 2048, 900),   # in two, beside two
+    (cases.general_delta(16, 64, 3072), 1024, 1601),                                                             # in two
+    (cases.general_delta(16, 64, 384), 1024, 1601),                                                              # whole
+])
+def test_down_projection_in_pieces(decoder, tmp_path, layer, width, rows):
+    """A prompt in one pass, where pieces of the down projection's reduction fill idle CUs, against portions too short for that: streams behind
+    each layer and scores.  Both sides' sums are fp32; what they round to bf16 may part by a step, as against the oracle."""
+    cfg = cases.config(256, width, [layer, layer])
+    cases.write_model(str(tmp_path), cfg, cases.weights(cfg))
+    tokens = cases.tokens_of(cfg, rows)
+    places = sorted({0, 63, 127, 128, rows // 2, rows - 2, rows - 1})
+    whole = decoder.Decoder(str(tmp_path), rows, max_rows=rows)
+    logits, streams = whole.step(whole.open(), tokens, places, streams=True)
+    portions = decoder.Decoder(str(tmp_path), rows, max_rows=400)
+    s, parts, scores = portions.open(), [], []
+    for at in range(0, rows, 400):
+        got, stream = portions.step(s, tokens[at:at + 400], [p - at for p in places if at <= p < at + 400], streams=True)
+        parts.append(stream)
+        scores.append(got)
+    want = np.concatenate(parts, axis=1)
+    for i in range(2):
+        assert cases.error(streams[i], want[i]) < LIMIT[False], i
+    assert cases.error(logits, np.concatenate(scores)) < LIMIT[False]
