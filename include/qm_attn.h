@@ -856,6 +856,16 @@ int32_t qm_linear_rows_split(
     const uint16_t* input, const uint16_t* weight, const uint16_t* bias, const uint16_t* residual,
     uint16_t* output, int32_t rows, int32_t output_columns, int32_t reduction_columns,
     void* workspace, int64_t workspace_bytes, void* hip_stream);
+/*
+ * qm_linear_rows with a residual, and RMSNorm (qm_rmsnorm_rows) of the rows that it leaves.  With a workspace of
+ * qm_linear_rows_norm_workspace_bytes (0 where the shape is not cut; as above otherwise) a long reduction is cut into pieces that the norm's launch
+ * adds; without one exactly the two calls.
+ */
+int64_t qm_linear_rows_norm_workspace_bytes(int32_t rows, int32_t output_columns, int32_t reduction_columns);
+int32_t qm_linear_rows_norm(
+    const uint16_t* input, const uint16_t* weight, const uint16_t* bias, const uint16_t* residual, uint16_t* output,
+    const uint16_t* norm_weight, uint16_t* normalized, int32_t rows, int32_t output_columns, int32_t reduction_columns, float epsilon,
+    void* workspace, int64_t workspace_bytes, void* hip_stream);
 int32_t qm_gate_up_swiglu_rows_split(
     const uint16_t* input, const uint16_t* gate_weight, const uint16_t* up_weight, uint16_t* output,
     int32_t rows, int32_t hidden, int32_t intermediate,

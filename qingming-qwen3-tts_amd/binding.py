@@ -154,6 +154,8 @@ _SIGNATURES = {
     "qm_linear_rows": (_I32, [_PTR] * 5 + [_I32, _I32, _I32, _PTR]),
     "qm_gate_up_swiglu_rows": (_I32, [_PTR] * 4 + [_I32, _I32, _I32, _PTR]),
     "qm_linear_rows_split_workspace_bytes": (C.c_int64, [_I32, _I32, _I32, _I32]),
+    "qm_linear_rows_norm_workspace_bytes": (C.c_int64, [_I32, _I32, _I32]),
+    "qm_linear_rows_norm": (_I32, [_PTR] * 7 + [_I32, _I32, _I32, C.c_float, _PTR, C.c_int64, _PTR]),
     "qm_linear_rows_split": (_I32, [_PTR] * 5 + [_I32, _I32, _I32, _PTR, C.c_int64, _PTR]),
     "qm_gate_up_swiglu_rows_split": (_I32, [_PTR] * 4 + [_I32, _I32, _I32, _PTR, C.c_int64, _PTR]),
     "qm_qkv_rows": (_I32, [_PTR] * 10 + [_I32, _I32, _I32, _I32, _PTR]),

@@ -328,7 +328,7 @@ static const uint16_t* decode(qm_talker& e, const uint16_t* input_device, const 
 //   linear_generic (o_proj) + add             -> qm_linear_rows with the residual folded in
 //   rmsnorm                                   -> qm_rmsnorm_rows
 //   2 x linear_generic + swiglu               -> qm_gate_up_swiglu_rows
-//   linear_generic (down) + add               -> qm_linear_rows with the residual folded in
+//   linear_generic (down) + add, next rmsnorm  -> qm_linear_rows_norm
 // and the final RMSNorm, of the last row only (the one row the reference reads back).
 static const uint16_t* prefill(qm_talker& e, const uint16_t* input_device, const uint16_t* cosine, const uint16_t* sine,
                                int rows) {
@@ -359,7 +359,8 @@ static const uint16_t* prefill(qm_talker& e, const uint16_t* input_device, const
                                qm_linear_rows_split_workspace_bytes(rows, e.kv_dim, kHidden, 0),
                                qm_linear_rows_split_workspace_bytes(rows, kHidden, e.q_dim, 0),
                                qm_linear_rows_split_workspace_bytes(rows, e.intermediate, kHidden, 1),
-                               qm_linear_rows_split_workspace_bytes(rows, kHidden, e.intermediate, 0)})
+                               qm_linear_rows_split_workspace_bytes(rows, kHidden, e.intermediate, 0),
+                               qm_linear_rows_norm_workspace_bytes(rows, kHidden, e.intermediate)})
         rows_bytes = std::max(rows_bytes, need);
     if (static_cast<size_t>(rows_bytes) > e.p_rows_split.bytes()) {
         hip_check(hipStreamSynchronize(s), "prefill workspace growth");
@@ -373,10 +374,10 @@ static const uint16_t* prefill(qm_talker& e, const uint16_t* input_device, const
     hip_check(hipMemcpyAsync(e.p_sine.raw(), sine, rope_bytes, hipMemcpyHostToDevice, s), "prefill sine upload");
     DeviceBuffer* current = &e.p_hidden_a;
     DeviceBuffer* next = &e.p_hidden_b;
-    for (Layer& w : e.layers) {
+    op_check(qm_rmsnorm_rows(current->u16(), e.layers.front().input_norm.data(), e.p_norm.u16(), rows, kHidden, kEpsilon, s), "prefill input RMSNorm");
+    for (size_t i = 0; i < e.layers.size(); ++i) {
+        Layer& w = e.layers[i];
         const qm_kv_cache cache = flat_cache_of(e, w);
-        op_check(qm_rmsnorm_rows(current->u16(), w.input_norm.data(), e.p_norm.u16(), rows, kHidden, kEpsilon, s),
-                 "prefill input RMSNorm");
         op_check(qm_qkv_rows_split(e.p_norm.u16(), w.q_weight.data(), w.k_weight.data(), w.v_weight.data(), w.q_bias.data(),
                                    w.k_bias.data(), w.v_bias.data(), e.p_q.u16(), e.p_k.u16(), e.p_v.u16(), rows, e.q_dim, e.kv_dim,
                                    kHidden, rows_ws, rows_bytes, s), "prefill q/k/v_proj");
@@ -394,8 +395,13 @@ static const uint16_t* prefill(qm_talker& e, const uint16_t* input_device, const
                  "prefill post-attention RMSNorm");
         op_check(qm_gate_up_swiglu_rows_split(e.p_norm.u16(), w.gate_weight.data(), w.up_weight.data(), e.p_swiglu.u16(), rows,
                                               kHidden, e.intermediate, rows_ws, rows_bytes, s), "prefill gate/up/SwiGLU");
-        op_check(qm_linear_rows_split(e.p_swiglu.u16(), w.down_weight.data(), nullptr, e.p_residual.u16(), next->u16(), rows,
-                                      kHidden, e.intermediate, rows_ws, rows_bytes, s), "prefill down_proj + residual");
+        if (i + 1 < e.layers.size())
+            op_check(qm_linear_rows_norm(e.p_swiglu.u16(), w.down_weight.data(), nullptr, e.p_residual.u16(), next->u16(),
+                                         e.layers[i + 1].input_norm.data(), e.p_norm.u16(), rows, kHidden, e.intermediate, kEpsilon,
+                                         rows_ws, rows_bytes, s), "prefill down_proj + residual + input RMSNorm");
+        else
+            op_check(qm_linear_rows_split(e.p_swiglu.u16(), w.down_weight.data(), nullptr, e.p_residual.u16(), next->u16(), rows,
+                                          kHidden, e.intermediate, rows_ws, rows_bytes, s), "prefill down_proj + residual");
         std::swap(current, next);
     }
     op_check(qm_rmsnorm_rows(current->u16() + static_cast<size_t>(rows - 1) * kHidden, e.final_norm.data(),

@@ -289,6 +289,43 @@ extern "C" int64_t qm_linear_rows_split_workspace_bytes(int32_t rows, int32_t ou
     return static_cast<int64_t>(rows_mfma_workspace_bytes(rows, output_columns, reduction_columns, gate_up_pair != 0));
 }
 
+extern "C" int64_t qm_linear_rows_norm_workspace_bytes(int32_t rows, int32_t output_columns, int32_t reduction_columns) {
+    using namespace qm;
+    if (rows < kRowsMatrixMinimum || output_columns <= 0 || reduction_columns <= 0 || output_columns % 128 || reduction_columns % 128) return 0;
+    bool wide = false;
+    const int parts = rows_mfma_norm_parts(rows, output_columns, reduction_columns, &wide);
+    return parts > 1 ? static_cast<int64_t>(parts) * rows * output_columns * 4 : 0;
+}
+
+extern "C" int32_t qm_linear_rows_norm(const uint16_t* input, const uint16_t* weight, const uint16_t* bias, const uint16_t* residual, uint16_t* output,
+                                       const uint16_t* norm_weight, uint16_t* normalized, int32_t rows, int32_t output_columns,
+                                       int32_t reduction_columns, float epsilon, void* workspace, int64_t workspace_bytes, void* hip_stream) {
+    using namespace qm;
+    if (!input || !weight || !residual || !output || !norm_weight || !normalized) return QM_ERR_NULL;
+    if (workspace_bytes < 0 || (workspace_bytes > 0 && !workspace)) return QM_ERR_ARGUMENT;
+    if (reinterpret_cast<uintptr_t>(workspace) & 255) return QM_ERR_GEOMETRY;
+    LinearRowsParams prm = {};
+    prm.input = input; prm.weight[0] = weight; prm.weight[1] = weight; prm.bias = bias; prm.residual = residual;
+    prm.output = output; prm.rows = rows; prm.columns = output_columns; prm.reduction = reduction_columns;
+    int32_t rc = check_rows(prm, false);
+    int32_t matrix_cores = 0;
+    if (rc == QM_OK) rc = rows_on_matrix_cores(prm, &matrix_cores);
+    if (rc != QM_OK) return rc;
+    const int64_t need = workspace && matrix_cores ? qm_linear_rows_norm_workspace_bytes(rows, output_columns, reduction_columns) : 0;
+    if (need > workspace_bytes) return QM_ERR_WORKSPACE;
+    if (need > 0) {
+        prm.reduction_parts = rows_mfma_norm_parts(rows, output_columns, reduction_columns, &prm.wide_tiles);
+        prm.partials = static_cast<float*>(workspace);
+        prm.groups = 1;
+        prm.norm_weight = norm_weight;
+        prm.normalized = normalized;
+        prm.epsilon = epsilon;
+        return launch_rows_mfma(prm, false, static_cast<hipStream_t>(hip_stream));
+    }
+    rc = qm_linear_rows(input, weight, bias, residual, output, rows, output_columns, reduction_columns, hip_stream);
+    return rc == QM_OK ? qm_rmsnorm_rows(output, norm_weight, normalized, rows, output_columns, epsilon, hip_stream) : rc;
+}
+
 extern "C" int32_t qm_linear_rows_split(const uint16_t* input, const uint16_t* weight, const uint16_t* bias,
                                         const uint16_t* residual, uint16_t* output, int32_t rows, int32_t output_columns,
                                         int32_t reduction_columns, void* workspace, int64_t workspace_bytes, void* hip_stream) {

@@ -596,6 +596,48 @@ __global__ __launch_bounds__(256) void linear_rows_parts_kernel(LinearRowsParams
     *reinterpret_cast<uint2*>(prm.output + static_cast<int64_t>(m) * prm.columns + n) = packed;
 }
 
+// The pieces of a cut reduction added in order, the roundings of the epilogue, and RMSNorm of the row that they make, in rmsnorm_held_rows_kernel's
+// order: block = row, thread t = columns t, t + 256, ... (N of them), two pieces asked for at once (there are 2, 4 or 8).  Bound by the pieces' bytes:
+// 1000 rows of 2048 in two 6.9 us, where the norm alone takes 5.2.
+template <int N>
+__global__ __launch_bounds__(256) void linear_rows_parts_norm_kernel(LinearRowsParams prm) {
+    request_arguments(prm);
+    __shared__ float sh_waves[8];
+    __shared__ float sh_total;
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * (N * 256) + threadIdx.x, plane = static_cast<int64_t>(prm.rows) * (N * 256);
+    uint16_t res[N], weight[N];
+    float sum[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        sum[i] = 0.0f;
+        res[i] = prm.residual[base + i * 256];
+        weight[i] = prm.norm_weight[threadIdx.x + i * 256];
+    }
+    for (int z = 0; z < prm.reduction_parts; z += 2) {
+        const float* at = prm.partials + z * plane + base;
+        float one[N], two[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) one[i] = at[i * 256];
+#pragma unroll
+        for (int i = 0; i < N; ++i) two[i] = at[plane + i * 256];
+#pragma unroll
+        for (int i = 0; i < N; ++i) sum[i] = (sum[i] + one[i]) + two[i];
+    }
+    float squares = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        if (prm.bias) sum[i] += bf2f(prm.bias[threadIdx.x + i * 256]);
+        const uint16_t out = f2bf(bf2f(res[i]) + round_bf16(sum[i]));
+        prm.output[base + i * 256] = out;
+        sum[i] = bf2f(out);
+        squares = fmaf(sum[i], sum[i], squares);
+    }
+    const float total = block_sum_256_like_reference(squares, sh_waves, &sh_total);
+    const float inverse_rms = 1.0f / sqrtf(total / static_cast<float>(N * 256) + prm.epsilon);
+#pragma unroll
+    for (int i = 0; i < N; ++i) prm.normalized[base + i * 256] = f2bf(round_bf16(sum[i] * inverse_rms) * bf2f(weight[i]));
+}
+
 template <bool DUAL, int BM, int BN, int KSTEP, int WAVES>
 int32_t launch_rows_mfma_as(const LinearRowsParams& given, hipStream_t stream) {
     LinearRowsParams prm = given;
@@ -618,7 +660,11 @@ int32_t launch_rows_mfma_as(const LinearRowsParams& given, hipStream_t stream) {
     if (rc != QM_OK) return rc;
     hipLaunchKernelGGL((linear_rows_mfma_kernel<DUAL, BM, BN, KSTEP, WAVES>), grid, dim3(64 * WAVES), smem, stream, prm);
     int32_t status = launch_status();
-    if (status == QM_OK && prm.reduction_parts > 1) {
+    if (status == QM_OK && prm.reduction_parts > 1 && prm.norm_weight) {
+        const auto kernel = prm.columns == 2048 ? linear_rows_parts_norm_kernel<8> : linear_rows_parts_norm_kernel<4>;
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(prm.rows)), dim3(256), 0, stream, prm);
+        status = launch_status();
+    } else if (status == QM_OK && prm.reduction_parts > 1) {
         const int64_t quads = static_cast<int64_t>(prm.rows) * (prm.columns / 4);
         hipLaunchKernelGGL((linear_rows_parts_kernel<DUAL>), dim3(static_cast<unsigned>((quads + 255) / 256)), dim3(256), 0, stream, prm);
         status = launch_status();
@@ -641,6 +687,20 @@ int rows_mfma_reduction_parts(int rows, int columns, int reduction, bool dual) {
     for (int p = 2; p <= 8; p *= 2)
         if (blocks * p <= 256 && steps % p == 0) parts = p;
     return parts;
+}
+
+// With a norm behind, whose launch adds the pieces for the price of their bytes, a long reduction is also cut in two where 64-row tiles would just
+// give every CU a block: as many blocks of 128 x 128 walk half the steps for two thirds of the requests an output takes (1000 tokens, 2048 columns of
+// 6144, with the norm behind: 52.1 -> 44.8 us).
+int rows_mfma_norm_parts(int rows, int columns, int reduction, bool* wide) {
+    *wide = false;
+    if (columns != 1024 && columns != 2048) return 1;
+    const int parts = rows_mfma_reduction_parts(rows, columns, reduction, false);
+    if (parts > 1 || rows <= 0 || reduction < kGmStep) return parts;
+    const int64_t blocks = static_cast<int64_t>(columns / 128) * ((rows + 127) / 128) * 2;
+    const int steps = reduction / kGmStep;
+    *wide = steps >= 64 && steps % 2 == 0 && blocks >= 200 && blocks <= 256;
+    return *wide ? 2 : 1;
 }
 
 size_t rows_mfma_workspace_bytes(int rows, int columns, int reduction, bool dual) {
@@ -677,6 +737,7 @@ int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t str
     int64_t columns = prm.columns;
     for (int g = 1; g < prm.groups; ++g) columns += prm.group_columns[g - 1];
     const int64_t blocks_128 = columns / kGmTile * row_tiles;
+    if (prm.wide_tiles) return launch_rows_mfma_as<false, 128, 128, 64, 8>(prm, stream);
     const bool small = blocks_128 < 200;
     // Measured (us, 64 x 128 / 64 x 64 tiles): 2048 columns of 6144 at 16 / 64 / 300 / 500 rows 24 / 28 / 27 / 28 against 17 / 20 / 20 / 22,
     // 4096 of 2048 at 128 / 200 / 300 rows 10.9 / 11.1 / 11.4 against 8.7 / 9.5 / 16.2, pairs of 6144 of 2048 at 64 / 128 / 200 rows

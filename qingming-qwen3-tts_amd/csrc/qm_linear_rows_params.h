@@ -48,6 +48,12 @@ struct LinearRowsParams {
     int tile_rows;
     // (matrix cores) column tiles of the launch, which sets it: the grid may be wider
     int column_tiles;
+    // (a cut reduction of 1024 or 2048 columns) norm_weight != NULL: the launch that adds the pieces also leaves RMSNorm of the output's rows
+    const uint16_t* norm_weight;
+    uint16_t* normalized;
+    float epsilon;
+    // (a cut reduction) 128 x 128 tiles
+    bool wide_tiles;
 };
 
 // The row linears on the matrix cores (qm_linear_rows_mfma.hip).  `dual`: weight[0] / weight[1] are the gate and up
@@ -58,5 +64,7 @@ int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t str
 // function of the shape), and the bytes that workspace must hold (0: the shape is not cut).
 int rows_mfma_reduction_parts(int rows, int columns, int reduction, bool dual);
 size_t rows_mfma_workspace_bytes(int rows, int columns, int reduction, bool dual);
+// The same where the pieces are added by the launch of a norm that is there anyway; *wide: in 128 x 128 tiles.
+int rows_mfma_norm_parts(int rows, int columns, int reduction, bool* wide);
 
 }  // namespace qm

@@ -316,3 +316,36 @@ def test_swiglu_of_every_bf16_gate(qm, dev, rows_kernel):
             got.append(out)
         torch.cuda.synchronize()
         assert bool((got[0] == got[1]).all()), part
+
+
+@pytest.mark.parametrize("rows,cols,red", [(16, 2048, 6144), (100, 1024, 4096), (785, 2048, 6144), (1000, 2048, 6144), (1024, 2048, 4224), (1601, 1024, 4096),
+                                           (2048, 1024, 6144), (1025, 2048, 6144), (300, 1536, 4096), (900, 2048, 2048)])
+@pytest.mark.parametrize("rows_kernel", [MATRIX, EXACT], indirect=True)
+@pytest.mark.parametrize("bias", [False, True])
+def test_linear_and_norm_of_its_rows(qm, dev, rows, cols, red, rows_kernel, bias):
+    """Cut in 128-row tiles, cut in smaller ones, not cut, on the exact chain: the sum with its residual against 64 bits, the norm the bits that
+    qm_rmsnorm_rows gives for the output."""
+    import torch
+    if rows_kernel == EXACT and rows > 100:
+        rows = 17
+    gen = torch.Generator(device=dev).manual_seed(rows + cols + red)
+    x, w, res, gamma = (torch.randn(*shape, device=dev, generator=gen).bfloat16() for shape in ((rows, red), (cols, red), (rows, cols), (cols,)))
+    b = torch.randn(cols, device=dev, generator=gen).bfloat16() if bias else None
+    need = qm.lib().qm_linear_rows_norm_workspace_bytes(rows, cols, red)
+    ws = torch.empty(max(need, 256), dtype=torch.uint8, device=dev)
+    out, normed = (torch.full((rows + 1, cols), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(2))
+    call = lambda bytes_: qm.lib().qm_linear_rows_norm(x.data_ptr(), w.data_ptr(), b.data_ptr() if bias else None, res.data_ptr(), out.data_ptr(),
+                                                       gamma.data_ptr(), normed.data_ptr(), rows, cols, red, 1e-6, ws.data_ptr(), bytes_, None)
+    if need > 0 and rows_kernel == MATRIX:
+        assert call(need - 256) < 0
+    assert call(need) == 0
+    again = torch.empty(rows, cols, dtype=torch.bfloat16, device=dev)
+    qm.rmsnorm_rows(out, gamma, again, rows, cols, 1e-6)
+    torch.cuda.synchronize()
+    assert bool((normed[:rows].view(torch.int16) == again.view(torch.int16)).all())
+    assert bool(out[rows].isnan().all() and normed[rows].isnan().all())
+    sums = x.double() @ w.double().t() + (b.double() if bias else 0.0)
+    want = sums + res.double()
+    # two roundings, each half a bf16 spacing at most, and the fp32 sum's own error: red * 2^-24 of the sum of magnitudes
+    bound = (sums.abs() + want.abs()) * 2.0 ** -8 + (x.double().abs() @ w.double().abs().t()) * red * 2.0 ** -24
+    assert bool(((out[:rows].double() - want).abs() <= bound).all())
