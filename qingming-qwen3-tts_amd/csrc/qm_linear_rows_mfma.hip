@@ -690,8 +690,10 @@ int rows_mfma_reduction_parts(int rows, int columns, int reduction, bool dual) {
 }
 
 // With a norm behind, whose launch adds the pieces for the price of their bytes, a long reduction is also cut in two where 64-row tiles would just
-// give every CU a block: as many blocks of 128 x 128 walk half the steps for two thirds of the requests an output takes (1000 tokens, 2048 columns of
-// 6144, with the norm behind: 52.1 -> 44.8 us).
+// give every CU a block: as many blocks of 128 x 128 walk half the steps for two thirds of the requests an output takes.  (us, 2048 columns with the
+// norm behind, 64-row tiles / cut: of 6144, weights from memory, 1000 tokens 52.1 / 44.8; weights still in the caches, 785, 900, 1000 and 1024 tokens
+// 35.2 / 34.0, 37.9 / 38.1, 39.7 / 41.1 and 40.4 / 41.9; 1024 columns, 1600 tokens 39.0 / 36.0.  Of 2048, from memory, 24.1 / 23.9, and of 4096, from the
+// caches, 29.0 / 34.7: shorter ones stay.)
 int rows_mfma_norm_parts(int rows, int columns, int reduction, bool* wide) {
     *wide = false;
     if (columns != 1024 && columns != 2048) return 1;
@@ -699,7 +701,7 @@ int rows_mfma_norm_parts(int rows, int columns, int reduction, bool* wide) {
     if (parts > 1 || rows <= 0 || reduction < kGmStep) return parts;
     const int64_t blocks = static_cast<int64_t>(columns / 128) * ((rows + 127) / 128) * 2;
     const int steps = reduction / kGmStep;
-    *wide = steps >= 64 && steps % 2 == 0 && blocks >= 200 && blocks <= 256;
+    *wide = steps >= 96 && steps % 2 == 0 && blocks >= 200 && blocks <= 256;
     return *wide ? 2 : 1;
 }
 
