@@ -648,11 +648,9 @@ int32_t launch_rows_mfma_as(const LinearRowsParams& given, hipStream_t stream) {
     int column_tiles = prm.columns / BN;
     for (int g = 1; g < prm.groups; ++g) column_tiles += prm.group_columns[g - 1] / BN;
     prm.column_tiles = column_tiles;
-    // Blocks go to the eight dies in turn: where 8 divides the column tiles, the row tiles of one read its weights on one die.  Many column tiles are
-    // rounded up to that, the blocks beyond end at once (1024 tokens, 81 column tiles of 2048: 64.8 -> 56.1 us, 80: 54.2); of few the dies' shares would
-    // be too uneven.
-    if (column_tiles > 40 && prm.rows > BM && !prm.linear_by_linear) column_tiles = (column_tiles + 7) / 8 * 8;
-    const dim3 grid(static_cast<unsigned>(column_tiles), static_cast<unsigned>((prm.rows + BM - 1) / BM),
+    const int row_tiles = (prm.rows + BM - 1) / BM;
+    if (!prm.linear_by_linear) column_tiles = rows_grid_columns(column_tiles, row_tiles, prm.reduction_parts);
+    const dim3 grid(static_cast<unsigned>(column_tiles), static_cast<unsigned>(row_tiles),
                     static_cast<unsigned>(prm.reduction_parts));
     if (grid.y > 65535u) return QM_ERR_ARGUMENT;
     static std::atomic<bool> lds_raised[kMaxDevices];
