@@ -156,7 +156,7 @@ struct GmSchedule {
 
 template <bool DUAL, int BM, int BN, int KSTEP, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRowsParams prm) {
-    request_arguments(prm);
+    request_large_argument(prm);
     extern __shared__ __attribute__((aligned(16))) unsigned char gm_smem[];
     constexpr int kStages = GmShape<DUAL, BM, BN, KSTEP>::kStages;
     constexpr int kRowBytes = KSTEP * 2, kSlots = kRowBytes / 16, kKb = KSTEP / 16;
@@ -184,7 +184,6 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
     int m0 = static_cast<int>(blockIdx.y) * BM;
     // (several linears of one input in one grid: which of them this block's column tile belongs to)
     int tile = static_cast<int>(blockIdx.x);
-    if (tile >= prm.column_tiles) return;                         // (the grid's width is rounded up)
     if (!DUAL && prm.linear_by_linear) {
         int at = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x), first = 0, next = prm.group_first_tile[0];
         for (int g = 1; g < prm.groups && at >= static_cast<int>(gridDim.y) * (next - first); ++g) {
@@ -218,6 +217,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
         }
     }
     const int n0 = tile * BN;
+    if (n0 >= columns) return;                                    // (the grid's width may be rounded up)
     if (pitch == 0) pitch = K;
     int64_t matrix_at = 0;
     if (prm.tile_matrix) {
@@ -565,7 +565,7 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
 // The pieces of a cut reduction added in order, then what the epilogue above does: thread = four output columns of a row.
 template <bool DUAL>
 __global__ __launch_bounds__(256) void linear_rows_parts_kernel(LinearRowsParams prm) {
-    request_arguments(prm);
+    request_large_argument(prm);
     const int64_t quad = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const int quads_per_row = prm.columns / 4;
     if (quad >= static_cast<int64_t>(prm.rows) * quads_per_row) return;
@@ -601,7 +601,7 @@ __global__ __launch_bounds__(256) void linear_rows_parts_kernel(LinearRowsParams
 // 1000 rows of 2048 in two 6.9 us, where the norm alone takes 5.2.
 template <int N>
 __global__ __launch_bounds__(256) void linear_rows_parts_norm_kernel(LinearRowsParams prm) {
-    request_arguments(prm);
+    request_large_argument(prm);
     __shared__ float sh_waves[8];
     __shared__ float sh_total;
     const int64_t base = static_cast<int64_t>(blockIdx.x) * (N * 256) + threadIdx.x, plane = static_cast<int64_t>(prm.rows) * (N * 256);
@@ -647,7 +647,6 @@ int32_t launch_rows_mfma_as(const LinearRowsParams& given, hipStream_t stream) {
     constexpr int smem = Shape::kStages * Shape::kStageBytes + (Shape::kStages == 2 ? 256 * WAVES : 0);
     int column_tiles = prm.columns / BN;
     for (int g = 1; g < prm.groups; ++g) column_tiles += prm.group_columns[g - 1] / BN;
-    prm.column_tiles = column_tiles;
     const int row_tiles = (prm.rows + BM - 1) / BM;
     if (!prm.linear_by_linear) column_tiles = rows_grid_columns(column_tiles, row_tiles, prm.reduction_parts);
     const dim3 grid(static_cast<unsigned>(column_tiles), static_cast<unsigned>(row_tiles),

@@ -46,8 +46,6 @@ struct LinearRowsParams {
     // tile_rows rows (64 or 128) takes matrix tile_matrix[t], or is left out where that is negative
     const int32_t* tile_matrix;
     int tile_rows;
-    // (matrix cores) column tiles of the launch, which sets it: the grid may be wider
-    int column_tiles;
     // (a cut reduction of 1024 or 2048 columns) norm_weight != NULL: the launch that adds the pieces also leaves RMSNorm of the output's rows
     const uint16_t* norm_weight;
     uint16_t* normalized;
