@@ -1,6 +1,7 @@
 """CPU-only checks of rules that choose a launch's shape: small programs over the kernels' own headers, linked with the built library where the rule
 lives in it."""
 import os
+import re
 import subprocess
 
 import pytest
@@ -47,3 +48,42 @@ int main() {
             rounded += 1
     assert rounded > 5000
     assert "81 8 1 88" in lines and "42 6 1 42" in lines and "42 3 2 42" in lines
+
+
+def test_a_steps_weights_stay_in_flight(tmp_path):
+    """A long row's dot products, the first weights asked for at one of several places as in a step's output launch: in the loop over the row nothing waits
+    for all loads (vmcnt(0)), a piece's products leave the requests behind it under way."""
+    (tmp_path / "loop.hip").write_text("""
+#include "decoder/qm_decoder_device.h"
+#include "decoder/qm_decoder_dot.h"
+using namespace qm;
+extern "C" __global__ __launch_bounds__(256) void long_row(DecLinearGroup group, const uint16_t* x, int kind) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    uint16_t* xs = reinterpret_cast<uint16_t*>(smem);
+    const auto d = dot_rows<2, false>(group, static_cast<int>(blockIdx.x));
+    uint4 piece[kDotAhead][2];
+    if (kind == 0) {
+        dot_request(d, group.k, piece);
+        for (int c = threadIdx.x; c < group.k; c += 256) xs[c] = x[c];
+    } else {
+        const uint16_t first = x[threadIdx.x];
+        dot_request(d, group.k, piece);
+        for (int c = threadIdx.x; c < group.k; c += 256) xs[c] = first;
+    }
+    __syncthreads();
+    dot_finish<uint16_t, 1>(group, d, piece, xs, 0, 1);
+}
+""")
+    subprocess.run(["hipcc", "--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                    "-I" + CSRC, "--cuda-device-only", "-S", str(tmp_path / "loop.hip"), "-o", str(tmp_path / "loop.s")], check=True, capture_output=True)
+    text = (tmp_path / "loop.s").read_text()
+    body = text[text.index("\nlong_row:"):text.index(".Lfunc_end0")]
+    # the loop: the shortest stretch between a label and a branch back to it with products and requests in it
+    loops = []
+    for m in re.finditer(r"s_cbranch_\w+ (\.LBB\d+_\d+)", body):
+        start = body.find("\n" + m.group(1) + ":")
+        if 0 <= start < m.start():
+            loop = body[start:m.start()]
+            if "v_dot2" in loop and "global_load_dwordx4" in loop:
+                loops.append(loop)
+    assert not re.search(r"s_waitcnt[^\n]*vmcnt\(0\)", min(loops, key=len))
