@@ -14,12 +14,13 @@
 // (histogram passes of 12 bits, sixteen bins per thread, ended as soon as few enough keys lie at or above it to be
 // ranked), those keys are gathered and ranked by counting, several threads to a key where there are threads for it, and
 // the first `keep` ranks are the sequence.  The select looks at each thread's largest key first: the keep-th largest of
-// those is such a bound, with an eighth of the additions to LDS; only where it lets too many keys through (equal scores, or
-// one thread holding many of the largest) does it look at all of them.  The exponentials are computed by `keep` threads at once; the sums
+// those is such a bound, with an eighth of the additions to LDS; only where it would let too many keys through (`keep` beyond half of the
+// threads) or does (one thread holding many of the largest) are all keys looked at, in passes of 8 bits.  The exponentials are computed by `keep` threads at once; the sums
 // are added in the reference's order: the running sum of the second loop repeats the partial sums of the first, so one pass
 // gives both.
 // Bound: a chain of LDS exchanges.  Cycles for 50 of 2048 16-bit scores: 14 400 with 64-bit keys, 8-bit digits of all keys until the bin is
-// wanted whole, a thread per key and the sums of one thread through LDS; 9 900 as it stands.
+// wanted whole, a thread per key and the sums of one thread through LDS; 9 900 as it stands.  (us a draw of many in a row, 200 of 2048: 16-bit scores
+// 14.5 so at first, 13.0 from the largest keys and then from all, 11.5 from all at once; 32-bit ones 11.5, 14.4 and 11.7.)
 // One block of 256 threads; vocab <= 4096 (the reference's sort size), top_k <= 256.
 #pragma once
 
@@ -33,6 +34,9 @@ constexpr int kSmpPerThread = kSmpMaxVocab / kSmpThreads;
 constexpr int kSmpMaxKeep = 256;
 constexpr int kSmpBins = 4096;                           // of a histogram pass: 16-bit counters, two to a word
 constexpr int kSmpWords = kSmpBins / 2 / kSmpThreads;    // counter words of a thread
+// Most entries that the select finds from each thread's largest key.  Of random scores the keep-th largest of 256 maxima lets through about
+// -256 ln(1 - keep / 256) keys, 177 for 128 and more than can be ranked from 160 on: its passes would be for nothing.
+constexpr int kSmpFromLargest = 128;
 
 struct SamplerParams {
     const void* logits;          // float or bf16 bits
@@ -90,8 +94,9 @@ __device__ __forceinline__ int wave_inclusive_scan(int v, int lane) {
     return v;
 }
 
-// A score and its id as one number: larger key = earlier in the order; 0 is below every key.  kPasses radix digits of `width(p)` bits
-// from bit `shift(p)` on cover the significant bits; those that no pass looks at (kFree) are set in every key.
+// A score and its id as one number: larger key = earlier in the order; 0 is below every key.  kPasses radix digits of 12 bits (`mask(p)`)
+// from bit `shift(p)` on cover the significant bits, or kBytePasses of 8 (`byte_mask(p)`, `byte_shift(p)`); those that no pass looks at (kFree)
+// are set in every key.
 template <bool NARROW>
 struct SamplerKey;
 template <>
@@ -101,6 +106,9 @@ struct SamplerKey<false> {                               // any score: 32 bits o
     static constexpr type kFree = 0xfffff000ULL;
     static __device__ __forceinline__ int shift(int p) { return p == 0 ? 52 : p == 1 ? 40 : p == 2 ? 32 : 0; }
     static __device__ __forceinline__ unsigned mask(int p) { return p == 2 ? 0xffU : 0xfffU; }
+    static constexpr int kBytePasses = 6;
+    static __device__ __forceinline__ int byte_shift(int p) { return p < 4 ? 56 - 8 * p : p == 4 ? 4 : 0; }
+    static __device__ __forceinline__ unsigned byte_mask(int p) { return p == 5 ? 0xfU : 0xffU; }
     static __device__ __forceinline__ type make(float v, int id) {
         return (static_cast<type>(ordered_bits(v)) << 32) | (0xffffffffU - static_cast<uint32_t>(id));
     }
@@ -114,6 +122,9 @@ struct SamplerKey<true> {                                // scores that are bf16
     static constexpr type kFree = 0xf000U;
     static __device__ __forceinline__ int shift(int p) { return p == 0 ? 20 : p == 1 ? 16 : 0; }
     static __device__ __forceinline__ unsigned mask(int p) { return p == 1 ? 0xfU : 0xfffU; }
+    static constexpr int kBytePasses = 4;
+    static __device__ __forceinline__ int byte_shift(int p) { return p == 0 ? 24 : p == 1 ? 16 : p == 2 ? 4 : 0; }
+    static __device__ __forceinline__ unsigned byte_mask(int p) { return p == 3 ? 0xfU : 0xffU; }
     static __device__ __forceinline__ type make(float v, int id) {
         return (ordered_bits(v) & 0xffff0000U) | (0xffffU - static_cast<uint32_t>(id));
     }
@@ -126,7 +137,7 @@ struct SamplerKey<true> {                                // scores that are bf16
 // The block's scratch memory (LDS): 14.6 KiB.
 struct SamplerScratch {
     uint32_t seen[kSmpMaxVocab / 32];                    // tokens present in the history
-    __attribute__((aligned(16))) uint32_t hist[kSmpBins / 2];    // bin 2 w in the low half of word w; later the parts of the ranks
+    __attribute__((aligned(16))) uint32_t hist[kSmpBins / 2];    // bin 2 w in the low half of word w, or bin b in words 8 b ..; later the parts of the ranks
     int wave_total[4], wave_first[4];
     int digit, remaining, count;
     __attribute__((aligned(16))) unsigned long long cand[kSmpMaxKeep];
@@ -203,38 +214,15 @@ __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, Sampl
     // its digits have been looked at, most significant first.  Equal scores are told apart by their ids when they are ranked, not in
     // passes over bits that they share.  (Half a block's threads rank 128 keys in less time than a pass takes.) ----
     const int rankable = keep <= 64 ? 128 : kSmpMaxKeep;
-    key_t largest = 0;
-#pragma unroll
-    for (int j = 0; j < kSmpPerThread; ++j) largest = key[j] > largest ? key[j] : largest;
     key_t prefix = 0, prefix_mask = 0, threshold = 0;
     int remaining = keep, candidates = kSmpMaxVocab + 1, place = 0;
-    bool all_keys = false;
-    // (kept as a loop: unrolled, the compiler computes the digits of all passes ahead and runs out of registers)
-#pragma unroll 1
-    for (int pass = 0; candidates > rankable; ++pass) {
-        const int shift = Key::shift(pass);
-        const unsigned digit_mask = Key::mask(pass);
-        sync();                                   // the bins are clear (and, later, the last pass's results read)
-        auto count = [&](key_t k) __attribute__((always_inline)) {
-            if (k != 0 && (k & prefix_mask) == prefix) {
-                const unsigned digit = static_cast<unsigned>(k >> shift) & digit_mask;
-                atomicAdd(&sh_hist[digit >> 1], 1U << (16 * (digit & 1U)));          // (at most 4096 in a counter)
-            }
-        };
-        if (!all_keys) {
-            count(largest);
-        } else {
-#pragma unroll
-            for (int j = 0; j < kSmpPerThread; ++j) count(key[j]);
-        }
-        sync();
-        // keys in bins above this thread's sixteen: inside the wave from a prefix sum, then the waves above
-        const uint4 low = own_words[0], high = own_words[1];
+    // counters of this thread's bins, and the keys in all bins above those: inside the wave from a prefix sum, then the waves above
+    auto bins_above = [&](uint4& low, uint4& high, int& own) __attribute__((always_inline)) {
+        low = own_words[0];
+        high = own_words[1];
         own_words[0] = own_words[1] = make_uint4(0, 0, 0, 0);
-        const uint32_t high_pairs = (high.x + high.y) + (high.z + high.w);
-        const uint32_t all_pairs = (low.x + low.y) + (low.z + low.w) + high_pairs;
-        auto both = [](uint32_t pair) { return static_cast<int>((pair & 0xffffU) + (pair >> 16)); };
-        const int own = both(all_pairs);
+        const uint32_t all = ((low.x + low.y) + (low.z + low.w)) + ((high.x + high.y) + (high.z + high.w));
+        own = static_cast<int>((all & 0xffffU) + (all >> 16));
         const int upto = wave_inclusive_scan(own, lane);
         const int wave_sum = __builtin_amdgcn_readlane(upto, 63);
         if (lane == 0) sh_wave_total[wave] = wave_sum;
@@ -242,54 +230,104 @@ __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, Sampl
         int above = wave_sum - upto;
 #pragma unroll
         for (int w = 1; w < 4; ++w) above += w > wave ? sh_wave_total[w] : 0;
-        if (above < remaining && remaining <= above + own) {       // exactly one thread; its bins by halves, from the top
-            int rest = remaining - above, digit = 16 * tid;
-            bool upper = rest <= both(high_pairs);
-            if (!upper) rest -= both(high_pairs);
-            digit += upper ? 8 : 0;
-            const uint32_t w0 = upper ? high.x : low.x, w1 = upper ? high.y : low.y, w2 = upper ? high.z : low.z, w3 = upper ? high.w : low.w;
-            upper = rest <= both(w2 + w3);
-            if (!upper) rest -= both(w2 + w3);
-            digit += upper ? 4 : 0;
-            const uint32_t v0 = upper ? w2 : w0, v1 = upper ? w3 : w1;
-            upper = rest <= both(v1);
-            if (!upper) rest -= both(v1);
-            digit += upper ? 2 : 0;
-            const uint32_t word = upper ? v1 : v0;
-            upper = rest <= static_cast<int>(word >> 16);
-            if (!upper) rest -= static_cast<int>(word >> 16);
-            digit += upper ? 1 : 0;
-            sh_digit = digit;
-            sh_remaining = rest;
-        }
+        return above;
+    };
+    auto digit_found = [&](int shift, unsigned digit_mask) __attribute__((always_inline)) {
         sync();
         prefix |= static_cast<key_t>(sh_digit) << shift;
         prefix_mask |= static_cast<key_t>(digit_mask) << shift;
         remaining = sh_remaining;
-        // the bound starts with the digits in `prefix`; those not looked at are free (zero here)
+    };
+    // how many keys reach the bound that starts with the digits in `prefix` (those not looked at are free, zero here), and where this
+    // thread's go (a prefix sum over the block: no counter to queue at)
+    auto reach = [&]() __attribute__((always_inline)) {
         threshold = prefix | Key::kFree;
-        // how many keys reach it, and where this thread's go (a prefix sum over the block: no counter to queue at)
         int mine = 0;
 #pragma unroll
         for (int j = 0; j < kSmpPerThread; ++j) mine += key[j] >= threshold ? 1 : 0;
-        const int upto_mine = wave_inclusive_scan(mine, lane);
-        if (lane == 63) sh_wave_first[wave] = upto_mine;
+        const int upto = wave_inclusive_scan(mine, lane);
+        if (lane == 63) sh_wave_first[wave] = upto;
         sync();
-        place = upto_mine - mine;
+        place = upto - mine;
         candidates = 0;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             place += w < wave ? sh_wave_first[w] : 0;
             candidates += sh_wave_first[w];
         }
-        // the largest keys have told all they can, and too many keys reach the bound: from all of them (the last pass of that
-        // tells all keys apart and leaves `keep`)
-        if (!all_keys && pass + 1 == Key::kPasses && candidates > rankable) {
-            all_keys = true;
-            pass = -1;
-            prefix = prefix_mask = 0;
-            remaining = keep;
+    };
+    if (keep <= kSmpFromLargest) {
+        key_t largest = 0;
+#pragma unroll
+        for (int j = 0; j < kSmpPerThread; ++j) largest = key[j] > largest ? key[j] : largest;
+        // (kept as a loop: unrolled, the compiler computes the digits of all passes ahead and runs out of registers)
+#pragma unroll 1
+        for (int pass = 0; pass < Key::kPasses && candidates > rankable; ++pass) {
+            const int shift = Key::shift(pass);
+            const unsigned digit_mask = Key::mask(pass);
+            sync();                                // the bins are clear (and, later, the last pass's results read)
+            if (largest != 0 && (largest & prefix_mask) == prefix) {
+                const unsigned digit = static_cast<unsigned>(largest >> shift) & digit_mask;
+                atomicAdd(&sh_hist[digit >> 1], 1U << (16 * (digit & 1U)));
+            }
+            sync();
+            uint4 low, high;
+            int own;
+            const int above = bins_above(low, high, own);
+            if (above < remaining && remaining <= above + own) {   // exactly one thread; its bins by halves, from the top
+                auto both = [](uint32_t pair) { return static_cast<int>((pair & 0xffffU) + (pair >> 16)); };
+                const uint32_t high_pairs = (high.x + high.y) + (high.z + high.w);
+                int rest = remaining - above, digit = 16 * tid;
+                bool upper = rest <= both(high_pairs);
+                if (!upper) rest -= both(high_pairs);
+                digit += upper ? 8 : 0;
+                const uint32_t w0 = upper ? high.x : low.x, w1 = upper ? high.y : low.y, w2 = upper ? high.z : low.z, w3 = upper ? high.w : low.w;
+                upper = rest <= both(w2 + w3);
+                if (!upper) rest -= both(w2 + w3);
+                digit += upper ? 4 : 0;
+                const uint32_t v0 = upper ? w2 : w0, v1 = upper ? w3 : w1;
+                upper = rest <= both(v1);
+                if (!upper) rest -= both(v1);
+                digit += upper ? 2 : 0;
+                const uint32_t word = upper ? v1 : v0;
+                upper = rest <= static_cast<int>(word >> 16);
+                if (!upper) rest -= static_cast<int>(word >> 16);
+                digit += upper ? 1 : 0;
+                sh_digit = digit;
+                sh_remaining = rest;
+            }
+            digit_found(shift, digit_mask);
+            reach();
         }
+        prefix = candidates > rankable ? 0 : prefix;
+        prefix_mask = 0;
+        remaining = keep;
+    }
+    // From all keys: a bin to a thread, and eight counters to a bin, since scores share their leading bits and additions to one word take turns.
+    // (The last pass tells all keys apart and leaves `keep`.)
+    if (candidates > rankable) {
+#pragma unroll 1
+        for (int pass = 0; candidates > rankable; ++pass) {
+            const int shift = Key::byte_shift(pass);
+            const unsigned digit_mask = Key::byte_mask(pass);
+            sync();
+#pragma unroll
+            for (int j = 0; j < kSmpPerThread; ++j)
+                if (key[j] != 0 && (key[j] & prefix_mask) == prefix)
+                    atomicAdd(&sh_hist[(static_cast<unsigned>(key[j] >> shift) & digit_mask) * kSmpWords + (lane & (kSmpWords - 1))], 1U);
+            sync();
+            uint4 low, high;
+            int own;
+            const int above = bins_above(low, high, own);
+            if (above < remaining && remaining <= above + own) {
+                sh_digit = tid;
+                sh_remaining = remaining - above;
+                sh_count = keep - (remaining - above) + own;       // so many reach the bin
+            }
+            digit_found(shift, digit_mask);
+            candidates = sh_count;
+        }
+        reach();
     }
 
     // ---- gather the keys that reach the bound, rank them by counting ----------------------------------------

@@ -174,3 +174,41 @@ def test_selection_where_the_bound_lets_many_keys_through(oracle, qm, dev, top_k
             scores = oracle.f32_to_bf16(scores)
         want = _cpu_sample(oracle, scores, bf16, 0, vocab, top_k, 0.9, 31 + i, draws=12)
         assert _gpu_sample(qm, dev, scores, bf16, 0, vocab, top_k, 0.9, 31 + i, draws=12) == want, (i, vocab)
+
+
+@pytest.mark.parametrize("top_k", [127, 129, 150, 199, 255])
+@pytest.mark.parametrize("bf16", [True, False])
+def test_selection_from_all_scores_at_once(oracle, qm, dev, top_k, bf16):
+    """Around the number of entries (128) from which no bound is looked for among the threads' largest scores: the same vocabularies and scores."""
+    test_selection_where_the_bound_lets_many_keys_through(oracle, qm, dev, top_k, bf16)
+
+
+@pytest.mark.parametrize("bf16", [True, False])
+def test_many_entries_cost_what_they_cost(qm, dev, bf16):
+    """200 entries of 4096 scores against 128: more of them are ranked and summed, but the select is no longer (1.28 times the time; 1.55 and 1.64 with passes
+    over the threads' largest scores whose bound lets too many through).  Best of several replays of forty draws each."""
+    import torch
+    scores = torch.from_numpy(np.random.default_rng(5).standard_normal(4096).astype(np.float32)).to(dev)
+    if bf16:
+        scores = scores.bfloat16()
+    state, out = torch.zeros(1, dtype=torch.int64, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
+    draw = lambda top_k, stream: qm.lib().qm_sample_topk(scores.data_ptr(), int(bf16), 0, 4096, top_k, 0.9, state.data_ptr(), out.data_ptr(), stream)
+    stream, best = torch.cuda.Stream(), {}
+    for top_k in (128, 200):
+        assert draw(top_k, None) == 0
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            for _ in range(40):
+                draw(top_k, stream.cuda_stream)
+        graph.replay()
+        times = []
+        for _ in range(20):
+            first, last = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            first.record()
+            graph.replay()
+            last.record()
+            torch.cuda.synchronize()
+            times.append(first.elapsed_time(last))
+        best[top_k] = min(times)
+    assert best[200] < 1.4 * best[128], best
