@@ -858,8 +858,8 @@ int32_t qm_linear_rows_split(
     void* workspace, int64_t workspace_bytes, void* hip_stream);
 /*
  * qm_linear_rows with a residual, and RMSNorm (qm_rmsnorm_rows) of the rows that it leaves.  With a workspace of
- * qm_linear_rows_norm_workspace_bytes (0 where the shape is not cut; as above otherwise) a long reduction is cut into pieces that the norm's launch
- * adds; without one exactly the two calls.
+ * qm_linear_rows_norm_workspace_bytes (0 where the shape is not cut; as above otherwise) a long reduction is cut into pieces, which for 1024 and
+ * 2048 output columns the norm's launch adds; without one exactly the two calls.
  */
 int64_t qm_linear_rows_norm_workspace_bytes(int32_t rows, int32_t output_columns, int32_t reduction_columns);
 int32_t qm_linear_rows_norm(

@@ -294,7 +294,8 @@ extern "C" int64_t qm_linear_rows_norm_workspace_bytes(int32_t rows, int32_t out
     if (rows < kRowsMatrixMinimum || output_columns <= 0 || reduction_columns <= 0 || output_columns % 128 || reduction_columns % 128) return 0;
     bool wide = false;
     const int parts = rows_mfma_norm_parts(rows, output_columns, reduction_columns, &wide);
-    return parts > 1 ? static_cast<int64_t>(parts) * rows * output_columns * 4 : 0;
+    if (parts > 1) return static_cast<int64_t>(parts) * rows * output_columns * 4;
+    return static_cast<int64_t>(rows_mfma_workspace_bytes(rows, output_columns, reduction_columns, false));    // (other widths: the two calls)
 }
 
 extern "C" int32_t qm_linear_rows_norm(const uint16_t* input, const uint16_t* weight, const uint16_t* bias, const uint16_t* residual, uint16_t* output,
@@ -313,8 +314,9 @@ extern "C" int32_t qm_linear_rows_norm(const uint16_t* input, const uint16_t* we
     if (rc != QM_OK) return rc;
     const int64_t need = workspace && matrix_cores ? qm_linear_rows_norm_workspace_bytes(rows, output_columns, reduction_columns) : 0;
     if (need > workspace_bytes) return QM_ERR_WORKSPACE;
-    if (need > 0) {
-        prm.reduction_parts = rows_mfma_norm_parts(rows, output_columns, reduction_columns, &prm.wide_tiles);
+    const int parts = need > 0 ? rows_mfma_norm_parts(rows, output_columns, reduction_columns, &prm.wide_tiles) : 1;
+    if (parts > 1) {
+        prm.reduction_parts = parts;
         prm.partials = static_cast<float*>(workspace);
         prm.groups = 1;
         prm.norm_weight = norm_weight;
@@ -322,7 +324,7 @@ extern "C" int32_t qm_linear_rows_norm(const uint16_t* input, const uint16_t* we
         prm.epsilon = epsilon;
         return launch_rows_mfma(prm, false, static_cast<hipStream_t>(hip_stream));
     }
-    rc = qm_linear_rows(input, weight, bias, residual, output, rows, output_columns, reduction_columns, hip_stream);
+    rc = qm_linear_rows_split(input, weight, bias, residual, output, rows, output_columns, reduction_columns, workspace, workspace_bytes, hip_stream);
     return rc == QM_OK ? qm_rmsnorm_rows(output, norm_weight, normalized, rows, output_columns, epsilon, hip_stream) : rc;
 }
 

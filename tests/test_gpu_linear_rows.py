@@ -318,8 +318,12 @@ def test_swiglu_of_every_bf16_gate(qm, dev, rows_kernel):
         assert bool((got[0] == got[1]).all()), part
 
 
-@pytest.mark.parametrize("rows,cols,red", [(16, 2048, 6144), (100, 1024, 4096), (785, 2048, 6144), (1000, 2048, 6144), (1024, 2048, 4224), (1601, 1024, 4096),
-                                           (2048, 1024, 6144), (1025, 2048, 6144), (300, 1536, 4096), (900, 2048, 2048)])
+# rows, columns, reduction: pieces of the reduction with a norm behind (0: whole)
+NORM_PIECES = {(16, 2048, 6144): 8, (100, 1024, 4096): 8, (785, 2048, 6144): 2, (1000, 2048, 6144): 2, (1024, 2048, 4224): 0, (1601, 1024, 4096): 0,
+               (2048, 1024, 6144): 2, (1025, 2048, 6144): 0, (300, 1536, 4096): 4, (900, 2048, 2048): 0}
+
+
+@pytest.mark.parametrize("rows,cols,red", list(NORM_PIECES))
 @pytest.mark.parametrize("rows_kernel", [MATRIX, EXACT], indirect=True)
 @pytest.mark.parametrize("bias", [False, True])
 def test_linear_and_norm_of_its_rows(qm, dev, rows, cols, red, rows_kernel, bias):
@@ -332,6 +336,8 @@ def test_linear_and_norm_of_its_rows(qm, dev, rows, cols, red, rows_kernel, bias
     x, w, res, gamma = (torch.randn(*shape, device=dev, generator=gen).bfloat16() for shape in ((rows, red), (cols, red), (rows, cols), (cols,)))
     b = torch.randn(cols, device=dev, generator=gen).bfloat16() if bias else None
     need = qm.lib().qm_linear_rows_norm_workspace_bytes(rows, cols, red)
+    if rows_kernel == MATRIX:
+        assert need == NORM_PIECES[rows, cols, red] * rows * cols * 4
     ws = torch.empty(max(need, 256), dtype=torch.uint8, device=dev)
     out, normed = (torch.full((rows + 1, cols), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(2))
     call = lambda bytes_: qm.lib().qm_linear_rows_norm(x.data_ptr(), w.data_ptr(), b.data_ptr() if bias else None, res.data_ptr(), out.data_ptr(),

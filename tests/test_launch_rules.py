@@ -50,6 +50,19 @@ int main() {
     assert "81 8 1 88" in lines and "42 6 1 42" in lines and "42 3 2 42" in lines
 
 
+def test_a_norm_behind_a_linear_takes_no_cut_away(qm):
+    """Whatever the width, a reduction that is cut by itself is cut with the norm behind as well, and the workspace holds its pieces."""
+    L, cut, more = qm.lib(), 0, 0
+    for cols in (128, 512, 1024, 1536, 2048, 3072, 4096):
+        for red in (128, 2048, 4096, 6144, 8192):
+            for rows in (1, 15, 16, 64, 100, 200, 300, 520, 768, 769, 900, 1024, 1025, 1600, 2048):
+                alone, behind = L.qm_linear_rows_split_workspace_bytes(rows, cols, red, 0), L.qm_linear_rows_norm_workspace_bytes(rows, cols, red)
+                assert behind >= alone and behind % (rows * cols * 4) == 0, (rows, cols, red)
+                cut += alone > 0
+                more += behind > alone
+    assert cut > 40 and more > 4, (cut, more)
+
+
 def test_a_steps_weights_stay_in_flight(tmp_path):
     """A long row's dot products, the first weights asked for at one of several places as in a step's output launch: in the loop over the row nothing waits
     for all loads (vmcnt(0)), a piece's products leave the requests behind it under way."""
