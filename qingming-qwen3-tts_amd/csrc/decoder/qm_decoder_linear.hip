@@ -186,7 +186,7 @@ static int64_t steps_of_busiest(const DecLinearParams& prm, int parts) {
 // fill them.  (us, 1024 rows, 2048 outputs of 6144: beside 2048 of 2048, three pieces, 66 -> 55; beside twice that, two pieces, 70 -> 65; the norm
 // behind, which adds the pieces, 11.5 -> 14.)  A piece more is a plane of sums written and read, rows x outputs x 8 bytes: a step's time (0.73 us)
 // for each 3 MB.
-static int reduction_pieces(const DecLinearParams& prm) {
+int reduction_pieces(const DecLinearParams& prm) {
     const DecLinearGroup& last = prm.group[prm.groups - 1];
     int64_t blocks = 0;
     for (int g = 0; g < prm.groups; ++g) blocks += static_cast<int64_t>(prm.group[g].n / 128) * ((prm.rows + 127) / 128);
@@ -202,6 +202,16 @@ static int reduction_pieces(const DecLinearParams& prm) {
         }
     }
     return best;
+}
+
+int64_t reduction_cut_floats(const DecLinearParams& prm, int max_rows) {
+    int64_t most = 0;
+    DecLinearParams tile = prm;
+    for (int row = 0; row < max_rows; row += 128) {                            // (of a row tile's rows the first has the most pieces, the last the most rows)
+        tile.rows = row + 1;
+        most = std::max(most, static_cast<int64_t>(reduction_pieces(tile) - 1) * std::min(row + 128, max_rows) * prm.group[prm.groups - 1].n);
+    }
+    return most;
 }
 
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut) {
@@ -229,10 +239,11 @@ int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t 
         if (prm.group[g].w_up) cut = nullptr;
     }
     if (cut) {
-        const int pieces = reduction_pieces(prm);
         DecLinearGroup& last = all[count - 1];
-        last.k /= pieces;
         cut->plane = static_cast<int64_t>(prm.rows) * last.n;
+        int pieces = reduction_pieces(prm);
+        if ((pieces - 1) * cut->plane > cut->room) pieces = 1;
+        last.k /= pieces;
         for (; cut->planes < pieces - 1; ++cut->planes, ++count) {
             all[count] = last;
             all[count].x = static_cast<const uint16_t*>(last.x) + (cut->planes + 1) * last.k;

@@ -60,13 +60,17 @@ int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipSt
 int32_t launch_gated_norm(const GatedNormParams& prm, int rows, int f32, hipStream_t stream);
 // Many rows of bf16 go to the matrix cores (linears of one launch in one grid, a gate/up pair in its own), few rows and
 // fp32 to the streaming kernel.
-// cut: the last linear's reduction may be taken in pieces, whose sums behind the first's go to cut->sums (room for kMorePlanes planes of
-// [rows][n]); how many do is left in cut->planes.
+// cut: the last linear's reduction may be taken in pieces, whose sums behind the first's go to cut->sums in planes of [rows][n], as many as `room`
+// floats hold; how many do is left in cut->planes.
 struct ReductionCut {
     float* sums;
+    int64_t room;
     int64_t plane;
     int planes;
 };
+// Into how many pieces that is, and the most floats that they take with any number of rows up to max_rows.
+int reduction_pieces(const DecLinearParams& prm);
+int64_t reduction_cut_floats(const DecLinearParams& prm, int max_rows);
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut = nullptr);
 int32_t launch_split_linears(const DecLinearParams& prm, hipStream_t stream);    // fp32 rows on the matrix cores
 // Rotation and cache write, then the attention.

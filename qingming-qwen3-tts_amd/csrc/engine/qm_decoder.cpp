@@ -359,6 +359,8 @@ int64_t token_bytes(const qm_decoder& d) {
 }
 constexpr int64_t kStreamingTokenBytes = 256ll << 20;
 
+int64_t cut_floats(const qm_decoder& d);
+
 std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int capacity, int sequences, int max_rows, hipStream_t stream) {
     if (capacity <= 0 || sequences <= 0 || max_rows < 0 || (f32 != 0 && f32 != 1))
         throw ApiError(QM_ERR_ARGUMENT, "capacity and sequences must be positive");
@@ -483,9 +485,7 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
     d->attended = zeros(rows * attended * item);
     d->gated = zeros(rows * gated * item);
     for (DeviceBuffer& y : d->y) y = zeros(rows * d->width_p * 4);
-    if (!f32)
-        for (const DecoderLayer& w : d->layers)
-            if (w.config.ff && w.config.form != LayerForm::Sandwich && !d->y_more.raw()) d->y_more = zeros(qm::kMorePlanes * rows * d->width_p * 4);
+    if (const int64_t more = f32 ? 0 : cut_floats(*d)) d->y_more = zeros(static_cast<size_t>(more) * 4);
     d->q_rot = zeros(rows * q_rot * item);
     d->raw = zeros(rows * raw * 4);
     d->ml = zeros(ml * 4);
@@ -767,6 +767,16 @@ qm::DecLinearParams linears_out(const qm_decoder& d, const DecoderLayer& w, int 
     return p;
 }
 
+// Floats for the further pieces of any layer's output linears.
+int64_t cut_floats(const qm_decoder& d) {
+    int64_t most = 0;
+    for (const DecoderLayer& w : d.layers) {
+        Pending none;
+        most = std::max(most, qm::reduction_cut_floats(linears_out(d, w, d.max_rows, none), d.max_rows));
+    }
+    return most;
+}
+
 // A sandwich layer's feed-forward: what reads norm2, and (dense) the linear behind it.
 qm::DecLinearParams feed_in(const qm_decoder& d, const DecoderLayer& w, int rows) {
     qm::DecLinearParams p = {};
@@ -819,7 +829,7 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
         }
         if (w.config.mixer != MixerKind::LatentAttention) op_check(qm::launch_gated_norm(gated_of(d, w), rows, d.f32, s), "gated norm");
         const qm::DecLinearParams outputs = linears_out(d, w, rows, pending);
-        qm::ReductionCut cut = {f32_of(d.y_more), 0, 0};
+        qm::ReductionCut cut = {f32_of(d.y_more), static_cast<int64_t>(d.y_more.bytes() / 4), 0, 0};
         op_check(qm::launch_decoder_linears(outputs, d.f32, s, cut.sums ? &cut : nullptr), "output projections");
         pending.more = {cut.sums, cut.plane, cut.planes};
         if (sandwich(w) && w.config.ff) {

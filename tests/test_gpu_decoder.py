@@ -413,7 +413,7 @@ def test_weights_beyond_the_cache_give_the_same_bits(decoder, tmp_path, design):
 @pytest.mark.parametrize("layer,width,rows", [
     (cases.general_delta(32, 64, 6144), 2048, 1000),                                                             # in three pieces
     (cases.parallel(cases.left(16, 4, 128, 128, 512, 64), cases.right(16, 64, 128, [0.95] * 16), 6144), 2048, 900),   # in two, beside two
-    (cases.general_delta(16, 64, 3072), 1024, 1601),                                                             # in two
+    (cases.general_delta(16, 64, 3072), 1024, 1601),                                                             # in three
     (cases.general_delta(16, 64, 384), 1024, 1601),                                                              # whole
 ])
 def test_down_projection_in_pieces(decoder, tmp_path, layer, width, rows):
@@ -435,3 +435,22 @@ def test_down_projection_in_pieces(decoder, tmp_path, layer, width, rows):
     for i in range(2):
         assert cases.error(streams[i], want[i]) < LIMIT[False], i
     assert cases.error(logits, np.concatenate(scores)) < LIMIT[False]
+
+
+def test_pieces_of_a_reduction_take_memory_only_where_one_is_cut(decoder, tmp_path):
+    """A narrow model's output linears are never cut: its feed-forward takes the rows of its channels more than the same model without, and no planes for
+    sums (64 MiB here)."""
+    import torch
+    rows, used = 65536, []
+    for i, ff in enumerate((None, None, 300)):                 # (the first loads the library's code as well)
+        where = tmp_path / str(i)
+        where.mkdir()
+        cfg = cases.config(100, 128, [cases.parallel(cases.left(2, 1, 32, 32, 64, 32), cases.right(2, 16, 32, [0.9, 0.99]), ff)])
+        cases.write_model(str(where), cfg, cases.weights(cfg))
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        engine = decoder.Decoder(str(where), rows, max_rows=rows)
+        used.append(before - torch.cuda.mem_get_info()[0])
+        engine.close_model()
+    channels = rows * 384 * 2                                  # 300 padded to 384, bf16
+    assert used[2] - used[1] < channels + (16 << 20), used     # (allocations come in pieces of two MiB)

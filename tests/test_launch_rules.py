@@ -50,6 +50,49 @@ int main() {
     assert "81 8 1 88" in lines and "42 6 1 42" in lines and "42 3 2 42" in lines
 
 
+# output linears as (columns, reduction) each, the last the one that may be cut; rows; its pieces (the first four are the layers of
+# test_gpu_decoder.py's test_down_projection_in_pieces)
+CUTS = [([(2048, 2048), (2048, 6144)], 1000, 3), ([(2048, 2048), (2048, 2048), (2048, 6144)], 900, 2), ([(1024, 1024), (1024, 3072)], 1601, 3),
+        ([(1024, 1024), (1024, 384)], 1601, 1), ([(2048, 2048), (2048, 6144)], 700, 1), ([(2048, 6144)], 1024, 1)]
+
+
+def test_pieces_of_a_decoders_reduction_and_their_memory(tmp_path):
+    """Into how many pieces the last of several output linears is cut, and that the memory for it holds the pieces of every number of rows."""
+    shapes = [linears for linears, _, _ in CUTS] + [[(3072, 3072), (3072, 9216)], [(1280, 640), (1280, 2560), (1280, 5120)]]
+    source = """
+#include <cstdio>
+#include "decoder/qm_decoder_ops.h"
+static qm::DecLinearParams of(std::initializer_list<std::pair<int, int>> linears, int rows) {
+    qm::DecLinearParams p = {};
+    p.rows = rows;
+    for (const auto& [n, k] : linears) {
+        p.group[p.groups].n = n;
+        p.group[p.groups++].k = k;
+    }
+    return p;
+}
+int main() {
+"""
+    for linears in shapes:
+        text = "{" + ", ".join("{%d, %d}" % l for l in linears) + "}"
+        source += f"""
+    for (int rows = 1; rows <= 2300; ++rows)
+        std::printf("%d %lld\\n", qm::reduction_pieces(of({text}, rows)), (long long)qm::reduction_cut_floats(of({text}, rows), rows));
+"""
+    lines = [tuple(map(int, line.split())) for line in run(tmp_path, source + "}", "qm_decoder")]
+    assert len(lines) == 2300 * len(shapes)
+    for i, linears in enumerate(shapes):
+        of_rows = lines[2300 * i:2300 * (i + 1)]
+        most = 0
+        for rows, (pieces, floats) in enumerate(of_rows, 1):
+            assert 1 <= pieces <= 3 and linears[-1][1] % (128 * pieces) == 0
+            most = max(most, (pieces - 1) * rows * linears[-1][0])
+            assert most <= floats, (linears, rows)                    # enough for as many rows and for fewer
+            assert floats <= 2 * (rows + 127) * linears[-1][0] and (floats > 0) == (most > 0), (linears, rows)
+    for i, (linears, rows, pieces) in enumerate(CUTS):
+        assert lines[2300 * i + rows - 1][0] == pieces, (linears, rows)
+
+
 def test_a_norm_behind_a_linear_takes_no_cut_away(qm):
     """Whatever the width, a reduction that is cut by itself is cut with the norm behind as well, and the workspace holds its pieces."""
     L, cut, more = qm.lib(), 0, 0
