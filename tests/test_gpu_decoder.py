@@ -383,14 +383,15 @@ def test_generate_program(decoder, models):
     assert [json.loads(line) for line in p.stdout.splitlines()] == [greedy(m, prompt, 6) for prompt in prompts]
 
 
-@pytest.mark.parametrize("design", ["parallel", "sandwich"])
-def test_weights_beyond_the_cache_give_the_same_bits(decoder, tmp_path, design):
+@pytest.mark.parametrize("float32", [False, True])
+@pytest.mark.parametrize("design", ["parallel", "sandwich", "looped"])
+def test_weights_beyond_the_cache_give_the_same_bits(decoder, tmp_path, design, float32):
     """A model whose head alone is more than the last-level cache keeps reads a step's weights with the non-temporal hint: the small model's scores, bit for
     bit (the large vocabulary's rows repeat the small one's)."""
     small, times = 1000, 1100                                  # 1 100 000 x 128 values of two bytes: 268 MiB
-    if design == "parallel":
+    if design != "sandwich":
         layers = [cases.parallel(cases.left(4, 2, 32, 48, 40, 16), cases.right(2, 32, 64, [0.9, 0.99]), 300), cases.general_delta(2, 32, 200)]
-        make = lambda vocab: cases.config(vocab, 128, layers)
+        make = lambda vocab: cases.config(vocab, 128, layers, loop=(0, 1, 3) if design == "looped" else None)
     else:
         layers = [cases.latent(4, 16, 8, 24, 48, 40, cases.moe(6, 2, 48)), cases.retention(2, 16, 24, [0.9, 0.99], cases.dense(300))]
         make = lambda vocab: cases.sandwich(vocab, 128, layers, (11, 6, 7))
@@ -401,7 +402,7 @@ def test_weights_beyond_the_cache_give_the_same_bits(decoder, tmp_path, design):
         where = tmp_path / str(count)
         where.mkdir()
         cases.write_model(str(where), make(small * count), {name: np.tile(w, (count, 1)) if name in ("embed", "head") else w for name, w in weights.items()})
-        engine = decoder.Decoder(str(where), 32)
+        engine = decoder.Decoder(str(where), 32, float32=float32)
         s = engine.open()
         rows.append([engine.step(s, tokens[:5], [4])[0]] + [engine.step(s, [t], [0])[0] for t in tokens[5:]])
         engine.close(s)
@@ -454,3 +455,26 @@ def test_pieces_of_a_reduction_take_memory_only_where_one_is_cut(decoder, tmp_pa
         engine.close_model()
     channels = rows * 384 * 2                                  # 300 padded to 384, bf16
     assert used[2] - used[1] < channels + (16 << 20), used     # (allocations come in pieces of two MiB)
+
+
+@pytest.mark.parametrize("rows", [1601, 1900])                   # in two; below 1537 rows whole
+def test_a_layer_without_feed_forward_is_cut_in_front_of_its_norm(decoder, tmp_path, rows):
+    """The last output linear of a parallel layer without feed-forward is the decayed attention's, whose sum is normed before it is added: its pieces come
+    together first.  Between layers with one; against portions too short for a cut, as above."""
+    mixers = cases.left(4, 2, 64, 64, 512, 64), cases.right(16, 64, 128, [0.95] * 16)
+    cfg = cases.config(256, 1024, [cases.parallel(*mixers, 3072), cases.parallel(*mixers, None), cases.general_delta(16, 64, 3072)])
+    cases.write_model(str(tmp_path), cfg, cases.weights(cfg))
+    tokens = cases.tokens_of(cfg, rows)
+    places = [0, 127, rows // 2, rows - 1]
+    whole = decoder.Decoder(str(tmp_path), rows, max_rows=rows)
+    logits, streams = whole.step(whole.open(), tokens, places, streams=True)
+    portions = decoder.Decoder(str(tmp_path), rows, max_rows=400)
+    s, parts, scores = portions.open(), [], []
+    for at in range(0, rows, 400):
+        got, stream = portions.step(s, tokens[at:at + 400], [p - at for p in places if at <= p < at + 400], streams=True)
+        parts.append(stream)
+        scores.append(got)
+    want = np.concatenate(parts, axis=1)
+    for i in range(3):
+        assert cases.error(streams[i], want[i]) < LIMIT[False], i
+    assert cases.error(logits, np.concatenate(scores)) < LIMIT[False]

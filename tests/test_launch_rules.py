@@ -51,9 +51,10 @@ int main() {
 
 
 # output linears as (columns, reduction) each, the last the one that may be cut; rows; its pieces (the first four are the layers of
-# test_gpu_decoder.py's test_down_projection_in_pieces)
+# test_gpu_decoder.py's test_down_projection_in_pieces, the last of its test_a_layer_without_feed_forward_is_cut_in_front_of_its_norm)
 CUTS = [([(2048, 2048), (2048, 6144)], 1000, 3), ([(2048, 2048), (2048, 2048), (2048, 6144)], 900, 2), ([(1024, 1024), (1024, 3072)], 1601, 3),
-        ([(1024, 1024), (1024, 384)], 1601, 1), ([(2048, 2048), (2048, 6144)], 700, 1), ([(2048, 6144)], 1024, 1)]
+        ([(1024, 1024), (1024, 384)], 1601, 1), ([(2048, 2048), (2048, 6144)], 700, 1), ([(2048, 6144)], 1024, 1),
+        ([(1024, 256), (1024, 2048)], 1601, 2), ([(1024, 256), (1024, 2048)], 1536, 1)]
 
 
 def test_pieces_of_a_decoders_reduction_and_their_memory(tmp_path):
