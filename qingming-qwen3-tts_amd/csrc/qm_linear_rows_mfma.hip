@@ -72,8 +72,8 @@ __device__ __forceinline__ uint32_t finish_pair(float s0, float s1, bool has_bia
     return v;
 }
 
-// g / (1 + exp(-g)) of a bf16 value, good for its rounding to bf16: the bits that expf and the correctly rounded division give, for every one of
-// the 65 536 (compared exhaustively on the device), in ten instructions where those take some forty.  The denominator is kept down by 2^32, so that its
+// g / (1 + exp(-g)) of a bf16 value, good for its rounding to bf16: the bits that expf and the correctly rounded division give, for every finite one
+// (all compared on the device; infinity stays infinity, minus infinity and NaN make NaN there and here), in ten instructions where those take some forty.  The denominator is kept down by 2^32, so that its
 // reciprocal does not go below the normal numbers where exp(-g) is near the largest; one Newton step makes the reciprocal good to the last bit.
 // (The pair's epilogue is as long as five of its steps: 1000 tokens x 6144 channels of 2048 54.6 -> 52.1 us, 777 x 3072 of 1024 22.1 -> 20.9.)
 __device__ __forceinline__ float silu_of_bf16(float g) {
@@ -687,10 +687,10 @@ int rows_mfma_reduction_parts(int rows, int columns, int reduction, bool dual) {
 }
 
 // With a norm behind, whose launch adds the pieces for the price of their bytes, a long reduction is also cut in two where 64-row tiles would just
-// give every CU a block: as many blocks of 128 x 128 walk half the steps for two thirds of the requests an output takes.  (us, 2048 columns with the
-// norm behind, 64-row tiles / cut: of 6144, weights from memory, 1000 tokens 52.1 / 44.8; weights still in the caches, 785, 900, 1000 and 1024 tokens
-// 35.2 / 34.0, 37.9 / 38.1, 39.7 / 41.1 and 40.4 / 41.9; 1024 columns, 1600 tokens 39.0 / 36.0.  Of 2048, from memory, 24.1 / 23.9, and of 4096, from the
-// caches, 29.0 / 34.7: shorter ones stay.)
+// give every CU a block: as many blocks of 128 x 128 walk half the steps for two thirds of the requests an output takes.  (us, 2048 columns of 6144 and
+// the norm behind, as two calls / cut: weights from memory, 785, 850, 900, 1000 and 1024 tokens 43.6 / 35.1, 43.9 / 39.0, 43.3 / 36.6, 46.9 / 42.3 and
+// 48.4 / 43.0; still in the caches 36.0 / 33.1, 36.9 / 33.6, 36.2 / 36.6, 39.7 / 36.6 and 39.1 / 37.2; 1024 columns, 1600 tokens 39.1 / 36.1.  Of 2048,
+// from memory, 24.1 / 23.9, and of 4096, from the caches, 29.0 / 34.7: shorter ones stay.)
 int rows_mfma_norm_parts(int rows, int columns, int reduction, bool* wide) {
     *wide = false;
     if (columns != 1024 && columns != 2048) return 1;

@@ -300,7 +300,7 @@ def test_more_than_forty_column_tiles_that_eight_does_not_divide(qm, dev, rows, 
 
 @pytest.mark.parametrize("rows_kernel", [MATRIX], indirect=True)
 def test_swiglu_of_every_bf16_gate(qm, dev, rows_kernel):
-    """Each gate value once, through an identity on the matrix cores: the bits of the exact chain's expf and division (a NaN is a NaN)."""
+    """Each finite gate value once, through an identity on the matrix cores: the bits of the exact chain's expf and division."""
     import torch
     x = torch.eye(128, device=dev).bfloat16()
     up = torch.ones(128, 128, device=dev).bfloat16()
@@ -316,6 +316,26 @@ def test_swiglu_of_every_bf16_gate(qm, dev, rows_kernel):
             got.append(out)
         torch.cuda.synchronize()
         assert bool((got[0] == got[1]).all()), part
+
+
+@pytest.mark.parametrize("rows_kernel", [MATRIX], indirect=True)
+def test_swiglu_of_gates_that_are_no_numbers(qm, dev, rows_kernel):
+    """Through the same identity, a column of infinite and undefined gate weights: the first token's gates are those, every other's 0 times them.  What the
+    exact chain makes of them, a NaN being a NaN."""
+    import torch
+    x, up = torch.eye(128, device=dev).bfloat16(), torch.ones(128, 128, device=dev).bfloat16()
+    gate = torch.full((128, 128), 0.5, device=dev).bfloat16()
+    gate[0, 0], gate[1, 0], gate[2, 0] = float("inf"), float("-inf"), float("nan")
+    got = []
+    for kernel in (MATRIX, EXACT):
+        qm.set_option(qm.OPT_LINEAR_ROWS_KERNEL, kernel)
+        out = torch.zeros(128, 128, dtype=torch.bfloat16, device=dev)
+        qm.gate_up_swiglu_rows(x, gate, up, out, 128, 128, 128)
+        got.append(out.float())
+    torch.cuda.synchronize()
+    assert got[1][0, 0] == float("inf") and bool(got[1][0, 1:3].isnan().all()) and bool(got[1][1:, :3].isnan().all())
+    assert torch.equal(got[0].isnan(), got[1].isnan())
+    assert torch.equal(got[0].nan_to_num(7.0, float("inf"), float("-inf")), got[1].nan_to_num(7.0, float("inf"), float("-inf")))
 
 
 # rows, columns, reduction: pieces of the reduction with a norm behind (0: whole)
