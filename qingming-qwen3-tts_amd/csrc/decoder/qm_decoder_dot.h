@@ -88,8 +88,8 @@ struct NoRefill {
 };
 
 // One tile: xs holds R input rows [R][k] in LDS, `piece` the first pieces.  `refill` is called with a piece's number when the tile has no
-// more use for it.
-template <class T, int R, int NR, bool STREAM, class Refill = NoRefill>
+// more use for it.  ROUNDS: rows of many rounds (see below).
+template <class T, int R, bool ROUNDS = R == 1, int NR, bool STREAM, class Refill = NoRefill>
 __device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRows<NR, STREAM>& d, uint4 (&piece)[kDotAhead][NR], const T* xs, int row0,
                                            int rows, Refill&& refill = Refill()) {
     const int lane = threadIdx.x & 63;
@@ -107,7 +107,7 @@ __device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRow
     };
     constexpr int kRound = kDotAhead * 512;
     int k0 = 0;
-    if constexpr (R == 1) {
+    if constexpr (ROUNDS) {
         // All rounds but the last are whole, and nothing branches between a piece's products and the next request into its registers: behind a
         // branch the compiler waits for every load under way before it asks for more (2048 outputs of 6144 in a step: 8.6 us, 6.3 so).
         for (; k0 + kRound < k; k0 += kRound) {
@@ -125,7 +125,7 @@ __device__ __forceinline__ void dot_finish(const DecLinearGroup& g, const DotRow
             if (at < k) products(u, at);
             refill(u);
         }
-    } else {                                   // (several rows: the products of a piece are long, and the round's loads come back together)
+    } else {                                   // (several input rows: a piece's products are long, the round's loads come back together; fewer registers)
         for (; k0 < k; k0 += kRound) {
 #pragma unroll
             for (int u = 0; u < kDotAhead; ++u) {

@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kDecThreads) void expert_in_kernel(ExpertParams prm
     const auto d = dot_rows<kExpertInRows>(g, tile);
     uint4 piece[kDotAhead][kExpertInRows];
     dot_request(d, g.k, piece);
-    dot_finish<T, 1>(g, d, piece, xs, 0, 1);
+    dot_finish<T, 1, false>(g, d, piece, xs, 0, 1);                            // (a model's width is a round or two: 2 % of 300 fp32 rows)
 }
 
 // Down of row blockIdx.y: the chosen experts' reductions one behind the other, each weighted.
