@@ -55,14 +55,15 @@ struct LinearRowsParams {
 };
 
 // The grid's width for so many column tiles, by row tiles and pieces of the reduction.  Blocks go to the eight dies of 32 CUs in turn, one to a CU:
-// where 8 divides the width, the row tiles of a column read its weights on one die.  Many columns are rounded up to that, the blocks beyond end at
-// once (us, 1024 tokens of 2048, 81 column tiles of 128 by 8 row tiles 64.8 -> 56.1, 80 take 54.2), unless the dies with a column more would then
-// walk a round of blocks more than all of them do when the tiles are dealt out one by one (130 tokens of 1024, 84 column tiles of 64 by 3 row
-// tiles: 7.4 as they are, 11.0 as 88; 700 tokens, 41 of 128 by 6: 16.2 and 20.7).
+// where 8 divides the width, the row tiles of a column read its weights on one die, but the dies with a column more may walk a round of blocks more
+// than all of them do when the tiles are dealt out one by one.  Rounded up (the blocks beyond end at once) a grid takes, of its time as it is, reductions
+// of 1024 and 2048, weights in the caches and from memory: with more than forty columns 0.57 to 1.00 where the rounds stay the same, 0.83 to 0.95 where
+// three or more become one more, 0.93 to 1.18 where two become three and 0.90 to 1.71 where one becomes two; with fewer columns 0.60 to 1.21 even where
+// the rounds stay the same.  (us: 1024 tokens, 81 columns by 8 row tiles of 2048 64.8 -> 56.1; 130 tokens, 84 by 3 of 1024 7.4 -> 11.0.)
 inline int rows_grid_columns(int column_tiles, int row_tiles, int pieces) {
     const int64_t rounded = (column_tiles + 7) / 8 * 8, rows = static_cast<int64_t>(row_tiles) * pieces;
-    const int64_t busiest = rounded / 8 * rows, even = (column_tiles * rows + 7) / 8;
-    return column_tiles > 40 && row_tiles > 1 && (busiest + 31) / 32 == (even + 31) / 32 ? static_cast<int>(rounded) : column_tiles;
+    const int64_t busiest = (rounded / 8 * rows + 31) / 32, even = ((column_tiles * rows + 7) / 8 + 31) / 32;
+    return column_tiles > 40 && row_tiles > 1 && 3 * busiest <= 4 * even ? static_cast<int>(rounded) : column_tiles;
 }
 
 // The row linears on the matrix cores (qm_linear_rows_mfma.hip).  `dual`: weight[0] / weight[1] are the gate and up

@@ -21,9 +21,9 @@ def run(tmp_path, source, library=None):
     return subprocess.run([str(tmp_path / "rule")], check=True, capture_output=True, text=True).stdout.splitlines()
 
 
-def test_a_rounded_grid_keeps_no_die_longer_than_an_even_deal(tmp_path):
-    """Row linears: blocks go to the eight dies of 32 CUs in turn, one to a CU.  Whatever the grid's width is rounded to, no die walks more rounds of
-    blocks than all of them do when the tiles are dealt out one by one; and where that holds, many column tiles are rounded."""
+def test_a_rounded_grid_keeps_no_die_much_longer_than_an_even_deal(tmp_path):
+    """Row linears: blocks go to the eight dies of 32 CUs in turn, one to a CU.  Where a grid's width is rounded up, no die walks more rounds of blocks than
+    all of them do when the tiles are dealt out one by one, or a third more at most (three rounds become four)."""
     lines = run(tmp_path, """
 #include <cstdio>
 #include "qm_linear_rows_params.h"
@@ -44,10 +44,11 @@ int main() {
             assert width == columns
             busiest = -(-tiles // 8)
         if width != columns:
-            assert -(-busiest // 32) <= -(-(-(-tiles // 8)) // 32), line
+            rounds, even = -(-busiest // 32), -(-(-(-tiles // 8)) // 32)
+            assert rounds == even or (even >= 3 and 3 * rounds <= 4 * even), line
             rounded += 1
     assert rounded > 5000
-    assert "81 8 1 88" in lines and "42 6 1 42" in lines and "42 3 2 42" in lines
+    assert "81 8 1 88" in lines and "81 9 1 88" in lines and "42 6 1 42" in lines and "42 3 2 42" in lines and "42 12 1 42" in lines
 
 
 # output linears as (columns, reduction) each, the last the one that may be cut; rows; its pieces (the first four are the layers of
