@@ -707,7 +707,7 @@ __global__ __launch_bounds__(kFrThreads, 1) void predictor_frame_kernel(FrParams
             sp.vocab = kFrVocab;
             sp.top_k = prm.top_k;
             sp.temperature = prm.temperature;
-            const int32_t chosen = sampler_block<true>(sp, *reinterpret_cast<SamplerScratch*>(smem + kFrLdsScratch), score, rng);
+            const int32_t chosen = sampler_block<true, true>(sp, *reinterpret_cast<SamplerScratch*>(smem + kFrLdsScratch), score, rng);
             if (tid == 0) {
                 sh.code = chosen;
                 if (samples) prm.codes[step + 1] = chosen;

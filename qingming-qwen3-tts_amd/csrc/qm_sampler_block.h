@@ -152,8 +152,9 @@ struct SamplerScratch {
 // thread when prm.process_only stops after the processed scores.  Nothing is read from prm.logits or
 // prm.rng_state and nothing written to prm.output_id / prm.history / prm.rng_state: that is the caller's.
 // `sync` is the barrier of the kSmpThreads calling threads (the block's barrier where they are the whole block).
-// NARROW: every score is a bf16 value and prm.process is 0.
-template <bool NARROW, class Sync>
+// NARROW: every score is a bf16 value and prm.process is 0.  COMPACT: all keys go through the passes of the largest ones instead of their own, for a
+// kernel that has other uses for its registers (the second loop made the predictor's frame 1.7 % longer, 1132 -> 1151 us, with 50 entries).
+template <bool NARROW, bool COMPACT, class Sync>
 __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, SamplerScratch& sh, const float (&score)[kSmpPerThread],
                                                  unsigned long long& rng, Sync&& sync) {
     using Key = SamplerKey<NARROW>;
@@ -214,15 +215,38 @@ __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, Sampl
     // its digits have been looked at, most significant first.  Equal scores are told apart by their ids when they are ranked, not in
     // passes over bits that they share.  (Half a block's threads rank 128 keys in less time than a pass takes.) ----
     const int rankable = keep <= 64 ? 128 : kSmpMaxKeep;
+    key_t largest = 0;
+#pragma unroll
+    for (int j = 0; j < kSmpPerThread; ++j) largest = key[j] > largest ? key[j] : largest;
     key_t prefix = 0, prefix_mask = 0, threshold = 0;
     int remaining = keep, candidates = kSmpMaxVocab + 1, place = 0;
-    // counters of this thread's bins, and the keys in all bins above those: inside the wave from a prefix sum, then the waves above
-    auto bins_above = [&](uint4& low, uint4& high, int& own) __attribute__((always_inline)) {
-        low = own_words[0];
-        high = own_words[1];
+    bool all_keys = keep > kSmpFromLargest;
+    // (kept as a loop: unrolled, the compiler computes the digits of all passes ahead and runs out of registers)
+#pragma unroll 1
+    for (int pass = COMPACT || !all_keys ? 0 : Key::kPasses; (COMPACT || pass < Key::kPasses) && candidates > rankable; ++pass) {
+        const int shift = Key::shift(pass);
+        const unsigned digit_mask = Key::mask(pass);
+        sync();                                   // the bins are clear (and, later, the last pass's results read)
+        auto count = [&](key_t k) __attribute__((always_inline)) {
+            if (k != 0 && (k & prefix_mask) == prefix) {
+                const unsigned digit = static_cast<unsigned>(k >> shift) & digit_mask;
+                atomicAdd(&sh_hist[digit >> 1], 1U << (16 * (digit & 1U)));          // (at most 4096 in a counter)
+            }
+        };
+        if (COMPACT && all_keys) {
+#pragma unroll
+            for (int j = 0; j < kSmpPerThread; ++j) count(key[j]);
+        } else {
+            count(largest);
+        }
+        sync();
+        // keys in bins above this thread's sixteen: inside the wave from a prefix sum, then the waves above
+        const uint4 low = own_words[0], high = own_words[1];
         own_words[0] = own_words[1] = make_uint4(0, 0, 0, 0);
-        const uint32_t all = ((low.x + low.y) + (low.z + low.w)) + ((high.x + high.y) + (high.z + high.w));
-        own = static_cast<int>((all & 0xffffU) + (all >> 16));
+        const uint32_t high_pairs = (high.x + high.y) + (high.z + high.w);
+        const uint32_t all_pairs = (low.x + low.y) + (low.z + low.w) + high_pairs;
+        auto both = [](uint32_t pair) { return static_cast<int>((pair & 0xffffU) + (pair >> 16)); };
+        const int own = both(all_pairs);
         const int upto = wave_inclusive_scan(own, lane);
         const int wave_sum = __builtin_amdgcn_readlane(upto, 63);
         if (lane == 0) sh_wave_total[wave] = wave_sum;
@@ -230,82 +254,60 @@ __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, Sampl
         int above = wave_sum - upto;
 #pragma unroll
         for (int w = 1; w < 4; ++w) above += w > wave ? sh_wave_total[w] : 0;
-        return above;
-    };
-    auto digit_found = [&](int shift, unsigned digit_mask) __attribute__((always_inline)) {
+        if (above < remaining && remaining <= above + own) {       // exactly one thread; its bins by halves, from the top
+            int rest = remaining - above, digit = 16 * tid;
+            bool upper = rest <= both(high_pairs);
+            if (!upper) rest -= both(high_pairs);
+            digit += upper ? 8 : 0;
+            const uint32_t w0 = upper ? high.x : low.x, w1 = upper ? high.y : low.y, w2 = upper ? high.z : low.z, w3 = upper ? high.w : low.w;
+            upper = rest <= both(w2 + w3);
+            if (!upper) rest -= both(w2 + w3);
+            digit += upper ? 4 : 0;
+            const uint32_t v0 = upper ? w2 : w0, v1 = upper ? w3 : w1;
+            upper = rest <= both(v1);
+            if (!upper) rest -= both(v1);
+            digit += upper ? 2 : 0;
+            const uint32_t word = upper ? v1 : v0;
+            upper = rest <= static_cast<int>(word >> 16);
+            if (!upper) rest -= static_cast<int>(word >> 16);
+            digit += upper ? 1 : 0;
+            sh_digit = digit;
+            sh_remaining = rest;
+        }
         sync();
         prefix |= static_cast<key_t>(sh_digit) << shift;
         prefix_mask |= static_cast<key_t>(digit_mask) << shift;
         remaining = sh_remaining;
-    };
-    // how many keys reach the bound that starts with the digits in `prefix` (those not looked at are free, zero here), and where this
-    // thread's go (a prefix sum over the block: no counter to queue at)
-    auto reach = [&]() __attribute__((always_inline)) {
+        // the bound starts with the digits in `prefix`; those not looked at are free (zero here)
         threshold = prefix | Key::kFree;
+        // how many keys reach it, and where this thread's go (a prefix sum over the block: no counter to queue at)
         int mine = 0;
 #pragma unroll
         for (int j = 0; j < kSmpPerThread; ++j) mine += key[j] >= threshold ? 1 : 0;
-        const int upto = wave_inclusive_scan(mine, lane);
-        if (lane == 63) sh_wave_first[wave] = upto;
+        const int upto_mine = wave_inclusive_scan(mine, lane);
+        if (lane == 63) sh_wave_first[wave] = upto_mine;
         sync();
-        place = upto - mine;
+        place = upto_mine - mine;
         candidates = 0;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
             place += w < wave ? sh_wave_first[w] : 0;
             candidates += sh_wave_first[w];
         }
-    };
-    if (keep <= kSmpFromLargest) {
-        key_t largest = 0;
-#pragma unroll
-        for (int j = 0; j < kSmpPerThread; ++j) largest = key[j] > largest ? key[j] : largest;
-        // (kept as a loop: unrolled, the compiler computes the digits of all passes ahead and runs out of registers)
-#pragma unroll 1
-        for (int pass = 0; pass < Key::kPasses && candidates > rankable; ++pass) {
-            const int shift = Key::shift(pass);
-            const unsigned digit_mask = Key::mask(pass);
-            sync();                                // the bins are clear (and, later, the last pass's results read)
-            if (largest != 0 && (largest & prefix_mask) == prefix) {
-                const unsigned digit = static_cast<unsigned>(largest >> shift) & digit_mask;
-                atomicAdd(&sh_hist[digit >> 1], 1U << (16 * (digit & 1U)));
-            }
-            sync();
-            uint4 low, high;
-            int own;
-            const int above = bins_above(low, high, own);
-            if (above < remaining && remaining <= above + own) {   // exactly one thread; its bins by halves, from the top
-                auto both = [](uint32_t pair) { return static_cast<int>((pair & 0xffffU) + (pair >> 16)); };
-                const uint32_t high_pairs = (high.x + high.y) + (high.z + high.w);
-                int rest = remaining - above, digit = 16 * tid;
-                bool upper = rest <= both(high_pairs);
-                if (!upper) rest -= both(high_pairs);
-                digit += upper ? 8 : 0;
-                const uint32_t w0 = upper ? high.x : low.x, w1 = upper ? high.y : low.y, w2 = upper ? high.z : low.z, w3 = upper ? high.w : low.w;
-                upper = rest <= both(w2 + w3);
-                if (!upper) rest -= both(w2 + w3);
-                digit += upper ? 4 : 0;
-                const uint32_t v0 = upper ? w2 : w0, v1 = upper ? w3 : w1;
-                upper = rest <= both(v1);
-                if (!upper) rest -= both(v1);
-                digit += upper ? 2 : 0;
-                const uint32_t word = upper ? v1 : v0;
-                upper = rest <= static_cast<int>(word >> 16);
-                if (!upper) rest -= static_cast<int>(word >> 16);
-                digit += upper ? 1 : 0;
-                sh_digit = digit;
-                sh_remaining = rest;
-            }
-            digit_found(shift, digit_mask);
-            reach();
+        // (the largest keys have told all they can, and too many keys reach the bound: from all of them; the last pass of that tells all
+        // keys apart and leaves `keep`)
+        if (COMPACT && !all_keys && pass + 1 == Key::kPasses && candidates > rankable) {
+            all_keys = true;
+            pass = -1;
+            prefix = prefix_mask = 0;
+            remaining = keep;
         }
-        prefix = candidates > rankable ? 0 : prefix;
-        prefix_mask = 0;
-        remaining = keep;
     }
     // From all keys: a bin to a thread, and eight counters to a bin, since scores share their leading bits and additions to one word take turns.
     // (The last pass tells all keys apart and leaves `keep`.)
-    if (candidates > rankable) {
+    if (!COMPACT && __builtin_expect(candidates > rankable, false)) {
+        prefix = prefix_mask = 0;
+        remaining = keep;
 #pragma unroll 1
         for (int pass = 0; candidates > rankable; ++pass) {
             const int shift = Key::byte_shift(pass);
@@ -316,18 +318,35 @@ __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, Sampl
                 if (key[j] != 0 && (key[j] & prefix_mask) == prefix)
                     atomicAdd(&sh_hist[(static_cast<unsigned>(key[j] >> shift) & digit_mask) * kSmpWords + (lane & (kSmpWords - 1))], 1U);
             sync();
-            uint4 low, high;
-            int own;
-            const int above = bins_above(low, high, own);
+            const uint4 low = own_words[0], high = own_words[1];
+            own_words[0] = own_words[1] = make_uint4(0, 0, 0, 0);
+            const int own = static_cast<int>(((low.x + low.y) + (low.z + low.w)) + ((high.x + high.y) + (high.z + high.w)));
+            const int upto = wave_inclusive_scan(own, lane);
+            const int wave_sum = __builtin_amdgcn_readlane(upto, 63);
+            if (lane == 0) sh_wave_total[wave] = wave_sum;
+            sync();
+            int above = wave_sum - upto;
+            for (int w = wave + 1; w < 4; ++w) above += sh_wave_total[w];
             if (above < remaining && remaining <= above + own) {
                 sh_digit = tid;
                 sh_remaining = remaining - above;
                 sh_count = keep - (remaining - above) + own;       // so many reach the bin
             }
-            digit_found(shift, digit_mask);
+            sync();
+            prefix |= static_cast<key_t>(sh_digit) << shift;
+            prefix_mask |= static_cast<key_t>(digit_mask) << shift;
+            remaining = sh_remaining;
             candidates = sh_count;
         }
-        reach();
+        threshold = prefix | Key::kFree;
+        int mine = 0;
+#pragma unroll
+        for (int j = 0; j < kSmpPerThread; ++j) mine += key[j] >= threshold ? 1 : 0;
+        const int upto = wave_inclusive_scan(mine, lane);
+        if (lane == 63) sh_wave_first[wave] = upto;
+        sync();
+        place = upto - mine;
+        for (int w = 0; w < wave; ++w) place += sh_wave_first[w];
     }
 
     // ---- gather the keys that reach the bound, rank them by counting ----------------------------------------
@@ -470,10 +489,10 @@ __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, Sampl
 struct WholeBlockBarrier {
     __device__ __forceinline__ void operator()() const { __syncthreads(); }
 };
-template <bool NARROW>
+template <bool NARROW, bool COMPACT = false>
 __device__ __forceinline__ int32_t sampler_block(const SamplerParams& prm, SamplerScratch& sh, const float (&score)[kSmpPerThread],
                                                  unsigned long long& rng) {
-    return sampler_block<NARROW>(prm, sh, score, rng, WholeBlockBarrier());
+    return sampler_block<NARROW, COMPACT>(prm, sh, score, rng, WholeBlockBarrier());
 }
 
 }  // namespace qm

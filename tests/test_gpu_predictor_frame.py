@@ -154,6 +154,12 @@ def test_frame_steps_equal_the_operator_chain(frame, top_k):
         assert _same(got, want)
 
 
+@pytest.mark.parametrize("top_k", [128, 129, 256])
+def test_frame_steps_of_many_entries(frame, top_k):
+    """Around the number of entries from which the launch's sampler goes through all scores: the draws of the sampler's own launch, which does it its own way."""
+    test_frame_steps_equal_the_operator_chain(frame, top_k)
+
+
 @pytest.mark.parametrize("top_k", [50, 0], ids=["top50", "argmax"])
 def test_step_0_and_the_whole_frame_in_one_launch(frame, top_k):
     """Step 0 alone leaves what its row-by-row operators leave (caches rows 0 and 1, codes[1], selected[1], the next
