@@ -73,8 +73,8 @@ __device__ __forceinline__ uint32_t finish_pair(float s0, float s1, bool has_bia
 }
 
 // g / (1 + exp(-g)) of a bf16 value, good for its rounding to bf16: the bits that expf and the correctly rounded division give, for every finite one
-// (all compared on the device; infinity stays infinity, minus infinity and NaN make NaN there and here), in ten instructions where those take some forty.  The denominator is kept down by 2^32, so that its
-// reciprocal does not go below the normal numbers where exp(-g) is near the largest; one Newton step makes the reciprocal good to the last bit.
+// (all compared on the device; infinity stays infinity, minus infinity and NaN make NaN there and here), in ten instructions where those take some
+// forty.  The denominator is kept down by 2^32, so that its reciprocal does not go below the normal numbers where exp(-g) is near the largest; one Newton step makes the reciprocal good to the last bit.
 // (The pair's epilogue is as long as five of its steps: 1000 tokens x 6144 channels of 2048 54.6 -> 52.1 us, 777 x 3072 of 1024 22.1 -> 20.9.)
 __device__ __forceinline__ float silu_of_bf16(float g) {
     const float s = fmaf(__builtin_amdgcn_exp2f(g * -kLog2e), 0x1p-32f, 0x1p-32f);
@@ -689,8 +689,9 @@ int rows_mfma_reduction_parts(int rows, int columns, int reduction, bool dual) {
 // With a norm behind, whose launch adds the pieces for the price of their bytes, a long reduction is also cut in two where 64-row tiles would just
 // give every CU a block: as many blocks of 128 x 128 walk half the steps for two thirds of the requests an output takes.  (us, 2048 columns of 6144 and
 // the norm behind, as two calls / cut: weights from memory, 785, 850, 900, 1000 and 1024 tokens 43.6 / 35.1, 43.9 / 39.0, 43.3 / 36.6, 46.9 / 42.3 and
-// 48.4 / 43.0; still in the caches 36.0 / 33.1, 36.9 / 33.6, 36.2 / 36.6, 39.7 / 36.6 and 39.1 / 37.2; 1024 columns, 1600 tokens 39.1 / 36.1.  Of 2048,
-// from memory, 24.1 / 23.9, and of 4096, from the caches, 29.0 / 34.7: shorter ones stay.)
+// 48.4 / 43.0; still in the caches 36.0 / 33.1, 36.9 / 33.6, 36.2 / 36.6, 39.7 / 36.6 to 41.9 in runs with other buffers, and 39.1 / 37.2 to 41.6; 1024
+// columns, 1600 tokens 39.1 / 36.1.  Of 2048, from memory, 24.1 / 23.9, and of 4096, from the caches, 30.0 / 34.4: shorter ones stay.  Other row counts are
+// as the linear alone: 700 tokens would take 45.8 / 35.9 from memory and 1200 75.0 / 59.6, but 1700 59.3 / 67.3.)
 int rows_mfma_norm_parts(int rows, int columns, int reduction, bool* wide) {
     *wide = false;
     if (columns != 1024 && columns != 2048) return 1;

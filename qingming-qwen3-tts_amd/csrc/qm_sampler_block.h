@@ -15,8 +15,8 @@
 // ranked), those keys are gathered and ranked by counting, several threads to a key where there are threads for it, and
 // the first `keep` ranks are the sequence.  The select looks at each thread's largest key first: the keep-th largest of
 // those is such a bound, with an eighth of the additions to LDS; only where it would let too many keys through (`keep` beyond half of the
-// threads) or does (one thread holding many of the largest) are all keys looked at, in passes of 8 bits.  The exponentials are computed by `keep` threads at once; the sums
-// are added in the reference's order: the running sum of the second loop repeats the partial sums of the first, so one pass
+// threads) or does (one thread holding many of the largest) are all keys looked at, in passes of 8 bits.  The exponentials are computed by
+// `keep` threads at once; the sums are added in the reference's order: the running sum of the second loop repeats the partial sums of the first, so one pass
 // gives both.
 // Bound: a chain of LDS exchanges.  Cycles for 50 of 2048 16-bit scores: 14 400 with 64-bit keys, 8-bit digits of all keys until the bin is
 // wanted whole, a thread per key and the sums of one thread through LDS; 9 900 as it stands.  (us a draw of many in a row, 200 of 2048: 16-bit scores
