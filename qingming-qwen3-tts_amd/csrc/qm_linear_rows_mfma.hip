@@ -17,7 +17,7 @@
 // of a tile is KSTEP / 8 16-byte pieces in LDS, piece q of row r stored in slot q ^ key(r), the key chosen so that the
 // sixteen rows a fragment read touches in a cycle spread over all 64 banks.  An MFMA takes the weight rows as its A
 // operand and the token rows as B (D = W X^T): a lane then holds, for one token row, runs of four consecutive output
-// columns — 8-byte stores.
+// columns, which a linear's tile gathers to whole rows in LDS and a pair's lanes store as they are.
 // The tiles go from memory straight into a ring of LDS stages (buffer_load ... lds, no registers, the swizzle chosen by
 // which piece a lane fetches): four stages where they fit in 128 KiB (the 64 x 64 tile: eight, or six for a pair), else three,
 // two for the 192-column tile (64 KiB a stage).  A step's one barrier stands between the MFMAs of its last two k blocks, where a wave has read all it needs of
@@ -62,14 +62,15 @@ __device__ __forceinline__ void gm_wait_vm() {
 // What follows the fp32 sums of two neighbouring output columns, as a packed bf16 pair.  Every rounding is one half of a
 // v_cvt_pk_bf16_f32 (round to nearest even, a NaN quieted with its payload kept: the bits f2bf gives for every fp32 input).
 // Linear: bf16(sum + bias), then bf16(residual + that) (linear_bf16 and add_bf16, R17:126-245, 8772-8790).
-__device__ __forceinline__ uint32_t finish_pair(float s0, float s1, bool has_bias, uint32_t bias, bool has_residual, uint32_t residual) {
+__device__ __forceinline__ uint32_t finish_pair(float s0, float s1, bool has_bias, uint32_t bias) {
     if (has_bias) {
         s0 += lo_bf16(bias);
         s1 += hi_bf16(bias);
     }
-    uint32_t v = pack_bf16_pair(s0, s1);
-    if (has_residual) v = pack_bf16_pair(lo_bf16(residual) + lo_bf16(v), hi_bf16(residual) + hi_bf16(v));
-    return v;
+    return pack_bf16_pair(s0, s1);
+}
+__device__ __forceinline__ uint32_t add_residual_pair(uint32_t v, uint32_t residual) {
+    return pack_bf16_pair(lo_bf16(residual) + lo_bf16(v), hi_bf16(residual) + hi_bf16(v));
 }
 
 // g / (1 + exp(-g)) of a bf16 value, good for its rounding to bf16: the bits that expf and the correctly rounded division give, for every finite one
@@ -491,73 +492,118 @@ __global__ __launch_bounds__(64 * WAVES) void linear_rows_mfma_kernel(LinearRows
 
     // ---- epilogue: accumulator register r of a lane is output column 8 (r / 4) + 4 (lane / 32) + r % 4 of the MFMA
     // tile's 32, token row lane % 32 ----
-    if (prm.reduction_parts > 1) {
-        // a piece of the reduction: the sums as they are, for linear_rows_parts_kernel
-        const int64_t plane = static_cast<int64_t>(prm.rows) * prm.columns;
-        float* const part = prm.partials + static_cast<int64_t>(blockIdx.z) * (DUAL ? 2 : 1) * plane;
+    if constexpr (DUAL) {
+        // A pair's lanes store from there: a store's 64 lanes go to 32 rows, one lane a cycle in the address path, but behind the next values' SwiGLU
+        // (through LDS, as below: 777 tokens x 3072 channels of 1024 20.2 -> 20.5 us, 300 x 3072 8.4 -> 8.7, 1000 x 6144 of 2048 57.8 -> 58.9).
+        if (prm.reduction_parts > 1) {
+            // a piece of the reduction: the sums as they are, for linear_rows_parts_kernel
+            const int64_t plane = static_cast<int64_t>(prm.rows) * prm.columns;
+            float* const part = prm.partials + static_cast<int64_t>(blockIdx.z) * 2 * plane;
 #pragma unroll
-        for (int a = 0; a < kTn; ++a) {
+            for (int a = 0; a < kTn; ++a) {
 #pragma unroll
-            for (int b = 0; b < kTm; ++b) {
-                const int m = m0 + 32 * (kTm * wave_m + b) + (lane & 31);
-                if (m >= prm.rows) continue;
+                for (int b = 0; b < kTm; ++b) {
+                    const int m = m0 + 32 * (kTm * wave_m + b) + (lane & 31);
+                    if (m >= prm.rows) continue;
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const int n = n0 + 32 * (kTn * wave_n + a) + 8 * g + 4 * (lane >> 5);
-                    float* at = part + static_cast<int64_t>(m) * prm.columns + n;
-                    *reinterpret_cast<float4*>(at) = make_float4(acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
-                    if (DUAL)
+                    for (int g = 0; g < 4; ++g) {
+                        const int n = n0 + 32 * (kTn * wave_n + a) + 8 * g + 4 * (lane >> 5);
+                        float* at = part + static_cast<int64_t>(m) * prm.columns + n;
+                        *reinterpret_cast<float4*>(at) = make_float4(acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
                         *reinterpret_cast<float4*>(at + plane) =
                             make_float4(acc_up[a][b][4 * g], acc_up[a][b][4 * g + 1], acc_up[a][b][4 * g + 2], acc_up[a][b][4 * g + 3]);
+                    }
                 }
             }
+            return;
         }
-        return;
-    }
-    if (!DUAL && sums) {
 #pragma unroll
         for (int a = 0; a < kTn; ++a) {
 #pragma unroll
             for (int b = 0; b < kTm; ++b) {
                 const int m = m0 + 32 * (kTm * wave_m + b) + (lane & 31);
-                if (m >= prm.rows) continue;
+                const bool inside = m < prm.rows;
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
+                    if (!inside) break;
                     const int n = n0 + 32 * (kTn * wave_n + a) + 8 * g + 4 * (lane >> 5);
-                    *reinterpret_cast<float4*>(sums + static_cast<int64_t>(m) * columns + n) =
-                        make_float4(acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
+                    uint32_t packed[2];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        packed[e] = swiglu_pair(acc[a][b][4 * g + 2 * e], acc[a][b][4 * g + 2 * e + 1], acc_up[a][b][4 * g + 2 * e], acc_up[a][b][4 * g + 2 * e + 1]);
+                    *reinterpret_cast<uint2*>(output + static_cast<int64_t>(m) * columns + n) = make_uint2(packed[0], packed[1]);
                 }
             }
         }
-        return;
-    }
+    } else {
+        // A linear's have nothing to hide them behind: the tile passes through the stages' LDS and leaves as whole rows, 16 bytes a lane.
+        // (Of a 128 x 128 tile's 4900 cycles behind its last step the stores were 4000.  us, from the lanes / through LDS: 1000 tokens, 4096 outputs
+        // of 2048 23.0 / 21.4, 1024 tokens, 11264 fp32 sums 63 / 58, 8192 42 / 40; 777 tokens, 6144 of 1024 21.3 / 18.7, 1024 6.3 / 6.0.)
+        asm volatile("s_barrier" ::: "memory");                   // (everybody's reads and requests are over)
+        const int64_t corner = static_cast<int64_t>(m0) * columns + n0;
+        if (prm.reduction_parts > 1 || sums) {
+            // the fp32 sums as they are: of a piece of the reduction, for linear_rows_parts_kernel, or for the caller
+            constexpr int kPitch = BN * 4 + 16, kChunks = BN / 4;
+            static_assert(BM * kPitch <= kStages * kStageBytes && BM * kChunks % (64 * WAVES) == 0, "the tile's sums");
+            float* to = (prm.reduction_parts > 1 ? prm.partials + static_cast<int64_t>(blockIdx.z) * prm.rows * prm.columns : sums) + corner;
 #pragma unroll
-    for (int a = 0; a < kTn; ++a) {
+            for (int a = 0; a < kTn; ++a) {
 #pragma unroll
-        for (int b = 0; b < kTm; ++b) {
-            const int m = m0 + 32 * (kTm * wave_m + b) + (lane & 31);
-            const bool inside = m < prm.rows;
+                for (int b = 0; b < kTm; ++b) {
+                    unsigned char* at = gm_smem + (32 * (kTm * wave_m + b) + (lane & 31)) * kPitch + (32 * (kTn * wave_n + a) + 4 * (lane >> 5)) * 4;
+#pragma unroll
+                    for (int g = 0; g < 4; ++g)
+                        *reinterpret_cast<float4*>(at + 32 * g) = make_float4(acc[a][b][4 * g], acc[a][b][4 * g + 1], acc[a][b][4 * g + 2], acc[a][b][4 * g + 3]);
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < BM * kChunks / (64 * WAVES); ++i) {
+                const int at = i * 64 * WAVES + tid, row = at / kChunks, chunk = at % kChunks;
+                if (row < x_rows) *reinterpret_cast<float4*>(to + static_cast<int64_t>(row) * columns + 4 * chunk) = *reinterpret_cast<const float4*>(gm_smem + row * kPitch + 16 * chunk);
+            }
+            return;
+        }
+        constexpr int kPitch = BN * 2 + 16, kChunks = BN / 8, kMine = BM * kChunks / (64 * WAVES);
+        static_assert(BM * kPitch <= kStages * kStageBytes && BM * kChunks % (64 * WAVES) == 0, "the tile's outputs");
+        typedef uint32_t row_piece_t __attribute__((ext_vector_type(4), aligned(8)));     // (outputs and residuals begin at any eight bytes)
+        row_piece_t residual[kMine];
+        if (prm.residual) {
+#pragma unroll
+            for (int i = 0; i < kMine; ++i) {
+                const int at = i * 64 * WAVES + tid, row = at / kChunks, chunk = at % kChunks;
+                residual[i] = *reinterpret_cast<const row_piece_t*>(prm.residual + corner + static_cast<int64_t>(min(row, x_rows - 1)) * columns + 8 * chunk);
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < kTn; ++a) {
+            uint2 bias_pair[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
-                if (!inside) break;
-                const int n = n0 + 32 * (kTn * wave_n + a) + 8 * g + 4 * (lane >> 5);
-                uint2 res = make_uint2(0, 0);
-                if (!DUAL && prm.residual) res = *reinterpret_cast<const uint2*>(prm.residual + static_cast<int64_t>(m) * columns + n);
-                uint2 bias_pair = make_uint2(0, 0);
-                if (!DUAL && bias) bias_pair = *reinterpret_cast<const uint2*>(bias + n);
-                uint32_t packed[2];
-#pragma unroll
-                for (int e = 0; e < 2; ++e) {
-                    const float s0 = acc[a][b][4 * g + 2 * e], s1 = acc[a][b][4 * g + 2 * e + 1];
-                    if (DUAL) {
-                        packed[e] = swiglu_pair(s0, s1, acc_up[a][b][4 * g + 2 * e], acc_up[a][b][4 * g + 2 * e + 1]);
-                    } else {
-                        packed[e] = finish_pair(s0, s1, bias != nullptr, e == 0 ? bias_pair.x : bias_pair.y, prm.residual != nullptr,
-                                                e == 0 ? res.x : res.y);
-                    }
-                }
-                *reinterpret_cast<uint2*>(output + static_cast<int64_t>(m) * columns + n) = make_uint2(packed[0], packed[1]);
+                bias_pair[g] = make_uint2(0, 0);
+                if (bias) bias_pair[g] = *reinterpret_cast<const uint2*>(bias + n0 + 32 * (kTn * wave_n + a) + 8 * g + 4 * (lane >> 5));
             }
+#pragma unroll
+            for (int b = 0; b < kTm; ++b) {
+                unsigned char* at = gm_smem + (32 * (kTm * wave_m + b) + (lane & 31)) * kPitch + (32 * (kTn * wave_n + a) + 4 * (lane >> 5)) * 2;
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    *reinterpret_cast<uint2*>(at + 16 * g) =
+                        make_uint2(finish_pair(acc[a][b][4 * g], acc[a][b][4 * g + 1], bias != nullptr, bias_pair[g].x),
+                                   finish_pair(acc[a][b][4 * g + 2], acc[a][b][4 * g + 3], bias != nullptr, bias_pair[g].y));
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < kMine; ++i) {
+            const int at = i * 64 * WAVES + tid, row = at / kChunks, chunk = at % kChunks;
+            if (row >= x_rows) continue;
+            row_piece_t v = *reinterpret_cast<const row_piece_t*>(gm_smem + row * kPitch + 16 * chunk);
+            if (prm.residual) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = add_residual_pair(v[e], residual[i][e]);
+            }
+            *reinterpret_cast<row_piece_t*>(output + corner + static_cast<int64_t>(row) * columns + 8 * chunk) = v;
         }
     }
 }
@@ -590,8 +636,12 @@ __global__ __launch_bounds__(256) void linear_rows_parts_kernel(LinearRowsParams
         packed.x = swiglu_pair(sum.x, sum.y, up.x, up.y);
         packed.y = swiglu_pair(sum.z, sum.w, up.z, up.w);
     } else {
-        packed.x = finish_pair(sum.x, sum.y, prm.bias != nullptr, bias.x, prm.residual != nullptr, res.x);
-        packed.y = finish_pair(sum.z, sum.w, prm.bias != nullptr, bias.y, prm.residual != nullptr, res.y);
+        packed.x = finish_pair(sum.x, sum.y, prm.bias != nullptr, bias.x);
+        packed.y = finish_pair(sum.z, sum.w, prm.bias != nullptr, bias.y);
+        if (prm.residual) {
+            packed.x = add_residual_pair(packed.x, res.x);
+            packed.y = add_residual_pair(packed.y, res.y);
+        }
     }
     *reinterpret_cast<uint2*>(prm.output + static_cast<int64_t>(m) * prm.columns + n) = packed;
 }

@@ -61,6 +61,26 @@ def test_linear_rows_against_the_oracle(oracle, qm, dev, rows, cols, red, bias, 
     _check(oracle, to_u16(out), want, _on_matrix_cores(rows_kernel, rows, cols, red), r)
 
 
+# (a tile of each width and height the rules choose, its last row tile of one row, of all but one and whole)
+@pytest.mark.parametrize("rows,cols,red", [(17, 128, 256), (63, 384, 256), (700, 1024, 256), (777, 2048, 128), (1025, 3328, 128), (2048, 2048, 128), (100, 4096, 4096)])
+@pytest.mark.parametrize("rows_kernel", [MATRIX], indirect=True)
+def test_outputs_and_residuals_that_begin_at_eight_bytes(oracle, qm, dev, rows, cols, red, rows_kernel):
+    """Output, residual and bias at eight bytes of a line, the residual added in place, nothing written around the output."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows + cols)
+    x = torch.randn((rows, red), generator=gen, device=dev).to(torch.bfloat16)
+    w = (torch.randn((cols, red), generator=gen, device=dev) * red ** -0.5).to(torch.bfloat16)
+    memory = torch.randn(rows * cols + 12 + cols, generator=gen, device=dev).to(torch.bfloat16)
+    out, bias, before = memory[4:4 + rows * cols].view(rows, cols), memory[8 + rows * cols:8 + rows * cols + cols], memory.clone()
+    v = (x.float() @ w.float().t() + bias.float()).to(torch.bfloat16)
+    qm.linear_rows(x, w, bias, out, out, rows, cols, red)
+    torch.cuda.synchronize()
+    residual = before[4:4 + rows * cols].view(rows, cols)
+    want = (residual.float() + v.float()).to(torch.bfloat16)
+    _check(oracle, to_u16(out.contiguous().view(torch.int16)), to_u16(want.view(torch.int16)), True, to_u16(residual.contiguous().view(torch.int16)))
+    assert torch.equal(memory[:4], before[:4]) and torch.equal(memory[4 + rows * cols:], before[4 + rows * cols:])
+
+
 def test_a_prompt_row_equals_the_decode_linear_of_that_row(oracle, qm, dev, rows_kernel):
     """(the exact chain; with 64 rows and 128 columns the default kernel is the matrix cores, the other is asked for)"""
     import torch
