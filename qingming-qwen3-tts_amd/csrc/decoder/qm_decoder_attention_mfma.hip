@@ -1,17 +1,24 @@
 // qm_decoder_attention_mfma.hip — the chunked attention of a prompt's rows on the bf16 matrix cores (gfx950).
 //
-// A block of eight waves takes 64 query rows of one key/value head (a query row is a position and one of the head's query
-// heads: they share keys and values) and walks the keys that any of them sees in tiles of 128.  Four waves work on the same
-// 32 rows, each on a quarter of every tile, and combine at the end: a prompt of a thousand tokens gives a grid that fills the
-// chip, its longest block walks eight tiles, and a wave needs nothing from another while it walks.  Blocks of one key/value
-// head share a die's L2 (block numbers go round the dies).
+// A block of four or eight waves takes 32 query rows of one key/value head (a query row is a position and one of the head's
+// query heads: they share keys and values); the waves take turns at the tiles of 32 keys that any of them sees and combine
+// at the end.  A wave's keys and values are its own: it brings them straight into its part of the LDS
+// (buffer_load ... lds, a tile of keys and a tile of values) and asks for the next keys when the products with these have read
+// them, for the next values likewise, so that nothing waits for another wave and either is under way during the other's
+// product; two blocks of four waves share a CU.  Blocks of one key/value head share a die's L2 (block numbers go round the dies).
 //
 // Scores are S^T = K Q^T (v_mfma_f32_32x32x16_bf16): a lane then holds sixteen keys of one query, the softmax is in the lane
 // but for one exchange with the other half of the wave, and the weights stand where the second product O^T = V^T P^T wants
 // its operand, if it takes the keys of a block in the order the scores left them.  Scores and weights are fp32; the second
 // product takes a weight as the sum of two bf16 numbers (its rounding and the rounding of what is left: 16 bits).  Values
-// are transposed on their way into LDS.  Bound: bf16 MFMA and the vector work per score; flops 2 (dim + vdim) per visible
-// key and query (the second product's doubled weights not counted).
+// are transposed on their way out of LDS (ds_read_b64_tr_b16).  Bound: the chain of a tile in its wave (two products, the
+// softmax between them); flops 2 (dim + vdim) per visible key and query (the second product's doubled weights not counted).
+// (us, by blocks of eight waves that staged 128 keys for 64 rows through registers, values transposed on the way in, two barriers a
+// tile / so: 8 heads of 192 and 128 channels, 777 rows 25.9 / 15.4; 16 query heads on 8 of 128, 1024 rows 28.7 / 19.5, of 64, 1000 rows
+// 12.3 / 10.4; 32 heads of 128, 1500 rows 79 / 61; 4 on 2 of 250, 200 rows 24.9 / 12.0.)
+#include <algorithm>
+#include <utility>
+
 #include "../qm_host.h"
 #include "qm_decoder_device.h"
 
@@ -21,153 +28,238 @@ typedef float dec_f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t dec_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t dec_u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kFlashKeys = 128;                // keys per tile
-constexpr int kFlashParts = kFlashKeys / 32;   // waves that share 32 query rows
-constexpr int kFlashThreads = 2 * kFlashParts * 64;
-constexpr int kFlashRows = 64;                 // query rows per block
-constexpr int kFlashVStride = kFlashKeys + 4;  // bf16 per value channel in LDS: the 32 rows of a fragment lie in different banks
+constexpr int kFlashKeys = 32;                 // keys per tile of a wave
+constexpr int kFlashRows = 32;                 // query rows per block
 
-// CK, CV: channels of a key and of a value, rounded up to multiples of 32
-template <int CK, int CV>
-struct FlashShape {
-    static constexpr int kKStride = CK + 8;
-    static constexpr int kKBytes = kFlashKeys * kKStride * 2;
-    static constexpr int kVBytes = CV * kFlashVStride * 2;
-    // (the other parts' sums arrive two channel tiles at a time)
-    static constexpr int kCombineTiles = CV / 32 < 2 ? 1 : 2;
-    static constexpr int kCombineBytes = 2 * (kFlashParts - 1) * (kCombineTiles * 16 * 64 + 2 * 32) * 4;
-    static constexpr int kLds = kKBytes + kVBytes > kCombineBytes ? kKBytes + kVBytes : kCombineBytes;
+// A tile in LDS: rows of CHANNELS bf16, in 16-byte pieces; piece c of row r stands in slot c ^ key(r).
+// KEYS: the sixteen rows whose piece c a fragment read takes in a cycle stand in different banks; else the four rows of a
+// transposing read do (it takes two pieces of each).
+template <int CHANNELS, bool KEYS>
+struct FlashTile {
+    static constexpr int kPieces = CHANNELS / 8, kRowBytes = CHANNELS * 2, kBytes = kFlashKeys * kRowBytes;
+    static constexpr int kRequests = kBytes / 1024;                            // instructions of a wave
+    static constexpr int kPeriod = kPieces % 16 == 0 ? 1 : kPieces % 8 == 0 ? 2 : 4;    // rows to 256 bytes' multiple
+    static constexpr int kSwap = KEYS ? 16 / kPeriod : 1;                      // (keys) pieces that change places with one another
+    static __device__ __forceinline__ int key(int row) {
+        if (KEYS) return row / kPeriod & (kSwap - 1);
+        return kPeriod == 1 ? 4 * (row & 3) : kPeriod == 2 ? 4 * (row >> 1 & 1) : 0;
+    }
+    // instructions after which a lane's row has the same key: their offsets differ by rows only
+    static constexpr int kOffsets = kRequests > kPieces / 4 ? kPieces / 4 : kRequests;
+    static constexpr int kOffsetRows = kOffsets * 64 / kPieces;
+    static_assert(kOffsets >= 1 && kOffsetRows % 16 == 0 && kRequests % kOffsets == 0, "");
 };
 
-template <int CK, int CV>
-__global__ __launch_bounds__(kFlashThreads) void chunk_attention_mfma_kernel(ChunkAttentionParams prm) {
-    using Shape = FlashShape<CK, CV>;
+template <int CK, int CV, int PARTS>
+struct FlashShape {
+    using Keys = FlashTile<CK, true>;
+    using Values = FlashTile<CV, false>;
+    static constexpr int kWaveBytes = Keys::kBytes + Values::kBytes;
+    // the parts' sums meet in LDS, and their largest scores and sums of weights
+    static constexpr int kSumBytes = PARTS * (CV / 32) * 4096, kCombineBytes = kSumBytes + PARTS * 2 * 32 * 4;
+    static constexpr int kLds = PARTS * kWaveBytes > kCombineBytes ? PARTS * kWaveBytes : kCombineBytes;
+};
+
+template <class F, int... I>
+__device__ __forceinline__ void flash_each_of(F&& f, std::integer_sequence<int, I...>) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, class F>
+__device__ __forceinline__ void flash_each(F&& f) { flash_each_of(f, std::make_integer_sequence<int, N>{}); }
+
+// LDS reads and the waits for them, as assembly: the compiler would have each read wait for all requests under way
+template <int OFFSET>
+__device__ __forceinline__ void flash_read(dec_u32x4& to, uint32_t at) { asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(to) : "v"(at), "n"(OFFSET)); }
+template <int OFFSET>
+__device__ __forceinline__ void flash_read_transposed(dec_u32x2& to, uint32_t at) {
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(to) : "v"(at), "n"(OFFSET));
+}
+template <int LATER>
+__device__ __forceinline__ void flash_arrived(dec_u32x4& a, dec_u32x4& b) { asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(a), "+v"(b) : "n"(LATER) : "memory"); }
+__device__ __forceinline__ void flash_arrived(dec_u32x2 (&v)[4]) { asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3])::"memory"); }
+template <int LATER>
+__device__ __forceinline__ void flash_landed() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LATER) : "memory"); }
+
+template <int CK, int CV, int PARTS>
+__global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void chunk_attention_mfma_kernel(ChunkAttentionParams prm) {
+    using Shape = FlashShape<CK, CV, PARTS>;
+    using Keys = typename Shape::Keys;
+    using Values = typename Shape::Values;
+    request_arguments(prm);
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    uint16_t* ks = reinterpret_cast<uint16_t*>(smem);                          // [keys][kKStride]
-    uint16_t* vt = reinterpret_cast<uint16_t*>(smem + Shape::kKBytes);         // [CV][kFlashVStride]
     constexpr int kKb = CK / 16, kVt = CV / 32;
     const int tid = threadIdx.x, lane = tid & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int pair = wave / kFlashParts, part = wave % kFlashParts, half = lane >> 5;
+    const int part = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5;
     const int kv_head = static_cast<int>(blockIdx.x);
     const int group = prm.heads / prm.kv_heads;
     const int total = prm.rows * group;
     const int row0 = static_cast<int>(gridDim.y - 1 - blockIdx.y) * kFlashRows;      // (late rows, which may see more keys, first)
-    auto position_at = [&](int query_row) { return prm.position + min(query_row, total - 1) / group; };
     auto chunk_start = [&](int position) { return position - position % prm.chunk; };
-    // what the block, this wave and this lane see: keys [.., ..]
-    const int block_lo = chunk_start(position_at(row0)), block_hi = position_at(row0 + kFlashRows - 1);
-    const int wave_first = position_at(row0 + 32 * pair), wave_last = position_at(row0 + 32 * pair + 31);
-    const int wave_lo = chunk_start(wave_first), wave_lo_most = chunk_start(wave_last);
-    const int query_row = row0 + 32 * pair + (lane & 31);
-    const int local = min(query_row, total - 1) / group;
-    const int head = kv_head * group + min(query_row, total - 1) % group;
+    // what the block and this lane see: keys [.., ..]
+    const int first_position = prm.position + row0 / group, last_position = prm.position + min(row0 + kFlashRows - 1, total - 1) / group;
+    const int block_lo = chunk_start(first_position), block_lo_most = chunk_start(last_position);
+    const int query_row = min(row0 + (lane & 31), total - 1);
+    const int local = query_row / group;
     const int position = prm.position + local;
-    const int lo = chunk_start(position);
+    const int lo = block_lo == block_lo_most ? block_lo : chunk_start(position);
 
-    dec_u32x4 q[kKb];
-    const uint16_t* q_row = static_cast<const uint16_t*>(prm.q_rot) + (static_cast<int64_t>(local) * prm.heads + head) * prm.k_stride;
+    // ---- requests: a tile goes out through a descriptor that begins at its first key and ends behind the last one that the block sees: a lane's
+    // offset is the same for every tile, what lies past the last key or past a row's channels is out of range and reads as zero.  Past a wave's last
+    // tile the requests stay (the waits count them) and ask for nothing. ----
+    const uint16_t* k_head = static_cast<const uint16_t*>(prm.k_cache) + static_cast<int64_t>(kv_head) * prm.ring * prm.k_stride;
+    const uint16_t* v_head = static_cast<const uint16_t*>(prm.v_cache) + static_cast<int64_t>(kv_head) * prm.ring * prm.v_stride;
+    constexpr uint32_t kOutOfRange = 0x7ffffff0U;
+    auto offsets_of = [&](auto tile_, int stride, auto& off) __attribute__((always_inline)) {
+        using Tile = decltype(tile_);
 #pragma unroll
-    for (int kb = 0; kb < kKb; ++kb) {
-        const int c = kb * 16 + 8 * half;
-        const dec_u32x4 read = *reinterpret_cast<const dec_u32x4*>(q_row + min(c, prm.k_stride - 8));
-        q[kb] = c < prm.k_stride ? read : dec_u32x4{0, 0, 0, 0};
+        for (int i = 0; i < Tile::kOffsets; ++i) {
+            const int at = 64 * i + lane, row = at / Tile::kPieces, c = 8 * (at % Tile::kPieces ^ Tile::key(row));
+            off[i] = c < stride ? static_cast<uint32_t>(row * stride + c) * 2u : kOutOfRange;
+        }
+    };
+    uint32_t k_off[Keys::kOffsets], v_off[Values::kOffsets];
+    offsets_of(Keys{}, prm.k_stride, k_off);
+    offsets_of(Values{}, prm.v_stride, v_off);
+    unsigned char* const k_lds = smem + part * Shape::kWaveBytes;
+    unsigned char* const v_lds = k_lds + Keys::kBytes;
+    auto request = [&](auto tile_, const uint16_t* head_rows, int stride, const auto& off, unsigned char* to, int k0, int base) __attribute__((always_inline)) {
+        using Tile = decltype(tile_);
+        const int keys = max(min(last_position + 1 - k0, kFlashKeys), 0), ahead = prm.ring - base;
+        auto rows_from = [&](const uint16_t* first, int count) {
+            return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(first), 0, count * stride * 2, 0x00020000);
+        };
+        auto bring = [&](const __amdgpu_buffer_rsrc_t& rsrc, int i, uint32_t from) __attribute__((always_inline)) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)(to + 1024 * i), 16, static_cast<int>(from), 0, 0, 0);
+        };
+        const __amdgpu_buffer_rsrc_t rsrc = rows_from(head_rows + static_cast<int64_t>(base) * stride, min(keys, ahead));
+        if (keys <= ahead) {
+#pragma unroll
+            for (int i = 0; i < Tile::kRequests; ++i)
+                bring(rsrc, i, off[i % Tile::kOffsets] + static_cast<uint32_t>(i / Tile::kOffsets * Tile::kOffsetRows * stride * 2));
+            return;
+        }
+        // (the rest at the ring's beginning, by other lanes of two instructions for one: the waits take that as longer ones)
+        const __amdgpu_buffer_rsrc_t rest = rows_from(head_rows, keys - ahead);
+#pragma unroll
+        for (int i = 0; i < Tile::kRequests; ++i) {
+            const int row = (64 * i + lane) / Tile::kPieces;
+            const uint32_t from = off[i % Tile::kOffsets] + static_cast<uint32_t>(i / Tile::kOffsets * Tile::kOffsetRows * stride * 2);
+            if (row < ahead) bring(rsrc, i, from);
+            else bring(rest, i, from - static_cast<uint32_t>(ahead * stride * 2));
+        }
+    };
+    auto request_keys = [&](int k0, int slot) __attribute__((always_inline)) { request(Keys{}, k_head, prm.k_stride, k_off, k_lds, k0, slot); };
+    auto request_values = [&](int k0, int slot) __attribute__((always_inline)) { request(Values{}, v_head, prm.v_stride, v_off, v_lds, k0, slot); };
+
+    // ---- fragment reads ----
+    auto lds_of = [](unsigned char* at) { return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)at)); };
+    // keys: lane's row lane % 32, piece 2 kb + half
+    constexpr int kSwapKb = Keys::kSwap / 2;
+    uint32_t k_at[kSwapKb];
+#pragma unroll
+    for (int i = 0; i < kSwapKb; ++i)
+        k_at[i] = lds_of(k_lds) + static_cast<uint32_t>((lane & 31) * Keys::kRowBytes + 16 * (2 * i ^ half ^ Keys::key(lane & 31)));
+    // queries: rows as a tile of keys, in KiB dealt to the waves' value tiles, every wave's piece brought by itself (straight into a matrix operand's
+    // order a load goes to 32 rows, one lane a cycle: 24 KiB took a block 3000 cycles)
+    auto query_lds = [&](int i) { return smem + i % PARTS * Shape::kWaveBytes + Keys::kBytes + i / PARTS * 1024; };
+    {
+        const int first_local = row0 / group, locals = min(row0 + kFlashRows - 1, total - 1) / group - first_local + 1;
+        const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<uint16_t*>(static_cast<const uint16_t*>(prm.q_rot) + static_cast<int64_t>(first_local) * prm.heads * prm.k_stride), 0,
+            locals * prm.heads * prm.k_stride * 2, 0x00020000);
+#pragma unroll
+        for (int n = 0; n < (Keys::kRequests + PARTS - 1) / PARTS; ++n) {
+            const int i = PARTS * n + part;
+            if (i >= Keys::kRequests) break;
+            const int at = 64 * i + lane, row = at / Keys::kPieces, c = 8 * (at % Keys::kPieces ^ Keys::key(row)), query = min(row0 + row, total - 1);
+            const int from = (query / group - first_local) * prm.heads + kv_head * group + query % group;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void*)query_lds(i), 16,
+                                                     static_cast<int>(c < prm.k_stride ? static_cast<uint32_t>(from * prm.k_stride + c) * 2u : kOutOfRange), 0, 0, 0);
+        }
     }
+    const int first_key = block_lo + kFlashKeys * part;
+    int slot = first_key % prm.ring;
+    request_keys(first_key, slot);
+    flash_landed<Keys::kRequests>();
+    asm volatile("s_barrier" ::: "memory");
+    dec_u32x4 q[kKb];
+    flash_each<kKb>([&](auto kb) {
+        constexpr int i = decltype(kb)::value;
+        const int at = (lane & 31) * Keys::kRowBytes + 16 * ((2 * i ^ half) ^ Keys::key(lane & 31));
+        flash_read<0>(q[i], lds_of(smem) + static_cast<uint32_t>((at >> 10) % PARTS * Shape::kWaveBytes + Keys::kBytes + (at >> 10) / PARTS * 1024 + (at & 1023)));
+    });
+    flash_each<kKb / 2>([&](auto pair) { flash_arrived<0>(q[2 * decltype(pair)::value], q[2 * decltype(pair)::value + 1]); });
+    asm volatile("s_barrier" ::: "memory");
+    request_values(first_key, slot);
+    // values: sixteen lanes take four keys x sixteen channels, lane 4 j + q of them channels 4 q .. of key j, and lane i gets the keys of channel i.
+    // The product's k index 8 half + e of 16 keys is key 8 (e / 4) + 4 half + e % 4 (the order the scores left them in): two such reads.
+    uint32_t v_at[kVt];
+    const int v_row = 4 * half + (lane >> 2 & 3);
+#pragma unroll
+    for (int t = 0; t < kVt; ++t)
+        v_at[t] = lds_of(v_lds) + static_cast<uint32_t>(v_row * Values::kRowBytes + 16 * ((4 * t + 2 * (lane >> 4 & 1) + (lane >> 1 & 1)) ^ Values::key(v_row)) + 8 * (lane & 1));
+
     dec_f32x16 o[kVt];
 #pragma unroll
     for (int t = 0; t < kVt; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) o[t][r] = 0.0f;
     float m = -INFINITY, l = 0.0f;
-    const float to_log2 = prm.scale * kLog2e;
+    // (of scores times a positive factor the largest is the largest score's; others are multiplied first)
+    const float to_log2 = prm.scale * kLog2e, factor_of_score = to_log2 > 0.0f ? to_log2 : 1.0f;
 
-    const uint16_t* k_head = static_cast<const uint16_t*>(prm.k_cache) + static_cast<int64_t>(kv_head) * prm.ring * prm.k_stride;
-    const uint16_t* v_head = static_cast<const uint16_t*>(prm.v_cache) + static_cast<int64_t>(kv_head) * prm.ring * prm.v_stride;
-    constexpr int kKPieces = kFlashKeys * (CK / 8) / kFlashThreads;                // 16-byte pieces of keys per thread
-    constexpr int kVBlocks = (kFlashKeys / 4 * (CV / 4) + kFlashThreads - 1) / kFlashThreads;    // blocks of 4 keys x 4 channels per thread
-    dec_u32x4 k_piece[kKPieces];
-    dec_u32x2 v_piece[kVBlocks][4];
-    // (keys past the last one that the block sees repeat it, channels past the head's repeat others: the first are masked,
-    // the second meet zeros of the query or are not stored; no branch around a load)
-    auto request = [&](int tile) __attribute__((always_inline)) {
-        const int base = tile % prm.ring, last = block_hi - tile;
-        auto slot_of = [&](int key) {
-            const int s = base + min(key, last);
-            return s >= prm.ring ? s - prm.ring : s;
-        };
-#pragma unroll
-        for (int i = 0; i < kKPieces; ++i) {
-            const int at = tid + i * kFlashThreads, key = at / (CK / 8), c = at % (CK / 8) * 8;
-            k_piece[i] = *reinterpret_cast<const dec_u32x4*>(k_head + slot_of(key) * prm.k_stride + min(c, prm.k_stride - 8));
-        }
-#pragma unroll
-        for (int i = 0; i < kVBlocks; ++i) {
-            const int at = tid + i * kFlashThreads, key = at / (CV / 4) * 4, c = at % (CV / 4) * 4;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                v_piece[i][j] = *reinterpret_cast<const dec_u32x2*>(v_head + slot_of(key + j) * prm.v_stride + min(c, prm.v_stride - 4));
-        }
-    };
-    auto deposit = [&]() __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < kKPieces; ++i) {
-            const int at = tid + i * kFlashThreads, key = at / (CK / 8), c = at % (CK / 8) * 8;
-            *reinterpret_cast<dec_u32x4*>(ks + key * Shape::kKStride + c) = k_piece[i];
-        }
-#pragma unroll
-        for (int i = 0; i < kVBlocks; ++i) {
-            const int at = tid + i * kFlashThreads, key = at / (CV / 4) * 4, c = at % (CV / 4) * 4;
-            if (at >= kFlashKeys / 4 * (CV / 4)) break;
-            const dec_u32x2 p0 = v_piece[i][0], p1 = v_piece[i][1], p2 = v_piece[i][2], p3 = v_piece[i][3];
-            uint16_t* to = vt + c * kFlashVStride + key;
-            auto pair_low = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x05040100U); };
-            auto pair_high = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302U); };
-            *reinterpret_cast<dec_u32x2*>(to) = dec_u32x2{pair_low(p0[0], p1[0]), pair_low(p2[0], p3[0])};
-            *reinterpret_cast<dec_u32x2*>(to + kFlashVStride) = dec_u32x2{pair_high(p0[0], p1[0]), pair_high(p2[0], p3[0])};
-            *reinterpret_cast<dec_u32x2*>(to + 2 * kFlashVStride) = dec_u32x2{pair_low(p0[1], p1[1]), pair_low(p2[1], p3[1])};
-            *reinterpret_cast<dec_u32x2*>(to + 3 * kFlashVStride) = dec_u32x2{pair_high(p0[1], p1[1]), pair_high(p2[1], p3[1])};
-        }
-    };
-
-    request(block_lo);
-    for (int tile = block_lo; tile <= block_hi; tile += kFlashKeys) {
-        __syncthreads();                                           // the tile before has been read
-        deposit();
-        __syncthreads();
-        if (tile + kFlashKeys <= block_hi) request(tile + kFlashKeys);
-        const int k0 = tile + 32 * part;
-        if (k0 > wave_last || k0 + 31 < wave_lo) continue;         // nothing here for this wave's rows
+    for (int k0 = first_key; k0 <= last_position; k0 += PARTS * kFlashKeys) {
+        const int next = k0 + PARTS * kFlashKeys;
+        slot += PARTS * kFlashKeys;
+        if (slot >= prm.ring) slot %= prm.ring;
+        flash_landed<Values::kRequests>();
+        dec_u32x4 key[kKb];
+        flash_each<kKb>([&](auto kb) {
+            constexpr int i = decltype(kb)::value;
+            flash_read<16 * Keys::kSwap * (i / kSwapKb)>(key[i], k_at[i % kSwapKb]);
+        });
         dec_f32x16 s;
 #pragma unroll
         for (int r = 0; r < 16; ++r) s[r] = 0.0f;
-        const uint16_t* k_row = ks + (32 * part + (lane & 31)) * Shape::kKStride + 8 * half;
-#pragma unroll
-        for (int kb = 0; kb < kKb; ++kb) {
-            const dec_u32x4 a = *reinterpret_cast<const dec_u32x4*>(k_row + kb * 16);
-            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, q[kb]), s, 0, 0, 0);
-        }
+        flash_each<kKb / 2>([&](auto pair) {
+            constexpr int i = 2 * decltype(pair)::value;
+            flash_arrived<kKb - 2 - i>(key[i], key[i + 1]);
+            if constexpr (i + 2 == kKb) request_keys(next, slot);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, key[i]), __builtin_bit_cast(bf16x8_t, q[i]), s, 0, 0, 0);
+            s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, key[i + 1]), __builtin_bit_cast(bf16x8_t, q[i + 1]), s, 0, 0, 0);
+        });
+        flash_landed<Keys::kRequests>();
+        dec_u32x2 value[kVt][4];
+        flash_each<kVt>([&](auto tile) {
+            constexpr int t = decltype(tile)::value;
+            flash_read_transposed<0>(value[t][0], v_at[t]);
+            flash_read_transposed<8 * Values::kRowBytes>(value[t][1], v_at[t]);
+            flash_read_transposed<16 * Values::kRowBytes>(value[t][2], v_at[t]);
+            flash_read_transposed<24 * Values::kRowBytes>(value[t][3], v_at[t]);
+        });
         // register r is key k0 + 8 (r / 4) + 4 half + r % 4
-        float p[16];
-        const bool whole = k0 >= wave_lo_most && k0 + 31 <= wave_first;
+        const bool whole = k0 >= block_lo_most && k0 + kFlashKeys - 1 <= first_position;
+        if (!(to_log2 > 0.0f)) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) p[r] = s[r] * to_log2;
+            for (int r = 0; r < 16; ++r) s[r] *= to_log2;
+        }
         if (!whole) {
             const int first = lo - k0 - 4 * half, last = position - k0 - 4 * half;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) p[r] = 8 * (r / 4) + r % 4 >= first && 8 * (r / 4) + r % 4 <= last ? p[r] : -INFINITY;
+            for (int r = 0; r < 16; ++r) s[r] = 8 * (r / 4) + r % 4 >= first && 8 * (r / 4) + r % 4 <= last ? s[r] : -INFINITY;
         }
-        float largest = p[0];
-#pragma unroll
-        for (int r = 1; r < 16; ++r) largest = fmaxf(largest, p[r]);
-        largest = xor32_max(largest);
+        float largest = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+        largest = fmaxf(largest, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])), fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
+        largest = xor32_max(largest) * factor_of_score;
         const float before = m;
         m = fmaxf(m, largest);
         const float reference = m == -INFINITY ? 0.0f : m;         // (a row that has seen no key yet: all its weights are zero)
         const float alpha = fast_exp2(before - reference);
-        float sum = 0.0f;
+#pragma unroll
+        for (int t = 0; t < kVt; ++t) flash_arrived(value[t]);
+        request_values(next, slot);
+        float p[16], sum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            p[r] = fast_exp2(p[r] - reference);
+            p[r] = fast_exp2(fmaf(s[r], factor_of_score, -reference));
             sum += p[r];
         }
         l = l * alpha + sum;
@@ -189,76 +281,66 @@ __global__ __launch_bounds__(kFlashThreads) void chunk_attention_mfma_kernel(Chu
             }
         }
 #pragma unroll
-        for (int t = 0; t < kVt; ++t) {
-            const uint16_t* v_row = vt + (32 * t + (lane & 31)) * kFlashVStride + 32 * part + 4 * half;
+        for (int b = 0; b < 2; ++b) {
 #pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const dec_u32x2 first = *reinterpret_cast<const dec_u32x2*>(v_row + 16 * b), second = *reinterpret_cast<const dec_u32x2*>(v_row + 16 * b + 8);
-                const dec_u32x4 a = {first[0], first[1], second[0], second[1]};
-                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, high[b]), o[t], 0, 0, 0);
-                o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, low[b]), o[t], 0, 0, 0);
+            for (int t = 0; t < 2 * kVt; ++t) {                    // (a sum is not asked for again right behind its last product)
+                const dec_u32x2 *v = value[t % kVt] + 2 * b;
+                const dec_u32x4 a = {v[0][0], v[0][1], v[1][0], v[1][1]};
+                o[t % kVt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, t < kVt ? high[b] : low[b]), o[t % kVt], 0, 0, 0);
             }
         }
     }
 
-    // the four parts of the keys, combined by the first
+    // The parts of the keys, combined: all leave their sums in LDS, and each takes its share of the rows.
     l = xor32_sum(l);
-    constexpr int kAtOnce = Shape::kCombineTiles;
-    float* shared = reinterpret_cast<float*>(smem);
-    float* sh_ml = shared + 2 * (kFlashParts - 1) * kAtOnce * 16 * 64;         // [2 pairs][parts - 1][2][32]
-    auto sums_of = [&](int p) { return shared + (pair * (kFlashParts - 1) + p - 1) * kAtOnce * 16 * 64; };
-    auto ml_of = [&](int p) { return sh_ml + (pair * (kFlashParts - 1) + p - 1) * 64; };
-    float factor[kFlashParts], scale = 0.0f;
+    flash_landed<0>();               // (the requests past the last tile)
+    __syncthreads();
+    float* sums = reinterpret_cast<float*>(smem);                  // [parts][kVt][register / 4][lane][4]
+    float* ml = reinterpret_cast<float*>(smem + Shape::kSumBytes); // [parts][2][32]
 #pragma unroll
-    for (int t0 = 0; t0 < kVt; t0 += kAtOnce) {
-        __syncthreads();
-        if (part > 0) {
+    for (int t = 0; t < kVt; ++t)
 #pragma unroll
-            for (int t = 0; t < kAtOnce; ++t)
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<float4*>(sums + (((part * kVt + t) * 4 + g) * 64 + lane) * 4) = make_float4(o[t][4 * g], o[t][4 * g + 1], o[t][4 * g + 2], o[t][4 * g + 3]);
+    if (lane < 32) {
+        ml[part * 64 + lane] = m;
+        ml[part * 64 + 32 + lane] = l;
+    }
+    __syncthreads();
+    constexpr int kLanes = 2 * PARTS;                              // to a row
+    const int mine = 32 / PARTS * part + lane / kLanes, mine_row = row0 + mine;
+    if (mine_row < total) {
+        float most = ml[mine], factor[PARTS], total_l = 0.0f;
 #pragma unroll
-                for (int r = 0; r < 16; ++r) sums_of(part)[(t * 16 + r) * 64 + lane] = o[t0 + t][r];
-            if (t0 == 0 && lane < 32) {
-                ml_of(part)[lane] = m;
-                ml_of(part)[32 + lane] = l;
-            }
+        for (int p = 1; p < PARTS; ++p) most = fmaxf(most, ml[p * 64 + mine]);
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) {
+            factor[p] = fast_exp2(ml[p * 64 + mine] - most);
+            total_l = fmaf(ml[p * 64 + 32 + mine], factor[p], total_l);
         }
-        __syncthreads();
-        if (part > 0) continue;
-        if (t0 == 0) {
-            float most = m;
+        const float scale = 1.0f / total_l;
+        uint16_t* out = static_cast<uint16_t*>(prm.out) + mine_row / group * prm.ld_out + (kv_head * group + mine_row % group) * prm.vdim;
 #pragma unroll
-            for (int p = 1; p < kFlashParts; ++p) most = fmaxf(most, ml_of(p)[lane & 31]);
-            factor[0] = fast_exp2(m - most);
-            float total_l = l * factor[0];
+        for (int i = 0; i < (CV / 4 + kLanes - 1) / kLanes; ++i) {
+            const int c = 4 * (kLanes * i + lane % kLanes);
+            if (c >= prm.vdim) break;
+            float v[4] = {};
 #pragma unroll
-            for (int p = 1; p < kFlashParts; ++p) {
-                factor[p] = fast_exp2(ml_of(p)[lane & 31] - most);
-                total_l = fmaf(ml_of(p)[32 + (lane & 31)], factor[p], total_l);
+            for (int p = 0; p < PARTS; ++p) {
+                const float4 x = *reinterpret_cast<const float4*>(sums + ((p * (CV / 8) + (c >> 3)) * 64 + mine + 32 * (c >> 2 & 1)) * 4);
+                v[0] = fmaf(x.x, factor[p], v[0]);
+                v[1] = fmaf(x.y, factor[p], v[1]);
+                v[2] = fmaf(x.z, factor[p], v[2]);
+                v[3] = fmaf(x.w, factor[p], v[3]);
             }
-            scale = 1.0f / total_l;
-        }
-        if (query_row >= total) continue;
-        uint16_t* out = static_cast<uint16_t*>(prm.out) + local * prm.ld_out + head * prm.vdim;
 #pragma unroll
-        for (int t = 0; t < kAtOnce; ++t) {
+            for (int e = 0; e < 4; ++e) v[e] *= scale;
+            if (prm.vdim % 4 == 0) {
+                *reinterpret_cast<uint2*>(out + c) = make_uint2(pack_bf16_pair(v[0], v[1]), pack_bf16_pair(v[2], v[3]));
+            } else {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int c = 32 * (t0 + t) + 8 * g + 4 * half;
-                float v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    v[e] = o[t0 + t][4 * g + e] * factor[0];
-#pragma unroll
-                    for (int p = 1; p < kFlashParts; ++p) v[e] = fmaf(sums_of(p)[(t * 16 + 4 * g + e) * 64 + lane], factor[p], v[e]);
-                    v[e] *= scale;
-                }
-                if (prm.vdim % 4 == 0) {
-                    if (c < prm.vdim) *reinterpret_cast<uint2*>(out + c) = make_uint2(pack_bf16_pair(v[0], v[1]), pack_bf16_pair(v[2], v[3]));
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (c + e < prm.vdim) out[c + e] = f2bf(v[e]);
-                }
+                for (int e = 0; e < 4; ++e)
+                    if (c + e < prm.vdim) out[c + e] = f2bf(v[e]);
             }
         }
     }
@@ -266,22 +348,32 @@ __global__ __launch_bounds__(kFlashThreads) void chunk_attention_mfma_kernel(Chu
     if (kv_head == prm.kv_heads - 1) {
         const int first = row0 / group, last = min(row0 + kFlashRows - 1, total - 1) / group;
         const int from = prm.heads * prm.vdim, behind = static_cast<int>(prm.ld_out) - from;
-        for (int i = tid; i < (last - first + 1) * behind; i += kFlashThreads)
+        for (int i = tid; i < (last - first + 1) * behind; i += 64 * PARTS)
             static_cast<uint16_t*>(prm.out)[(first + i / behind) * prm.ld_out + from + i % behind] = 0;
     }
 }
 
+template <int CK, int CV, int PARTS>
+static int32_t flash_of(const ChunkAttentionParams& prm, unsigned blocks, hipStream_t stream) {
+    using Shape = FlashShape<CK, CV, PARTS>;
+    static std::atomic<bool> raised[kMaxDevices];
+    const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(chunk_attention_mfma_kernel<CK, CV, PARTS>), Shape::kLds, raised);
+    if (rc != QM_OK) return rc;
+    hipLaunchKernelGGL((chunk_attention_mfma_kernel<CK, CV, PARTS>), dim3(prm.kv_heads, blocks), dim3(64 * PARTS), Shape::kLds, stream, prm);
+    return launch_status();
+}
+// Eight waves where the grid leaves CUs without a second block and a block walks long: half the steps, for a longer combination (us, four waves /
+// eight: 8 heads of 192 and 128, 128 rows 7.4 / 9.3, 777 rows 18.2 / 15.4; 300 rows of 16 on 8 heads of 128 behind 876 keys 20.5 / 16.6; 512 blocks,
+// 1024 rows 19.5 / 24.5).  A step of 128 keys costs 1.8 us, of 256 with eight waves 2.05, the longer combination 1.9: they meet at some 330 keys.
+constexpr int kFlashLongWalk = 384, kFlashCus = 256;
 template <int CK, int CV>
 static int32_t flash_as(const ChunkAttentionParams& prm, hipStream_t stream) {
-    constexpr int kLds = FlashShape<CK, CV>::kLds;
-    static std::atomic<bool> raised[kMaxDevices];
-    const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(chunk_attention_mfma_kernel<CK, CV>), kLds, raised);
-    if (rc != QM_OK) return rc;
-    const int64_t total = static_cast<int64_t>(prm.rows) * (prm.heads / prm.kv_heads);
-    if ((total + kFlashRows - 1) / kFlashRows > 65535) return QM_ERR_GEOMETRY;
-    hipLaunchKernelGGL((chunk_attention_mfma_kernel<CK, CV>), dim3(prm.kv_heads, static_cast<unsigned>((total + kFlashRows - 1) / kFlashRows)),
-                       dim3(kFlashThreads), kLds, stream, prm);
-    return launch_status();
+    const int64_t blocks = (static_cast<int64_t>(prm.rows) * (prm.heads / prm.kv_heads) + kFlashRows - 1) / kFlashRows;
+    if (blocks > 65535) return QM_ERR_GEOMETRY;
+    if constexpr (FlashShape<CK, CV, 8>::kLds <= 160 * 1024)
+        if (blocks * prm.kv_heads <= kFlashCus && std::min<int64_t>(prm.chunk, static_cast<int64_t>(prm.position) + prm.rows) >= kFlashLongWalk)
+            return flash_of<CK, CV, 8>(prm, static_cast<unsigned>(blocks), stream);
+    return flash_of<CK, CV, 4>(prm, static_cast<unsigned>(blocks), stream);
 }
 
 int32_t launch_chunk_attention_mfma(const ChunkAttentionParams& prm, hipStream_t stream) {

@@ -437,6 +437,17 @@ def test_chunk_attention_over_a_ring(decoder, dev, shape):
         close(case.run(decoder, dev, False, portions, ring=ring), want, False, tol16=3e-2)
 
 
+@pytest.mark.parametrize("shape", [(2, 2, 192, 128, 900, 64), (4, 2, 64, 64, 450, 16), (3, 1, 128, 120, 1000, 128), (2, 1, 32, 32, 385, 0), (2, 1, 250, 136, 500, 6)])
+def test_chunk_attention_of_few_blocks_that_walk_far(decoder, dev, shape):
+    """Prompts behind 384 keys and more, whose few blocks take eight waves where these fit, on both sides of that line and with a ring that wraps
+    inside a wave's tile; tolerance and plain attention as above."""
+    case = AttentionCase(shape, 640, seed=13)
+    want = case.want()
+    for portions in ([640], [383, 17, 240], [384, 33, 31, 192]):
+        for ring in (640, min(640, case.chunk + max(portions) - 1)):
+            close(case.run(decoder, dev, False, portions, ring=ring), want, False, tol16=3e-2)
+
+
 def test_two_attention_kernels_agree(decoder, dev):
     case = AttentionCase((8, 4, 64, 64, 512, 32), 700, seed=9)
     a, b = case.run(decoder, dev, False, [700]), case.run(decoder, dev, False, [700], rows_only=True)
