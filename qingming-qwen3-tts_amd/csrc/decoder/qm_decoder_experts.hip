@@ -5,6 +5,8 @@
 // from the logits themselves.  Many bf16 rows are copied expert by expert, each expert's rows from a multiple of the matrix-core
 // linear's row tile on, and that linear takes every tile's weights from its expert.  Bound by HBM: the chosen experts' weights are
 // read once per row (few rows) or once per row tile.
+#include <algorithm>
+
 #include "../qm_host.h"
 #include "../qm_linear_rows_params.h"
 #include "qm_decoder_dot.h"
@@ -16,7 +18,9 @@ constexpr int kExpertOutRows = 2;              // down
 constexpr int kRouteRows = kDecThreads / 64;   // rows per block of the router: a wave each
 constexpr int kSortThreads = 1024;
 constexpr int kExpertMatrixRows = 16;          // rows from which bf16 goes to the matrix cores
-constexpr int kExpertLongTile = 256;           // rows per expert (on average) from which row tiles are 128 high, not 64
+constexpr int kExpertLongTile = 256;           // rows per expert (on average) from which row tiles are 128 high, not 64,
+constexpr int kExpertTwoTiles[2] = {72, 116};  // and between which, where that many experts' ..
+constexpr int kExpertLongGrid = 96;            // .. column tiles are many blocks
 
 // What the kernels share in the scratch.
 struct ExpertScratch {
@@ -203,6 +207,15 @@ __global__ __launch_bounds__(kDecThreads) void expert_combine_kernel(ExpertParam
 
 static bool by_matrix(int rows, int f32) { return !f32 && rows >= kExpertMatrixRows; }
 
+// Row tiles of 128 where an expert's rows come to two tiles of 64 but for few, and one of 128, and the tiles of 64 are about as many as CUs or more: an
+// expert's weights are read once, not on two dies.  (us, pair and down of bf16, 64 / 128: 32 experts of 1024 x 512 with 97 rows each 27.9 + 17.0 / 21.6 +
+// 16.0, with 64 22.1 + 15.6 / 21.7 + 15.8, with 128 36.0 + 21.6 / 25.6 + 22.4; 24 of 2048 x 1024 with 96 62.6 + 33.9 / 55.2 + 32.8; 12 of 1024 x 512 12.6 +
+// 6.4 / 15.0 + 7.5.  Over fourteen numbers of experts and three of rows within these lines 0.97 to 1.34 times, 1.12 in the mean.)
+static bool tall_tiles(int64_t assignments, int experts, int ff_p) {
+    const bool two = assignments >= static_cast<int64_t>(kExpertTwoTiles[0]) * experts && assignments <= static_cast<int64_t>(kExpertTwoTiles[1]) * experts;
+    return assignments / experts >= kExpertLongTile || (two && static_cast<int64_t>(experts) * (ff_p / 128) >= kExpertLongGrid);
+}
+
 // The scratch's parts from `base` on; returns its bytes.
 static int64_t lay_out(char* base, int rows, int experts, int top, int width_p, int ff_p, int f32, bool matrix, ExpertScratch& s) {
     const int64_t assignments = static_cast<int64_t>(rows) * top;
@@ -215,7 +228,7 @@ static int64_t lay_out(char* base, int rows, int experts, int top, int width_p, 
     s.id = reinterpret_cast<int32_t*>(take(assignments * 4));
     s.weight = reinterpret_cast<float*>(take(assignments * 4));
     s.place = reinterpret_cast<int32_t*>(take(assignments * 4));
-    s.tile_rows = assignments / experts >= kExpertLongTile ? 128 : 64;
+    s.tile_rows = tall_tiles(assignments, experts, ff_p) ? 128 : 64;
     const int64_t full = assignments / s.tile_rows, used = assignments < experts ? assignments : experts;
     s.tiles = static_cast<int>(full + used);
     s.tile_expert = reinterpret_cast<int32_t*>(take(static_cast<int64_t>(s.tiles) * 4));
@@ -229,7 +242,10 @@ static int64_t lay_out(char* base, int rows, int experts, int top, int width_p, 
 int64_t expert_scratch_bytes(int rows, int experts, int top, int width_p, int ff_p, int f32) {
     if (rows <= 0 || experts <= 0 || top <= 0 || width_p <= 0 || ff_p <= 0) return 0;
     ExpertScratch s;
-    return lay_out(nullptr, rows, experts, top, width_p, ff_p, f32, by_matrix(rows, f32), s);      // (more rows never need less)
+    // (more rows never need less: past the rows that take tall tiles for their two tiles the bytes stay at theirs)
+    const int tall = static_cast<int>(std::min<int64_t>(rows, static_cast<int64_t>(kExpertTwoTiles[1]) * experts / top));
+    const int64_t bytes = lay_out(nullptr, rows, experts, top, width_p, ff_p, f32, by_matrix(rows, f32), s);
+    return tall > 0 ? std::max(bytes, lay_out(nullptr, tall, experts, top, width_p, ff_p, f32, by_matrix(tall, f32), s)) : bytes;
 }
 
 template <class T>

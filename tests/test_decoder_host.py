@@ -282,6 +282,13 @@ def test_latent_attention_in_the_latents_space():
             assert np.allclose(o[t, h], up_v[6 * h:6 * h + 6] @ ((p / p.sum()) @ c[:t + 1]))
 
 
+@pytest.mark.parametrize("experts,top,width,ff", [(24, 6, 128, 512), (32, 4, 1024, 512), (8, 2, 256, 1536), (1, 1, 128, 128), (300, 3, 128, 128)])
+def test_experts_memory_of_more_rows_is_never_less(decoder, experts, top, width, ff):
+    """(row tiles change their height with the rows)"""
+    sizes = [decoder.lib().qm_expert_scratch_bytes(rows, experts, top, width, ff, 0) for rows in range(1, 320 * experts // top + 2)]
+    assert all(a <= b for a, b in zip(sizes, sizes[1:]))
+
+
 def test_experts_of_the_highest_scores_are_weighted_with_them():
     h = np.array([[1.0, -2.0], [0.5, 3.0]])
     router = np.array([[1.0, 0.0], [0.0, 1.0], [-1.0, 0.0]])

@@ -823,3 +823,9 @@ def test_experts(decoder, dev, f32, rows, experts, top, width, ff):
         got = get(out)
         close(got[:, :width], want, f32, tol32=5e-6, tol16=2e-2)
         assert np.all(got[:, width:] == 0)
+
+
+@pytest.mark.parametrize("rows", [287, 288, 464, 465])
+def test_experts_whose_rows_are_two_row_tiles(decoder, dev, rows):
+    """24 experts of four column tiles with 72 to 116 rows each take one tall row tile, those outside two or three low ones; one expert is crowded."""
+    test_experts(decoder, dev, False, rows, 24, 6, 128, 512)
