@@ -7,6 +7,7 @@
 #include <algorithm>
 #include <map>
 #include <numeric>
+#include <vector>
 
 #include "qm_decoder_device.h"
 #include "../qm_host.h"
@@ -159,28 +160,32 @@ static bool split_pays(const DecLinearParams& prm) {
     return dots > 33 + k * (pair ? 85 : prm.rows <= 16 ? 46 : 56) / 1024;
 }
 
+int64_t steps_of_busiest_cu(int kinds, const int64_t* count, const int64_t* steps) {
+    std::vector<int> order(static_cast<size_t>(kinds));
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return steps[a] > steps[b]; });
+    std::map<int64_t, int64_t> cus = {{0, 256}};                               // steps dealt so far -> how many CUs have as many
+    for (int kind : order)
+        for (int64_t left = count[kind]; left > 0;) {
+            const auto [at, many] = *cus.begin();
+            const int64_t taken = std::min(left, many);
+            cus.erase(cus.begin());
+            if (many > taken) cus[at] = many - taken;
+            cus[at + steps[kind]] += taken;
+            left -= taken;
+        }
+    return cus.rbegin()->first;
+}
 // Steps of 64 k that the busiest CU walks when blocks of 128 x 128 outputs are dealt out long reductions first, the last one in `parts` pieces; a
 // block's first stages and its outputs are about three steps more.
 static int64_t steps_of_busiest(const DecLinearParams& prm, int parts) {
     int64_t count[kDecGroups], steps[kDecGroups];
-    int order[kDecGroups] = {0, 1, 2};
     for (int g = 0; g < prm.groups; ++g) {
         const int pieces = g == prm.groups - 1 ? parts : 1;
         count[g] = static_cast<int64_t>(prm.group[g].n / 128) * ((prm.rows + 127) / 128) * pieces;
         steps[g] = prm.group[g].k / 64 / pieces + 3;
     }
-    std::stable_sort(order, order + prm.groups, [&](int a, int b) { return steps[a] > steps[b]; });
-    std::map<int64_t, int64_t> cus = {{0, 256}};                               // steps dealt so far -> how many CUs have as many
-    for (int i = 0; i < prm.groups; ++i)
-        for (int64_t left = count[order[i]]; left > 0;) {
-            const auto [at, many] = *cus.begin();
-            const int64_t taken = std::min(left, many);
-            cus.erase(cus.begin());
-            if (many > taken) cus[at] = many - taken;
-            cus[at + steps[order[i]]] += taken;
-            left -= taken;
-        }
-    return cus.rbegin()->first;
+    return steps_of_busiest_cu(prm.groups, count, steps);
 }
 // Into how many pieces the last linear's reduction is cut: where the linears' blocks leave CUs idle behind the longest reduction, its pieces
 // fill them.  (us, 1024 rows, 2048 outputs of 6144: beside 2048 of 2048, three pieces, 66 -> 55; beside twice that, two pieces, 70 -> 65; the norm
@@ -214,16 +219,25 @@ int64_t reduction_cut_floats(const DecLinearParams& prm, int max_rows) {
     return most;
 }
 
-int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut) {
-    if (cut) cut->planes = 0;
+int32_t check_linears(const DecLinearParams& prm) {
     if (prm.rows < 0 || prm.groups < 1 || prm.groups > kDecGroups) return QM_ERR_ARGUMENT;
     for (int g = 0; g < prm.groups; ++g) {
         const DecLinearGroup& d = prm.group[g];
         if (!d.x || !d.w || (d.w_up ? !d.out : !d.out32)) return QM_ERR_NULL;
         if (d.n <= 0 || d.k <= 0 || d.n % (d.w_up ? 128 : 16) || d.k % 128 || d.ldx < d.k || d.ldo < d.n || d.ldx % 8 || d.ldo % 4) return QM_ERR_GEOMETRY;
     }
-    if (prm.rows == 0) return QM_OK;
-    if (f32) return split_pays(prm) ? launch_split_linears(prm, stream) : streaming<float>(prm, stream);
+    return QM_OK;
+}
+
+int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut, const PlaneMemory& planes) {
+    if (cut) cut->planes = 0;
+    const int32_t checked = check_linears(prm);
+    if (checked != QM_OK || prm.rows == 0) return checked;
+    if (f32) {
+        if (!split_pays(prm)) return streaming<float>(prm, stream);
+        return plane_elements(prm) <= planes.elements && planes_pay(prm, cut ? plane_pieces(prm) : 1) ? launch_plane_linears(prm, planes, stream, cut)
+                                                                                                      : launch_split_linears(prm, stream);
+    }
     bool matrix = prm.rows >= kDecMatrixRows;
     if (matrix && prm.groups == 1 && prm.group[0].n <= kNarrowColumns && !prm.group[0].w_up)
         return prm.group[0].n <= 32 ? launch_narrow<2>(prm, stream) : launch_narrow<4>(prm, stream);

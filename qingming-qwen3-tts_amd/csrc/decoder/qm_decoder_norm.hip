@@ -50,10 +50,10 @@ int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipSt
     if (rows < 0) return QM_ERR_ARGUMENT;
     if (!prm.h) return QM_ERR_NULL;
     if (rows == 0) return QM_OK;
-    if (more.planes > 0) {                     // (only the matrix cores' bf16 rows leave a term in pieces)
+    if (more.planes > 0) {                     // (the matrix cores leave a term in pieces)
         if (!more.sums) return QM_ERR_NULL;
-        if (more.planes > kMorePlanes || prm.terms == 0 || f32) return QM_ERR_ARGUMENT;
-        return residual_as<uint16_t, true>(prm, rows, more, stream);
+        if (more.planes > kMorePlanes || prm.terms == 0) return QM_ERR_ARGUMENT;
+        return f32 ? residual_as<float, true>(prm, rows, more, stream) : residual_as<uint16_t, true>(prm, rows, more, stream);
     }
     return f32 ? residual_as<float, false>(prm, rows, more, stream) : residual_as<uint16_t, false>(prm, rows, more, stream);
 }

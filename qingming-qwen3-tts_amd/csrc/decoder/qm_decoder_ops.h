@@ -47,6 +47,7 @@ inline int row_vectors(int64_t ld) { return ld <= 1024 ? 1 : ld <= 2048 ? 2 : ld
 
 // Whether the kernels take these arguments.
 int32_t check_residual(const ResidualParams& prm);
+int32_t check_linears(const DecLinearParams& prm);
 int32_t check_attention(const ChunkAttentionParams& prm);
 int32_t check_decay_attention(const DecayAttentionParams& prm);
 // The last term in pieces: `planes` more of them, `plane` floats apart, laid out as the term's own and added to it in order.
@@ -71,8 +72,22 @@ struct ReductionCut {
 // Into how many pieces that is, and the most floats that they take with any number of rows up to max_rows.
 int reduction_pieces(const DecLinearParams& prm);
 int64_t reduction_cut_floats(const DecLinearParams& prm, int max_rows);
-int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut = nullptr);
+// Memory in which fp32 inputs are split into their three parts beforehand: three times rows x k elements for each of the linears' different inputs.
+struct PlaneMemory {
+    uint16_t* at = nullptr;
+    int64_t elements = 0;
+};
+int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut = nullptr, const PlaneMemory& planes = PlaneMemory());
 int32_t launch_split_linears(const DecLinearParams& prm, hipStream_t stream);    // fp32 rows on the matrix cores
+// The same with inputs split beforehand: whether they can be, and whether that ends first (given that the matrix cores do), with the last reduction in so
+// many pieces; into how many it is cut; the launch, which cuts if `cut` has room.
+bool planes_fit(const DecLinearParams& prm);
+bool planes_pay(const DecLinearParams& prm, int pieces);
+int plane_pieces(const DecLinearParams& prm);
+int64_t plane_elements(const DecLinearParams& prm);
+int32_t launch_plane_linears(const DecLinearParams& prm, const PlaneMemory& planes, hipStream_t stream, ReductionCut* cut);
+// Steps that the busiest of 256 CUs walks when `kinds` kinds of blocks, `count` of `steps` steps each, are dealt out one to a CU, long ones first.
+int64_t steps_of_busiest_cu(int kinds, const int64_t* count, const int64_t* steps);
 // Rotation and cache write, then the attention.
 int32_t launch_chunk_attention(const ChunkAttentionParams& prm, int f32, hipStream_t stream);
 int32_t launch_chunk_attention_mfma(const ChunkAttentionParams& prm, hipStream_t stream);

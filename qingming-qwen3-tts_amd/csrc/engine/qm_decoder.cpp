@@ -134,7 +134,7 @@ struct qm_decoder {
     hipStream_t stream = nullptr;
     bool own_stream = false;
     qm_engine::DeviceBuffer x[2], h, proj, mlp, attended, gated, y[3], y_more, q_rot, raw, ml, acc, scratch, tokens, wanted, head_h, logits, tap, tap_h,
-        step_words, q_latent, queries, q_scratch, expanded, expert_logits, expert_scratch;
+        step_words, q_latent, queries, q_scratch, expanded, expert_logits, expert_scratch, planes;
     std::vector<hipGraphExec_t> graphs;             // one-token step of each sequence
     std::vector<hipGraphExec_t> mail_graphs;        // the same between the mailbox's words and its scores
     qm_engine::Mailbox mailbox;
@@ -362,6 +362,7 @@ int64_t token_bytes(const qm_decoder& d) {
 constexpr int64_t kStreamingTokenBytes = 256ll << 20;
 
 int64_t cut_floats(const qm_decoder& d);
+int64_t plane_elements(const qm_decoder& d);
 
 std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int capacity, int sequences, int max_rows, hipStream_t stream) {
     if (capacity <= 0 || sequences <= 0 || max_rows < 0 || (f32 != 0 && f32 != 1))
@@ -487,7 +488,8 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
     d->attended = zeros(rows * attended * item);
     d->gated = zeros(rows * gated * item);
     for (DeviceBuffer& y : d->y) y = zeros(rows * d->width_p * 4);
-    if (const int64_t more = f32 ? 0 : cut_floats(*d)) d->y_more = zeros(static_cast<size_t>(more) * 4);
+    if (const int64_t more = cut_floats(*d)) d->y_more = zeros(static_cast<size_t>(more) * 4);
+    if (f32) d->planes = zeros(static_cast<size_t>(plane_elements(*d)) * 2);
     d->q_rot = zeros(rows * q_rot * item);
     d->raw = zeros(rows * raw * 4);
     d->ml = zeros(ml * 4);
@@ -774,7 +776,9 @@ int64_t cut_floats(const qm_decoder& d) {
     int64_t most = 0;
     for (const DecoderLayer& w : d.layers) {
         Pending none;
-        most = std::max(most, qm::reduction_cut_floats(linears_out(d, w, d.max_rows, none), d.max_rows));
+        const qm::DecLinearParams outputs = linears_out(d, w, d.max_rows, none);
+        if (!d.f32) most = std::max(most, qm::reduction_cut_floats(outputs, d.max_rows));
+        else if (outputs.groups > 1) most = static_cast<int64_t>(qm::kMorePlanes) * d.max_rows * d.width_p;
     }
     return most;
 }
@@ -792,6 +796,19 @@ qm::DecLinearParams feed_out(const qm_decoder& d, const DecoderLayer& w, int row
     p.group[p.groups++] = linear_of(w.down, d.mlp.raw(), f32_of(d.y[0]));
     return p;
 }
+// Elements for any layer's fp32 inputs, split.
+int64_t plane_elements(const qm_decoder& d) {
+    int64_t most = 0;
+    for (const DecoderLayer& w : d.layers) {
+        Pending none;
+        most = std::max({most, qm::plane_elements(linears_in(d, w, d.max_rows)), qm::plane_elements(linears_out(d, w, d.max_rows, none))});
+        if (sandwich(w) && w.config.ff) {
+            most = std::max(most, qm::plane_elements(feed_in(d, w, d.max_rows)));
+            if (!w.config.experts) most = std::max(most, qm::plane_elements(feed_out(d, w, d.max_rows)));
+        }
+    }
+    return most;
+}
 Pending feed_term(const qm_decoder& d, const DecoderLayer& w) {
     Pending pending;
     add_term(d, pending, f32_of(d.y[0]), f32_of(w.after_ff), static_cast<float>(d.config.residual_mult));
@@ -801,6 +818,7 @@ Pending feed_term(const qm_decoder& d, const DecoderLayer& w) {
 // Every layer run over `rows` tokens of d.tokens at `position`; leaves the stream and what is pending for the head.
 void run_layers(qm_decoder& d, int sequence, int rows, int position, const float** stream_out, Pending& pending, float* taps) {
     hipStream_t s = d.stream;
+    const qm::PlaneMemory planes = {static_cast<uint16_t*>(d.planes.raw()), static_cast<int64_t>(d.planes.bytes() / 2)};
     const float* x = nullptr;
     int next = 0;
     pending = Pending();
@@ -812,7 +830,7 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
                  "residual + norm");
         x = x_new;
         next ^= 1;
-        op_check(qm::launch_decoder_linears(linears_in(d, w, rows), d.f32, s), "input projections");
+        op_check(qm::launch_decoder_linears(linears_in(d, w, rows), d.f32, s, nullptr, planes), "input projections");
         if (w.config.mixer == MixerKind::AttentionBesideDecay) {
             op_check(qm::launch_chunk_attention(attention_of(d, w, d.states[i], sequence, rows, position), d.f32, s), "chunked attention");
             op_check(qm::launch_decay_attention(decay_of(d, w, d.states[i], sequence, rows, position), s), "decayed linear attention");
@@ -832,16 +850,16 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
         if (w.config.mixer != MixerKind::LatentAttention) op_check(qm::launch_gated_norm(gated_of(d, w), rows, d.f32, s), "gated norm");
         const qm::DecLinearParams outputs = linears_out(d, w, rows, pending);
         qm::ReductionCut cut = {f32_of(d.y_more), static_cast<int64_t>(d.y_more.bytes() / 4), 0, 0};
-        op_check(qm::launch_decoder_linears(outputs, d.f32, s, cut.sums ? &cut : nullptr), "output projections");
+        op_check(qm::launch_decoder_linears(outputs, d.f32, s, cut.sums ? &cut : nullptr, planes), "output projections");
         pending.more = {cut.sums, cut.plane, cut.planes};
         if (sandwich(w) && w.config.ff) {
             x_new = f32_of(d.x[next]);
             op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, nullptr, f32_of(w.norm2), d.h.raw()), rows, d.f32, s, pending.more), "residual + norm");
             x = x_new;
             next ^= 1;
-            op_check(qm::launch_decoder_linears(feed_in(d, w, rows), d.f32, s), "feed-forward");
+            op_check(qm::launch_decoder_linears(feed_in(d, w, rows), d.f32, s, nullptr, planes), "feed-forward");
             if (w.config.experts) op_check(qm::launch_experts(experts_of(d, w, rows, f32_of(d.y[0])), d.f32, s), "experts");
-            else op_check(qm::launch_decoder_linears(feed_out(d, w, rows), d.f32, s), "feed-forward");
+            else op_check(qm::launch_decoder_linears(feed_out(d, w, rows), d.f32, s, nullptr, planes), "feed-forward");
             pending = feed_term(d, w);
         }
         if (taps) {

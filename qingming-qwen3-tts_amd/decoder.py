@@ -52,6 +52,8 @@ _SIGNATURES = {
     "qm_residual_norm_rows": (_I32, [C.POINTER(ResidualNorm), _I32, _I32, _P]),
     "qm_gated_norm_rows": (_I32, [C.POINTER(GatedNorm), _I32, _I32, _P]),
     "qm_decoder_linear_rows": (_I32, [C.POINTER(DecoderLinear), _I32, _I32, _I32, _P]),
+    "qm_decoder_linear_planes_bytes": (_I64, [C.POINTER(DecoderLinear), _I32, _I32]),
+    "qm_decoder_linear_rows_planes": (_I32, [C.POINTER(DecoderLinear), _I32, _I32, _P, _I64, _P]),
     "qm_chunk_attention_rows": (_I32, [C.POINTER(ChunkAttention), _I32, _P]),
     "qm_decay_attention_scratch_floats": (_I64, [_I32, _I32, _I32, _I32]),
     "qm_decay_attention_rows": (_I32, [C.POINTER(DecayAttention), _P]),

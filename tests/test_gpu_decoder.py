@@ -438,6 +438,31 @@ def test_down_projection_in_pieces(decoder, tmp_path, layer, width, rows):
     assert cases.error(logits, np.concatenate(scores)) < LIMIT[False]
 
 
+@pytest.mark.parametrize("layer,rows", [
+    (cases.general_delta(16, 64, 3072), 300),                                                                    # three pieces
+    (cases.parallel(cases.left(16, 4, 64, 64, 512, 64), cases.right(8, 64, 128, [0.95] * 8), 3072), 400),        # two, beside two; wide blocks in front
+])
+def test_linears_of_a_long_fp32_prompt(decoder, tmp_path, layer, rows):
+    """A prompt in one pass, whose linears have their inputs split beforehand and the down projection in pieces, against portions of nine rows at most, which
+    take the kernels of few rows: streams behind each layer and scores."""
+    cfg = cases.config(256, 1024, [layer, layer])
+    cases.write_model(str(tmp_path), cfg, cases.weights(cfg))
+    tokens = cases.tokens_of(cfg, rows)
+    places = sorted({0, 63, 64, 127, rows // 2, rows - 2, rows - 1})
+    whole = decoder.Decoder(str(tmp_path), rows, float32=True, max_rows=rows)
+    logits, streams = whole.step(whole.open(), tokens, places, streams=True)
+    portions = decoder.Decoder(str(tmp_path), rows, float32=True, max_rows=9)
+    s, parts, scores = portions.open(), [], []
+    for at in range(0, rows, 9):
+        got, stream = portions.step(s, tokens[at:at + 9], [p - at for p in places if at <= p < at + 9], streams=True)
+        parts.append(stream)
+        scores.append(got)
+    want = np.concatenate(parts, axis=1)
+    for i in range(2):
+        assert cases.error(streams[i], want[i]) < LIMIT[True], i
+    assert cases.error(logits, np.concatenate([x for x in scores if len(x)])) < LIMIT[True]
+
+
 def test_pieces_of_a_reduction_take_memory_only_where_one_is_cut(decoder, tmp_path):
     """A narrow model's output linears are never cut: its feed-forward takes the rows of its channels more than the same model without, and no planes for
     sums (64 MiB here)."""

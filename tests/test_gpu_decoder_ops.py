@@ -345,6 +345,71 @@ def test_many_fp32_rows_into_any_float_address(decoder, dev, pair, shift):
     assert float((got - want).abs().max()) <= 4e-6 * float(want[:, :n].abs().max())
 
 
+class ThroughPlanes:
+    """The decoder library with fp32 linears of more than eight rows by qm_decoder_linear_rows_planes."""
+
+    def __init__(self, decoder, dev):
+        self.decoder, self.dev = decoder, dev
+
+    def __getattr__(self, name):
+        return getattr(self.decoder, name)
+
+    def lib(self):
+        return self
+
+    def qm_decoder_linear_rows(self, linears, count, rows, f32, stream):
+        import torch
+        lib = self.decoder.lib()
+        if rows <= 8:
+            return lib.qm_decoder_linear_rows(linears, count, rows, f32, stream)
+        nbytes = lib.qm_decoder_linear_planes_bytes(linears, count, rows)
+        planes = torch.full((nbytes // 4 + 4,), float("nan"), device=self.dev)
+        assert lib.qm_decoder_linear_rows_planes(linears, count, rows, planes.data_ptr(), nbytes - 1, stream) == -4
+        rc = lib.qm_decoder_linear_rows_planes(linears, count, rows, planes.data_ptr(), nbytes, stream)
+        torch.cuda.synchronize()
+        assert bool(planes[nbytes // 4:].isnan().all())
+        return rc
+
+
+# (the last ones: grids that take blocks of 256 weight rows; a reduction of a single pair of steps; a last row tile of one row and of all but one)
+@pytest.mark.parametrize("rows,n,k,pair", SPLIT_LINEARS + [(600, 4112, 128, False), (577, 2176, 384, True), (64, 128, 128, False), (191, 256, 256, True)])
+def test_linears_of_fp32_rows_split_beforehand(decoder, dev, rows, n, k, pair):
+    """As the linears that split their inputs themselves: bounds against 64 bits, infinities, inputs down to the smallest normal numbers."""
+    planes = ThroughPlanes(decoder, dev)
+    test_linears_of_many_fp32_rows(planes, dev, rows, n, k, pair)
+    test_many_fp32_rows_meet_infinite_weights(planes, dev, rows, n, k, pair)
+    if not pair:
+        for exponent in (-122, -112, -108, -60):
+            test_many_fp32_rows_of_small_inputs(planes, dev, rows, n, k, exponent)
+
+
+@pytest.mark.parametrize("rows", [70, 300])
+def test_three_linears_of_fp32_rows_split_beforehand(decoder, dev, rows):
+    """Several linears in one launch, two of them of one input: the bits of one launch each, and errors no larger than the other kernel's."""
+    import torch
+    gen = torch.Generator(device=dev).manual_seed(rows)
+    shapes = [(1024, 1024, 0), (256, 1024, 0), (1040, 3072, 1)]
+    x = [torch.randn(rows, k, device=dev, generator=gen) for k in (1024, 3072)]
+    w = [(torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for n, k, _ in shapes]
+
+    def run(library, which):
+        outs = [torch.full((rows, shapes[i][0]), 7.0, device=dev) for i in which]
+        linears = (decoder.DecoderLinear * len(which))(*[
+            decoder.DecoderLinear(x=x[shapes[i][2]].data_ptr(), w=w[i].data_ptr(), out32=out.data_ptr(), ldx=shapes[i][1], ldo=shapes[i][0], n=shapes[i][0], k=shapes[i][1])
+            for i, out in zip(which, outs)])
+        assert library.lib().qm_decoder_linear_rows(linears, len(which), rows, 1, torch.cuda.current_stream().cuda_stream) == 0
+        torch.cuda.synchronize()
+        return outs
+
+    together, alone, plain_way = run(ThroughPlanes(decoder, dev), [0, 1, 2]), [run(ThroughPlanes(decoder, dev), [i])[0] for i in range(3)], run(decoder, [0, 1, 2])
+    for i in range(3):
+        assert torch.equal(together[i], alone[i])
+        want = x[shapes[i][2]].double() @ w[i].double().T
+        errors = [float((got.double() - want).norm() / want.norm()) for got in (together[i], plain_way[i])]
+        # (reductions of 1024 in four shares 7.5e-8, in two or here 7.9e-8; a draw of 70 x 256 sums scatters by a hundredth)
+        assert errors[0] <= 1.1 * errors[1], errors
+
+
 ATTENTION = [
     # heads, kv_heads, dim, vdim, chunk, rot_dims
     (4, 2, 16, 16, 50, 8), (3, 3, 24, 40, 37, 24), (5, 1, 36, 20, 64, 10), (6, 2, 64, 64, 200, 16), (2, 1, 136, 144, 300, 64), (8, 2, 128, 128, 256, 128),
