@@ -14,8 +14,8 @@
 // are transposed on their way out of LDS (ds_read_b64_tr_b16).  Bound: the chain of a tile in its wave (two products, the
 // softmax between them); flops 2 (dim + vdim) per visible key and query (the second product's doubled weights not counted).
 // (us, by blocks of eight waves that staged 128 keys for 64 rows through registers, values transposed on the way in, two barriers a
-// tile / so: 8 heads of 192 and 128 channels, 777 rows 25.9 / 15.4; 16 query heads on 8 of 128, 1024 rows 28.7 / 19.5, of 64, 1000 rows
-// 12.3 / 10.4; 32 heads of 128, 1500 rows 79 / 61; 4 on 2 of 250, 200 rows 24.9 / 12.0.)
+// tile / so: 8 heads of 192 and 128 channels, 777 rows 25.9 / 12.6; 16 query heads on 8 of 128, 1024 rows 28.7 / 14.7, of 64, 1000 rows
+// 12.3 / 8.6; 32 heads of 128, 1500 rows 79 / 47; 4 on 2 of 250, 200 rows 24.9 / 11.9.)
 #include <algorithm>
 #include <utility>
 
@@ -30,6 +30,7 @@ typedef uint32_t dec_u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kFlashKeys = 32;                 // keys per tile of a wave
 constexpr int kFlashRows = 32;                 // query rows per block
+constexpr float kFlashSlack = 8.0f;            // (powers of two)
 
 // A tile in LDS: rows of CHANNELS bf16, in 16-byte pieces; piece c of row r stands in slot c ^ key(r).
 // KEYS: the sixteen rows whose piece c a fragment read takes in a cycle stand in different banks; else the four rows of a
@@ -89,13 +90,16 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
     const int tid = threadIdx.x, lane = tid & 63;
     const int part = __builtin_amdgcn_readfirstlane(tid >> 6), half = lane >> 5;
     const int kv_head = static_cast<int>(blockIdx.x);
-    const int group = prm.heads / prm.kv_heads;
+    // (What divisions and a median leave in vector registers is the same in every lane, but a descriptor made of it would be taken lane by lane, in a loop
+    // around each request: 1024 rows of 16 query heads 19.5 us, so 15.8.)
+    auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int group = uniform(prm.heads / prm.kv_heads);
     const int total = prm.rows * group;
     const int row0 = static_cast<int>(gridDim.y - 1 - blockIdx.y) * kFlashRows;      // (late rows, which may see more keys, first)
     auto chunk_start = [&](int position) { return position - position % prm.chunk; };
     // what the block and this lane see: keys [.., ..]
-    const int first_position = prm.position + row0 / group, last_position = prm.position + min(row0 + kFlashRows - 1, total - 1) / group;
-    const int block_lo = chunk_start(first_position), block_lo_most = chunk_start(last_position);
+    const int first_position = uniform(prm.position + row0 / group), last_position = uniform(prm.position + min(row0 + kFlashRows - 1, total - 1) / group);
+    const int block_lo = uniform(chunk_start(first_position)), block_lo_most = uniform(chunk_start(last_position));
     const int query_row = min(row0 + (lane & 31), total - 1);
     const int local = query_row / group;
     const int position = prm.position + local;
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
     unsigned char* const v_lds = k_lds + Keys::kBytes;
     auto request = [&](auto tile_, const uint16_t* head_rows, int stride, const auto& off, unsigned char* to, int k0, int base) __attribute__((always_inline)) {
         using Tile = decltype(tile_);
-        const int keys = max(min(last_position + 1 - k0, kFlashKeys), 0), ahead = prm.ring - base;
+        const int keys = uniform(max(min(last_position + 1 - k0, kFlashKeys), 0)), ahead = prm.ring - base;
         auto rows_from = [&](const uint16_t* first, int count) {
             return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(first), 0, count * stride * 2, 0x00020000);
         };
@@ -161,7 +165,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
     // order a load goes to 32 rows, one lane a cycle: 24 KiB took a block 3000 cycles)
     auto query_lds = [&](int i) { return smem + i % PARTS * Shape::kWaveBytes + Keys::kBytes + i / PARTS * 1024; };
     {
-        const int first_local = row0 / group, locals = min(row0 + kFlashRows - 1, total - 1) / group - first_local + 1;
+        const int first_local = first_position - prm.position, locals = last_position - first_position + 1;
         const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
             const_cast<uint16_t*>(static_cast<const uint16_t*>(prm.q_rot) + static_cast<int64_t>(first_local) * prm.heads * prm.k_stride), 0,
             locals * prm.heads * prm.k_stride * 2, 0x00020000);
@@ -176,7 +180,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
         }
     }
     const int first_key = block_lo + kFlashKeys * part;
-    int slot = first_key % prm.ring;
+    int slot = uniform(first_key % prm.ring);
     request_keys(first_key, slot);
     flash_landed<Keys::kRequests>();
     asm volatile("s_barrier" ::: "memory");
@@ -209,7 +213,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
     for (int k0 = first_key; k0 <= last_position; k0 += PARTS * kFlashKeys) {
         const int next = k0 + PARTS * kFlashKeys;
         slot += PARTS * kFlashKeys;
-        if (slot >= prm.ring) slot %= prm.ring;
+        if (slot >= prm.ring) slot = uniform(slot % prm.ring);
         flash_landed<Values::kRequests>();
         dec_u32x4 key[kKb];
         flash_each<kKb>([&](auto kb) {
@@ -249,10 +253,19 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
         float largest = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
         largest = fmaxf(largest, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])), fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
         largest = xor32_max(largest) * factor_of_score;
-        const float before = m;
-        m = fmaxf(m, largest);
+        // (weights are taken of a largest score that may be up to kFlashSlack too low: it is raised, and the sums so far lowered, where one exceeds it by more:
+        // 1024 rows of 16 query heads 15.8 -> 14.7 us)
+        if (__any(largest > m + kFlashSlack)) {
+            const float before = m;
+            m = fmaxf(m, largest);
+            const float alpha = m == -INFINITY ? 1.0f : fast_exp2(before - m);
+            l *= alpha;
+#pragma unroll
+            for (int t = 0; t < kVt; ++t)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
+        }
         const float reference = m == -INFINITY ? 0.0f : m;         // (a row that has seen no key yet: all its weights are zero)
-        const float alpha = fast_exp2(before - reference);
 #pragma unroll
         for (int t = 0; t < kVt; ++t) flash_arrived(value[t]);
         request_values(next, slot);
@@ -262,13 +275,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
             p[r] = fast_exp2(fmaf(s[r], factor_of_score, -reference));
             sum += p[r];
         }
-        l = l * alpha + sum;
-        if (__any(alpha != 1.0f)) {
-#pragma unroll
-            for (int t = 0; t < kVt; ++t)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) o[t][r] *= alpha;
-        }
+        l += sum;
         dec_u32x4 high[2], low[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b) {
@@ -363,9 +370,9 @@ static int32_t flash_of(const ChunkAttentionParams& prm, unsigned blocks, hipStr
     return launch_status();
 }
 // Eight waves where the grid leaves CUs without a second block and a block walks long: half the steps, for a longer combination (us, four waves /
-// eight: 8 heads of 192 and 128, 128 rows 7.4 / 9.3, 777 rows 18.2 / 15.4; 300 rows of 16 on 8 heads of 128 behind 876 keys 20.5 / 16.6; 512 blocks,
-// 1024 rows 19.5 / 24.5).  A step of 128 keys costs 1.8 us, of 256 with eight waves 2.05, the longer combination 1.9: they meet at some 330 keys.
-constexpr int kFlashLongWalk = 384, kFlashCus = 256;
+// eight, 8 heads of 192 and 128: 100 rows behind 0, 500, 900, 1500 and 4000 keys 6.3 / 8.0, 10.2 / 10.6, 12.9 / 13.0, 17.4 / 15.9 and 34.8 / 28.4, 300 rows behind 1000
+// 15.9 / 14.9; 16 query heads on 8 of 128, 100 rows behind 900 11.4 / 11.7, 500 behind 1500 21.0 / 20.0, 850 rows, 432 blocks, 12.9 / 18.0).
+constexpr int kFlashLongWalk = 1200, kFlashCus = 256;
 template <int CK, int CV>
 static int32_t flash_as(const ChunkAttentionParams& prm, hipStream_t stream) {
     const int64_t blocks = (static_cast<int64_t>(prm.rows) * (prm.heads / prm.kv_heads) + kFlashRows - 1) / kFlashRows;

@@ -502,15 +502,25 @@ def test_chunk_attention_over_a_ring(decoder, dev, shape):
         close(case.run(decoder, dev, False, portions, ring=ring), want, False, tol16=3e-2)
 
 
-@pytest.mark.parametrize("shape", [(2, 2, 192, 128, 900, 64), (4, 2, 64, 64, 450, 16), (3, 1, 128, 120, 1000, 128), (2, 1, 32, 32, 385, 0), (2, 1, 250, 136, 500, 6)])
+@pytest.mark.parametrize("shape", [(2, 2, 192, 128, 1250, 64), (4, 2, 64, 64, 1300, 16), (3, 1, 128, 120, 1000, 128), (2, 1, 32, 32, 1201, 0), (2, 1, 250, 136, 1290, 6)])
 def test_chunk_attention_of_few_blocks_that_walk_far(decoder, dev, shape):
-    """Prompts behind 384 keys and more, whose few blocks take eight waves where these fit, on both sides of that line and with a ring that wraps
+    """Prompts behind 1200 keys and more, whose few blocks take eight waves where these fit, on both sides of that line and with a ring that wraps
     inside a wave's tile; tolerance and plain attention as above."""
-    case = AttentionCase(shape, 640, seed=13)
+    case = AttentionCase(shape, 1290, seed=13)
     want = case.want()
-    for portions in ([640], [383, 17, 240], [384, 33, 31, 192]):
-        for ring in (640, min(640, case.chunk + max(portions) - 1)):
+    for portions in ([1290], [1199, 17, 74], [1100, 33, 31, 126]):
+        for ring in (1290, min(1290, case.chunk + max(portions) - 1)):
             close(case.run(decoder, dev, False, portions, ring=ring), want, False, tol16=3e-2)
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.3, 3.0])
+def test_chunk_attention_of_other_scales(decoder, dev, scale):
+    """Scores that are all equal, whose order the factor turns round, and that run far apart, so that a row's largest rises again and again: against the
+    row kernel, which reads the same rounded queries and keys (at a scale of 3 their rounding alone moves a score by up to some 3 x 16 x 16 x 2^-8 = 3)."""
+    case = AttentionCase((4, 2, 64, 64, 200, 16), 230, seed=17)
+    case.scale = scale
+    got, want = case.run(decoder, dev, False, [230]), case.run(decoder, dev, False, [230], rows_only=True)
+    assert np.abs(got - want).max() <= 2e-2 * np.abs(want).max()
 
 
 def test_two_attention_kernels_agree(decoder, dev):
