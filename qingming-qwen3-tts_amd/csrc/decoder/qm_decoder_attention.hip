@@ -68,6 +68,80 @@ __global__ __launch_bounds__(kDecThreads) void rope_cache_kernel(ChunkAttentionP
     }
 }
 
+// The same for heads of whole pieces of eight channels whose halves turn in fours, projections of whole float4s: a thread holds four channels of both
+// halves of a head, asked for before the row's angles are known, and nothing but those passes through LDS.  Bound by memory: 16 + 8 heads of 128 and as
+// many values over 1024 rows, 25 MB, 11.2 -> 6.6 us (3.8 TB/s); 16 + 8 of 64 over 300 fp32 rows 7.0 -> 4.8, most of it the launch.  (Above, a value a
+// load, eight LDS reads of a stride of eight banks for a piece, a condition for each channel.)
+__device__ __forceinline__ float4 turned(float4 own, float4 other, float4 cosine, float4 sine, float sign) {
+    return make_float4(own.x * cosine.x + sign * other.x * sine.x, own.y * cosine.y + sign * other.y * sine.y,
+                       own.z * cosine.z + sign * other.z * sine.z, own.w * cosine.w + sign * other.w * sine.w);
+}
+template <class T>
+__global__ __launch_bounds__(kDecThreads) void rope_cache_vectors_kernel(ChunkAttentionParams prm) {
+    __shared__ __attribute__((aligned(16))) float sh_cos[kDecMaxHead / 2], sh_sin[kDecMaxHead / 2];
+    const int tid = threadIdx.x, row = static_cast<int>(blockIdx.x);
+    const int position = position_of(prm.position_dev, prm.position) + row;
+    const int half = prm.rot_dims >> 1, heads = prm.heads + prm.kv_heads;
+    const int64_t slot = position % prm.ring;
+    const float* proj = prm.proj + row * prm.ld_proj;
+    auto from = [&](int h) { return proj + (h < prm.heads ? h * prm.dim : prm.k_column + (h - prm.heads) * prm.dim); };
+    auto to = [&](int h) {
+        return h < prm.heads ? static_cast<T*>(prm.q_rot) + (static_cast<int64_t>(row) * prm.heads + h) * prm.dim
+                             : static_cast<T*>(prm.k_cache) + (static_cast<int64_t>(h - prm.heads) * prm.ring + slot) * prm.dim;
+    };
+    const int pairs = half >> 2, turning = heads * pairs, value_pieces = prm.vdim >> 2, values = prm.kv_heads * value_pieces;
+    constexpr int kHeld = 2;
+    float4 low[kHeld], high[kHeld], value[kHeld];
+    auto request = [&](int first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < kHeld; ++n) {
+            const int i = min(first + n * kDecThreads, turning - 1), h = i / pairs, c = (i - h * pairs) * 4;
+            low[n] = *reinterpret_cast<const float4*>(from(h) + c);
+            high[n] = *reinterpret_cast<const float4*>(from(h) + c + half);
+        }
+    };
+    auto request_values = [&](int first) __attribute__((always_inline)) {
+#pragma unroll
+        for (int n = 0; n < kHeld; ++n) value[n] = *reinterpret_cast<const float4*>(proj + prm.v_column + min(first + n * kDecThreads, values - 1) * 4);
+    };
+    if (turning > 0) request(tid);
+    request_values(tid);
+    for (int i = tid; i < half; i += kDecThreads) rotary(position, prm.frequency[i], sh_cos[i], sh_sin[i]);
+    for (int first = tid; first < values; first += kHeld * kDecThreads) {
+        if (first != tid) request_values(first);
+#pragma unroll
+        for (int n = 0; n < kHeld; ++n) {
+            const int i = first + n * kDecThreads, h = i / value_pieces;
+            if (i < values)
+                store4(static_cast<T*>(prm.v_cache) + (static_cast<int64_t>(h) * prm.ring + slot) * prm.vdim, i - h * value_pieces, value[n].x, value[n].y,
+                       value[n].z, value[n].w);
+        }
+    }
+    const int still = (prm.dim - prm.rot_dims) >> 2;
+    for (int i = tid; i < heads * still; i += kDecThreads) {
+        const int h = i / still, v = (prm.rot_dims >> 2) + i - h * still;
+        const float4 x = reinterpret_cast<const float4*>(from(h))[v];
+        store4(to(h), v, x.x, x.y, x.z, x.w);
+    }
+    __syncthreads();
+    for (int first = tid; first < turning; first += kHeld * kDecThreads) {
+        if (first != tid) request(first);
+#pragma unroll
+        for (int n = 0; n < kHeld; ++n) {
+            const int i = first + n * kDecThreads, h = i / pairs, c = (i - h * pairs) * 4;
+            if (i >= turning) break;
+            const float4 cosine = *reinterpret_cast<const float4*>(sh_cos + c), sine = *reinterpret_cast<const float4*>(sh_sin + c);
+            const float4 u = turned(low[n], high[n], cosine, sine, -1.0f), v = turned(high[n], low[n], cosine, sine, 1.0f);
+            store4(to(h), c >> 2, u.x, u.y, u.z, u.w);
+            store4(to(h), (c + half) >> 2, v.x, v.y, v.z, v.w);
+        }
+    }
+}
+static bool rope_in_vectors(const ChunkAttentionParams& p) {
+    return p.dim % 8 == 0 && p.vdim % 8 == 0 && p.rot_dims % 8 == 0 && p.ld_proj % 4 == 0 && p.k_column % 4 == 0 && p.v_column % 4 == 0 &&
+           reinterpret_cast<uintptr_t>(p.proj) % 16 == 0;
+}
+
 template <class T, int GQ, int VC>
 __global__ __launch_bounds__(kDecThreads) void chunk_attention_kernel(ChunkAttentionParams prm) {
     extern __shared__ __attribute__((aligned(16))) float lds[];
@@ -104,6 +178,10 @@ static int32_t rope_cache(const ChunkAttentionParams& prm, hipStream_t stream) {
     const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(rope_cache_kernel<T>), kDotLdsMost, raised);
     if (rc != QM_OK) return rc;
     if (lds > static_cast<size_t>(kDotLdsMost)) return QM_ERR_GEOMETRY;
+    if (rope_in_vectors(prm)) {
+        hipLaunchKernelGGL(rope_cache_vectors_kernel<T>, dim3(prm.rows), dim3(kDecThreads), 0, stream, prm);
+        return launch_status();
+    }
     hipLaunchKernelGGL(rope_cache_kernel<T>, dim3(prm.rows), dim3(kDecThreads), lds, stream, prm);
     return launch_status();
 }

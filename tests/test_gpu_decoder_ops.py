@@ -513,6 +513,46 @@ def test_chunk_attention_of_few_blocks_that_walk_far(decoder, dev, shape):
             close(case.run(decoder, dev, False, portions, ring=ring), want, False, tol16=3e-2)
 
 
+def rotated_alike(got, want, f32):
+    """The same products and sums, fused one way or the other: two roundings of the terms in fp32, one more of the result to bf16."""
+    got, want = get(got).astype(np.float64), get(want).astype(np.float64)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    keep = ~np.isnan(want)
+    assert np.all(np.abs(got - want)[keep] <= (0 if f32 else 2.0 ** -7) * np.abs(want[keep]) + 2.0 ** -21 * np.abs(want[keep]).max())
+
+
+@pytest.mark.parametrize("f32", [True, False])
+@pytest.mark.parametrize("heads,kv,dim,vdim,rot", [(4, 2, 64, 64, 64), (16, 8, 128, 128, 128), (3, 1, 24, 8, 16), (2, 1, 256, 136, 0), (36, 9, 64, 40, 8), (1, 1, 8, 8, 8),
+                                                   (64, 32, 64, 128, 64), (2, 2, 256, 256, 256)])
+def test_chunk_attention_rotates_in_vectors(decoder, dev, heads, kv, dim, vdim, rot, f32):
+    """Queries and keys that are turned four channels at a time, and values, as the kernel for any alignment leaves them: the same projections, begun a
+    float later in memory."""
+    import torch
+    rng = np.random.default_rng(heads + dim)
+    rows, position, ring = 19, 5, 21
+    k_at = heads * dim + 4
+    v_at = k_at + kv * dim + 4
+    ld = v_at + kv * vdim
+    flat = rng.standard_normal(rows * ld).astype(np.float32)
+    freq = put(700.0 ** (-2.0 * np.arange(max(1, rot // 2)) / max(1, rot)), dev)
+    left = []
+    for shift in (0, 1):
+        proj = torch.zeros(rows * ld + 4, device=dev)
+        proj[shift:shift + rows * ld] = put(flat, dev)
+        caches = [torch.full(s, float("nan"), device=dev, dtype=activation(f32)) for s in ((rows, heads, dim), (kv, ring, dim), (kv, ring, vdim))]
+        out = torch.zeros((rows, (heads * vdim + 127) // 128 * 128), device=dev, dtype=activation(f32))
+        ml, acc = torch.zeros(rows * heads * 2, device=dev), torch.zeros(rows * heads * vdim, device=dev)
+        op = decoder.ChunkAttention(proj=proj.data_ptr() + 4 * shift, frequency=freq.data_ptr(), q_rot=caches[0].data_ptr(), k_cache=caches[1].data_ptr(),
+                                    v_cache=caches[2].data_ptr(), out=out.data_ptr(), part=decoder.AttentionPartials(ml.data_ptr(), acc.data_ptr(), heads, vdim, 1, 3),
+                                    ld_proj=ld, ld_out=out.shape[1], position=position, rows=rows, heads=heads, kv_heads=kv, dim=dim, vdim=vdim, k_stride=dim,
+                                    v_stride=vdim, ring=ring, chunk=3, rot_dims=rot, k_column=k_at, v_column=v_at, scale=dim ** -0.5)
+        # (a chunk of three positions: the two behind it in the ring stay as they were)
+        assert decoder.lib().qm_chunk_attention_rows(C.byref(op), int(f32), torch.cuda.current_stream().cuda_stream) == 0
+        left.append(caches)
+    for got, want in zip(*left):
+        rotated_alike(got, want, f32)
+
+
 @pytest.mark.parametrize("scale", [0.0, -0.3, 3.0])
 def test_chunk_attention_of_other_scales(decoder, dev, scale):
     """Scores that are all equal, whose order the factor turns round, and that run far apart, so that a row's largest rises again and again: against the
