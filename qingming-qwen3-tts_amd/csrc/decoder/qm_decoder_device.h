@@ -87,9 +87,37 @@ __device__ __forceinline__ float4 weighted(float4 acc, float f, float4 y, float4
 struct NothingBehind {
     __device__ __forceinline__ void operator()() const {}
 };
-// MORE: the last term's further pieces are added to it.
-template <class T, int NV, bool EARLY = false, bool MORE = false, class Behind = NothingBehind>
-__device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int row, float* sh_red, T* h, bool write_x, Behind&& behind = Behind(),
+// The upper eight significant bits of x as a bf16 in the upper half of a word, and what is left of x.  (Infinities and NaNs
+// stay what they are, with nothing left.)
+__device__ __forceinline__ uint32_t take_upper(float& x) {
+    const uint32_t bits = __float_as_uint(x);
+    const bool finite = (bits & 0x7f800000U) != 0x7f800000U;
+    const uint32_t nan = (bits & 0x7fffffffU) > 0x7f800000U ? 0x00400000U : 0U;
+    const uint32_t upper = (bits | nan) & 0xffff0000U;
+    x = finite ? x - __uint_as_float(upper) : 0.0f;
+    return upper;
+}
+
+// A row of fp32 that is also left split into its three parts, `plane` elements apart.
+struct SplitRow {
+    float* whole;
+    uint16_t* parts;
+    int64_t plane;
+};
+__device__ __forceinline__ void store4(const SplitRow& to, int v, float a, float b, float c, float d) {
+    store4(to.whole, v, a, b, c, d);
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+        auto next = [&](float& x) { return part < 2 ? take_upper(x) : __float_as_uint(x); };
+        const uint32_t wa = next(a), wb = next(b), wc = next(c), wd = next(d);
+        reinterpret_cast<uint2*>(to.parts + part * to.plane)[v] =
+            make_uint2(__builtin_amdgcn_perm(wb, wa, 0x07060302U), __builtin_amdgcn_perm(wd, wc, 0x07060302U));
+    }
+}
+
+// MORE: the last term's further pieces are added to it.  H: where the norm's output goes.
+template <class T, int NV, bool EARLY = false, bool MORE = false, class Behind = NothingBehind, class H = T*>
+__device__ __forceinline__ void residual_norm_row(const ResidualParams& prm, int row, float* sh_red, H h, bool write_x, Behind&& behind = Behind(),
                                                   const MoreOfTerm& more = MoreOfTerm()) {
     const int tid = threadIdx.x;
     const int64_t src = prm.row_map ? prm.row_map[row] : row;

@@ -229,14 +229,18 @@ int32_t check_linears(const DecLinearParams& prm) {
     return QM_OK;
 }
 
+bool goes_through_planes(const DecLinearParams& prm, int f32, const ReductionCut* cut, const PlaneMemory& planes) {
+    return f32 && check_linears(prm) == QM_OK && prm.rows > 0 && split_pays(prm) && plane_elements(prm) <= planes.elements &&
+           planes_pay(prm, cut ? plane_pieces(prm) : 1);
+}
+
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut, const PlaneMemory& planes) {
     if (cut) cut->planes = 0;
     const int32_t checked = check_linears(prm);
     if (checked != QM_OK || prm.rows == 0) return checked;
     if (f32) {
         if (!split_pays(prm)) return streaming<float>(prm, stream);
-        return plane_elements(prm) <= planes.elements && planes_pay(prm, cut ? plane_pieces(prm) : 1) ? launch_plane_linears(prm, planes, stream, cut)
-                                                                                                      : launch_split_linears(prm, stream);
+        return goes_through_planes(prm, f32, cut, planes) ? launch_plane_linears(prm, planes, stream, cut) : launch_split_linears(prm, stream);
     }
     bool matrix = prm.rows >= kDecMatrixRows;
     if (matrix && prm.groups == 1 && prm.group[0].n <= kNarrowColumns && !prm.group[0].w_up)

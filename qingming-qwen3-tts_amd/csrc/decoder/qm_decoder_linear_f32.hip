@@ -29,17 +29,6 @@ struct SplitLinearParams {
     int first_tile[kDecGroups + 1];            // column tiles in front of each linear
 };
 
-// The upper eight significant bits of x as a bf16 in the upper half of a word, and what is left of x.  (Infinities and NaNs
-// stay what they are, with nothing left.)
-__device__ __forceinline__ uint32_t take_upper(float& x) {
-    const uint32_t bits = __float_as_uint(x);
-    const bool finite = (bits & 0x7f800000U) != 0x7f800000U;
-    const uint32_t nan = (bits & 0x7fffffffU) > 0x7f800000U ? 0x00400000U : 0U;
-    const uint32_t upper = (bits | nan) & 0xffff0000U;
-    x = finite ? x - __uint_as_float(upper) : 0.0f;
-    return upper;
-}
-
 // x . w in one chain.
 __device__ __forceinline__ float plain_dot(const float* x, const uint16_t* w, int k) {
     float sum = 0.0f;
@@ -730,9 +719,11 @@ int32_t launch_plane_linears(const DecLinearParams& given, const PlaneMemory& me
         split.first_block[i] = blocks;
         blocks += (split.input[i].k + kSplitColumns - 1) / kSplitColumns;
     }
-    hipLaunchKernelGGL(split_rows_kernel, dim3(blocks, given.rows), dim3(kSplitThreads), 0, stream, split);
-    const int32_t rc = launch_status();
-    if (rc != QM_OK) return rc;
+    if (!memory.split || split.inputs != 1) {
+        hipLaunchKernelGGL(split_rows_kernel, dim3(blocks, given.rows), dim3(kSplitThreads), 0, stream, split);
+        const int32_t rc = launch_status();
+        if (rc != QM_OK) return rc;
+    }
     // Wide blocks read less for their products; a step of theirs is as long as 1.75 of the others'.
     const int pieces = cut ? cut->planes + 1 : 1;
     return 7 * plane_steps(given, pieces, 256) < 4 * plane_steps(given, pieces, 128) ? launch_planes_as<256>(prm, stream) : launch_planes_as<128>(prm, stream);

@@ -57,7 +57,9 @@ struct MoreOfTerm {
     int64_t plane = 0;
     int planes = 0;
 };
-int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipStream_t stream, const MoreOfTerm& more = MoreOfTerm());
+// parts: h also goes there, split as PlaneMemory below has it (fp32 only).
+int32_t launch_residual_norm(const ResidualParams& prm, int rows, int f32, hipStream_t stream, const MoreOfTerm& more = MoreOfTerm(),
+                             uint16_t* parts = nullptr);
 int32_t launch_gated_norm(const GatedNormParams& prm, int rows, int f32, hipStream_t stream);
 // Many rows of bf16 go to the matrix cores (linears of one launch in one grid, a gate/up pair in its own), few rows and
 // fp32 to the streaming kernel.
@@ -76,12 +78,14 @@ int64_t reduction_cut_floats(const DecLinearParams& prm, int max_rows);
 struct PlaneMemory {
     uint16_t* at = nullptr;
     int64_t elements = 0;
+    bool split = false;              // the linears' one input is there, split
 };
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut = nullptr, const PlaneMemory& planes = PlaneMemory());
 int32_t launch_split_linears(const DecLinearParams& prm, hipStream_t stream);    // fp32 rows on the matrix cores
 // The same with inputs split beforehand: whether they can be, and whether that ends first (given that the matrix cores do), with the last reduction in so
 // many pieces; into how many it is cut; the launch, which cuts if `cut` has room.
 bool planes_fit(const DecLinearParams& prm);
+bool goes_through_planes(const DecLinearParams& prm, int f32, const ReductionCut* cut, const PlaneMemory& planes);    // (what launch_decoder_linears does)
 bool planes_pay(const DecLinearParams& prm, int pieces);
 int plane_pieces(const DecLinearParams& prm);
 int64_t plane_elements(const DecLinearParams& prm);

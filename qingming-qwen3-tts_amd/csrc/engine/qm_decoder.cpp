@@ -826,11 +826,13 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
         const LayerRun& run = d.runs[i];
         const DecoderLayer& w = d.layers[static_cast<size_t>(run.layer)];
         float* x_new = f32_of(d.x[next]);
-        op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, step_vec_of(d, run), f32_of(w.norm1), d.h.raw()), rows, d.f32, s, pending.more),
-                 "residual + norm");
+        const qm::DecLinearParams inputs = linears_in(d, w, rows);
+        const bool split = qm::goes_through_planes(inputs, d.f32, nullptr, planes);
+        op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, step_vec_of(d, run), f32_of(w.norm1), d.h.raw()), rows, d.f32, s, pending.more,
+                                          split ? planes.at : nullptr), "residual + norm");
         x = x_new;
         next ^= 1;
-        op_check(qm::launch_decoder_linears(linears_in(d, w, rows), d.f32, s, nullptr, planes), "input projections");
+        op_check(qm::launch_decoder_linears(inputs, d.f32, s, nullptr, {planes.at, planes.elements, split}), "input projections");
         if (w.config.mixer == MixerKind::AttentionBesideDecay) {
             op_check(qm::launch_chunk_attention(attention_of(d, w, d.states[i], sequence, rows, position), d.f32, s), "chunked attention");
             op_check(qm::launch_decay_attention(decay_of(d, w, d.states[i], sequence, rows, position), s), "decayed linear attention");
@@ -854,10 +856,13 @@ void run_layers(qm_decoder& d, int sequence, int rows, int position, const float
         pending.more = {cut.sums, cut.plane, cut.planes};
         if (sandwich(w) && w.config.ff) {
             x_new = f32_of(d.x[next]);
-            op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, nullptr, f32_of(w.norm2), d.h.raw()), rows, d.f32, s, pending.more), "residual + norm");
+            const qm::DecLinearParams feed = feed_in(d, w, rows);
+            const bool split = qm::goes_through_planes(feed, d.f32, nullptr, planes);
+            op_check(qm::launch_residual_norm(residual_of(d, pending, x, x_new, nullptr, f32_of(w.norm2), d.h.raw()), rows, d.f32, s, pending.more,
+                                              split ? planes.at : nullptr), "residual + norm");
             x = x_new;
             next ^= 1;
-            op_check(qm::launch_decoder_linears(feed_in(d, w, rows), d.f32, s, nullptr, planes), "feed-forward");
+            op_check(qm::launch_decoder_linears(feed, d.f32, s, nullptr, {planes.at, planes.elements, split}), "feed-forward");
             if (w.config.experts) op_check(qm::launch_experts(experts_of(d, w, rows, f32_of(d.y[0])), d.f32, s), "experts");
             else op_check(qm::launch_decoder_linears(feed_out(d, w, rows), d.f32, s, nullptr, planes), "feed-forward");
             pending = feed_term(d, w);

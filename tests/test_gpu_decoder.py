@@ -463,6 +463,25 @@ def test_linears_of_a_long_fp32_prompt(decoder, tmp_path, layer, rows):
     assert cases.error(logits, np.concatenate([x for x in scores if len(x)])) < LIMIT[True]
 
 
+@pytest.mark.parametrize("width,ff,rows", [(1100, 3072, 200), (2100, 2048, 300)])
+def test_norms_that_leave_their_rows_split(decoder, tmp_path, width, ff, rows):
+    """A prompt whose feed-forward takes the second norm's rows as that left them, rows of two and of four vectors a thread with zeros behind them, against
+    portions of nine rows, as above."""
+    cfg = cases.sandwich(200, width, [cases.retention(4, 64, 64, [0.9, 0.99, 0.5, 0.0], cases.dense(ff))], (11, 6, 7))
+    cases.write_model(str(tmp_path), cfg, cases.weights(cfg))
+    tokens, places = cases.tokens_of(cfg, rows), [0, 63, 64, rows - 1]
+    whole = decoder.Decoder(str(tmp_path), rows, float32=True, max_rows=rows)
+    logits, streams = whole.step(whole.open(), tokens, places, streams=True)
+    portions = decoder.Decoder(str(tmp_path), rows, float32=True, max_rows=9)
+    s, parts, scores = portions.open(), [], []
+    for at in range(0, rows, 9):
+        got, stream = portions.step(s, tokens[at:at + 9], [p - at for p in places if at <= p < at + 9], streams=True)
+        parts.append(stream)
+        scores.append(got)
+    assert cases.error(streams[0], np.concatenate(parts, axis=1)[0]) < LIMIT[True]
+    assert cases.error(logits, np.concatenate([x for x in scores if len(x)])) < LIMIT[True]
+
+
 def test_pieces_of_a_reduction_take_memory_only_where_one_is_cut(decoder, tmp_path):
     """A narrow model's output linears are never cut: its feed-forward takes the rows of its channels more than the same model without, and no planes for
     sums (64 MiB here)."""
