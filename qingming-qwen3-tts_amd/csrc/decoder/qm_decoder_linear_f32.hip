@@ -7,6 +7,8 @@
 // taken in two levels — 64 terms, the smallest parts first, then those sums one after the other — which keeps the chains of
 // roundings as short as a wave's lanes keep them in the dot-product kernel.
 //
+// Two kernels: few blocks or short reductions split the inputs in the blocks (as follows), a long prompt's are split once beforehand (the second part).
+//
 // A block of four waves takes 16 BT token rows and 64 TN weight rows (a gate/up pair: 32 TN channels, gate and up rows in the
 // same lanes), 64 k a step.  Weights are a wave's own and go straight to its registers, requested two steps ahead, a row's
 // 64 bytes per instruction; inputs are read once per block, split by the threads that fetched them and shared through two
@@ -655,9 +657,9 @@ bool planes_fit(const DecLinearParams& prm) {
 
 // Whether planes end first, and no further from 64 bits: where launch_split_linears would not share the reduction among groups of waves, or among two and
 // it is long, and where a long reduction can be cut.  The launch that splits is 4 to 7 us.  (us, split in the blocks / beforehand, relative error x 1e8: 5120 outputs
-// of 1024 inputs beside 3072 pairs, 100, 200, 300, 512 and 1024 rows 20.9 / 18.2, 34.3 / 27.9, 38.5 (14.4) / 31.3 (13.0), 57 / 48, 98 / 78; the three linears above, cut, 100
-// rows 22.0 (9.5) / 20.6 (9.2), 300 30.3 (11.1) / 25.0 (9.3), 512 46 / 33; 4096 of 4096, 129 rows 48.7 / 42.9, 300 rows 79.6 (15.8) / 48.7 (10.3); those that stay: 1024 of 1024,
-// 300 rows 9.8 (7.5) / 17.8 (7.9), 2048 of 2048, 300 rows 26.4 / 28.0, 2048 of 512, 1024 rows 16.7 / 18.4.)
+// of 1024 inputs beside 3072 pairs, 100, 200, 300, 512 and 1024 rows 20.8 (12.8) / 17.9 (12.7), 34.6 / 27.8, 38.5 (14.4) / 30.8 (12.7), 59 / 50, 108 / 83; the three linears
+// above, cut, 100 rows 21.5 (9.5) / 20.5 (8.6), 300 30.1 (11.1) / 25.0 (8.7), 512 46 / 40; 4096 of 4096, 300 rows 79.7 (15.8) / 49.2 (10.3); those that stay: 1024 of 1024, 300 rows
+// 9.7 (7.5) / 17.7 (7.9), 2048 of 2048, 300 rows 25.9 (9.6) / 27.5 (8.8), 2048 of 512, 1024 rows 16.4 (7.3) / 18.1 (7.3).)
 bool planes_pay(const DecLinearParams& prm, int pieces) {
     int longest = 0;
     bool pair = false;
