@@ -759,10 +759,10 @@ size_t rows_mfma_workspace_bytes(int rows, int columns, int reduction, bool dual
     return static_cast<size_t>(parts) * (dual ? 2 : 1) * rows * columns * sizeof(float);
 }
 
-// The longest chain of 64-k steps that a CU walks if the linears are dealt out in tiles of 64 rows and `bn` columns, a block per CU,
+// The longest chain of 64-k steps that a CU walks if the linears are dealt out in tiles of `bm` rows and `bn` columns, a block per CU,
 // long reductions first: the whole work over the CUs, in whole blocks of the shortest reduction.
-static int64_t rows_mfma_chain(const LinearRowsParams& prm, int bn) {
-    const int64_t row_tiles = (prm.rows + 63) / 64;
+static int64_t rows_mfma_chain(const LinearRowsParams& prm, int bm, int bn) {
+    const int64_t row_tiles = (prm.rows + bm - 1) / bm;
     int64_t total = 0, shortest = 0, longest = 0;
     for (int g = 0; g < prm.groups; ++g) {
         const int64_t columns = g == 0 ? prm.columns : prm.group_columns[g - 1];
@@ -782,19 +782,23 @@ int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t str
         if (prm.tile_rows == 64) return dual ? launch_rows_mfma_as<true, 64, 128, 64, 4>(prm, stream) : launch_rows_mfma_as<false, 64, 128, 64, 4>(prm, stream);
         return dual ? launch_rows_mfma_as<true, 128, 128, 64, 4>(prm, stream) : launch_rows_mfma_as<false, 128, 128, 64, 8>(prm, stream);
     }
-    // blocks of 64 token rows where blocks of 128 would leave CUs without one (one block per CU either way)
+    // Blocks of 64 token rows where blocks of 128 would leave CUs without one (one block per CU either way), unless some CU then walks its steps twice:
+    // a step of 128 rows takes 1.15 to 1.5 of one of 64.  (us, 64 / 128 rows, weights from memory, 64-row blocks of 264 to 400 on 256 CUs: pairs of 3072 of
+    // 1024, 700, 777 and 1000 tokens 20.0 / 15.6, 20.2 / 16.4, 21.0 / 17.1, of 3072 of 2048, 777 38.9 / 27.6, of 6144 of 2048, 400 41.2 / 28.8; 3072 columns of
+    // 2048, 777 21.6 / 15.6, 2048 of 2048, 1200 22.1 / 15.8, of 6144, 1200 78.6 / 50.2.  One round: pairs of 4608 of 1024, 400 12.2 / 17.8, of 6144 of 2048, 300 26.3 /
+    // 29.2; 2048 of 4096, 1000 22.4 / 28.1.)
     const int64_t row_tiles = (prm.rows + 127) / 128;
     int64_t columns = prm.columns;
     for (int g = 1; g < prm.groups; ++g) columns += prm.group_columns[g - 1];
     const int64_t blocks_128 = columns / kGmTile * row_tiles;
     if (prm.wide_tiles) return launch_rows_mfma_as<false, 128, 128, 64, 8>(prm, stream);
-    const bool small = blocks_128 < 200;
+    const bool small = blocks_128 < 200 && 2 * rows_mfma_chain(prm, 64, 128) < 3 * rows_mfma_chain(prm, 128, 128);
     // Measured (us, 64 x 128 / 64 x 64 tiles): 2048 columns of 6144 at 16 / 64 / 300 / 500 rows 24 / 28 / 27 / 28 against 17 / 20 / 20 / 22,
     // 4096 of 2048 at 128 / 200 / 300 rows 10.9 / 11.1 / 11.4 against 8.7 / 9.5 / 16.2, pairs of 6144 of 2048 at 64 / 128 / 200 rows
     // 26 / 25 / 25 against 18 / 18 / 30, three linears of 2048, 2048 and 6144 at 200 / 300 / 500 rows 36 / 41 / 44 against 25 / 36 / 52.
     // Smaller tiles with deeper rings where that shortens the grid's longest chain of steps or leaves it as it is: a step of a 64 x 64
     // tile takes about 0.7 of a 64 x 128 one's time (seven stages under way instead of three).
-    if (small && prm.reduction_parts == 1 && 7 * rows_mfma_chain(prm, 64) < 10 * rows_mfma_chain(prm, 128))
+    if (small && prm.reduction_parts == 1 && 7 * rows_mfma_chain(prm, 64, 64) < 10 * rows_mfma_chain(prm, 64, 128))
         return dual ? launch_rows_mfma_as<true, 64, 64, 64, 4>(prm, stream) : launch_rows_mfma_as<false, 64, 64, 64, 4>(prm, stream);
     if (dual) {
         // a gate/up pair whose grid of 128-column tiles is more than the CUs take at once and less than twice that: tiles

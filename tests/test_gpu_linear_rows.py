@@ -301,6 +301,15 @@ def test_matrix_core_tiles_against_64_bits(qm, dev, rows, cols, red, pair, rows_
     assert bool(((got - want).abs() <= bound + 1e-30).all()), float(((got - want).abs() / (bound + 1e-30)).max())
 
 
+@pytest.mark.parametrize("rows,cols,red", [(600, 3072, 256), (640, 3072, 256), (641, 3072, 256), (1024, 2048, 256), (1025, 2048, 256), (833, 2560, 256), (385, 4992, 256),
+                                           (897, 2304, 384), (65, 16384, 4096), (130, 10880, 4096), (130, 11008, 4096)])
+@pytest.mark.parametrize("pair", [False, True])
+@pytest.mark.parametrize("rows_kernel", [MATRIX], indirect=True)
+def test_grids_of_low_tiles_of_one_round_and_of_more(qm, dev, rows, cols, red, pair, rows_kernel):
+    """Tiles of 64 rows come to 240 to 288 blocks: up to 256 they are taken, above tiles of 128 rows are; tolerance as above."""
+    test_matrix_core_tiles_against_64_bits(qm, dev, rows, cols, red, pair, rows_kernel)
+
+
 @pytest.mark.parametrize("rows,cols,red", [(129, 5248, 128), (65, 5376, 256), (300, 5248, 128), (1024, 5888, 128)])
 @pytest.mark.parametrize("rows_kernel", [MATRIX], indirect=True)
 def test_more_than_forty_column_tiles_that_eight_does_not_divide(qm, dev, rows, cols, red, rows_kernel):
