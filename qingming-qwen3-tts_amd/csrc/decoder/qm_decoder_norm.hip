@@ -14,7 +14,7 @@ __global__ __launch_bounds__(kDecThreads) void residual_norm_kernel(ResidualPara
 }
 
 // The row of h also split into three parts, for linears that want their inputs so.  A launch of its own reads h again: 4.9 us for 300 rows of 1024,
-// where this kernel takes 6.2 us with the parts and without (a prompt of four layers 443 -> 435 us).
+// where this kernel takes 6.9 us with the parts and 6.2 without (a prompt of four layers 443 -> 435 us).
 template <int NV, bool MORE>
 __global__ __launch_bounds__(kDecThreads) void residual_norm_split_kernel(ResidualParams prm, MoreOfTerm more, uint16_t* parts, int64_t plane) {
     __shared__ float sh_red[16];
