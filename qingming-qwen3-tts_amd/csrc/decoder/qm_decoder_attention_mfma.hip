@@ -272,7 +272,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
         float p[16], sum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            p[r] = fast_exp2(fmaf(s[r], factor_of_score, -reference));
+            p[r] = fast_exp2(s[r] * factor_of_score - reference);       // (of rounded products, as the reference is: finite scores of any size come to kFlashSlack at most)
             sum += p[r];
         }
         l += sum;

@@ -563,6 +563,17 @@ def test_chunk_attention_of_other_scales(decoder, dev, scale):
     assert np.abs(got - want).max() <= 2e-2 * np.abs(want).max()
 
 
+@pytest.mark.parametrize("exponent", [20, 32, 48])
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 2, 64, 64), (2, 1, 192, 128)])
+def test_chunk_attention_of_large_scores(decoder, dev, heads, kv, dim, vdim, exponent):
+    """Finite scores around 2^exponent, of which an fp32 rounding alone comes to many powers of two: a row is the value of its largest score.  Queries and
+    keys are bf16 numbers that do not turn, and two scores of a row nearer to each other than fp32 tells apart do not occur."""
+    case = AttentionCase((heads, kv, dim, vdim, 200, 0), 230, seed=19)
+    case.proj = cases.bf16(case.proj)
+    case.proj[:, :case.v_at] *= 2.0 ** (exponent // 2)
+    close(case.run(decoder, dev, False, [230]), case.want(), False)
+
+
 def test_two_attention_kernels_agree(decoder, dev):
     case = AttentionCase((8, 4, 64, 64, 512, 32), 700, seed=9)
     a, b = case.run(decoder, dev, False, [700]), case.run(decoder, dev, False, [700], rows_only=True)
