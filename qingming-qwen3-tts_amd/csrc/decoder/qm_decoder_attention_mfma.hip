@@ -56,7 +56,7 @@ struct FlashShape {
     using Keys = FlashTile<CK, true>;
     using Values = FlashTile<CV, false>;
     static constexpr int kWaveBytes = Keys::kBytes + Values::kBytes;
-    // the parts' sums meet in LDS, and their largest scores and sums of weights
+    // the parts' sums meet in LDS, and the scores that their weights are taken of and sums of weights
     static constexpr int kSumBytes = PARTS * (CV / 32) * 4096, kCombineBytes = kSumBytes + PARTS * 2 * 32 * 4;
     static constexpr int kLds = PARTS * kWaveBytes > kCombineBytes ? PARTS * kWaveBytes : kCombineBytes;
 };
@@ -253,11 +253,12 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
         float largest = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
         largest = fmaxf(largest, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])), fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
         largest = xor32_max(largest) * factor_of_score;
-        // (weights are taken of a largest score that may be up to kFlashSlack too low: it is raised, and the sums so far lowered, where one exceeds it by more:
-        // 1024 rows of 16 query heads 15.8 -> 14.7 us)
-        if (__any(largest > m + kFlashSlack)) {
+        // (weights are taken of a score up to kFlashSlack above the largest so far: where one exceeds that, it is raised and the sums so far are lowered.
+        // 1024 rows of 16 query heads 15.8 -> 14.7 us.  Weights stay at one or below, so that no sum leaves the range that its result is in; what lies 2^118 below
+        // the largest is zero.)
+        if (__any(largest > m)) {
             const float before = m;
-            m = fmaxf(m, largest);
+            m = fmaxf(m, largest + kFlashSlack);
             const float alpha = m == -INFINITY ? 1.0f : fast_exp2(before - m);
             l *= alpha;
 #pragma unroll
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
         float p[16], sum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            p[r] = fast_exp2(s[r] * factor_of_score - reference);       // (of rounded products, as the reference is: finite scores of any size come to kFlashSlack at most)
+            p[r] = fast_exp2(s[r] * factor_of_score - reference);       // (of rounded products, as the reference is: finite scores of any size come to zero at most)
             sum += p[r];
         }
         l += sum;

@@ -574,6 +574,18 @@ def test_chunk_attention_of_large_scores(decoder, dev, heads, kv, dim, vdim, exp
     close(case.run(decoder, dev, False, [230]), case.want(), False)
 
 
+def test_chunk_attention_of_values_near_the_largest(decoder, dev):
+    """A key whose score is 2^6.5 times the others' in powers of two, with a value of 2^123, behind 128 keys that its wave has partly seen: weights are at
+    most one on the way, and so no sum leaves the range that the result is in."""
+    case = AttentionCase((1, 1, 32, 32, 300, 0), 300)
+    case.scale = 1.0
+    case.proj[:] = 0.0
+    case.proj[:, 0] = 1.0
+    case.proj[128, case.k_at] = 4.5
+    case.proj[128, case.v_at:case.v_at + 32] = 2.0 ** 123
+    close(case.run(decoder, dev, False, [300]), case.want(), False)
+
+
 def test_two_attention_kernels_agree(decoder, dev):
     case = AttentionCase((8, 4, 64, 64, 512, 32), 700, seed=9)
     a, b = case.run(decoder, dev, False, [700]), case.run(decoder, dev, False, [700], rows_only=True)
