@@ -208,11 +208,14 @@ int32_t launch_chunk_attention(const ChunkAttentionParams& prm, int f32, hipStre
     int32_t rc = check_attention(prm);
     if (rc != QM_OK || prm.rows == 0) return rc;
     if (!prm.q_rot) return QM_ERR_NULL;
+    // (positions that only the device knows belong to one-token steps)
+    const bool many = !prm.position_dev && !(prm.options & QM_ATTENTION_ROWS), matrix = many && !f32 && prm.rows >= kAttentionMatrixRows;
+    if (matrix) rc = check_chunk_attention_mfma(prm);              // (in front of the rotation, which writes the caches)
+    if (rc != QM_OK) return rc;
     rc = f32 ? rope_cache<float>(prm, stream) : rope_cache<uint16_t>(prm, stream);
     if (rc != QM_OK) return rc;
-    // (positions that only the device knows belong to one-token steps)
-    if (!f32 && prm.rows >= kAttentionMatrixRows && !prm.position_dev && !(prm.options & QM_ATTENTION_ROWS)) return launch_chunk_attention_mfma(prm, stream);
-    if (f32 && attention_f32_pays(prm) && !prm.position_dev && !(prm.options & QM_ATTENTION_ROWS)) return launch_chunk_attention_f32(prm, stream);
+    if (matrix) return launch_chunk_attention_mfma(prm, stream);
+    if (f32 && many && attention_f32_pays(prm)) return launch_chunk_attention_f32(prm, stream);
     return f32 ? attention_rows<float>(prm, stream) : attention_rows<uint16_t>(prm, stream);
 }
 

@@ -30,6 +30,8 @@ typedef uint32_t dec_u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kFlashKeys = 32;                 // keys per tile of a wave
 constexpr int kFlashRows = 32;                 // query rows per block
+constexpr int kFlashHigh = 65535;              // blocks of a key/value head in one layer of the grid
+constexpr int64_t kFlashMostRows = int64_t{64} * kFlashHigh;    // query rows of a key/value head (two layers)
 constexpr float kFlashSlack = 8.0f;            // (powers of two)
 
 // A tile in LDS: rows of CHANNELS bf16, in 16-byte pieces; piece c of row r stands in slot c ^ key(r).
@@ -95,7 +97,9 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
     auto uniform = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
     const int group = uniform(prm.heads / prm.kv_heads);
     const int total = prm.rows * group;
-    const int row0 = static_cast<int>(gridDim.y - 1 - blockIdx.y) * kFlashRows;      // (late rows, which may see more keys, first)
+    // late rows, which may see more keys, first
+    const int row0 = ((total + kFlashRows - 1) / kFlashRows - 1 - static_cast<int>(blockIdx.z * gridDim.y + blockIdx.y)) * kFlashRows;
+    if (row0 < 0) return;
     auto chunk_start = [&](int position) { return position - position % prm.chunk; };
     // what the block and this lane see: keys [.., ..]
     const int first_position = uniform(prm.position + row0 / group), last_position = uniform(prm.position + min(row0 + kFlashRows - 1, total - 1) / group);
@@ -367,7 +371,8 @@ static int32_t flash_of(const ChunkAttentionParams& prm, unsigned blocks, hipStr
     static std::atomic<bool> raised[kMaxDevices];
     const int32_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(chunk_attention_mfma_kernel<CK, CV, PARTS>), Shape::kLds, raised);
     if (rc != QM_OK) return rc;
-    hipLaunchKernelGGL((chunk_attention_mfma_kernel<CK, CV, PARTS>), dim3(prm.kv_heads, blocks), dim3(64 * PARTS), Shape::kLds, stream, prm);
+    const unsigned layers = (blocks + kFlashHigh - 1) / kFlashHigh;
+    hipLaunchKernelGGL((chunk_attention_mfma_kernel<CK, CV, PARTS>), dim3(prm.kv_heads, (blocks + layers - 1) / layers, layers), dim3(64 * PARTS), Shape::kLds, stream, prm);
     return launch_status();
 }
 // Eight waves where the grid leaves CUs without a second block and a block walks long: half the steps, for a longer combination (us, four waves /
@@ -377,15 +382,19 @@ constexpr int kFlashLongWalk = 1200, kFlashCus = 256;
 template <int CK, int CV>
 static int32_t flash_as(const ChunkAttentionParams& prm, hipStream_t stream) {
     const int64_t blocks = (static_cast<int64_t>(prm.rows) * (prm.heads / prm.kv_heads) + kFlashRows - 1) / kFlashRows;
-    if (blocks > 65535) return QM_ERR_GEOMETRY;
     if constexpr (FlashShape<CK, CV, 8>::kLds <= 160 * 1024)
         if (blocks * prm.kv_heads <= kFlashCus && std::min<int64_t>(prm.chunk, static_cast<int64_t>(prm.position) + prm.rows) >= kFlashLongWalk)
             return flash_of<CK, CV, 8>(prm, static_cast<unsigned>(blocks), stream);
     return flash_of<CK, CV, 4>(prm, static_cast<unsigned>(blocks), stream);
 }
 
-int32_t launch_chunk_attention_mfma(const ChunkAttentionParams& prm, hipStream_t stream) {
+int32_t check_chunk_attention_mfma(const ChunkAttentionParams& prm) {
     if (prm.ld_out % 4 || (reinterpret_cast<uintptr_t>(prm.out) & 7)) return QM_ERR_GEOMETRY;
+    return static_cast<int64_t>(prm.rows) * (prm.heads / prm.kv_heads) > kFlashMostRows ? QM_ERR_GEOMETRY : QM_OK;
+}
+int32_t launch_chunk_attention_mfma(const ChunkAttentionParams& prm, hipStream_t stream) {
+    const int32_t rc = check_chunk_attention_mfma(prm);
+    if (rc != QM_OK) return rc;
     const int c = prm.dim > prm.vdim ? prm.dim : prm.vdim;
     if (c <= 32) return flash_as<32, 32>(prm, stream);
     if (c <= 64) return flash_as<64, 64>(prm, stream);

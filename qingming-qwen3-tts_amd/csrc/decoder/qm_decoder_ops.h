@@ -94,6 +94,7 @@ int32_t launch_plane_linears(const DecLinearParams& prm, const PlaneMemory& plan
 int64_t steps_of_busiest_cu(int kinds, const int64_t* count, const int64_t* steps);
 // Rotation and cache write, then the attention.
 int32_t launch_chunk_attention(const ChunkAttentionParams& prm, int f32, hipStream_t stream);
+int32_t check_chunk_attention_mfma(const ChunkAttentionParams& prm);              // what it asks for beside check_attention
 int32_t launch_chunk_attention_mfma(const ChunkAttentionParams& prm, hipStream_t stream);
 bool attention_f32_pays(const ChunkAttentionParams& prm);                         // whether many fp32 rows go to the matrix cores
 int32_t launch_chunk_attention_f32(const ChunkAttentionParams& prm, hipStream_t stream);

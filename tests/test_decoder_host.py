@@ -144,6 +144,9 @@ def test_operators_check_their_arguments(decoder):
     for change in (dict(kv_heads=3), dict(k_stride=20), dict(rot_dims=18), dict(rot_dims=7), dict(chunk=0), dict(dim=300), dict(ring=0), dict(ld_out=60),
                    dict(chunk=200), dict(position=-1), dict(proj=None), dict(frequency=None)):
         assert lib.qm_chunk_attention_rows(C.byref(decoder.ChunkAttention(**{**attention, **change})), 0, None) < 0, change
+    # more query rows than the matrix cores' grid takes: refused in front of the rotation, which would write the caches (and needs a device)
+    many = dict(rows=65535, heads=65, kv_heads=1, dim=8, vdim=8, k_stride=8, v_stride=8, ld_out=640, part=decoder.AttentionPartials(at, at, 65, 8, 1, 128))
+    assert lib.qm_chunk_attention_rows(C.byref(decoder.ChunkAttention(**{**attention, **many})), 0, None) == -2
     decay = dict(proj=at, powers=at, state=at, out=at, ld_proj=100, rows=0, heads=2, dim=16, vdim=16)
     assert lib.qm_decay_attention_rows(C.byref(decoder.DecayAttention(**decay)), None) == 0
     for change in (dict(dim=257), dict(vdim=0), dict(heads=0), dict(rows=-1), dict(state=None)):

@@ -586,6 +586,32 @@ def test_chunk_attention_of_values_near_the_largest(decoder, dev):
     close(case.run(decoder, dev, False, [300]), case.want(), False)
 
 
+def test_chunk_attention_of_more_query_rows_than_a_grid_is_high(decoder, dev):
+    """32 800 rows of 64 query heads on one key head are 65 600 blocks of 32 query rows."""
+    import torch
+    rows, heads, dim, chunk = 32800, 64, 8, 32
+    gen = torch.Generator(device=dev).manual_seed(23)
+    ld = heads * dim + 2 * dim
+    proj = torch.randn(rows, ld, device=dev, generator=gen).bfloat16().float()
+    k, v, q_rot = [torch.full((n,), float("nan"), device=dev, dtype=torch.bfloat16) for n in (rows * dim, rows * dim, rows * heads * dim)]
+    out = torch.full((rows, heads * dim), 7.0, device=dev, dtype=torch.bfloat16)
+    ml, acc = torch.empty(rows * heads * 2, device=dev), torch.empty(rows * heads * dim, device=dev)
+    op = decoder.ChunkAttention(proj=proj.data_ptr(), q_rot=q_rot.data_ptr(), k_cache=k.data_ptr(), v_cache=v.data_ptr(), out=out.data_ptr(),
+                                part=decoder.AttentionPartials(ml.data_ptr(), acc.data_ptr(), heads, dim, 1, chunk), ld_proj=ld, ld_out=heads * dim, rows=rows,
+                                heads=heads, kv_heads=1, dim=dim, vdim=dim, k_stride=dim, v_stride=dim, ring=rows, chunk=chunk, k_column=heads * dim,
+                                v_column=heads * dim + dim, scale=dim ** -0.5)
+    assert decoder.lib().qm_chunk_attention_rows(C.byref(op), 0, torch.cuda.current_stream().cuda_stream) == 0
+    parts = proj.double().reshape(rows // chunk, chunk, ld)
+    q, keys, values = parts[..., :heads * dim].reshape(-1, chunk, heads, dim), parts[..., heads * dim:heads * dim + dim], parts[..., heads * dim + dim:]
+    hidden = torch.ones(chunk, chunk, device=dev, dtype=torch.bool).triu(1)
+    for first in range(0, rows // chunk, 205):
+        at = slice(first, first + 205)
+        s = (q[at].unsqueeze(3) * keys[at].unsqueeze(1).unsqueeze(1)).sum(-1) * dim ** -0.5                # [chunks][row][head][key]
+        p = s.permute(0, 2, 1, 3).masked_fill(hidden, -float("inf")).softmax(-1)                           # [chunks][head][row][key]
+        want = (p.unsqueeze(-1) * values[at].unsqueeze(1).unsqueeze(1)).sum(-2).permute(0, 2, 1, 3).reshape(-1, heads * dim)
+        close(get(out[first * chunk:first * chunk + want.shape[0]]), want.cpu().numpy(), False)
+
+
 def test_two_attention_kernels_agree(decoder, dev):
     case = AttentionCase((8, 4, 64, 64, 512, 32), 700, seed=9)
     a, b = case.run(decoder, dev, False, [700]), case.run(decoder, dev, False, [700], rows_only=True)
