@@ -317,11 +317,11 @@ struct SplitRowsParams {
 constexpr int kSplitThreads = 64, kSplitColumns = 8 * kSplitThreads;
 __global__ __launch_bounds__(kSplitThreads) void split_rows_kernel(SplitRowsParams prm) {
     request_arguments(prm);
-    const int row = static_cast<int>(blockIdx.y);
+    const int row = static_cast<int>(blockIdx.x);                  // (a grid is higher than 65535 in its first dimension only)
     int which = 0;
-    while (which + 1 < prm.inputs && static_cast<int>(blockIdx.x) >= prm.first_block[which + 1]) ++which;
+    while (which + 1 < prm.inputs && static_cast<int>(blockIdx.y) >= prm.first_block[which + 1]) ++which;
     const PlaneInput& in = prm.input[which];
-    const int c = (static_cast<int>(blockIdx.x) - prm.first_block[which]) * kSplitColumns + 8 * threadIdx.x;
+    const int c = (static_cast<int>(blockIdx.y) - prm.first_block[which]) * kSplitColumns + 8 * threadIdx.x;
     if (c >= in.k) return;
     const float* from = in.x + row * in.ldx + c;
     const float4 a = *reinterpret_cast<const float4*>(from), b = *reinterpret_cast<const float4*>(from + 4);
@@ -722,7 +722,7 @@ int32_t launch_plane_linears(const DecLinearParams& given, const PlaneMemory& me
         blocks += (split.input[i].k + kSplitColumns - 1) / kSplitColumns;
     }
     if (!memory.split || split.inputs != 1) {
-        hipLaunchKernelGGL(split_rows_kernel, dim3(blocks, given.rows), dim3(kSplitThreads), 0, stream, split);
+        hipLaunchKernelGGL(split_rows_kernel, dim3(given.rows, blocks), dim3(kSplitThreads), 0, stream, split);
         const int32_t rc = launch_status();
         if (rc != QM_OK) return rc;
     }

@@ -383,6 +383,18 @@ def test_linears_of_fp32_rows_split_beforehand(decoder, dev, rows, n, k, pair):
             test_many_fp32_rows_of_small_inputs(planes, dev, rows, n, k, exponent)
 
 
+def test_more_rows_than_a_grid_is_high_are_split_beforehand(decoder, dev):
+    import torch
+    rows, n, k = 65600, 16, 128
+    gen = torch.Generator(device=dev).manual_seed(29)
+    x, w = torch.randn(rows, k, device=dev, generator=gen), (torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16()
+    out = torch.full((rows, n), 7.0, device=dev)
+    linear = decoder.DecoderLinear(x=x.data_ptr(), w=w.data_ptr(), out32=out.data_ptr(), ldx=k, ldo=n, n=n, k=k)
+    assert ThroughPlanes(decoder, dev).qm_decoder_linear_rows(C.byref(linear), 1, rows, 1, torch.cuda.current_stream().cuda_stream) == 0
+    want = x.double() @ w.double().T
+    assert float((out.double() - want).abs().max()) <= 2e-6 * float(want.abs().max())
+
+
 @pytest.mark.parametrize("rows", [70, 300])
 def test_three_linears_of_fp32_rows_split_beforehand(decoder, dev, rows):
     """Several linears in one launch, two of them of one input: the bits of one launch each, and errors no larger than the other kernel's."""
