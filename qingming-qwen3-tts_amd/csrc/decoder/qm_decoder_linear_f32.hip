@@ -246,10 +246,11 @@ static int32_t launch_split_as(const DecLinearParams& linears, hipStream_t strea
     return launch_status();
 }
 
-int32_t launch_split_linears(const DecLinearParams& given, hipStream_t stream) {
-    DecLinearParams linears = given;
-    // long reductions first, so that none of them starts late
-    std::stable_sort(linears.group, linears.group + linears.groups, [](const DecLinearGroup& a, const DecLinearGroup& b) { return a.k > b.k; });
+// What launch_split_linears takes: 16 ROWS token rows and 64 WEIGHTS weight rows a block, the reduction shared among SHARES groups of waves.
+struct SplitShape {
+    int rows, weights, shares;
+};
+static SplitShape split_shape(const DecLinearParams& linears) {
     bool pair = false, quarters = true;
     int64_t tiles64 = 0, tiles128 = 0;                             // of 64 and of 128 weight rows
     for (int g = 0; g < linears.groups; ++g) {
@@ -266,14 +267,29 @@ int32_t launch_split_linears(const DecLinearParams& given, hipStream_t stream) {
     // <4,2,2> 18 / 19 / 20 / 38 / 56, <4,2,1> 24 / 24 / 25 / 36 / 55 us; 1024, 1024 and 3072 inputs to 1024 outputs each: <1,1,4> 19 / 19 / 27 / 52,
     // <2,1,4> 20 / 21 / 21 / 38 / 52, <2,1,2> 23 / 23 / 23 / 30 / 51, <2,1,1> 36 / 36 / 36 / 40 / 46, <4,2,1> 65 / 66 / 66 / 67 / 68 us.
     if (pair) {
-        if (linears.rows <= 16) return launch_split_as<1, 2, 2>(linears, stream);
-        if (tiles128 * rows32 <= 256) return launch_split_as<2, 2, 2>(linears, stream);
-        return tiles128 * rows64 <= 256 ? launch_split_as<4, 2, 2>(linears, stream) : launch_split_as<4, 2, 1>(linears, stream);
+        if (linears.rows <= 16) return {1, 2, 2};
+        if (tiles128 * rows32 <= 256) return {2, 2, 2};
+        return {4, 2, tiles128 * rows64 <= 256 ? 2 : 1};
     }
-    if (linears.rows <= 16) return quarters ? launch_split_as<1, 1, 4>(linears, stream) : launch_split_as<1, 1, 2>(linears, stream);
-    if (quarters && tiles64 * rows32 <= 256) return launch_split_as<2, 1, 4>(linears, stream);
-    if (tiles64 * rows32 <= 512) return launch_split_as<2, 1, 2>(linears, stream);
-    return tiles64 * rows32 <= 1024 ? launch_split_as<2, 1, 1>(linears, stream) : launch_split_as<4, 2, 1>(linears, stream);
+    if (linears.rows <= 16) return {1, 1, quarters ? 4 : 2};
+    if (quarters && tiles64 * rows32 <= 256) return {2, 1, 4};
+    if (tiles64 * rows32 <= 512) return {2, 1, 2};
+    return tiles64 * rows32 <= 1024 ? SplitShape{2, 1, 1} : SplitShape{4, 2, 1};
+}
+
+int32_t launch_split_linears(const DecLinearParams& given, hipStream_t stream) {
+    DecLinearParams linears = given;
+    // long reductions first, so that none of them starts late
+    std::stable_sort(linears.group, linears.group + linears.groups, [](const DecLinearGroup& a, const DecLinearGroup& b) { return a.k > b.k; });
+    const SplitShape shape = split_shape(linears);
+    if (shape.weights == 2) {
+        if (shape.rows == 1) return launch_split_as<1, 2, 2>(linears, stream);
+        if (shape.rows == 2) return launch_split_as<2, 2, 2>(linears, stream);
+        return shape.shares == 2 ? launch_split_as<4, 2, 2>(linears, stream) : launch_split_as<4, 2, 1>(linears, stream);
+    }
+    if (shape.rows == 1) return shape.shares == 4 ? launch_split_as<1, 1, 4>(linears, stream) : launch_split_as<1, 1, 2>(linears, stream);
+    if (shape.shares == 4) return launch_split_as<2, 1, 4>(linears, stream);
+    return shape.shares == 2 ? launch_split_as<2, 1, 2>(linears, stream) : launch_split_as<2, 1, 1>(linears, stream);
 }
 
 // ---- inputs split beforehand ---------------------------------------------------------------------------------------------
@@ -655,27 +671,30 @@ bool planes_fit(const DecLinearParams& prm) {
     return true;
 }
 
-// Whether planes end first, and no further from 64 bits: where launch_split_linears would not share the reduction among groups of waves, or among two and
-// it is long, and where a long reduction can be cut.  The launch that splits is 4 to 7 us.  (us, split in the blocks / beforehand, relative error x 1e8: 5120 outputs
-// of 1024 inputs beside 3072 pairs, 100, 200, 300, 512 and 1024 rows 20.8 (12.8) / 17.9 (12.7), 34.6 / 27.8, 38.5 (14.4) / 30.8 (12.7), 59 / 50, 108 / 83; the three linears
-// above, cut, 100 rows 21.5 (9.5) / 20.5 (8.6), 300 30.1 (11.1) / 25.0 (8.7), 512 46 / 40; 4096 of 4096, 300 rows 79.7 (15.8) / 49.2 (10.3); those that stay: 1024 of 1024, 300 rows
-// 9.7 (7.5) / 17.7 (7.9), 2048 of 2048, 300 rows 25.9 (9.6) / 27.5 (8.8), 2048 of 512, 1024 rows 16.4 (7.3) / 18.1 (7.3).)
+// Whether planes end first, and no linear of the launch comes out further from 64 bits.  A plane's sums are the same whatever the grid; those of
+// launch_split_linears are the closer the more groups of waves share a reduction, so that the shortest one decides.  (Relative error x 1e8, split in the blocks /
+// beforehand.  One walks it all: 1024 inputs 9.15 / 7.92, 512 7.34 / 7.33, 384 6.79 / 7.23; two groups: 1024 7.94 / 7.92, 896 7.69 / 7.83, pairs of them 13.0 / 12.9
+// and 12.7 / 12.8; four: 3072 9.63 / 9.57, 2560 9.15 / 9.21, 1024 7.54 / 7.92.)  The launch that splits is 4 to 7 us, so that planes end first where no groups share,
+// or where they do and the reduction is long and can be cut or has many blocks (us, split in the blocks / beforehand: 5120 outputs of 1024 inputs beside 3072 pairs,
+// 100, 200, 300, 512 and 1024 rows 20.8 / 17.9, 34.6 / 27.8, 38.5 / 30.8, 59 / 50, 108 / 83; the three linears above, the last one cut, 300 rows 30.1 / 25.0, 512
+// 46 / 40; 4096 of 4096, 300 rows 79.7 / 49.2; those that stay: 1024 of 1024, 300 rows 9.7 / 17.7, 2048 of 2048, 300 rows 25.9 / 27.5, 2048 of 512, 1024 rows 16.4 /
+// 18.1, and, for their shorter reductions, the three at 100 rows 21.5 / 20.5).
 bool planes_pay(const DecLinearParams& prm, int pieces) {
-    int longest = 0;
+    if (prm.rows <= 16 || !planes_fit(prm)) return false;
+    int longest = 0, shortest = prm.group[0].k;
+    int64_t tiles64 = 0;
     bool pair = false;
-    int64_t tiles64 = 0, tiles128 = 0;
     for (int g = 0; g < prm.groups; ++g) {
         const DecLinearGroup& d = prm.group[g];
         longest = std::max(longest, d.k);
-        pair = pair || d.w_up;
+        shortest = std::min(shortest, d.k);
         tiles64 += (d.n + 63) / 64;
-        tiles128 += d.w_up ? d.n / 64 : (d.n + 127) / 128;
+        pair = pair || d.w_up;
     }
-    if (!planes_fit(prm)) return false;
-    const int64_t rows32 = (prm.rows + 31) / 32;
-    if (prm.rows <= 16 || longest < 768) return false;
-    if (pair) return tiles128 * rows32 > 256;
-    return tiles64 * rows32 > (longest >= 3072 ? (pieces > 1 ? 0 : 256) : 512);
+    const SplitShape shape = split_shape(prm);
+    if (longest < 768 || shortest < (shape.shares == 4 ? 3072 : shape.shares == 2 ? 1024 : 512)) return false;
+    if (pair) return shape.rows == 4;
+    return shape.shares == 1 || (longest >= 3072 && (pieces > 1 || tiles64 * ((prm.rows + 31) / 32) > 256));
 }
 
 int32_t launch_plane_linears(const DecLinearParams& given, const PlaneMemory& memory, hipStream_t stream, ReductionCut* cut) {

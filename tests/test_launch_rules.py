@@ -95,6 +95,53 @@ int main() {
         assert lines[2300 * i + rows - 1][0] == pieces, (linears, rows)
 
 
+# fp32 linears as (columns, reduction), negative columns a pair's channels; rows; whether their inputs are split beforehand, and the last one's pieces (the first
+# three are the prompts of test_gpu_decoder.py's test_linears_of_a_long_fp32_prompt and test_norms_that_leave_their_rows_split)
+PLANES = [([(1024, 1024), (1024, 3072)], 300, True, 3), ([(1024, 1024), (1024, 1024), (1024, 3072)], 400, True, 2), ([(-3072, 1152)], 200, True, 1),
+          ([(-2048, 2176)], 300, True, 1), ([(5120, 1024), (-3072, 1024)], 100, True, 1), ([(4096, 4096)], 300, True, 1),
+          # four groups of waves share the reductions, and the shorter ones would lose by planes; then only long ones
+          ([(1024, 1024), (1024, 1024), (1024, 3072)], 160, False, 1), ([(1024, 1024), (1024, 1024), (1024, 3072)], 17, False, 1),
+          ([(2048, 2048), (2048, 6144)], 100, False, 1), ([(1024, 3072), (1024, 9216)], 100, True, 3),
+          # two groups: from 1024 inputs on
+          ([(1024, 512), (1024, 4096)], 300, False, 1), ([(1024, 1024), (1024, 4096)], 300, True, 2), ([(-1024, 896), (4096, 896)], 200, False, 1),
+          # none: from 512 on
+          ([(2048, 512), (2048, 4096)], 600, True, 1), ([(2048, 384), (2048, 4096)], 600, False, 1), ([(4096, 640)], 2000, False, 1),
+          # few rows; few outputs
+          ([(4096, 4096)], 16, False, 1), ([(16, 1024)], 300, False, 1)]
+
+
+def test_which_fp32_inputs_are_split_beforehand(tmp_path):
+    source = """
+#include <cstdio>
+#include "decoder/qm_decoder_ops.h"
+alignas(16) static char somewhere[16];
+static void of(std::initializer_list<std::pair<int, int>> linears, int rows) {
+    qm::DecLinearParams p = {};
+    p.rows = rows;
+    for (const auto& [n, k] : linears) {
+        qm::DecLinearGroup& g = p.group[p.groups++];
+        g.x = g.out = somewhere;
+        g.out32 = reinterpret_cast<float*>(somewhere);
+        g.w = reinterpret_cast<const uint16_t*>(somewhere);
+        g.w_up = n < 0 ? g.w : nullptr;
+        g.ldx = g.k = k;
+        g.ldo = g.n = n < 0 ? -n : n;
+    }
+    qm::ReductionCut cut = {};
+    const qm::PlaneMemory all = {reinterpret_cast<uint16_t*>(somewhere), qm::plane_elements(p)}, less = {all.at, all.elements - 1};
+    std::printf("%d %d %d %d %d\\n", qm::goes_through_planes(p, 1, &cut, all), qm::plane_pieces(p), qm::goes_through_planes(p, 1, &cut, less),
+                qm::goes_through_planes(p, 0, &cut, all), qm::goes_through_planes(p, 1, &cut, qm::PlaneMemory()));
+}
+int main() {
+"""
+    for linears, rows, _, _ in PLANES:
+        source += "    of({" + ", ".join("{%d, %d}" % l for l in linears) + "}, %d);\n" % rows
+    for line, (linears, rows, takes, pieces) in zip(run(tmp_path, source + "}", "qm_decoder"), PLANES):
+        got = list(map(int, line.split()))
+        assert got[0] == takes and got[2:] == [0, 0, 0], (linears, rows, got)
+        assert not takes or got[1] == pieces, (linears, rows, got)
+
+
 def test_a_norm_behind_a_linear_takes_no_cut_away(qm):
     """Whatever the width, a reduction that is cut by itself is cut with the norm behind as well, and the workspace holds its pieces."""
     L, cut, more = qm.lib(), 0, 0
