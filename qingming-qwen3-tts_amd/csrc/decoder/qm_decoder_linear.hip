@@ -229,9 +229,30 @@ int32_t check_linears(const DecLinearParams& prm) {
     return QM_OK;
 }
 
+static bool planes_end_first(const DecLinearParams& prm, bool cut) {
+    return split_pays(prm) && (planes_pay(prm, 1) || (cut && planes_pay(prm, 2) && plane_pieces(prm) > 1));
+}
 bool goes_through_planes(const DecLinearParams& prm, int f32, const ReductionCut* cut, const PlaneMemory& planes) {
-    return f32 && check_linears(prm) == QM_OK && prm.rows > 0 && split_pays(prm) && plane_elements(prm) <= planes.elements &&
-           planes_pay(prm, cut ? plane_pieces(prm) : 1);
+    return f32 && check_linears(prm) == QM_OK && prm.rows > 0 && plane_elements(prm) <= planes.elements && planes_end_first(prm, cut != nullptr);
+}
+int64_t plane_elements_up_to(const DecLinearParams& prm, int max_rows, bool cut) {
+    DecLinearParams some = prm;
+    for (some.rows = max_rows; some.rows > 0; --some.rows)                     // (more rows take more)
+        if (planes_end_first(some, cut)) return plane_elements(some);
+    return 0;
+}
+int64_t plane_cut_floats(const DecLinearParams& prm, int max_rows) {
+    int64_t most = 0;
+    DecLinearParams tile = prm;
+    for (int row = 0; row < max_rows; row += kPlaneRows) {                     // (of a row tile's rows the first has the most pieces, the last the most rows)
+        const int last = std::min(row + kPlaneRows, max_rows);
+        tile.rows = row + 1;
+        const int more = plane_pieces(tile) - 1;
+        const int64_t floats = static_cast<int64_t>(more) * last * prm.group[prm.groups - 1].n;
+        for (; floats > most && tile.rows <= last; ++tile.rows)
+            if (planes_end_first(tile, true)) most = floats;
+    }
+    return most;
 }
 
 int32_t launch_decoder_linears(const DecLinearParams& prm, int f32, hipStream_t stream, ReductionCut* cut, const PlaneMemory& planes) {

@@ -302,7 +302,6 @@ int32_t launch_split_linears(const DecLinearParams& given, hipStream_t stream) {
 // a wave takes 64 for all token rows, of 128 for 32 of them; a step's 56 KiB (40) are as long in the address path (46 bytes a cycle) as its matrix
 // instructions (1536 cycles, 768).  The parts below the first gather in sums of their own, whose roundings lie 2^-8 lower, and the first's in two
 // levels of 128 terms, added while the last of the lower parts are multiplied.  A step's one barrier stands in front of its last k block.
-constexpr int kPlaneRows = 64;
 constexpr int kPlaneLinears = kDecGroups + kMorePlanes;
 
 struct PlaneLinear {

@@ -74,6 +74,7 @@ struct ReductionCut {
 // Into how many pieces that is, and the most floats that they take with any number of rows up to max_rows.
 int reduction_pieces(const DecLinearParams& prm);
 int64_t reduction_cut_floats(const DecLinearParams& prm, int max_rows);
+constexpr int kPlaneRows = 64;            // token rows of a block whose inputs are split beforehand
 // Memory in which fp32 inputs are split into their three parts beforehand: three times rows x k elements for each of the linears' different inputs.
 struct PlaneMemory {
     uint16_t* at = nullptr;
@@ -89,6 +90,9 @@ bool goes_through_planes(const DecLinearParams& prm, int f32, const ReductionCut
 bool planes_pay(const DecLinearParams& prm, int pieces);
 int plane_pieces(const DecLinearParams& prm);
 int64_t plane_elements(const DecLinearParams& prm);
+// What they take at most with any number of rows up to max_rows: elements of split inputs, and floats of pieces (given that memory).
+int64_t plane_elements_up_to(const DecLinearParams& prm, int max_rows, bool cut);
+int64_t plane_cut_floats(const DecLinearParams& prm, int max_rows);
 int32_t launch_plane_linears(const DecLinearParams& prm, const PlaneMemory& planes, hipStream_t stream, ReductionCut* cut);
 // Steps that the busiest of 256 CUs walks when `kinds` kinds of blocks, `count` of `steps` steps each, are dealt out one to a CU, long ones first.
 int64_t steps_of_busiest_cu(int kinds, const int64_t* count, const int64_t* steps);

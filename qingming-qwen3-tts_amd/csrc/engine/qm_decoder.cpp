@@ -489,7 +489,7 @@ std::unique_ptr<qm_decoder> create_decoder(const std::string& dir, int f32, int 
     d->gated = zeros(rows * gated * item);
     for (DeviceBuffer& y : d->y) y = zeros(rows * d->width_p * 4);
     if (const int64_t more = cut_floats(*d)) d->y_more = zeros(static_cast<size_t>(more) * 4);
-    if (f32) d->planes = zeros(static_cast<size_t>(plane_elements(*d)) * 2);
+    if (const int64_t elements = f32 ? plane_elements(*d) : 0) d->planes = zeros(static_cast<size_t>(elements) * 2);
     d->q_rot = zeros(rows * q_rot * item);
     d->raw = zeros(rows * raw * 4);
     d->ml = zeros(ml * 4);
@@ -777,8 +777,7 @@ int64_t cut_floats(const qm_decoder& d) {
     for (const DecoderLayer& w : d.layers) {
         Pending none;
         const qm::DecLinearParams outputs = linears_out(d, w, d.max_rows, none);
-        if (!d.f32) most = std::max(most, qm::reduction_cut_floats(outputs, d.max_rows));
-        else if (outputs.groups > 1) most = static_cast<int64_t>(qm::kMorePlanes) * d.max_rows * d.width_p;
+        most = std::max(most, d.f32 ? qm::plane_cut_floats(outputs, d.max_rows) : qm::reduction_cut_floats(outputs, d.max_rows));
     }
     return most;
 }
@@ -799,12 +798,14 @@ qm::DecLinearParams feed_out(const qm_decoder& d, const DecoderLayer& w, int row
 // Elements for any layer's fp32 inputs, split.
 int64_t plane_elements(const qm_decoder& d) {
     int64_t most = 0;
+    auto take = [&](const qm::DecLinearParams& linears, bool cut) { most = std::max(most, qm::plane_elements_up_to(linears, d.max_rows, cut)); };
     for (const DecoderLayer& w : d.layers) {
         Pending none;
-        most = std::max({most, qm::plane_elements(linears_in(d, w, d.max_rows)), qm::plane_elements(linears_out(d, w, d.max_rows, none))});
+        take(linears_in(d, w, d.max_rows), false);
+        take(linears_out(d, w, d.max_rows, none), d.y_more.raw() != nullptr);
         if (sandwich(w) && w.config.ff) {
-            most = std::max(most, qm::plane_elements(feed_in(d, w, d.max_rows)));
-            if (!w.config.experts) most = std::max(most, qm::plane_elements(feed_out(d, w, d.max_rows)));
+            take(feed_in(d, w, d.max_rows), false);
+            if (!w.config.experts) take(feed_out(d, w, d.max_rows), false);
         }
     }
     return most;

@@ -482,9 +482,10 @@ def test_norms_that_leave_their_rows_split(decoder, tmp_path, width, ff, rows):
     assert cases.error(logits, np.concatenate([x for x in scores if len(x)])) < LIMIT[True]
 
 
-def test_pieces_of_a_reduction_take_memory_only_where_one_is_cut(decoder, tmp_path):
-    """A narrow model's output linears are never cut: its feed-forward takes the rows of its channels more than the same model without, and no planes for
-    sums (64 MiB here)."""
+@pytest.mark.parametrize("float32", [False, True])
+def test_pieces_of_a_reduction_take_memory_only_where_one_is_cut(decoder, tmp_path, float32):
+    """A narrow model's output linears are never cut, nor are its inputs split in the 32-bit mode: its feed-forward takes the rows of its channels more than
+    the same model without, and no planes for sums (64 MiB here) or parts (144 MiB)."""
     import torch
     rows, used = 65536, []
     for i, ff in enumerate((None, None, 300)):                 # (the first loads the library's code as well)
@@ -494,10 +495,10 @@ def test_pieces_of_a_reduction_take_memory_only_where_one_is_cut(decoder, tmp_pa
         cases.write_model(str(where), cfg, cases.weights(cfg))
         torch.cuda.synchronize()
         before = torch.cuda.mem_get_info()[0]
-        engine = decoder.Decoder(str(where), rows, max_rows=rows)
+        engine = decoder.Decoder(str(where), rows, float32=float32, max_rows=rows)
         used.append(before - torch.cuda.mem_get_info()[0])
         engine.close_model()
-    channels = rows * 384 * 2                                  # 300 padded to 384, bf16
+    channels = rows * 384 * (4 if float32 else 2)              # 300 padded to 384
     assert used[2] - used[1] < channels + (16 << 20), used     # (allocations come in pieces of two MiB)
 
 

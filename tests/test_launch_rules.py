@@ -110,12 +110,12 @@ PLANES = [([(1024, 1024), (1024, 3072)], 300, True, 3), ([(1024, 1024), (1024, 1
           ([(4096, 4096)], 16, False, 1), ([(16, 1024)], 300, False, 1)]
 
 
-def test_which_fp32_inputs_are_split_beforehand(tmp_path):
-    source = """
+# fp32 linears of `rows` rows, at one address where only their sizes matter
+OF_SIZES = """
 #include <cstdio>
 #include "decoder/qm_decoder_ops.h"
 alignas(16) static char somewhere[16];
-static void of(std::initializer_list<std::pair<int, int>> linears, int rows) {
+static qm::DecLinearParams of(std::initializer_list<std::pair<int, int>> linears, int rows) {
     qm::DecLinearParams p = {};
     p.rows = rows;
     for (const auto& [n, k] : linears) {
@@ -127,19 +127,64 @@ static void of(std::initializer_list<std::pair<int, int>> linears, int rows) {
         g.ldx = g.k = k;
         g.ldo = g.n = n < 0 ? -n : n;
     }
+    return p;
+}
+static bool goes(const qm::DecLinearParams& p, int f32, int64_t elements) {
     qm::ReductionCut cut = {};
-    const qm::PlaneMemory all = {reinterpret_cast<uint16_t*>(somewhere), qm::plane_elements(p)}, less = {all.at, all.elements - 1};
-    std::printf("%d %d %d %d %d\\n", qm::goes_through_planes(p, 1, &cut, all), qm::plane_pieces(p), qm::goes_through_planes(p, 1, &cut, less),
-                qm::goes_through_planes(p, 0, &cut, all), qm::goes_through_planes(p, 1, &cut, qm::PlaneMemory()));
+    return qm::goes_through_planes(p, f32, &cut, {reinterpret_cast<uint16_t*>(somewhere), elements});
 }
 int main() {
 """
+
+
+def sizes(linears):
+    return "{" + ", ".join("{%d, %d}" % l for l in linears) + "}"
+
+
+def test_which_fp32_inputs_are_split_beforehand(tmp_path):
+    source = OF_SIZES
     for linears, rows, _, _ in PLANES:
-        source += "    of({" + ", ".join("{%d, %d}" % l for l in linears) + "}, %d);\n" % rows
-    for line, (linears, rows, takes, pieces) in zip(run(tmp_path, source + "}", "qm_decoder"), PLANES):
+        source += """
+    {
+        const qm::DecLinearParams p = of(%s, %d);
+        const int64_t all = qm::plane_elements(p);
+        std::printf("%%d %%d %%d %%d\\n", goes(p, 1, all), qm::plane_pieces(p), goes(p, 1, all - 1), goes(p, 0, all));
+    }""" % (sizes(linears), rows)
+    lines = run(tmp_path, source + "}", "qm_decoder")
+    assert len(lines) == len(PLANES)
+    for line, (linears, rows, takes, pieces) in zip(lines, PLANES):
         got = list(map(int, line.split()))
-        assert got[0] == takes and got[2:] == [0, 0, 0], (linears, rows, got)
+        assert got[0] == takes and got[2:] == [0, 0], (linears, rows, got)
         assert not takes or got[1] == pieces, (linears, rows, got)
+
+
+def test_memory_for_fp32_inputs_that_are_split_beforehand(tmp_path):
+    """What a prompt of up to so many rows takes of it: as much as the largest that goes that way, and for pieces of a reduction at most a row tile more;
+    nothing where none goes."""
+    shapes = [linears for linears, _, _, _ in PLANES] + [[(128, 128), (128, 128), (128, 384)], [(2048, 640), (2048, 640), (2048, 640)]]
+    most = 700
+    source = OF_SIZES
+    for linears in shapes:
+        text = sizes(linears)
+        source += f"""
+    for (int rows = 1; rows <= {most}; ++rows) {{
+        const qm::DecLinearParams p = of({text}, rows);
+        const bool takes = goes(p, 1, int64_t{{1}} << 40);
+        std::printf("%lld %lld %lld %lld\\n", takes ? (long long)qm::plane_elements(p) : 0, (long long)qm::plane_elements_up_to(p, rows, true),
+                    takes ? (qm::plane_pieces(p) - 1ll) * rows * p.group[p.groups - 1].n : 0, (long long)qm::plane_cut_floats(p, rows));
+    }}"""
+    lines = [tuple(map(int, line.split())) for line in run(tmp_path, source + "}", "qm_decoder")]
+    assert len(lines) == most * len(shapes)
+    used = 0
+    for i, linears in enumerate(shapes):
+        elements = floats = 0
+        for rows, (needs, has, cut_needs, cut_has) in enumerate(lines[most * i:most * (i + 1)], 1):
+            elements, floats = max(elements, needs), max(floats, cut_needs)
+            assert has == elements, (linears, rows)
+            assert floats <= cut_has <= 2 * (rows + 63) * abs(linears[-1][0]), (linears, rows)
+        used += elements > 0
+        assert (cut_has > 0) == (floats > 0), linears
+    assert 8 <= used <= len(shapes) - 4 and lines[-1] == (0, 0, 0, 0) and lines[-1 - most] == (0, 0, 0, 0)
 
 
 def test_a_norm_behind_a_linear_takes_no_cut_away(qm):
