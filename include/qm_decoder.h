@@ -78,7 +78,8 @@ typedef struct {
 } qm_decoder_linear;
 int32_t qm_decoder_linear_rows(const qm_decoder_linear* linears, int32_t count, int32_t rows, int32_t f32, void* hip_stream);
 /* The same in fp32 with memory (16-byte aligned) for three bf16 parts of every input, which a launch of its own makes before the linears: for hundreds
- * of rows and thousands of outputs.  Outputs are 16-byte aligned, ldo a multiple of 4. */
+ * of rows and thousands of outputs.  Inputs, weights and outputs are 16-byte aligned, ldo is a multiple of 4, k is at most 2^20 and rows * k at most 2^28;
+ * other linears take no bytes and QM_ERR_GEOMETRY. */
 int64_t qm_decoder_linear_planes_bytes(const qm_decoder_linear* linears, int32_t count, int32_t rows);
 int32_t qm_decoder_linear_rows_planes(const qm_decoder_linear* linears, int32_t count, int32_t rows, void* planes, int64_t planes_bytes, void* hip_stream);
 

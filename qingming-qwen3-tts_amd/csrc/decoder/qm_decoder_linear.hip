@@ -219,12 +219,16 @@ int64_t reduction_cut_floats(const DecLinearParams& prm, int max_rows) {
     return most;
 }
 
+static bool has_sizes(const DecLinearGroup& d) {
+    return d.n > 0 && d.k > 0 && d.n % (d.w_up ? 128 : 16) == 0 && d.k % 128 == 0 && d.ldx >= d.k && d.ldo >= d.n && d.ldx % 8 == 0 && d.ldo % 4 == 0;
+}
+bool linears_have_sizes(const DecLinearParams& prm) { return std::all_of(prm.group, prm.group + prm.groups, has_sizes); }
 int32_t check_linears(const DecLinearParams& prm) {
     if (prm.rows < 0 || prm.groups < 1 || prm.groups > kDecGroups) return QM_ERR_ARGUMENT;
     for (int g = 0; g < prm.groups; ++g) {
         const DecLinearGroup& d = prm.group[g];
         if (!d.x || !d.w || (d.w_up ? !d.out : !d.out32)) return QM_ERR_NULL;
-        if (d.n <= 0 || d.k <= 0 || d.n % (d.w_up ? 128 : 16) || d.k % 128 || d.ldx < d.k || d.ldo < d.n || d.ldx % 8 || d.ldo % 4) return QM_ERR_GEOMETRY;
+        if (!has_sizes(d)) return QM_ERR_GEOMETRY;
     }
     return QM_OK;
 }

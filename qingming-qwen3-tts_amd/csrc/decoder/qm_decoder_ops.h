@@ -48,6 +48,7 @@ inline int row_vectors(int64_t ld) { return ld <= 1024 ? 1 : ld <= 2048 ? 2 : ld
 // Whether the kernels take these arguments.
 int32_t check_residual(const ResidualParams& prm);
 int32_t check_linears(const DecLinearParams& prm);
+bool linears_have_sizes(const DecLinearParams& prm);            // (of that, what no pointer is needed for)
 int32_t check_attention(const ChunkAttentionParams& prm);
 int32_t check_decay_attention(const DecayAttentionParams& prm);
 // The last term in pieces: `planes` more of them, `plane` floats apart, laid out as the term's own and added to it in order.

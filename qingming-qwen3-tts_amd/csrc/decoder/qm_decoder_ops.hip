@@ -23,7 +23,7 @@ extern "C" int32_t qm_decoder_linear_rows(const qm_decoder_linear* linears, int3
 }
 extern "C" int64_t qm_decoder_linear_planes_bytes(const qm_decoder_linear* linears, int32_t count, int32_t rows) {
     qm::DecLinearParams prm = {};
-    return linears_of(linears, count, rows, prm) && rows > 0 ? 2 * qm::plane_elements(prm) : 0;
+    return linears_of(linears, count, rows, prm) && rows > 0 && qm::linears_have_sizes(prm) && qm::planes_fit(prm) ? 2 * qm::plane_elements(prm) : 0;
 }
 extern "C" int32_t qm_decoder_linear_rows_planes(const qm_decoder_linear* linears, int32_t count, int32_t rows, void* planes, int64_t planes_bytes, void* hip_stream) {
     qm::DecLinearParams prm = {};

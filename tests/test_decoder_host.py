@@ -137,6 +137,19 @@ def test_operators_check_their_arguments(decoder):
         setattr(other, field, bad)
         assert lib.qm_decoder_linear_rows(C.byref(other), 1, 0, 0, None) < 0, field
     assert lib.qm_decoder_linear_rows(C.byref(linear), 4, 0, 0, None) < 0
+    # inputs split beforehand: what is refused takes no memory either
+    place = at + -at % 16
+    planes = dict(x=place, w=place, out32=place, ldx=128, ldo=128, n=128, k=128)
+
+    def split(rows, **change):
+        linear = decoder.DecoderLinear(**{**planes, **change})
+        return lib.qm_decoder_linear_planes_bytes(C.byref(linear), 1, rows), lib.qm_decoder_linear_rows_planes(C.byref(linear), 1, rows, place, 0, None)
+
+    assert split(5) == (5 * 128 * 6, -4)
+    assert split(1 << 21) == ((1 << 21) * 128 * 6, -4)
+    for rows, change in ((5, dict(n=100)), (5, dict(k=64)), (5, dict(ldo=130)), (5, dict(x=place + 8)), (5, dict(w=place + 2)), (5, dict(w_up=place + 8, out=place)),
+                         (5, dict(out32=place + 4)), (5, dict(k=(1 << 20) + 128, ldx=(1 << 20) + 128)), ((1 << 21) + 1, {})):
+        assert split(rows, **change) == (0, -2), change
     attention = dict(proj=at, frequency=at, q_rot=at, k_cache=at, v_cache=at, out=at,
                      part=decoder.AttentionPartials(at, at, 4, 16, 1, 128), ld_proj=256, ld_out=128, position=0, rows=0, heads=4, kv_heads=2, dim=16,
                      vdim=16, k_stride=16, v_stride=16, ring=100, chunk=50, rot_dims=8)
