@@ -383,6 +383,116 @@ def test_linears_of_fp32_rows_split_beforehand(decoder, dev, rows, n, k, pair):
             test_many_fp32_rows_of_small_inputs(planes, dev, rows, n, k, exponent)
 
 
+class InnerTypes:
+    """The decoder kernels' launchers as the engine calls them: structures of qm_decoder_ops.h, and functions by their C++ names."""
+
+    class Linears(C.Structure):
+        pass
+
+    class Planes(C.Structure):
+        _fields_ = [("at", C.c_void_p), ("elements", C.c_int64), ("split", C.c_bool)]
+
+    class Cut(C.Structure):
+        _fields_ = [("sums", C.c_void_p), ("room", C.c_int64), ("plane", C.c_int64), ("planes", C.c_int)]
+
+    class More(C.Structure):
+        _fields_ = [("sums", C.c_void_p), ("plane", C.c_int64), ("planes", C.c_int)]
+
+    def __init__(self, decoder):
+        if not hasattr(self.Linears, "_fields_"):
+            self.Linears._fields_ = [("group", decoder.DecoderLinear * 3), ("groups", C.c_int), ("rows", C.c_int), ("streaming", C.c_int)]
+        handle = C.CDLL(decoder.lib_path())
+        self.linears = handle._ZN2qm22launch_decoder_linearsERKNS_15DecLinearParamsEiP12ihipStream_tPNS_12ReductionCutERKNS_11PlaneMemoryE
+        self.linears.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]
+        self.norm = handle._ZN2qm20launch_residual_normERK16qm_residual_normiiP12ihipStream_tRKNS_10MoreOfTermEPt
+        self.norm.argtypes = [C.c_void_p, C.c_int, C.c_int, C.c_void_p, C.c_void_p, C.c_void_p]
+
+
+def upper_parts(x):
+    """The three bf16 parts of fp32 numbers, as floats: eight significant bits each, cut off."""
+    parts = []
+    for _ in range(3):
+        upper = (x.view(np.uint32) & 0xffff0000).view(np.float32)
+        parts.append(upper)
+        x = x - upper
+    return parts
+
+
+@pytest.mark.parametrize("width,ld,rows,pieces", [(1000, 1024, 5, 1), (1024, 1024, 3, 3), (1500, 1536, 2, 1), (4000, 4096, 2, 2), (9000, 9088, 2, 1)])
+def test_norms_leave_the_parts_of_their_rows(decoder, dev, width, ld, rows, pieces):
+    """A norm that leaves its rows split as well: the rows and the stream with the bits that it has alone, and the parts of those rows, bit for bit; the last
+    term in pieces, too."""
+    import torch
+    inner, gen = InnerTypes(decoder), torch.Generator(device=dev).manual_seed(width)
+    x, y, w = [torch.randn(n, ld, device=dev, generator=gen) for n in (rows, rows, 1)]
+    more = torch.randn(2, rows, ld, device=dev, generator=gen)
+    for t in (x, y, w, more):
+        t[..., width:] = 0.0
+    left = []
+    for split in (False, True):
+        x_out, h = torch.full((rows, ld), 7.0, device=dev), torch.full((rows, ld), 7.0, device=dev)
+        parts = torch.full((3 * rows * ld + 8,), 7.0, device=dev, dtype=torch.bfloat16)
+        op = decoder.ResidualNorm(x_in=x.data_ptr(), x_out=x_out.data_ptr(), norm_w=w.data_ptr(), h=h.data_ptr(), ld_h=ld, width=width, eps=1e-5, terms=1)
+        op.term[0] = decoder.ResidualTerm(y=y.data_ptr(), ld=ld, scale=0.5)
+        pending = inner.More(more.data_ptr() if pieces > 1 else None, rows * ld, pieces - 1)
+        assert inner.norm(C.addressof(op), rows, 1, torch.cuda.current_stream().cuda_stream, C.addressof(pending), parts.data_ptr() if split else None) == 0
+        left.append([get(t) for t in (x_out, h, parts)])
+    (x_alone, h_alone, untouched), (x_out, h, parts) = left
+    assert np.array_equal(x_out, x_alone) and np.array_equal(h, h_alone) and np.all(untouched == 7.0) and np.all(parts[3 * rows * ld:] == 7.0)
+    want = (x.double() + 0.5 * (y.double() + more[:pieces - 1].double().sum(0))).cpu().numpy()
+    assert np.abs(x_out - want).max() <= 1e-6 * np.abs(want).max()
+    for got, part in zip(parts[:3 * rows * ld].reshape(3, rows, ld), upper_parts(h)):
+        assert np.array_equal(got, part)
+
+
+@pytest.mark.parametrize("rows,sizes,pieces", [(300, [(1024, 1024), (1024, 3072)], 3), (400, [(1024, 1024), (1024, 1024), (1024, 3072)], 2),
+                                               (70, [(1024, 3072), (1024, 9216)], 3)])
+def test_pieces_of_a_fp32_reduction(decoder, dev, rows, sizes, pieces):
+    """The engine's launch with memory for split inputs and for pieces of the last reduction: so many pieces, whose sums come to the linear, and the bits
+    of the others as they are without a cut.  A linear whose input is there already, split, takes the parts and not the rows."""
+    import torch
+    inner, gen = InnerTypes(decoder), torch.Generator(device=dev).manual_seed(rows)
+    x = [torch.randn(rows, k, device=dev, generator=gen) for _, k in sizes]
+    w = [(torch.randn(n, k, device=dev, generator=gen) * k ** -0.5).bfloat16() for n, k in sizes]
+    stream = torch.cuda.current_stream().cuda_stream
+    planes = torch.full((3 * rows * sum(k for _, k in sizes),), float("nan"), device=dev, dtype=torch.bfloat16)
+
+    def launch(which, cut, split=False):
+        outs = [torch.full((rows, sizes[i][0]), 7.0, device=dev) for i in which]
+        p = inner.Linears(groups=len(which), rows=rows)
+        for g, (i, out) in enumerate(zip(which, outs)):
+            p.group[g] = decoder.DecoderLinear(x=x[i].data_ptr(), w=w[i].data_ptr(), out32=out.data_ptr(), ldx=sizes[i][1], ldo=sizes[i][0], n=sizes[i][0], k=sizes[i][1])
+        memory = inner.Planes(planes.data_ptr(), planes.numel(), split)
+        assert inner.linears(C.addressof(p), 1, stream, C.addressof(cut) if cut else None, C.addressof(memory)) == 0
+        torch.cuda.synchronize()
+        return outs
+
+    sizes, every = list(sizes), list(range(len(sizes)))
+    n = sizes[-1][0]
+    more = torch.full((2, rows, n), float("nan"), device=dev)
+    cut = inner.Cut(more.data_ptr(), more.numel(), 0, 0)
+    outs = launch(every, cut)
+    assert (cut.planes, cut.plane) == (pieces - 1, rows * n)
+    assert bool(more[pieces - 1:].isnan().all())
+    small = inner.Cut(more.data_ptr(), (pieces - 1) * rows * n - 1, 0, 0)          # no room for them: whole
+    uncut = launch(every, small)
+    assert small.planes == 0
+    for i in every:
+        want = x[i].double() @ w[i].double().T
+        got = outs[i] + more[:pieces - 1].sum(0) if i == every[-1] else outs[i]
+        # (pieces of 1024 to 3072 inputs, each 8e-8 to 9.6e-8 of its own sums, and their sum's roundings)
+        assert float((got.double() - want).norm() / want.norm()) <= 1.1e-7
+        assert float((uncut[i].double() - want).norm() / want.norm()) <= 1.5e-7
+        assert i == every[-1] or torch.equal(outs[i], uncut[i])
+    if rows == 400:
+        sizes[:] = [(4096, 1024)]
+        w[0] = (torch.randn(4096, 1024, device=dev, generator=gen) / 32).bfloat16()
+        before = launch([0], None)[0]
+        x[0].normal_(generator=gen)
+        assert torch.equal(launch([0], None, split=True)[0], before)
+        assert not torch.equal(launch([0], None)[0], before)
+
+
 def test_more_rows_than_a_grid_is_high_are_split_beforehand(decoder, dev):
     import torch
     rows, n, k = 65600, 16, 128
@@ -528,14 +638,6 @@ def test_chunk_attention_of_few_blocks_that_walk_far(decoder, dev, shape):
             close(case.run(decoder, dev, False, portions, ring=ring), want, False, tol16=3e-2)
 
 
-def rotated_alike(got, want, f32):
-    """The same products and sums, fused one way or the other: two roundings of the terms in fp32, one more of the result to bf16."""
-    got, want = get(got).astype(np.float64), get(want).astype(np.float64)
-    assert np.array_equal(np.isnan(got), np.isnan(want))
-    keep = ~np.isnan(want)
-    assert np.all(np.abs(got - want)[keep] <= (0 if f32 else 2.0 ** -7) * np.abs(want[keep]) + 2.0 ** -21 * np.abs(want[keep]).max())
-
-
 @pytest.mark.parametrize("f32", [True, False])
 @pytest.mark.parametrize("heads,kv,dim,vdim,rot", [(4, 2, 64, 64, 64), (16, 8, 128, 128, 128), (3, 1, 24, 8, 16), (2, 1, 256, 136, 0), (36, 9, 64, 40, 8), (1, 1, 8, 8, 8),
                                                    (64, 32, 64, 128, 64), (2, 2, 256, 256, 256)])
@@ -565,7 +667,7 @@ def test_chunk_attention_rotates_in_vectors(decoder, dev, heads, kv, dim, vdim, 
         assert decoder.lib().qm_chunk_attention_rows(C.byref(op), int(f32), torch.cuda.current_stream().cuda_stream) == 0
         left.append(caches)
     for got, want in zip(*left):
-        rotated_alike(got, want, f32)
+        assert np.array_equal(get(got), get(want), equal_nan=True)     # the same products and sums (a zero behind the turning channels keeps its sign in vectors)
 
 
 @pytest.mark.parametrize("scale", [0.0, -0.3, 3.0])
