@@ -5,7 +5,7 @@
 // at the end.  A wave's keys and values are its own: it brings them straight into its part of the LDS
 // (buffer_load ... lds, a tile of keys and a tile of values) and asks for the next keys when the products with these have read
 // them, for the next values likewise, so that nothing waits for another wave and either is under way during the other's
-// product; two blocks of four waves share a CU.  Blocks of one key/value head share a die's L2 (block numbers go round the dies).
+// product; two blocks of four waves share a CU (not of 256 channels, 129 KiB).  Blocks of one key/value head share a die's L2 (block numbers go round the dies).
 //
 // Scores are S^T = K Q^T (v_mfma_f32_32x32x16_bf16): a lane then holds sixteen keys of one query, the softmax is in the lane
 // but for one exchange with the other half of the wave, and the weights stand where the second product O^T = V^T P^T wants
@@ -14,8 +14,9 @@
 // are transposed on their way out of LDS (ds_read_b64_tr_b16).  Bound: the chain of a tile in its wave (two products, the
 // softmax between them); flops 2 (dim + vdim) per visible key and query (the second product's doubled weights not counted).
 // (us, by blocks of eight waves that staged 128 keys for 64 rows through registers, values transposed on the way in, two barriers a
-// tile / so: 8 heads of 192 and 128 channels, 777 rows 25.9 / 12.6; 16 query heads on 8 of 128, 1024 rows 28.7 / 14.7, of 64, 1000 rows
-// 12.3 / 8.6; 32 heads of 128, 1500 rows 79 / 47; 4 on 2 of 250, 200 rows 24.9 / 11.9.)
+// tile / so, one shape again and again behind its rotation: 8 heads of 192 and 128 channels, 777 rows 25.8 / 13.1; 16 query heads on 8 of 128, 1024
+// rows 28.0 / 15.4, of 64, 1000 rows 18.8 / 10.5; 32 heads of 128, 1500 rows 74 / 44; 4 on 2 of 250, 200 rows 32 / 14.  In a prompt of several layers the
+// first two take 14.0 and 16.6.)
 #include <algorithm>
 #include <utility>
 
@@ -277,7 +278,7 @@ __global__ __launch_bounds__(64 * PARTS, PARTS == 8 || CK <= 192 ? 2 : 1) void c
         float p[16], sum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            p[r] = fast_exp2(s[r] * factor_of_score - reference);       // (of rounded products, as the reference is: finite scores of any size come to zero at most)
+            p[r] = fast_exp2(s[r] * factor_of_score - reference);       // (of rounded products, as the reference is: finite scores of any size come to zero at most; fused, 0.3 us less of 15)
             sum += p[r];
         }
         l += sum;
@@ -376,8 +377,8 @@ static int32_t flash_of(const ChunkAttentionParams& prm, unsigned blocks, hipStr
     return launch_status();
 }
 // Eight waves where the grid leaves CUs without a second block and a block walks long: half the steps, for a longer combination (us, four waves /
-// eight, 8 heads of 192 and 128: 100 rows behind 0, 500, 900, 1500 and 4000 keys 6.3 / 8.0, 10.2 / 10.6, 12.9 / 13.0, 17.4 / 15.9 and 34.8 / 28.4, 300 rows behind 1000
-// 15.9 / 14.9; 16 query heads on 8 of 128, 100 rows behind 900 11.4 / 11.7, 500 behind 1500 21.0 / 20.0, 850 rows, 432 blocks, 12.9 / 18.0).
+// eight, 8 heads of 192 and 128: 100 rows behind 0, 500, 900, 1500 and 4000 keys 6.6 / 8.4, 10.6 / 11.1, 13.4 / 13.6, 18.4 / 16.9 and 35.7 / 28.6, 300 rows behind 1000
+// 16.7 / 15.5; 16 query heads on 8 of 128, 100 rows behind 900 11.9 / 12.0, 500 behind 1500 21.2 / 20.2, 850 rows, 432 blocks, 13.2 / 18.3).
 constexpr int kFlashLongWalk = 1200, kFlashCus = 256;
 template <int CK, int CV>
 static int32_t flash_as(const ChunkAttentionParams& prm, hipStream_t stream) {

@@ -210,7 +210,8 @@ static bool by_matrix(int rows, int f32) { return !f32 && rows >= kExpertMatrixR
 // Row tiles of 128 where an expert's rows come to two tiles of 64 but for few, and one of 128, and the tiles of 64 are about as many as CUs or more: an
 // expert's weights are read once, not on two dies.  (us, pair and down of bf16, 64 / 128: 32 experts of 1024 x 512 with 97 rows each 27.9 + 17.0 / 21.6 +
 // 16.0, with 64 22.1 + 15.6 / 21.7 + 15.8, with 128 36.0 + 21.6 / 25.6 + 22.4; 24 of 2048 x 1024 with 96 62.6 + 33.9 / 55.2 + 32.8; 12 of 1024 x 512 12.6 +
-// 6.4 / 15.0 + 7.5.  Over fourteen numbers of experts and three of rows within these lines 0.97 to 1.34 times, 1.12 in the mean.)
+// 6.4 / 15.0 + 7.5.  Over fourteen numbers of experts and three of rows within these lines 0.97 to 1.34 times, 1.12 in the mean.  The upper line is where an expert
+// of somewhat more rows than the mean fills its one tile; between it and kExpertLongTile low tiles are kept unmeasured but for the 128 rows above, which gain as well.)
 static bool tall_tiles(int64_t assignments, int experts, int ff_p) {
     const bool two = assignments >= static_cast<int64_t>(kExpertTwoTiles[0]) * experts && assignments <= static_cast<int64_t>(kExpertTwoTiles[1]) * experts;
     return assignments / experts >= kExpertLongTile || (two && static_cast<int64_t>(experts) * (ff_p / 128) >= kExpertLongGrid);
