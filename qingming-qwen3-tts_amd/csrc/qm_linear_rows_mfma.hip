@@ -690,6 +690,7 @@ __global__ __launch_bounds__(256) void linear_rows_parts_norm_kernel(LinearRowsP
 
 template <bool DUAL, int BM, int BN, int KSTEP, int WAVES>
 int32_t launch_rows_mfma_as(const LinearRowsParams& given, hipStream_t stream) {
+    if (!rows_are_whole_tiles(given, BN, KSTEP)) return QM_ERR_GEOMETRY;
     LinearRowsParams prm = given;
     if (BN == 64)                                                 // (given in tiles of 128 columns)
         for (int& first : prm.group_first_tile) first *= 2;

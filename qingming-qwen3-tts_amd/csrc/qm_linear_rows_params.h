@@ -66,8 +66,27 @@ inline int rows_grid_columns(int column_tiles, int row_tiles, int pieces) {
     return column_tiles > 40 && row_tiles > 1 && 3 * busiest <= 4 * even ? static_cast<int>(rounded) : column_tiles;
 }
 
+// Whether tiles of `tile_columns` columns and `step` k cover every linear exactly.  The kernel bounds token rows only: a tile that hangs over a linear's
+// last column would read weight rows past the matrix (half a tile of 2048 inputs: 256 KiB, past the allocation as well) and write the
+// columns it has too many over the next row, past the output in the last; a piece that is no whole number of steps would leave inputs out; planes of
+// pieces are laid out for one linear, and the norm behind them takes two planes at a time of rows that 256 threads hold.
+inline bool rows_are_whole_tiles(const LinearRowsParams& prm, int tile_columns, int step) {
+    if (prm.rows <= 0 || prm.groups < 1 || prm.groups > kRowsGroups || prm.reduction_parts < 1) return false;
+    int64_t before = 0;
+    for (int g = 0; g < prm.groups; ++g) {
+        const int columns = g == 0 ? prm.columns : prm.group_columns[g - 1];
+        const int reduction = g == 0 || !prm.group_reduction[g - 1] ? prm.reduction : prm.group_reduction[g - 1];
+        if (columns <= 0 || columns % 128 || columns % tile_columns) return false;
+        if (reduction <= 0 || reduction % 128 || reduction % (static_cast<int64_t>(step) * prm.reduction_parts)) return false;
+        if (g > 0 && prm.group_first_tile[g - 1] != before / 128) return false;
+        before += columns;
+    }
+    if (prm.reduction_parts == 1) return true;
+    return prm.groups == 1 && prm.partials && (!prm.norm_weight || (prm.reduction_parts % 2 == 0 && (prm.columns == 1024 || prm.columns == 2048)));
+}
+
 // The row linears on the matrix cores (qm_linear_rows_mfma.hip).  `dual`: weight[0] / weight[1] are the gate and up
-// matrices and the epilogue is SwiGLU.  Needs columns % 128 == 0 and reduction % 128 == 0 (checked by the caller).
+// matrices and the epilogue is SwiGLU.  Columns and reductions that are not multiples of 128: QM_ERR_GEOMETRY, nothing is launched.
 int32_t launch_rows_mfma(const LinearRowsParams& prm, bool dual, hipStream_t stream);
 
 // Into how many pieces launch_rows_mfma cuts the reduction when it is given a workspace for the partial sums (a pure

@@ -11,14 +11,15 @@ CSRC = os.path.join(ROOT, "qingming-qwen3-tts_amd", "csrc")
 LIB = os.path.join(ROOT, "qingming-qwen3-tts_amd", "lib")
 
 
-def run(tmp_path, source, library=None):
-    """The output lines of a program of one `main`."""
+def run(tmp_path, source, *libraries):
+    """The output lines of a program of one `main`, which sees no GPU."""
     path = tmp_path / "rule.cpp"
     path.write_text(source)
-    link = ["-L" + LIB, "-l" + library, "-Wl,-rpath," + LIB] if library else []
+    link = ["-L" + LIB, "-L/opt/rocm/lib", *("-l" + name for name in libraries), "-Wl,-rpath," + LIB + ":/opt/rocm/lib"] if libraries else []
     subprocess.run(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I" + CSRC, "-I" + os.path.join(ROOT, "include"), "-o",
                     str(tmp_path / "rule"), str(path), *link], check=True)
-    return subprocess.run([str(tmp_path / "rule")], check=True, capture_output=True, text=True).stdout.splitlines()
+    hidden = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1")
+    return subprocess.run([str(tmp_path / "rule")], check=True, capture_output=True, text=True, env=hidden).stdout.splitlines()
 
 
 def test_a_rounded_grid_keeps_no_die_much_longer_than_an_even_deal(tmp_path):
@@ -49,6 +50,100 @@ int main() {
             rounded += 1
     assert rounded > 5000
     assert "81 8 1 88" in lines and "81 9 1 88" in lines and "42 6 1 42" in lines and "42 3 2 42" in lines and "42 12 1 42" in lines
+
+
+ROWS_OF = """
+#include <cstdio>
+#include <vector>
+#include "qm_attn.h"
+#include "qm_linear_rows_params.h"
+static float planes[1];
+static uint16_t weight[1];
+static qm::LinearRowsParams of(int rows, std::vector<std::pair<int, int>> linears, int parts = 1, bool norm = false) {
+    qm::LinearRowsParams p = {};
+    p.rows = rows;
+    p.groups = static_cast<int>(linears.size());
+    p.reduction_parts = parts;
+    if (parts > 1) p.partials = planes;
+    if (norm) p.norm_weight = weight;
+    p.columns = linears[0].first;
+    p.reduction = linears[0].second;
+    int columns = p.columns;
+    for (int g = 1; g < p.groups; ++g) {
+        p.group_first_tile[g - 1] = columns / 128;
+        p.group_columns[g - 1] = linears[g].first;
+        p.group_reduction[g - 1] = linears[g].second;
+        columns += linears[g].first;
+    }
+    return p;
+}
+int main() {
+"""
+
+
+# rows; (columns, reduction) each; whether a gate/up pair; pieces; whether a norm adds them
+HANGING = [(1024, [(10176, 2048)], 0, 1, 0), (1024, [(10176, 2048)], 1, 1, 0), (16, [(64, 128)], 0, 1, 0), (777, [(2048, 1088)], 0, 1, 0),
+           (1024, [(6144, 2080)], 1, 1, 0), (1000, [(2048, 2048), (1088, 2048)], 0, 1, 0), (1000, [(2048, 2048), (1024, 2048), (1024, 2112)], 0, 1, 0),
+           (300, [(2048, 4160)], 0, 1, 0), (64, [(2048, 6144)], 0, 5, 0), (64, [(2048, 4224)], 0, 4, 0), (64, [(2048, 6144)], 1, 7, 0),
+           (64, [(2048, 6144), (2048, 6144)], 0, 4, 0), (64, [(2048, 6144)], 0, 3, 1), (64, [(4096, 6144)], 0, 2, 1)]
+
+
+@pytest.mark.parametrize("library", ["qm_attn", "qm_decoder"])
+def test_no_tile_of_the_row_linears_hangs_over_a_matrix(tmp_path, library):
+    """The launch itself refuses what its tiles and steps do not cover exactly, whoever calls it."""
+    calls = "".join("""
+    std::printf("%%d\\n", qm::launch_rows_mfma(of(%d, {%s}, %d, %d), %d, nullptr));""" % (rows, ", ".join("{%d, %d}" % l for l in linears), parts, norm, dual)
+                    for rows, linears, dual, parts, norm in HANGING)
+    calls += """
+    qm::LinearRowsParams shifted = of(1024, {{2048, 2048}, {2048, 2048}});
+    shifted.group_first_tile[0] = 15;                        // a linear's tiles begin inside the one before
+    std::printf("%d\\n", qm::launch_rows_mfma(shifted, false, nullptr));
+    qm::LinearRowsParams nowhere = of(64, {{2048, 6144}}, 4);
+    nowhere.partials = nullptr;
+    std::printf("%d\\n", qm::launch_rows_mfma(nowhere, false, nullptr));
+    std::printf("%d\\n", QM_ERR_GEOMETRY);
+}"""
+    *got, geometry = map(int, run(tmp_path, ROWS_OF + calls, library))
+    assert got == [geometry] * (len(HANGING) + 2)
+
+
+def test_the_row_linears_take_what_their_entry_points_let_through(tmp_path):
+    """Whole tiles and steps, for every choice of tile and for the pieces that are chosen."""
+    lines = run(tmp_path, ROWS_OF + """
+    for (int rows : {16, 100, 520, 777, 1024, 4096})
+        for (int columns = 128; columns <= 12288; columns += columns < 2048 ? 128 : 896)
+            for (int reduction = 128; reduction <= 16384; reduction += reduction < 1024 ? 128 : 896) {
+                bool wide = false;
+                const int parts = qm::rows_mfma_reduction_parts(rows, columns, reduction, false), behind = qm::rows_mfma_norm_parts(rows, columns, reduction, &wide);
+                bool fits = true;
+                for (int tile : {64, 128})
+                    fits = fits && qm::rows_are_whole_tiles(of(rows, {{columns, reduction}, {columns, 128}, {128, reduction}}), tile, 128) &&
+                           qm::rows_are_whole_tiles(of(rows, {{columns, reduction}}, parts), tile, 64) &&
+                           qm::rows_are_whole_tiles(of(rows, {{columns, reduction}}, behind, true), tile, 64);
+                std::printf("%d %d %d\\n", fits && qm::rows_are_whole_tiles(of(rows, {{columns, reduction}}), 192, 64) == (columns % 192 == 0), parts, behind);
+            }
+}""", "qm_attn")
+    got = [tuple(map(int, line.split())) for line in lines]
+    assert all(fits for fits, _, _ in got) and len(got) > 3000
+    assert {1, 2, 4, 8} <= {parts for _, parts, _ in got} and any(behind > parts for _, parts, behind in got)
+
+
+def test_the_row_linears_take_a_decoders_launches(tmp_path):
+    """Linears of several inputs and widths, pairs and the pieces of a reduction get as far as the device, which is not there."""
+    shapes = [(list(linears), rows) for linears, rows, _ in CUTS] + [([(11264, 2048)], 1024), ([(128, 128), (3072, 640), (1024, 6144)], 16), ([(128, 128), (-384, 256)], 100)]
+    source = OF_SIZES.replace("int main() {", """int main() {
+    int devices = 0;
+    if (hipGetDeviceCount(&devices) == hipSuccess && devices > 0) return 1;              // (nothing below may be launched: the addresses are made up)
+""")
+    for linears, rows in shapes:
+        source += """
+    {
+        qm::ReductionCut cut = {reinterpret_cast<float*>(somewhere), int64_t{1} << 40, 0, 0};
+        const int rc = qm::launch_decoder_linears(of(%s, %d), 0, nullptr, &cut);
+        std::printf("%%d %%d\\n", rc <= QM_ERR_HIP_BASE, cut.planes + 1);
+    }""" % (sizes(linears), rows)
+    got = [tuple(map(int, line.split())) for line in run(tmp_path, source + "}", "qm_decoder", "amdhip64")]
+    assert got[:len(CUTS)] == [(1, pieces) for _, _, pieces in CUTS] and got[len(CUTS):] == [(1, 1)] * 3
 
 
 # output linears as (columns, reduction) each, the last the one that may be cut; rows; its pieces (the first four are the layers of
