@@ -13,11 +13,13 @@
 // The 16 row-streams of a block are merged through LDS; blocks write fp32 partials
 // (acc, max, sum) to the caller's workspace and a small second kernel merges the splits.
 // Blocks are dispatched by the hardware as earlier ones retire, which balances ragged lengths;
-// letting the last block to arrive at a per-(stream, head) counter merge in place needs one
-// device-scope fence per block (write-back and invalidate of the XCD's L2): measured, with
-// bit-identical results, at 17 us instead of 6.6 us for one stream of 512 tokens and 17x slower
-// on the ragged batch (a persistent variant pulling work items from a counter: 8x slower), so the
-// merge stays a second launch.
+// letting the last block to arrive at a per-(stream, head) counter merge in place was built twice,
+// with bit-identical results: behind one device-scope fence per block (write-back and invalidate
+// of the XCD's L2) 17 us instead of 6.6 us for one stream of 512 tokens and 17x slower on the
+// ragged batch; with records written by acknowledged agent-scope stores and a ticket 106 against
+// 102 us on the batch, 10.4 against 9.7 us for the fused step at 2048 tokens, 14.8 against 15.0 at
+// 8192 (a persistent variant pulling work items from a counter: 8x slower).  The merge stays a
+// second launch.
 //
 // Rounding: scores are rounded to bf16 before and after scaling as the reference does
 // (R17:16102-16116); probabilities stay fp32 (the reference's bf16(P) after a full-row

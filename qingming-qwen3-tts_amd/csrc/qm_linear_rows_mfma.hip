@@ -8,7 +8,10 @@
 //
 // A block owns a tile of BM token rows x BN output columns: 128 x 128 (eight waves 2 x 4, each 64 rows x 32 columns, two to a
 // SIMD so that one multiplies while the other waits to issue: three linears of 2048, 2048 and 6144 inputs over 1024 rows
-// 71.3 -> 68.6 us against four waves of 64 x 64; the other tiles gain nothing from it and keep four); 64 x 128 for calls whose
+// 71.3 -> 68.6 us against four waves of 64 x 64 when a tile's outputs still left from the products' layout.  Since they leave as whole
+// rows the two are within 4 % of each other: on seven grids four waves were ahead in six with weights in the caches, 56.1 against 57.9 us at 11264 columns
+// of 2048, and in two (a third a tie) with weights from memory, 58.9 us in eight against 59.8 in four for two outputs and a cut down projection; the other tiles gained nothing
+// from eight and keep four); 64 x 128 for calls whose
 // grid of 128-row tiles would leave CUs without a block; 64 x 64 with up to eight stages where most CUs would still be empty
 // and a block's time is its chain of round trips to memory (waves 2 x 2); 128 x 192 for a gate/up pair whose 128-column tiles
 // come to between one and two rounds of the CUs and whose 192-column tiles fit in one (1024 tokens x 6144 channels: 256
@@ -40,7 +43,7 @@
 namespace qm {
 
 constexpr int kGmTile = 128;                 // output columns per block (192 for a gate/up pair that it divides), token rows 128 or 64
-constexpr int kGmStep = 64;                  // k per step (32 with the 192-column tile)
+constexpr int kGmStep = 64;                  // k per step (128 for 64-row tiles with a long reduction)
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
